@@ -12,17 +12,31 @@
 // counts do not depend on the order of the vertices: they are compared bit for bit
 // with the oracle.
 //
-// Per epoch: the active bitmap is compacted into a queue; one lane per vertex of at
-// most KC_SMALL neighbours counts them in a byte histogram of its own in LDS; longer
-// adjacencies whose answer cannot exceed KC_HIST (min(length, estimate) <= KC_HIST) go to
-// a second queue handled one wave per vertex with a KC_HIST-bin LDS histogram, and the
-// others (adjacencies above KC_HUGE, or estimates above KC_HIST) to a third, one
-// 1024-thread block per vertex with a KC_HHIST-bin histogram (when the answer reaches
-// its last bin, a binary search over [KC_HHIST, est] with block-wide counts finishes
-// the job); adjacencies above KC_GIANT are cut into chunks whose block histograms add
-// up in global memory, so no block walks a giant alone.
-// Modified vertices set their neighbours' bits in the next bitmap (test, then atomic
-// OR, as the reference's get_bit / set_bit).  Then estimate = coreness for the queue.
+// On a symmetrized graph the adjacency is its own reverse, and most active vertices keep
+// their value, so the device carries cnt(v) = the neighbours u with estimate[u] >=
+// estimate[v] along with the estimates: v is modified in an epoch exactly when cnt(v) <
+// estimate[v].  A vertex that drops from `old` to `now` takes one from cnt(u) of every
+// unmodified neighbour u with now < estimate[u] <= old and re-counts its own, so an epoch
+// reads the adjacencies of the modified vertices (twice) instead of those of all active
+// ones; the active set is still marked and counted, for the per-epoch log.  In epoch 0
+// everything is active; a vertex that keeps its adjacency length has cnt(v) equal to it.
+// RMAT scale 22 symmetrized, degree-relabeled, 39 epochs, whole call: 51 ms re-counting every
+// active vertex, 20 ms with the counts.  Bound by the random 4-byte reads of the estimates in
+// the first ten epochs, when most vertices are modified (0.5 ms per scan of the 2^27 entries).
+// Other adjacencies (in-edges or out-edges of a directed graph) have no counts: every
+// active vertex is re-counted.
+//
+// Per epoch: the candidate bitmap (vertices with cnt < estimate; the active set without
+// counts) is cut into queues by adjacency length, then
+//   h-index:  one lane per vertex of at most KC_SMALL neighbours (byte histogram of its own
+//             in LDS), one wave up to KC_HUGE when the answer cannot exceed KC_HIST (KC_HIST
+//             + 1 LDS bins per wave), one 1024-thread block up to KC_GIANT, and chunks over
+//             all blocks beyond (their histograms add up in global memory); answers above
+//             KC_HHIST take a histogram of value ranges first and one of the range's values
+//             next, each halving the candidates' bits by 14;
+//   spread:   modified vertices activate their neighbours and update the counts;
+//   commit:   estimate = coreness, next epoch's candidates and the log's counters, which
+//             reach the host in one mail.
 #include <algorithm>
 #include <vector>
 
@@ -37,25 +51,39 @@ static constexpr uint32_t KC_PER = 17;      // bins per lane in its scan (64 * 1
 static constexpr int KC_THREADS = 256;
 static constexpr uint32_t KC_HUGE = 4096;    // longer adjacencies take one block each
 static constexpr int KC_HTHREADS = 1024;
-static constexpr uint32_t KC_HHIST = 16384;  // histogram bins 0..KC_HHIST of the block pass
+static constexpr uint32_t KC_HBITS = 14;
+static constexpr uint32_t KC_HHIST = 1u << KC_HBITS;  // histogram bins 0..KC_HHIST of the block pass
 static constexpr uint32_t KC_HPER = 17;      // bins per thread in its scan (1024 * 17 > KC_HHIST)
 static constexpr uint64_t KC_GIANT = 65536;  // longer adjacencies are cut into chunks over many blocks
 static constexpr uint64_t KC_GCHUNK = 16384;
+static constexpr int KC_U = 4;               // neighbours a lane of the wave and block passes has in flight
+static_assert(64 * (KC_SMALL + 1) <= 64 * KC_PER * 4, "a wave's byte histograms fit in the space of its bins");
 
 struct kc_counters {
-  unsigned long long queued;    // active vertices this epoch
-  unsigned long long nbig;      // of them, with KC_SMALL < neighbours <= KC_HUGE and min(neighbours, estimate) <= KC_HIST
-  unsigned long long nhuge;     // of them, the other ones above KC_SMALL neighbours
-  unsigned long long modified;  // vertices whose coreness dropped
+  unsigned long long nsmall, nbig, nhuge;  // queued candidates by adjacency length
+  unsigned long long modified;             // vertices whose coreness dropped
+  unsigned long long next_active;          // size of the next active set
+  unsigned long long next_cand;            // candidates of the next epoch
+  unsigned long long giant_top;            // largest estimate among the giants re-counted in this epoch
+};
+static constexpr uint32_t KC_CW = sizeof(kc_counters) / 8;
+
+// where a giant's h-index stands between two histogram rounds: it lies in the bins base +
+// [j << shift, (j + 1) << shift), j <= nb, of the round to come, with `above` neighbours over
+// them; shift -1: done
+struct kc_giant {
+  uint32_t base, above, nb;
+  int32_t shift;
 };
 
 __global__ void k_kc_init(const uint64_t* __restrict__ ptr, uint32_t V, uint32_t* __restrict__ core,
-                          uint32_t* __restrict__ est) {
+                          uint32_t* __restrict__ est, uint32_t* __restrict__ cnt) {
   for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x) {
     const uint64_t len = ptr[v + 1] - ptr[v];
     const uint32_t c = len ? (uint32_t)std::min<uint64_t>(len, 0xFFFFFFFEull) : KC_UNSET;
     core[v] = c;
     est[v] = c;
+    if (cnt) cnt[v] = c;
   }
 }
 
@@ -74,90 +102,123 @@ __global__ void k_kc_zero(uint64_t* __restrict__ w, uint64_t n) {
     w[i] = 0ull;
 }
 
-__global__ void k_kc_reset(kc_counters* c) {
-  c->queued = 0;
-  c->nbig = 0;
-  c->nhuge = 0;
-  c->modified = 0;
-}
-
-// the reference's `if (!get_bit(u)) set_bit(u)` on the next active bitmap
-__device__ __forceinline__ void kc_activate(uint64_t* next_bits, uint32_t u) {
+// the reference's `if (!get_bit(u)) set_bit(u)`
+__device__ __forceinline__ void kc_set_bit(uint64_t* bits, uint32_t u) {
   const uint64_t m = 1ull << (u & 63);
-  if (!(next_bits[u >> 6] & m)) atomicOr((unsigned long long*)&next_bits[u >> 6], (unsigned long long)m);
+  if (!(bits[u >> 6] & m)) atomicOr((unsigned long long*)&bits[u >> 6], (unsigned long long)m);
 }
 
-// One lane per queued vertex of at most KC_SMALL neighbours (byte counts suffice).
-// Grid-stride over the queue; longer adjacencies are marked in the big / huge bitmaps
-// (one atomic OR per marked vertex, on its own word) and queued by compaction after the
-// pass, and the modified count is summed once per wave: no per-wave atomics on a shared
-// counter.
-__global__ __launch_bounds__(KC_THREADS) void k_kc_small(
-    const uint32_t* __restrict__ queue, uint64_t n, const uint64_t* __restrict__ ptr,
-    const uint32_t* __restrict__ idx, const uint32_t* __restrict__ est, uint32_t* __restrict__ core,
-    uint64_t* __restrict__ next_bits, uint64_t* __restrict__ big_bits, uint64_t* __restrict__ huge_bits,
-    kc_counters* __restrict__ cnt) {
-  __shared__ uint8_t hist[KC_THREADS][KC_SMALL + 1];
-  uint8_t* h = hist[threadIdx.x];
-  unsigned long long nmod = 0;
-  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
-    const uint32_t v = queue[i];
-    const uint64_t b = ptr[v], e = ptr[v + 1];
-    const uint64_t len = e - b;
-    if (len == 0) {
-      core[v] = 0;  // kcore.hpp:214-218
-    } else if (len > KC_SMALL) {
-      // the block pass also takes the vertices whose answer may exceed the wave pass's
-      // KC_HIST bins (which would need its binary search over the adjacency)
-      const bool block = len > KC_HUGE || std::min<uint64_t>(len, est[v]) > KC_HIST;
-      atomicOr((unsigned long long*)&(block ? huge_bits : big_bits)[v >> 6], 1ull << (v & 63));
-    } else {
-      const uint32_t cap = std::min<uint32_t>((uint32_t)len, est[v]);
-      for (uint32_t j = 0; j <= cap; ++j) h[j] = 0;
-      for (uint64_t k = b; k < e; ++k) {
-        const uint32_t eu = est[idx[k]];
-        ++h[eu < cap ? eu : cap];
+// ---- queues ------------------------------------------------------------------------------
+// Candidate bitmap -> queues by adjacency length, the bitmap cleared for the next epoch's
+// marks.  One wave per word, lane = bit, so the offsets are read coalesced; a block takes 64
+// words at a time and reserves its slots of the three queues with one atomic each.  Giants
+// go to no queue: their bits are kept in `act` (nullptr without giants).
+static constexpr int KC_CW_WORDS = 4;  // words per wave and step
+__global__ __launch_bounds__(1024) void k_kc_classify(uint64_t* __restrict__ cand, uint64_t* __restrict__ act,
+                                                      uint64_t nwords, uint32_t V, const uint64_t* __restrict__ ptr,
+                                                      const uint32_t* __restrict__ est, uint32_t* __restrict__ qsmall,
+                                                      uint32_t* __restrict__ qbig, uint32_t* __restrict__ qhuge_end,
+                                                      kc_counters* __restrict__ cnt) {
+  __shared__ uint32_t s_cnt[3][16];
+  __shared__ unsigned long long s_base[3];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint64_t below = (1ull << lane) - 1ull;
+  constexpr uint64_t STEP = 16 * KC_CW_WORDS;
+  for (uint64_t w0 = blockIdx.x * STEP; w0 < nwords; w0 += (uint64_t)gridDim.x * STEP) {
+    uint64_t m[3][KC_CW_WORDS];
+    uint32_t n[3] = {0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < KC_CW_WORDS; ++j) {
+      const uint64_t word = w0 + (uint64_t)wave * KC_CW_WORDS + j;  // wave-uniform
+      uint64_t bits = 0;
+      if (word < nwords) {
+        bits = cand[word];
+        if (act && lane == 0) act[word] = bits;
+        if (bits && lane == 0) cand[word] = 0ull;
       }
-      uint32_t sum = 0, best = 0;
-      for (uint32_t j = cap; j > 0; --j) {
-        sum += h[j];
-        if (sum >= j) {
-          best = j;
-          break;
-        }
+      int cls = -1;
+      const uint64_t v = word * 64 + lane;
+      if (bits && v < V && ((bits >> lane) & 1ull)) {
+        const uint64_t len = ptr[v + 1] - ptr[v];
+        if (len <= KC_SMALL) cls = 0;
+        else if (len > KC_GIANT) cls = -1;
+        // the block pass also takes the vertices whose answer may exceed the wave pass's bins
+        else if (len > KC_HUGE || std::min<uint64_t>(len, est[v]) > KC_HIST) cls = 2;
+        else cls = 1;
       }
-      if (best && best < core[v]) {
-        core[v] = best;
-        ++nmod;
-        for (uint64_t k = b; k < e; ++k) kc_activate(next_bits, idx[k]);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        m[c][j] = __ballot(cls == c);
+        n[c] += (uint32_t)__popcll(m[c][j]);
       }
     }
+    if (!__syncthreads_or((int)(n[0] | n[1] | n[2]))) continue;
+    if (lane == 0)
+      for (int c = 0; c < 3; ++c) s_cnt[c][wave] = n[c];
+    __syncthreads();
+    if (threadIdx.x < 3) {
+      uint32_t t = 0;
+      for (int i = 0; i < 16; ++i) t += s_cnt[threadIdx.x][i];
+      s_base[threadIdx.x] = t ? atomicAdd(threadIdx.x == 0 ? &cnt->nsmall : threadIdx.x == 1 ? &cnt->nbig : &cnt->nhuge,
+                                          (unsigned long long)t)
+                              : 0ull;
+    }
+    __syncthreads();
+    if (n[0] | n[1] | n[2]) {
+      uint64_t at[3];
+      for (int c = 0; c < 3; ++c) {
+        at[c] = s_base[c];
+        for (int i = 0; i < wave; ++i) at[c] += s_cnt[c][i];
+      }
+#pragma unroll
+      for (int j = 0; j < KC_CW_WORDS; ++j) {
+        const uint32_t v = (uint32_t)((w0 + (uint64_t)wave * KC_CW_WORDS + j) * 64 + lane);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          if ((m[c][j] >> lane) & 1ull) {
+            const uint64_t p = at[c] + (uint64_t)__popcll(m[c][j] & below);
+            if (c == 0) qsmall[p] = v;
+            else if (c == 1) qbig[p] = v;
+            else *(qhuge_end - p) = v;  // the block pass's queue grows down from the end of qbig's array
+          }
+          at[c] += (uint64_t)__popcll(m[c][j]);
+        }
+      }
+    }
+    __syncthreads();  // s_cnt and s_base are rewritten by the next step
   }
-  block_add2(nmod, 0, &cnt->modified, &cnt->modified);
 }
 
-// One wave per queued vertex with more than KC_SMALL neighbours.
-__global__ __launch_bounds__(KC_THREADS) void k_kc_big(
-    const uint32_t* __restrict__ big, const kc_counters* __restrict__ cnt_in, const uint64_t* __restrict__ ptr,
-    const uint32_t* __restrict__ idx, const uint32_t* __restrict__ est, uint32_t* __restrict__ core,
-    uint64_t* __restrict__ next_bits, kc_counters* __restrict__ cnt) {
+// ---- h-index: lanes and waves -------------------------------------------------------------
+// The wave pass's vertices first (the longer ones), then one lane per vertex of the small
+// queue.  A wave's LDS share serves both: KC_PER words per lane as one histogram of the
+// wave, or KC_SMALL + 1 bytes per lane.
+__global__ __launch_bounds__(KC_THREADS) void k_kc_hindex(
+    const uint32_t* __restrict__ qsmall, const uint32_t* __restrict__ qbig, const kc_counters* __restrict__ cnt_in,
+    const uint64_t* __restrict__ ptr, const uint32_t* __restrict__ idx, const uint32_t* __restrict__ est,
+    uint32_t* __restrict__ core) {
   __shared__ uint32_t hist_all[KC_THREADS / 64][64 * KC_PER];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   uint32_t* hist = hist_all[wave];
-  const uint64_t nbig = cnt_in->nbig;
+  const uint64_t nbig = cnt_in->nbig, nsmall = cnt_in->nsmall;
   const uint64_t wave_id = grid_wave_id(), nwaves = grid_waves();
-  uint32_t nmod = 0;
   for (uint64_t q = wave_id; q < nbig; q += nwaves) {
-    const uint32_t v = big[q];
+    const uint32_t v = qbig[q];
     const uint64_t b = ptr[v], e = ptr[v + 1];
-    const uint32_t cap = (uint32_t)std::min<uint64_t>(e - b, (uint64_t)est[v]);
-    const uint32_t top = std::min(cap, KC_HIST);
+    const uint32_t top = (uint32_t)std::min<uint64_t>(e - b, (uint64_t)est[v]);  // at most KC_HIST
     for (uint32_t j = lane; j <= top; j += 64) hist[j] = 0;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    for (uint64_t k = b + lane; k < e; k += 64) {
-      const uint32_t eu = est[idx[k]];
-      atomicAdd(&hist[eu < top ? eu : top], 1u);
+    for (uint64_t k0 = b; k0 < e; k0 += 64 * KC_U) {
+      uint32_t eu[KC_U];
+#pragma unroll
+      for (int i = 0; i < KC_U; ++i) {
+        const uint64_t k = k0 + (uint64_t)i * 64 + lane;
+        eu[i] = k < e ? est[idx[k]] : 0u;
+      }
+#pragma unroll
+      for (int i = 0; i < KC_U; ++i)
+        if (k0 + (uint64_t)i * 64 + lane < e) atomicAdd(&hist[eu[i] < top ? eu[i] : top], 1u);
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -180,133 +241,148 @@ __global__ __launch_bounds__(KC_THREADS) void k_kc_big(
       }
     }
     for (int off = 32; off > 0; off >>= 1) best = std::max(best, (uint32_t)__shfl_xor(best, off, 64));
-    if (best && best < core[v]) {
-      if (lane == 0) core[v] = best;
-      for (uint64_t k = b + lane; k < e; k += 64) kc_activate(next_bits, idx[k]);
-      ++nmod;
-    }
+    if (lane == 0 && best && best < core[v]) core[v] = best;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
   }
-  if (lane == 0 && nmod) atomicAdd(&cnt->modified, (unsigned long long)nmod);
+  uint8_t* h = reinterpret_cast<uint8_t*>(hist) + lane * (KC_SMALL + 1);
+  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < nsmall;
+       i += (uint64_t)gridDim.x * blockDim.x) {
+    const uint32_t v = qsmall[i];
+    const uint64_t b = ptr[v], e = ptr[v + 1];
+    if (b == e) {
+      core[v] = 0;  // kcore.hpp:214-218
+      continue;
+    }
+    const uint32_t cap = std::min<uint32_t>((uint32_t)(e - b), est[v]);
+    for (uint32_t j = 0; j <= cap; ++j) h[j] = 0;
+    for (uint64_t k = b; k < e; ++k) {
+      const uint32_t eu = est[idx[k]];
+      ++h[eu < cap ? eu : cap];
+    }
+    uint32_t sum = 0, best = 0;
+    for (uint32_t j = cap; j > 0; --j) {
+      sum += h[j];
+      if (sum >= j) {
+        best = j;
+        break;
+      }
+    }
+    if (best && best < core[v]) core[v] = best;
+  }
 }
 
-// Block-wide h-index from a histogram in LDS (hist[j] = neighbours whose estimate, capped
-// at top, is j, for j <= top = min(cap, KC_HHIST)): the largest j in [1, top] whose suffix
-// sum reaches j; when that is KC_HHIST and cap is larger, a binary search on
-// [KC_HHIST, cap] with block-wide counts over the adjacency [b, e) finishes it.  0 when
-// no j qualifies.  Every thread of the block calls it and gets the answer.
-__device__ uint32_t kc_block_hindex(const uint32_t* hist, uint32_t top, uint32_t cap, uint64_t b, uint64_t e,
-                                    const uint32_t* __restrict__ idx, const uint32_t* __restrict__ est) {
+// ---- h-index: blocks -------------------------------------------------------------------------
+// shift of the first round over values up to cap: cap >> shift fits the bins
+__device__ __forceinline__ int kc_first_shift(uint32_t cap) {
+  int s = 0;
+  while ((cap >> s) > KC_HHIST) ++s;
+  return s;
+}
+
+// One round over bins hist[0..nb] of width 2^shift that start at base, with `above`
+// neighbours over them: J = the largest j with above + (bins >= j) >= base + (j << shift)
+// (j = 0 always holds) and the count over bin J.  Every thread calls it.
+__device__ void kc_block_pick(const uint32_t* hist, uint32_t nb, uint32_t base, int shift, uint32_t above,
+                              uint32_t* J, uint32_t* over) {
   __shared__ uint32_t s_wave[KC_HTHREADS / 64];
-  __shared__ uint32_t s_best;
+  __shared__ uint32_t s_best, s_over;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   constexpr int WAVES = KC_HTHREADS / 64;
   // thread t owns bins [17 t, 17 t + 17); suffix sums over the threads above it
   const uint32_t j0 = (uint32_t)tid * KC_HPER;
   uint32_t own = 0;
-  for (uint32_t j = j0; j < j0 + KC_HPER && j <= top; ++j) own += hist[j];
+  for (uint32_t j = j0; j < j0 + KC_HPER && j <= nb; ++j) own += hist[j];
   uint32_t incl = own;
   for (int off = 1; off < 64; off <<= 1) {
     const uint32_t t = __shfl_down(incl, off, 64);
     if (lane + off < 64) incl += t;
   }
   if (lane == 0) s_wave[wave] = incl;  // the wave's total
-  if (tid == 0) s_best = 0;
+  if (tid == 0) {
+    s_best = 0;
+    s_over = 0;
+  }
   __syncthreads();
-  uint32_t sum = incl - own;
+  uint32_t sum = above + incl - own;
   for (int w = wave + 1; w < WAVES; ++w) sum += s_wave[w];
-  uint32_t best = 0;
-  for (int j = (int)std::min(j0 + KC_HPER - 1, top); j >= (int)j0 && j >= 1; --j) {
+  uint32_t best = 0, mine = 0;
+  bool has = false;
+  for (int64_t j = (int64_t)std::min(j0 + KC_HPER - 1, nb); j >= (int64_t)j0; --j) {
+    const uint32_t o = sum;
     sum += hist[j];
-    if (sum >= (uint32_t)j) {
+    if (j == 0 || sum >= base + ((uint32_t)j << shift)) {
       best = (uint32_t)j;
+      mine = o;
+      has = true;
       break;
     }
   }
-  for (int off = 32; off > 0; off >>= 1) best = std::max(best, (uint32_t)__shfl_xor(best, off, 64));
-  if (lane == 0 && best) atomicMax(&s_best, best);
+  uint32_t wbest = best;
+  for (int off = 32; off > 0; off >>= 1) wbest = std::max(wbest, (uint32_t)__shfl_xor(wbest, off, 64));
+  if (lane == 0 && wbest) atomicMax(&s_best, wbest);
   __syncthreads();
-  best = s_best;
-  if (best == KC_HHIST && cap > KC_HHIST) {
-    // binary search on [KC_HHIST, cap] with block-wide counts
-    uint32_t lo = KC_HHIST, hi = cap;
-    while (lo < hi) {
-      const uint32_t mid = lo + (hi - lo + 1) / 2;
-      uint32_t c = 0;
-      for (uint64_t k = b + tid; k < e; k += KC_HTHREADS) c += est[idx[k]] >= mid ? 1u : 0u;
-      for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
-      __syncthreads();
-      if (tid == 0) s_best = 0;
-      __syncthreads();
-      if (lane == 0 && c) atomicAdd(&s_best, c);
-      __syncthreads();
-      if (s_best >= mid) lo = mid;
-      else hi = mid - 1;
-    }
-    best = lo;
-  }
-  __syncthreads();  // s_best and s_wave are free again
-  return best;
+  if (has && best == s_best) s_over = mine;  // one thread owns bin J
+  __syncthreads();
+  *J = s_best;
+  *over = s_over;
+  __syncthreads();  // the shared words are free again
 }
 
-// A block's vertex v with h-index `best`: a drop below its coreness is recorded and its
-// neighbours are activated.  Returns 1 for a modified vertex.
-__device__ uint32_t kc_block_finish(uint32_t v, uint32_t best, uint64_t b, uint64_t e,
-                                    const uint32_t* __restrict__ idx, uint32_t* __restrict__ core,
-                                    uint64_t* __restrict__ next_bits) {
-  const bool mod = best && best < core[v];
-  __syncthreads();  // every thread has read core[v]
-  if (mod) {
-    if (threadIdx.x == 0) core[v] = best;
-    for (uint64_t k = b + threadIdx.x; k < e; k += KC_HTHREADS) kc_activate(next_bits, idx[k]);
-  }
-  __syncthreads();
-  return mod ? 1u : 0u;
-}
-
-// One block per queued vertex with more than KC_HUGE neighbours (the hubs, whose
-// adjacency would otherwise keep one wave busy for the whole epoch), up to KC_GIANT;
-// longer ones are left to the chunked passes below.
+// One block per queued vertex of up to KC_GIANT neighbours.
 __global__ __launch_bounds__(KC_HTHREADS) void k_kc_huge(
-    const uint32_t* __restrict__ huge, const kc_counters* __restrict__ cnt_in, const uint64_t* __restrict__ ptr,
-    const uint32_t* __restrict__ idx, const uint32_t* __restrict__ est, uint32_t* __restrict__ core,
-    uint64_t* __restrict__ next_bits, kc_counters* __restrict__ cnt) {
+    const uint32_t* __restrict__ qhuge_end, const kc_counters* __restrict__ cnt_in, const uint64_t* __restrict__ ptr,
+    const uint32_t* __restrict__ idx, const uint32_t* __restrict__ est, uint32_t* __restrict__ core) {
   __shared__ uint32_t hist[KC_HTHREADS * KC_HPER];
   const int tid = threadIdx.x;
   const uint64_t nhuge = cnt_in->nhuge;
-  uint32_t nmod = 0;
   for (uint64_t q = blockIdx.x; q < nhuge; q += gridDim.x) {
-    const uint32_t v = huge[q];
+    const uint32_t v = *(qhuge_end - q);
     const uint64_t b = ptr[v], e = ptr[v + 1];
-    if (e - b > KC_GIANT) continue;  // uniform: k_kc_giant_*
     const uint32_t cap = (uint32_t)std::min<uint64_t>(e - b, (uint64_t)est[v]);
-    const uint32_t top = std::min(cap, KC_HHIST);
-    for (uint32_t j = tid; j <= top; j += KC_HTHREADS) hist[j] = 0;
-    __syncthreads();
-    for (uint64_t k = b + tid; k < e; k += KC_HTHREADS) {
-      const uint32_t eu = est[idx[k]];
-      atomicAdd(&hist[eu < top ? eu : top], 1u);
+    int shift = kc_first_shift(cap);
+    uint32_t base = 0, above = 0, nb = cap >> shift;
+    for (;;) {  // two rounds at most: cap < 2^28
+      for (uint32_t j = tid; j <= nb; j += KC_HTHREADS) hist[j] = 0;
+      __syncthreads();
+      for (uint64_t k0 = b; k0 < e; k0 += KC_HTHREADS * KC_U) {
+        uint32_t eu[KC_U];
+#pragma unroll
+        for (int i = 0; i < KC_U; ++i) {
+          const uint64_t k = k0 + (uint64_t)i * KC_HTHREADS + tid;
+          eu[i] = k < e ? est[idx[k]] : 0u;
+        }
+#pragma unroll
+        for (int i = 0; i < KC_U; ++i) {
+          const uint32_t x = std::min(eu[i], cap);
+          const uint32_t j = (x - base) >> shift;
+          if (k0 + (uint64_t)i * KC_HTHREADS + tid < e && x >= base && j <= nb) atomicAdd(&hist[j], 1u);
+        }
+      }
+      __syncthreads();
+      uint32_t J, over;
+      kc_block_pick(hist, nb, base, shift, above, &J, &over);
+      base += J << shift;
+      above = over;
+      if (shift == 0) break;
+      const int ns = std::max(0, shift - (int)KC_HBITS);
+      nb = (1u << (shift - ns)) - 1u;
+      shift = ns;
     }
-    __syncthreads();
-    const uint32_t best = kc_block_hindex(hist, top, cap, b, e, idx, est);
-    nmod += kc_block_finish(v, best, b, e, idx, core, next_bits);
+    if (tid == 0 && base && base < core[v]) core[v] = base;
   }
-  if (tid == 0 && nmod) atomicAdd(&cnt->modified, (unsigned long long)nmod);
 }
 
 // Giants (more than KC_GIANT neighbours): their adjacencies in chunks of KC_GCHUNK, one
-// block per chunk, each adding its LDS histogram of the neighbours' capped estimates
-// into the giant's histogram in global memory (ghist, KC_HHIST + 1 bins per giant);
-// then one block per giant finds the h-index from it.  Inactive giants are skipped.
-__global__ void k_kc_giant_zero(uint32_t* __restrict__ ghist, uint64_t n) {
-  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-    ghist[i] = 0u;
-}
-
+// block per chunk, each adding its LDS histogram of the neighbours' capped estimates into
+// the giant's histogram in global memory (ghist, KC_HHIST + 1 bins per giant, zero between
+// launches); then one block per giant picks from it.  Answers above KC_HHIST take another
+// round.  Only giants with their bit in `act` are counted.
 __global__ __launch_bounds__(KC_HTHREADS) void k_kc_giant_hist(
     const uint64_t* __restrict__ ptr, const uint32_t* __restrict__ idx, const uint32_t* __restrict__ giants,
     const unsigned long long* __restrict__ ngiant, const uint64_t* __restrict__ start,
-    const uint64_t* __restrict__ active, const uint32_t* __restrict__ est, uint32_t* __restrict__ ghist) {
+    const uint64_t* __restrict__ act, const uint32_t* __restrict__ est, const kc_giant* __restrict__ state, int round,
+    uint32_t* __restrict__ ghist) {
   __shared__ uint32_t hist[KC_HHIST + 1];
   const int tid = threadIdx.x;
   const uint64_t n = *ngiant;
@@ -315,55 +391,256 @@ __global__ __launch_bounds__(KC_HTHREADS) void k_kc_giant_hist(
   for (uint64_t c = blockIdx.x; c < total; c += gridDim.x) {
     uint64_t k0, k1, gi;
     const uint32_t v = hub_chunk(ptr, giants, start, n, KC_GCHUNK, c, &k0, &k1, &gi);
-    if (!((active[v >> 6] >> (v & 63)) & 1ull)) continue;  // uniform
-    const uint64_t len = ptr[v + 1] - ptr[v];
-    const uint32_t cap = (uint32_t)std::min<uint64_t>(len, (uint64_t)est[v]);
-    const uint32_t top = std::min(cap, KC_HHIST);
-    for (uint32_t j = tid; j <= top; j += KC_HTHREADS) hist[j] = 0;
+    if (!((act[v >> 6] >> (v & 63)) & 1ull)) continue;  // uniform
+    const uint32_t cap = (uint32_t)std::min<uint64_t>(ptr[v + 1] - ptr[v], (uint64_t)est[v]);
+    int shift = kc_first_shift(cap);
+    uint32_t base = 0, nb = cap >> shift;
+    if (round) {
+      const kc_giant g = state[gi];
+      if (g.shift < 0) continue;  // uniform
+      base = g.base;
+      shift = g.shift;
+      nb = g.nb;
+    }
+    for (uint32_t j = tid; j <= nb; j += KC_HTHREADS) hist[j] = 0;
     __syncthreads();
-    for (uint64_t k = k0 + tid; k < k1; k += KC_HTHREADS) {
-      const uint32_t eu = est[idx[k]];
-      atomicAdd(&hist[eu < top ? eu : top], 1u);
+    for (uint64_t kk = k0; kk < k1; kk += KC_HTHREADS * KC_U) {
+      uint32_t eu[KC_U];
+#pragma unroll
+      for (int i = 0; i < KC_U; ++i) {
+        const uint64_t k = kk + (uint64_t)i * KC_HTHREADS + tid;
+        eu[i] = k < k1 ? est[idx[k]] : 0u;
+      }
+#pragma unroll
+      for (int i = 0; i < KC_U; ++i) {
+        const uint32_t x = std::min(eu[i], cap);
+        const uint32_t j = (x - base) >> shift;
+        if (kk + (uint64_t)i * KC_HTHREADS + tid < k1 && x >= base && j <= nb) atomicAdd(&hist[j], 1u);
+      }
     }
     __syncthreads();
     uint32_t* gh = ghist + gi * (uint64_t)(KC_HHIST + 1);
-    for (uint32_t j = tid; j <= top; j += KC_HTHREADS)
+    for (uint32_t j = tid; j <= nb; j += KC_HTHREADS)
       if (hist[j]) atomicAdd(&gh[j], hist[j]);
     __syncthreads();
   }
 }
 
-__global__ __launch_bounds__(KC_HTHREADS) void k_kc_giant_final(
-    const uint64_t* __restrict__ ptr, const uint32_t* __restrict__ idx, const uint32_t* __restrict__ giants,
-    const unsigned long long* __restrict__ ngiant, const uint64_t* __restrict__ active,
-    const uint32_t* __restrict__ est, const uint32_t* __restrict__ ghist, uint32_t* __restrict__ core,
-    uint64_t* __restrict__ next_bits, kc_counters* __restrict__ cnt) {
+__global__ __launch_bounds__(KC_HTHREADS) void k_kc_giant_pick(
+    const uint64_t* __restrict__ ptr, const uint32_t* __restrict__ giants,
+    const unsigned long long* __restrict__ ngiant, const uint64_t* __restrict__ act,
+    const uint32_t* __restrict__ est, kc_giant* __restrict__ state, int round, uint32_t* __restrict__ ghist,
+    uint32_t* __restrict__ core, uint32_t* __restrict__ cnt_v, kc_counters* __restrict__ cnt) {
   __shared__ uint32_t hist[KC_HTHREADS * KC_HPER];
   const int tid = threadIdx.x;
   const uint64_t n = *ngiant;
-  uint32_t nmod = 0;
   for (uint64_t gi = blockIdx.x; gi < n; gi += gridDim.x) {
     const uint32_t v = giants[gi];
-    if (!((active[v >> 6] >> (v & 63)) & 1ull)) continue;  // uniform
-    const uint64_t b = ptr[v], e = ptr[v + 1];
-    const uint32_t cap = (uint32_t)std::min<uint64_t>(e - b, (uint64_t)est[v]);
-    const uint32_t top = std::min(cap, KC_HHIST);
-    const uint32_t* gh = ghist + gi * (uint64_t)(KC_HHIST + 1);
-    for (uint32_t j = tid; j <= top; j += KC_HTHREADS) hist[j] = gh[j];
+    if (!((act[v >> 6] >> (v & 63)) & 1ull)) continue;  // uniform
+    const uint32_t cap = (uint32_t)std::min<uint64_t>(ptr[v + 1] - ptr[v], (uint64_t)est[v]);
+    const int shift0 = kc_first_shift(cap);
+    kc_giant g{0u, 0u, cap >> shift0, shift0};
+    if (round) {
+      g = state[gi];
+      if (g.shift < 0) continue;  // uniform
+    }
+    uint32_t* gh = ghist + gi * (uint64_t)(KC_HHIST + 1);
+    for (uint32_t j = tid; j <= g.nb; j += KC_HTHREADS) {
+      hist[j] = gh[j];
+      gh[j] = 0u;
+    }
     __syncthreads();
-    const uint32_t best = kc_block_hindex(hist, top, cap, b, e, idx, est);
-    nmod += kc_block_finish(v, best, b, e, idx, core, next_bits);
+    uint32_t J, over;
+    kc_block_pick(hist, g.nb, g.base, g.shift, g.above, &J, &over);
+    if (tid == 0) {
+      g.base += J << g.shift;
+      g.above = over;
+      if (g.shift == 0) {
+        g.shift = -1;
+        if (g.base && g.base < core[v]) {
+          core[v] = g.base;
+          if (cnt_v) cnt_v[v] = 0u;  // re-counted chunk by chunk in the spread
+        }
+        atomicMax(&cnt->giant_top, (unsigned long long)core[v]);
+      } else {
+        const int ns = std::max(0, g.shift - (int)KC_HBITS);
+        g.nb = (1u << (g.shift - ns)) - 1u;
+        g.shift = ns;
+      }
+      state[gi] = g;
+    }
+    __syncthreads();
   }
-  if (tid == 0 && nmod) atomicAdd(&cnt->modified, (unsigned long long)nmod);
 }
 
-// estimate = coreness for the epoch's active vertices (kcore.hpp:248-258)
-__global__ void k_kc_sync(const uint32_t* __restrict__ queue, uint64_t n, const uint32_t* __restrict__ core,
-                          uint32_t* __restrict__ est) {
-  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
-    const uint32_t v = queue[i];
-    est[v] = core[v];
+// ---- spread ------------------------------------------------------------------------------------
+// The modified vertices (core below est) activate their neighbours; with counts (cnt_v) each
+// also takes itself out of the counts of the unmodified neighbours it fell below, marking those
+// that the last one leaves short as candidates, and returns how many neighbours it keeps at or
+// above its own new value.  act_bytes: the next active set, one byte per
+// vertex: a mark is a plain store of 1 that any number of waves may repeat, where an atomic OR
+// on a shared bitmap word is serialized in the memory-side atomic unit (RMAT scale 22, all epochs: 35 ms of
+// spreading with bits, 10 ms with bytes).
+struct kc_spread {
+  const uint32_t* idx;
+  const uint32_t* est;
+  const uint32_t* core;
+  uint32_t* cnt_v;
+  uint8_t* act_bytes;
+  uint64_t* cand;
+  __device__ __forceinline__ uint32_t one(uint32_t u, uint32_t cu, uint32_t old, uint32_t now) const {
+    if (!act_bytes[u]) act_bytes[u] = 1;
+    if (!cnt_v) return 0u;
+    if (cu > now && cu <= old && est[u] == cu && atomicSub(&cnt_v[u], 1u) == cu) kc_set_bit(cand, u);
+    return cu >= now ? 1u : 0u;
   }
+  // entries b + i0, b + i0 + step, ... below e
+  __device__ __forceinline__ uint32_t range(uint64_t b, uint64_t e, uint32_t i0, uint32_t step, uint32_t old,
+                                            uint32_t now) const {
+    uint32_t c = 0;
+    for (uint64_t k0 = b; k0 < e; k0 += (uint64_t)step * KC_U) {
+      uint32_t u[KC_U], cu[KC_U];
+#pragma unroll
+      for (int i = 0; i < KC_U; ++i) {
+        const uint64_t k = k0 + (uint64_t)i * step + i0;
+        u[i] = k < e ? idx[k] : 0u;
+        cu[i] = k < e && cnt_v ? core[u[i]] : 0u;
+      }
+#pragma unroll
+      for (int i = 0; i < KC_U; ++i)
+        if (k0 + (uint64_t)i * step + i0 < e) c += one(u[i], cu[i], old, now);
+    }
+    return c;
+  }
+};
+
+__global__ __launch_bounds__(KC_THREADS) void k_kc_spread(
+    const uint32_t* __restrict__ qsmall, const uint32_t* __restrict__ qbig, const kc_counters* __restrict__ cnt_in,
+    const uint64_t* __restrict__ ptr, kc_spread sp) {
+  const int lane = threadIdx.x & 63;
+  const uint64_t nbig = cnt_in->nbig, nsmall = cnt_in->nsmall;
+  const uint64_t wave_id = grid_wave_id(), nwaves = grid_waves();
+  for (uint64_t q = wave_id; q < nbig; q += nwaves) {
+    const uint32_t v = qbig[q];
+    const uint32_t old = sp.est[v], now = sp.core[v];
+    if (old == now) continue;  // uniform
+    uint32_t c = sp.range(ptr[v], ptr[v + 1], (uint32_t)lane, 64u, old, now);
+    if (sp.cnt_v) {
+      for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
+      if (lane == 0) sp.cnt_v[v] = c;
+    }
+  }
+  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < nsmall;
+       i += (uint64_t)gridDim.x * blockDim.x) {
+    const uint32_t v = qsmall[i];
+    const uint32_t old = sp.est[v], now = sp.core[v];
+    if (old == now) continue;
+    const uint32_t c = sp.range(ptr[v], ptr[v + 1], 0u, 1u, old, now);
+    if (sp.cnt_v) sp.cnt_v[v] = c;
+  }
+}
+
+__global__ __launch_bounds__(KC_HTHREADS) void k_kc_spread_huge(const uint32_t* __restrict__ qhuge_end,
+                                                                const kc_counters* __restrict__ cnt_in,
+                                                                const uint64_t* __restrict__ ptr, kc_spread sp) {
+  __shared__ uint32_t s_c;
+  const uint64_t nhuge = cnt_in->nhuge;
+  for (uint64_t q = blockIdx.x; q < nhuge; q += gridDim.x) {
+    const uint32_t v = *(qhuge_end - q);
+    const uint32_t old = sp.est[v], now = sp.core[v];
+    if (old == now) continue;  // uniform
+    if (threadIdx.x == 0) s_c = 0u;
+    __syncthreads();
+    uint32_t c = sp.range(ptr[v], ptr[v + 1], threadIdx.x, KC_HTHREADS, old, now);
+    if (sp.cnt_v) {
+      for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
+      if ((threadIdx.x & 63) == 0) atomicAdd(&s_c, c);
+      __syncthreads();
+      if (threadIdx.x == 0) sp.cnt_v[v] = s_c;
+    }
+    __syncthreads();
+  }
+}
+
+__global__ __launch_bounds__(KC_HTHREADS) void k_kc_spread_giant(const uint64_t* __restrict__ ptr,
+                                                                 const uint32_t* __restrict__ giants,
+                                                                 const unsigned long long* __restrict__ ngiant,
+                                                                 const uint64_t* __restrict__ start,
+                                                                 const uint64_t* __restrict__ act, kc_spread sp) {
+  const uint64_t n = *ngiant;
+  if (n == 0) return;
+  const uint64_t total = start[n];
+  for (uint64_t c = blockIdx.x; c < total; c += gridDim.x) {
+    uint64_t k0, k1;
+    const uint32_t v = hub_chunk(ptr, giants, start, n, KC_GCHUNK, c, &k0, &k1);
+    if (!((act[v >> 6] >> (v & 63)) & 1ull)) continue;  // uniform
+    const uint32_t old = sp.est[v], now = sp.core[v];
+    if (old == now) continue;
+    uint32_t k = sp.range(k0, k1, threadIdx.x, KC_HTHREADS, old, now);
+    if (sp.cnt_v) {
+      for (int off = 32; off > 0; off >>= 1) k += __shfl_xor(k, off, 64);
+      if ((threadIdx.x & 63) == 0 && k) atomicAdd(&sp.cnt_v[v], k);
+    }
+  }
+}
+
+// ---- commit --------------------------------------------------------------------------------------
+// estimate = coreness for the epoch's candidates (kcore.hpp:248-258); modified ones that are
+// already short again stay candidates.
+__global__ __launch_bounds__(KC_THREADS) void k_kc_commit(
+    const uint32_t* __restrict__ qsmall, const uint32_t* __restrict__ qbig, const uint32_t* __restrict__ qhuge_end,
+    const uint32_t* __restrict__ giants, const unsigned long long* __restrict__ ngiant,
+    const uint64_t* __restrict__ act, const uint32_t* __restrict__ core, uint32_t* __restrict__ est,
+    const uint32_t* __restrict__ cnt_v, uint64_t* __restrict__ cand, kc_counters* __restrict__ cnt) {
+  const uint64_t ns = cnt->nsmall, nb = cnt->nbig, nh = cnt->nhuge, ng = giants ? *ngiant : 0ull;
+  unsigned long long nmod = 0;
+  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < ns + nb + nh + ng;
+       i += (uint64_t)gridDim.x * blockDim.x) {
+    uint32_t v;
+    if (i < ns) {
+      v = qsmall[i];
+    } else if (i < ns + nb) {
+      v = qbig[i - ns];
+    } else if (i < ns + nb + nh) {
+      v = *(qhuge_end - (i - ns - nb));
+    } else {
+      v = giants[i - ns - nb - nh];
+      if (!((act[v >> 6] >> (v & 63)) & 1ull)) continue;
+    }
+    const uint32_t c = core[v], old = est[v];
+    if (c == old) continue;
+    est[v] = c;
+    nmod += old != KC_UNSET ? 1u : 0u;
+    if (cnt_v && cnt_v[v] < c) kc_set_bit(cand, v);
+  }
+  block_add2(nmod, 0, &cnt->modified, &cnt->modified);
+}
+
+// sizes of the next active set (its bytes, cleared here) and candidate set; without counts the
+// active set is the candidate set
+__global__ __launch_bounds__(256) void k_kc_next(uint64_t* __restrict__ act_bytes, uint64_t* __restrict__ cand,
+                                                 uint64_t nwords, int is_cand, kc_counters* __restrict__ cnt) {
+  const int lane = threadIdx.x & 63;
+  const uint64_t n = nwords * 8;  // 8-byte groups of marks; eight lanes cover one bitmap word
+  unsigned long long a = 0, c = 0;
+  for (uint64_t base = grid_wave_id() * 64; base < n; base += grid_waves() * 64) {
+    const uint64_t i = base + lane;
+    uint64_t w = 0;
+    if (i < n) {
+      w = act_bytes[i];
+      if (w) act_bytes[i] = 0ull;
+    }
+    a += (unsigned long long)__popcll(w);
+    if (is_cand) {
+      uint64_t bits = ((w * 0x0102040810204080ull) >> 56) << ((lane & 7) * 8);  // byte j's mark -> bit j
+      for (int off = 4; off > 0; off >>= 1) bits |= __shfl_xor(bits, off, 64);
+      if (i < n && (lane & 7) == 0) cand[i >> 3] = bits;
+    } else if (i < n && (lane & 7) == 0) {
+      c += (unsigned long long)__popcll(cand[i >> 3]);
+    }
+  }
+  if (is_cand) c = a;
+  block_add2(a, c, &cnt->next_active, &cnt->next_cand);
 }
 
 }  // namespace pe
@@ -380,71 +657,83 @@ extern "C" int pe_kcore(pe_graph_t* g, int out_edges, uint32_t* coreness, uint64
     const uint32_t V = g->V;
     const uint64_t* ptr = out_edges ? g->csr_ptr() : g->col_ptr.p;
     const uint32_t* idx = out_edges ? g->csr_idx() : g->row_idx.p;
+    const bool counts = g->csr_is_csc;  // the adjacency is its own reverse
     const uint64_t nwords = ((uint64_t)V >> 6) + 1;
     const uint32_t Vs = std::max<uint32_t>(1, V);
-    dbuf<uint32_t> core(ctx, Vs), est(ctx, Vs), queue(ctx, Vs), big(ctx, Vs), huge(ctx, Vs);
-    dbuf<uint64_t> cur(ctx, nwords), nxt(ctx, nwords), big_bits(ctx, nwords), huge_bits(ctx, nwords);
-    dbuf<kc_counters> cnt(ctx, 1);
-    kc_counters* h = static_cast<kc_counters*>(ctx->host_pinned);
+    dbuf<uint32_t> core(ctx, Vs), est(ctx, Vs), qsmall(ctx, Vs), qbig(ctx, Vs), cnt_v;
+    dbuf<uint64_t> cand(ctx, nwords), act, nxt(ctx, nwords * 8);  // nxt: one byte per vertex
+    if (counts) cnt_v.alloc(ctx, Vs);
+    uint32_t* qhuge_end = qbig.p + (Vs - 1);
+    dbuf<kc_counters> cnt(ctx, 2);  // two sets: consecutive epochs alternate
     PE_HIP(hipEventRecord(ctx->t0, s));
-    k_kc_init<<<grid_for(V, 256, 8192), 256, 0, s>>>(ptr, V, core.p, est.p);
-    k_kc_fill<<<grid_for(nwords, 256, 4096), 256, 0, s>>>(cur.p, nwords, V);  // active_current.fill()
+    k_kc_init<<<grid_for(V, 256, 8192), 256, 0, s>>>(ptr, V, core.p, est.p, cnt_v.p);
+    k_kc_fill<<<grid_for(nwords, 256, 4096), 256, 0, s>>>(cand.p, nwords, V);  // active_current.fill()
+    k_kc_zero<<<grid_for(nwords * 8, 256, 4096), 256, 0, s>>>(nxt.p, nwords * 8);
     PE_HIP(hipGetLastError());
-    const unsigned big_grid = persistent_grid(ctx, 1u << 20, 4);
-    const unsigned small_grid = persistent_grid(ctx, 1u << 20, 8);
-    const unsigned huge_grid = persistent_grid(ctx, 1u << 20, 1);
     // giants and their histograms (one per giant, KC_HHIST + 1 bins)
     hub_table giants;
     hub_table_build(ctx, ptr, V, g->nnz, KC_GIANT, KC_GCHUNK, giants);
-    unsigned long long ngiant = 0;
-    PE_HIP(hipMemcpyAsync(&ngiant, giants.count.p, sizeof(ngiant), hipMemcpyDeviceToHost, s));
-    PE_HIP(hipStreamSynchronize(s));
+    const uint64_t ngiant = mail_post(ctx, giants.count.p, 1, reinterpret_cast<unsigned long long*>(cnt.p), 2 * KC_CW)[0];
     const uint64_t ghist_words = ngiant * (uint64_t)(KC_HHIST + 1);
-    dbuf<uint32_t> ghist(ctx, std::max<uint64_t>(1, ghist_words));
-    uint32_t epoch = 0;
-    uint64_t total_mod = 0;
-    for (;;) {
-      k_kc_reset<<<1, 1, 0, s>>>(cnt.p);
-      frontier_compact(ctx, cur.p, nwords, V, queue.p, &cnt.p->queued);
-      PE_HIP(hipMemcpyAsync(h, cnt.p, sizeof(kc_counters), hipMemcpyDeviceToHost, s));
-      PE_HIP(hipStreamSynchronize(s));
-      const uint64_t n = h->queued;
-      if (epoch > 0) {
-        if (epoch - 1 < cap && epoch_next) epoch_next[epoch - 1] = n;  // need_modified of the last epoch
-        if (n == 0) break;                                              // kcore.hpp:264
-      }
-      k_kc_zero<<<grid_for(nwords, 256, 4096), 256, 0, s>>>(nxt.p, nwords);
-      if (n) {
-        k_kc_zero<<<grid_for(nwords, 256, 4096), 256, 0, s>>>(big_bits.p, nwords);
-        k_kc_zero<<<grid_for(nwords, 256, 4096), 256, 0, s>>>(huge_bits.p, nwords);
-        k_kc_small<<<std::min<unsigned>(small_grid, grid_for(n, KC_THREADS)), KC_THREADS, 0, s>>>(
-            queue.p, n, ptr, idx, est.p, core.p, nxt.p, big_bits.p, huge_bits.p, cnt.p);
-        frontier_compact(ctx, big_bits.p, nwords, V, big.p, &cnt.p->nbig);
-        frontier_compact(ctx, huge_bits.p, nwords, V, huge.p, &cnt.p->nhuge);
-        k_kc_big<<<big_grid, KC_THREADS, 0, s>>>(big.p, cnt.p, ptr, idx, est.p, core.p, nxt.p, cnt.p);
-        k_kc_huge<<<huge_grid, KC_HTHREADS, 0, s>>>(huge.p, cnt.p, ptr, idx, est.p, core.p, nxt.p, cnt.p);
-        if (ngiant) {
-          k_kc_giant_zero<<<grid_for(ghist_words, 256, 4096), 256, 0, s>>>(ghist.p, ghist_words);
-          k_kc_giant_hist<<<huge_grid, KC_HTHREADS, 0, s>>>(ptr, idx, giants.hubs.p, giants.count.p, giants.start.p,
-                                                            cur.p, est.p, ghist.p);
-          k_kc_giant_final<<<(unsigned)std::min<uint64_t>(ngiant, huge_grid), KC_HTHREADS, 0, s>>>(
-              ptr, idx, giants.hubs.p, giants.count.p, cur.p, est.p, ghist.p, core.p, nxt.p, cnt.p);
-        }
-        k_kc_sync<<<grid_for(n, 256, 8192), 256, 0, s>>>(queue.p, n, core.p, est.p);
-      }
+    dbuf<uint32_t> ghist;
+    dbuf<kc_giant> gstate;
+    if (ngiant) {
+      act.alloc(ctx, nwords);
+      ghist.alloc(ctx, ghist_words + 1);  // whole 8-byte words to clear
+      gstate.alloc(ctx, ngiant);
+      k_kc_zero<<<grid_for((ghist_words + 1) / 2, 256, 4096), 256, 0, s>>>(reinterpret_cast<uint64_t*>(ghist.p),
+                                                                          (ghist_words + 1) / 2);
       PE_HIP(hipGetLastError());
-      PE_HIP(hipMemcpyAsync(h, cnt.p, sizeof(kc_counters), hipMemcpyDeviceToHost, s));
-      PE_HIP(hipStreamSynchronize(s));
-      if (epoch < cap && epoch_modified) epoch_modified[epoch] = h->modified;
-      total_mod += h->modified;
-      std::swap(cur.p, nxt.p);
+    }
+    const kc_spread sp{idx, est.p, core.p, cnt_v.p, reinterpret_cast<uint8_t*>(nxt.p), cand.p};
+    const unsigned full_grid = persistent_grid(ctx, 1u << 20, 8), huge_max = persistent_grid(ctx, 1u << 20, 2);
+    const uint32_t* gl = ngiant ? giants.hubs.p : nullptr;
+    uint32_t epoch = 0;
+    uint64_t total_mod = 0, ncand = V, giant_top = g->nnz;
+    for (;;) {
+      kc_counters* c = cnt.p + (epoch & 1);
+      uint64_t modified = 0, next = 0;
+      if (ncand) {
+        const unsigned grid = (unsigned)std::min<uint64_t>(full_grid, (ncand + 3) / 4);
+        const unsigned hgrid = (unsigned)std::min<uint64_t>(huge_max, ncand);
+        k_kc_classify<<<grid_for(nwords, 16 * KC_CW_WORDS, (unsigned)std::max(1, ctx->num_cus) * 2), 1024, 0, s>>>(
+            cand.p, act.p, nwords, V, ptr, est.p, qsmall.p, qbig.p, qhuge_end, c);
+        k_kc_huge<<<hgrid, KC_HTHREADS, 0, s>>>(qhuge_end, c, ptr, idx, est.p, core.p);
+        k_kc_hindex<<<grid, KC_THREADS, 0, s>>>(qsmall.p, qbig.p, c, ptr, idx, est.p, core.p);
+        if (ngiant) {
+          // rounds: 14 bits of the answer each after the first
+          int rounds = 1;
+          for (uint64_t t = std::min<uint64_t>(giant_top, 0xFFFFFFFEull); t > KC_HHIST; t >>= KC_HBITS) ++rounds;
+          const unsigned pgrid = (unsigned)std::min<uint64_t>(ngiant, huge_max);
+          for (int r = 0; r < rounds; ++r) {
+            k_kc_giant_hist<<<huge_max, KC_HTHREADS, 0, s>>>(ptr, idx, gl, giants.count.p, giants.start.p, act.p, est.p,
+                                                             gstate.p, r, ghist.p);
+            k_kc_giant_pick<<<pgrid, KC_HTHREADS, 0, s>>>(ptr, gl, giants.count.p, act.p, est.p, gstate.p, r, ghist.p,
+                                                          core.p, cnt_v.p, c);
+          }
+          k_kc_spread_giant<<<huge_max, KC_HTHREADS, 0, s>>>(ptr, gl, giants.count.p, giants.start.p, act.p, sp);
+        }
+        k_kc_spread_huge<<<hgrid, KC_HTHREADS, 0, s>>>(qhuge_end, c, ptr, sp);
+        k_kc_spread<<<grid, KC_THREADS, 0, s>>>(qsmall.p, qbig.p, c, ptr, sp);
+        k_kc_commit<<<grid_for(ncand, KC_THREADS, full_grid), KC_THREADS, 0, s>>>(
+            qsmall.p, qbig.p, qhuge_end, gl, giants.count.p, act.p, core.p, est.p, cnt_v.p, cand.p, c);
+        k_kc_next<<<grid_for(nwords * 8, 256, (unsigned)std::max(1, ctx->num_cus) * 2), 256, 0, s>>>(nxt.p, cand.p, nwords, counts ? 0 : 1, c);
+        PE_HIP(hipGetLastError());
+        const kc_counters* h = reinterpret_cast<const kc_counters*>(
+            mail_post(ctx, reinterpret_cast<const unsigned long long*>(c), KC_CW,
+                      reinterpret_cast<unsigned long long*>(cnt.p + ((epoch + 1) & 1)), KC_CW));
+        modified = h->modified;
+        next = h->next_active;
+        ncand = h->next_cand;
+        if (epoch == 0) giant_top = h->giant_top;  // estimates only fall from here on
+      }
+      if (epoch < cap && epoch_modified) epoch_modified[epoch] = modified;
+      if (epoch < cap && epoch_next) epoch_next[epoch] = next;  // need_modified
+      total_mod += modified;
       ++epoch;
+      if (next == 0) break;  // kcore.hpp:264
       // every epoch but the last lowers some coreness, which starts at most at its length
       PE_REQUIRE((uint64_t)epoch <= g->nnz + 2, PE_ERR_INTERNAL, "k-core did not terminate");
-      if (n == 0) {  // nothing active in epoch 0: an empty graph
-        if (epoch - 1 < cap && epoch_next) epoch_next[epoch - 1] = 0;
-        break;
-      }
     }
     PE_HIP(hipEventRecord(ctx->t1, s));
     PE_HIP(hipEventSynchronize(ctx->t1));

@@ -108,3 +108,47 @@ def test_giant_hub(ctx):
     # directed: the hub's 70000 in-edges come from the rim's reversed edges
     s2, d2 = np.concatenate([s, r]), np.concatenate([d, np.zeros(rim, np.uint32)])
     _check(Graph.from_edges(ctx, s2, d2, V, build_csr=True), oracle.CSC(V, s2, d2))
+
+
+@pytest.mark.parametrize("n,mult", [(22, 820), (18, 965), (80, 1000)])
+@pytest.mark.parametrize("directed", [False, True])
+def test_answers_above_the_block_histogram(ctx, n, mult, directed):
+    """n vertices joined pairwise by 0.9 to 1.1 * mult parallel edges: h-indices around and
+    above the 16384 bins of the block pass (18 * 965 straddles them), which take a second
+    round over a value range, in one block per vertex and (n = 80) in chunks."""
+    from plato_amd import Graph
+    rng = np.random.default_rng(n)
+    a, b = np.triu_indices(n, 1)
+    m = rng.integers(int(mult * 0.9), int(mult * 1.1), a.size)
+    s, d = np.repeat(a, m).astype(np.uint32), np.repeat(b, m).astype(np.uint32)
+    if directed:
+        s, d = np.concatenate([s, d]), np.concatenate([d, s])
+    V = n + 1
+    print(f"case: kcore multigraph n={n} mult={mult} directed={directed}", flush=True)
+    g = Graph.from_edges(ctx, s, d, V, directed=directed, build_csr=True)
+    res = _check(g, oracle.CSC(V, s, d, symmetrize=not directed))
+    if n * mult > 15000:
+        assert res.coreness.max() > 14000
+    g.close()
+
+
+@pytest.mark.parametrize("length", [64, 65, 1024, 1025, 4096, 4097, 65536, 65537])
+@pytest.mark.parametrize("directed", [False, True])
+def test_adjacency_length_classes(ctx, length, directed):
+    """Eight vertices of exactly `length` neighbours (the last of one pass and the first of the
+    next) over a random graph, so their values move over several epochs."""
+    from plato_amd import Graph
+    rng = np.random.default_rng(length)
+    rim, hubs = max(4 * length // 3, 200), 8
+    s = np.concatenate([np.full(length, rim + h) for h in range(hubs)] + [rng.integers(0, rim, 6 * rim)])
+    d = np.concatenate([rng.choice(rim, length, replace=False) for _ in range(hubs)] + [rng.integers(0, rim, 6 * rim)])
+    s, d = s.astype(np.uint32), d.astype(np.uint32)
+    if directed:
+        s, d = np.concatenate([s, d]), np.concatenate([d, s])
+    V = rim + hubs
+    og = oracle.CSC(V, s, d, symmetrize=not directed)
+    assert int(np.diff(og.col_ptr)[rim]) == length
+    print(f"case: kcore length={length} directed={directed}", flush=True)
+    g = Graph.from_edges(ctx, s, d, V, directed=directed, relabel=length % 2 == 1)
+    _check(g, og)
+    g.close()
