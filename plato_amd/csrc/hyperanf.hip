@@ -13,13 +13,22 @@
 // than DBL_EPSILON (that anf is dropped).  The average distance is GetAvgDistance over
 // the anfs (hyperanf.hpp:58-67).
 //
-// Layout: counters [V][2^P] bytes, double-buffered (Jacobi).  Pull: one wave per
-// vertex, registers handled as 32-bit words of four; 64- and 128-register counters take
-// 4 or 2 in-edges per wave step (a row is 16 or 32 lanes), larger ones one edge per step
-// with each lane owning 2^P / 256 words; several rows are loaded before they are merged.
-// Vertices with more than HANF_HUB_DEG in-edges (the hubs) only copy their own row in
-// that pass; a second pass cuts their in-edges into chunks spread over all waves, each
-// merging its chunk's maximum into the hub's row, so no wave walks a hub alone.
+// Layout: counters [V][2^P] bytes, double-buffered (Jacobi), read as 16 registers per lane
+// and load: LPR = 2^P / 16 lanes hold a row (at most 64; counters above 1024 registers walk
+// the in-edges once per 1024), so a wave's load brings 64 / LPR rows.  A row that the last
+// iteration left as it was has already been merged by its out-neighbours, so a bitmap of the
+// changed rows decides per in-edge whether the row is read at all, a vertex without changed
+// in-neighbours is not touched, and its estimate is kept.  No row of a vertex that someone
+// pulls from can pass the register-wise max over the first counters of all such vertices (the
+// bound row): a pull stops at the first row that reaches it, and a vertex that has reached it
+// is done.  The pull's bound is the random
+// 2^P-byte rows of the first iterations, then the in-edge lists.  RMAT scale 23
+// symmetrized, P = 6, 8 pulls: 5.2 ms each with one 4-byte word per lane and every row read;
+// here 3.4, 3.4 and 2.5 ms, then 0.8 falling to 0.15 ms (without the bound row 3.4 four times,
+// then 0.8); the whole call 44.7 -> 16.0 ms.
+// Three passes by in-degree: fewer than HANF_LOW_DEG, a group of LPR lanes per vertex; up to
+// HANF_HUB_DEG, a wave per vertex; the hubs' in-edges in chunks over all waves, each merging
+// its chunk's maximum into the hub's row, so no wave walks a hub alone.
 #include <cfloat>
 #include <cmath>
 #include <vector>
@@ -30,9 +39,8 @@ namespace pe {
 
 static constexpr uint64_t HANF_HUB_DEG = 4096;    // in-edges above which a vertex is a hub
 static constexpr uint64_t HANF_HUB_CHUNK = 2048;  // in-edges of a hub per wave task
-static constexpr int HANF_HUB_U = 8;             // rows each lane of the hub pass keeps in flight
-static constexpr uint64_t HANF_LOW_DEG = 32;    // counters of up to 128 registers: fewer in-edges
-                                                 // take a lane group per vertex
+static constexpr uint64_t HANF_LOW_DEG = 32;    // fewer in-edges take a lane group per vertex
+static constexpr int HANF_U = 8;                 // rows a lane keeps in flight at most
 
 __device__ __forceinline__ uint32_t hanf_rotl(uint32_t x, int r) { return (x << r) | (x >> (32 - r)); }
 
@@ -54,15 +62,22 @@ __device__ __forceinline__ uint32_t hanf_murmur_u32(uint32_t key, uint32_t seed)
   return h;
 }
 
+// register and rank of a vertex's own id
+__device__ __forceinline__ void hanf_first(uint32_t id, int P, uint32_t* reg, uint32_t* rank) {
+  const uint32_t h = hanf_murmur_u32(id, 0x5f61767au);
+  const uint32_t w = h << P;
+  const uint32_t q = 32u - (uint32_t)P;
+  const uint32_t r = w ? (uint32_t)__clz(w) + 1u : q + 1u;
+  *reg = h >> q;
+  *rank = r < q + 1u ? r : q + 1u;
+}
+
 __global__ void k_hanf_init(uint8_t* __restrict__ regs, uint32_t V, int P, const uint32_t* __restrict__ perm) {
   const uint64_t m = 1ull << P;
   for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x) {
-    const uint32_t id = perm ? perm[v] : (uint32_t)v;  // counters hash input ids
-    const uint32_t h = hanf_murmur_u32(id, 0x5f61767au);
-    const uint32_t w = h << P;
-    const uint32_t q = 32u - (uint32_t)P;
-    const uint32_t rank = w ? (uint32_t)__clz(w) + 1u : q + 1u;
-    regs[v * m + (h >> q)] = (uint8_t)(rank < q + 1u ? rank : q + 1u);
+    uint32_t reg, rank;
+    hanf_first(perm ? perm[v] : (uint32_t)v, P, &reg, &rank);  // counters hash input ids
+    regs[v * m + reg] = (uint8_t)rank;
   }
 }
 
@@ -71,176 +86,350 @@ __global__ void k_hanf_zero(uint32_t* __restrict__ p, uint64_t n) {
     p[i] = 0u;
 }
 
-__device__ __forceinline__ uint32_t byte_max4(uint32_t a, uint32_t b) {
-  uint32_t r = 0;
-#pragma unroll
-  for (int i = 0; i < 32; i += 8) r |= max((a >> i) & 0xFFu, (b >> i) & 0xFFu) << i;
-  return r;
+// Byte-wise max of many words: the odd bytes in 16-bit maxima of the words as they are (the
+// high byte decides, the low byte only breaks ties), the even bytes in those of the words
+// shifted up by one byte: three instructions per word of four registers, where unpacking
+// each byte takes about sixteen.
+typedef uint16_t hanf_u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t max_u16x2(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(hanf_u16x2, a),
+                                                                __builtin_bit_cast(hanf_u16x2, b)));
 }
 
-// Pull for counters of 64 or 128 registers (16 or 32 words): a wave takes EPS in-edges
-// per step (64 / EPS lanes per row, one word each), U steps in flight, and folds the
-// EPS partial rows together with shuffles at the end.  0 is the identity of max.
-template <int EPS, int U>
-__global__ __launch_bounds__(256) void k_hanf_pull_small(const uint64_t* __restrict__ col_ptr,
-                                                         const uint32_t* __restrict__ row_idx, uint32_t V,
-                                                         uint64_t min_deg, const uint32_t* __restrict__ cur,
-                                                         uint32_t* __restrict__ nxt) {
-  constexpr int WPR = 64 / EPS;  // words per counter
-  const int lane = threadIdx.x & 63, slot = lane / WPR, w = lane % WPR;
-  const uint64_t wave_id = grid_wave_id(), nwaves = grid_waves();
-  for (uint64_t v = wave_id; v < V; v += nwaves) {
-    const uint64_t b = col_ptr[v], e = col_ptr[v + 1];
-    if (e - b < min_deg) continue;  // k_hanf_pull_lowdeg
-    uint32_t acc = slot == 0 ? cur[v * WPR + w] : 0u;
-    if (e - b > HANF_HUB_DEG) {  // a hub: its own row now, its in-edges in k_hanf_pull_hubs
-      if (slot == 0) nxt[v * WPR + w] = acc;
-      continue;
-    }
-    for (uint64_t k0 = b; k0 < e; k0 += (uint64_t)EPS * U) {
-      uint32_t val[U];
+__device__ __forceinline__ uint32_t byte_max4(uint32_t a, uint32_t b) {
+  return (max_u16x2(a, b) & 0xFF00FF00u) | ((max_u16x2(a << 8, b << 8) >> 8) & 0x00FF00FFu);
+}
+
+struct row_max {  // 16 registers
+  uint32_t odd[4] = {0, 0, 0, 0}, even[4] = {0, 0, 0, 0};
+  __device__ __forceinline__ void add(const uint4& r) {
+    const uint32_t w[4] = {r.x, r.y, r.z, r.w};
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const uint64_t k = k0 + (uint64_t)u * EPS + slot;
-        val[u] = k < e ? cur[(uint64_t)row_idx[k] * WPR + w] : 0u;
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) acc = byte_max4(acc, val[u]);
+    for (int i = 0; i < 4; ++i) {
+      odd[i] = max_u16x2(odd[i], w[i]);
+      even[i] = max_u16x2(even[i], w[i] << 8);
     }
-    for (int off = WPR; off < 64; off <<= 1) acc = byte_max4(acc, (uint32_t)__shfl_xor(acc, off, 64));
-    if (slot == 0) nxt[v * WPR + w] = acc;
+  }
+  __device__ __forceinline__ uint4 row() const {
+    uint32_t w[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) w[i] = (odd[i] & 0xFF00FF00u) | ((even[i] >> 8) & 0x00FF00FFu);
+    return make_uint4(w[0], w[1], w[2], w[3]);
+  }
+};
+
+__device__ __forceinline__ uint4 row_max2(const uint4& a, const uint4& b) {
+  return make_uint4(byte_max4(a.x, b.x), byte_max4(a.y, b.y), byte_max4(a.z, b.z), byte_max4(a.w, b.w));
+}
+__device__ __forceinline__ uint4 row_shfl_xor(const uint4& a, int off) {
+  return make_uint4((uint32_t)__shfl_xor((int)a.x, off, 64), (uint32_t)__shfl_xor((int)a.y, off, 64),
+                    (uint32_t)__shfl_xor((int)a.z, off, 64), (uint32_t)__shfl_xor((int)a.w, off, 64));
+}
+__device__ __forceinline__ bool row_differs(const uint4& a, const uint4& b) {
+  return ((a.x ^ b.x) | (a.y ^ b.y) | (a.z ^ b.z) | (a.w ^ b.w)) != 0u;
+}
+
+// the lanes g * LPR of the groups of LPR lanes that are all set in m
+template <int LPR>
+__device__ __forceinline__ uint64_t full_groups(uint64_t m) {
+#pragma unroll
+  for (int k = 1; k < LPR; k <<= 1) m &= m >> k;
+  constexpr uint64_t first = LPR == 64 ? 1ull : ~0ull / ((1ull << (LPR & 63)) - 1ull);  // every LPR-th bit
+  return m & first;
+}
+
+// The bound row: register-wise max of the first counters of the vertices with out-degree (od),
+// or with entries in their own list (ptr), one word per register, zeroed before.  Registers
+// that fit are collected per block in LDS.
+static constexpr uint32_t HANF_LDS_REGS = 4096;
+__global__ __launch_bounds__(256) void k_hanf_bound(uint32_t V, int P, const uint32_t* __restrict__ perm,
+                                                    const uint32_t* __restrict__ od, const uint64_t* __restrict__ ptr,
+                                                    uint32_t* __restrict__ top) {
+  __shared__ uint32_t s_top[HANF_LDS_REGS];
+  const uint32_t m = 1u << P;
+  const bool lds = m <= HANF_LDS_REGS;
+  if (lds) {
+    for (uint32_t i = threadIdx.x; i < m; i += blockDim.x) s_top[i] = 0u;
+    __syncthreads();
+  }
+  for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x) {
+    if (od ? od[v] == 0u : ptr[v] == ptr[v + 1]) continue;
+    uint32_t reg, rank;
+    hanf_first(perm ? perm[v] : (uint32_t)v, P, &reg, &rank);
+    uint32_t* t = lds ? &s_top[reg] : &top[reg];
+    if (*t < rank) atomicMax(t, rank);
+  }
+  if (lds) {
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < m; i += blockDim.x)
+      if (s_top[i] > top[i]) atomicMax(&top[i], s_top[i]);
   }
 }
 
-// Pull for the vertices with fewer than max_deg in-edges and counters of WPR <= 32
-// words: one group of WPR lanes per vertex, 64 / WPR vertices per wave step, U in-edges
-// of each in flight, so the vertices' short chains of dependent loads overlap.
-template <int WPR, int U>
-__global__ __launch_bounds__(256) void k_hanf_pull_lowdeg(const uint64_t* __restrict__ col_ptr,
-                                                          const uint32_t* __restrict__ row_idx, uint32_t V,
-                                                          uint64_t max_deg, const uint32_t* __restrict__ cur,
-                                                          uint32_t* __restrict__ nxt) {
-  constexpr int G = 64 / WPR;  // vertices per wave step
-  const int lane = threadIdx.x & 63, grp = lane / WPR, w = lane % WPR;
-  const uint64_t wave_id = grid_wave_id(), nwaves = grid_waves();
-  for (uint64_t v0 = wave_id * G; v0 < V; v0 += nwaves * G) {
+__global__ void k_hanf_bound_row(const uint32_t* __restrict__ top, uint32_t m, uint8_t* __restrict__ row) {
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < m; i += gridDim.x * blockDim.x) row[i] = (uint8_t)top[i];
+}
+
+__global__ void k_hanf_fill_bits(uint64_t* __restrict__ w, uint64_t nwords, uint32_t V) {
+  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < nwords; i += (uint64_t)gridDim.x * blockDim.x) {
+    const uint64_t lo = i * 64;
+    w[i] = lo + 64 <= V ? ~0ull : (lo < V ? (1ull << (V - lo)) - 1ull : 0ull);
+  }
+}
+
+// vertices of the wave-per-vertex pass: lo <= in-degree <= HANF_HUB_DEG
+__global__ __launch_bounds__(256) void k_hanf_mid_bits(const uint64_t* __restrict__ ptr, uint32_t V, uint64_t nwords,
+                                                       uint64_t lo, uint64_t* __restrict__ bits) {
+  const int lane = threadIdx.x & 63;
+  for (uint64_t word = grid_wave_id(); word < nwords; word += grid_waves()) {
+    const uint64_t v = word * 64 + lane;
+    bool in = false;
+    if (v < V) {
+      const uint64_t d = ptr[v + 1] - ptr[v];
+      in = d >= lo && d <= HANF_HUB_DEG;
+    }
+    const uint64_t m = __ballot(in);
+    if (lane == 0) bits[word] = m;
+  }
+}
+
+// One byte per vertex: bit 0, its row changed in the last pull; bit 1, it has reached the bound.
+static constexpr uint8_t HANF_CHANGED = 1, HANF_DONE = 2;
+
+// The changed marks as a bitmap, and whether there is any.
+__global__ __launch_bounds__(256) void k_hanf_bits(const uint64_t* __restrict__ bytes, uint64_t nwords,
+                                                   uint64_t* __restrict__ bits, unsigned long long* __restrict__ any) {
+  const int lane = threadIdx.x & 63;
+  const uint64_t n = nwords * 8;
+  bool got = false;
+  for (uint64_t base = grid_wave_id() * 64; base < n; base += grid_waves() * 64) {
+    const uint64_t i = base + lane;
+    const uint64_t w = i < n ? bytes[i] & 0x0101010101010101ull : 0ull;
+    uint64_t b = ((w * 0x0102040810204080ull) >> 56) << ((lane & 7) * 8);  // byte j's mark -> bit j
+    for (int off = 4; off > 0; off >>= 1) b |= __shfl_xor(b, off, 64);
+    if (i < n && (lane & 7) == 0) bits[i >> 3] = b;
+    got |= w != 0;
+  }
+  if (__ballot(got) && lane == 0) *any = 1ull;
+}
+
+// Max over the rows of the changed in-neighbours in [b, e) (words c0.. of each row), folded
+// over the wave's 64 / LPR row slots: every lane gets its 16 registers.  Returns whether there
+// was any.  The ids come 64 at a time, one per lane; the changed ones are packed to the front
+// with one forward permute, so that every row load of the wave is full.  A slot that reaches
+// the bound row's words (bound) ends the walk.
+template <int LPR>
+__device__ __forceinline__ bool hanf_range(uint64_t b, uint64_t e, const uint32_t* __restrict__ row_idx,
+                                           const uint64_t* __restrict__ changed, const uint4* __restrict__ cur,
+                                           uint64_t wpr4, uint64_t c0, const uint4& bound, uint4* out) {
+  constexpr int S = 64 / LPR, U = S * HANF_U > 64 ? 64 / S : HANF_U;
+  const int lane = threadIdx.x & 63, slot = lane / LPR, w = lane % LPR;
+  const uint64_t below = (1ull << lane) - 1ull;
+  row_max acc;
+  bool any = false;
+  for (uint64_t k0 = b; k0 < e; k0 += 64) {
+    uint32_t u = 0;
+    bool on = false;
+    if (k0 + lane < e) {
+      u = row_idx[k0 + lane];
+      on = (changed[u >> 6] >> (u & 63)) & 1ull;
+    }
+    const uint64_t m = __ballot(on);
+    const uint32_t n = (uint32_t)__popcll(m);
+    if (n == 0) continue;
+    any = true;
+    const uint32_t to = on ? (uint32_t)__popcll(m & below) : n + (uint32_t)__popcll(~m & below);
+    const uint32_t id = (uint32_t)__builtin_amdgcn_ds_permute((int)(to << 2), (int)u);
+    for (uint32_t t = 0; t < n; t += S * U) {
+      uint4 r[U];
+#pragma unroll
+      for (int i = 0; i < U; ++i) {
+        const uint32_t k = t + (uint32_t)(i * S + slot);
+        const uint32_t x = (uint32_t)__shfl((int)id, (int)(k & 63u), 64);
+        r[i] = k < n ? cur[(uint64_t)x * wpr4 + c0 + w] : make_uint4(0, 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < U; ++i) acc.add(r[i]);
+    }
+    if (full_groups<LPR>(__ballot(!row_differs(acc.row(), bound)))) break;
+  }
+  uint4 r = acc.row();
+  if (any)
+    for (int off = LPR; off < 64; off <<= 1) r = row_max2(r, row_shfl_xor(r, off));
+  *out = r;
+  return any;
+}
+
+// A vertex's row is written to the next buffer when it changes now, or when it changed last
+// time (the next buffer then still holds the row before that).
+template <int LPR>
+__global__ __launch_bounds__(256) void k_hanf_pull_wave(const uint64_t* __restrict__ col_ptr,
+                                                        const uint32_t* __restrict__ row_idx,
+                                                        const uint32_t* __restrict__ queue,
+                                                        const unsigned long long* __restrict__ nq, uint64_t wpr4,
+                                                        const uint64_t* __restrict__ changed,
+                                                        const uint4* __restrict__ bound_row,
+                                                        const uint4* __restrict__ cur, uint4* __restrict__ nxt,
+                                                        uint8_t* __restrict__ marks) {
+  const int lane = threadIdx.x & 63, w = lane % LPR;
+  const uint64_t n = *nq, nwaves = grid_waves();
+  for (uint64_t q = grid_wave_id(); q < n; q += nwaves) {
+    const uint32_t v = queue[q];
+    const uint8_t was = marks[v];
+    if (was == HANF_DONE) continue;  // done, and in both buffers
+    const uint64_t b = col_ptr[v], e = (was & HANF_DONE) ? b : col_ptr[v + 1];
+    const bool stale = (changed[v >> 6] >> (v & 63)) & 1ull;
+    bool mark = false, done = true;
+    for (uint64_t c0 = 0; c0 < wpr4; c0 += LPR) {
+      const uint4 bound = bound_row[c0 + w];
+      uint4 r;
+      const bool any = hanf_range<LPR>(b, e, row_idx, changed, cur, wpr4, c0, bound, &r);
+      if (!any && !stale) {
+        done = false;  // as it was: not done
+        continue;
+      }
+      const uint64_t at = (uint64_t)v * wpr4 + c0 + w;
+      const uint4 own = cur[at];
+      const uint4 now = row_max2(own, r);
+      const bool diff = __ballot(row_differs(own, now)) != 0ull;
+      mark |= diff;
+      done &= __ballot(row_differs(now, row_max2(now, bound))) == 0ull;
+      if ((diff || stale) && lane < LPR) nxt[at] = now;
+    }
+    if (lane == 0) marks[v] = (uint8_t)((mark ? HANF_CHANGED : 0) | (done ? HANF_DONE : 0));
+  }
+}
+
+// A group of LPR lanes per vertex of fewer than HANF_LOW_DEG in-edges, 64 / LPR vertices per
+// wave step, LPR in-edges of each at a time (an id per lane), so that the vertices' short
+// chains of dependent loads overlap.
+template <int LPR>
+__global__ __launch_bounds__(256) void k_hanf_pull_low(const uint64_t* __restrict__ col_ptr,
+                                                       const uint32_t* __restrict__ row_idx, uint32_t V,
+                                                       const uint64_t* __restrict__ changed,
+                                                       const uint4* __restrict__ bound_row,
+                                                       const uint4* __restrict__ cur, uint4* __restrict__ nxt,
+                                                       uint8_t* __restrict__ marks) {
+  constexpr int G = 64 / LPR, U = LPR < HANF_U ? LPR : HANF_U;
+  const int lane = threadIdx.x & 63, grp = lane / LPR, w = lane % LPR, g0 = grp * LPR;
+  const uint64_t nwaves = grid_waves();
+  const uint4 bound = bound_row[w];
+  for (uint64_t v0 = grid_wave_id() * G; v0 < V; v0 += nwaves * G) {
     const uint64_t v = v0 + grp;
     uint64_t b = 0, e = 0;
-    bool mine = false;
+    bool mine = false, stale = false;
+    uint8_t was = 0;
     if (v < V) {
+      was = marks[v];
       b = col_ptr[v];
       e = col_ptr[v + 1];
-      mine = e - b < max_deg;
+      mine = e - b < HANF_LOW_DEG && was != HANF_DONE;  // done, and in both buffers
+      stale = (changed[v >> 6] >> (v & 63)) & 1ull;
     }
-    if (!mine) e = b;
-    uint32_t acc = mine ? cur[v * WPR + w] : 0u;
-    // the wave steps until its longest list is done
-    uint64_t len = e - b;
-    for (int off = WPR; off < 64; off <<= 1) len = std::max<uint64_t>(len, (uint64_t)__shfl_xor((long long)len, off, 64));
-    for (uint64_t k0 = 0; k0 < len; k0 += U) {
-      uint32_t val[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const uint64_t k = b + k0 + u;
-        val[u] = k < e ? cur[(uint64_t)row_idx[k] * WPR + w] : 0u;
+    if (!mine || (was & HANF_DONE)) e = b;
+    row_max acc;
+    bool any = false;
+    for (uint64_t k0 = b; __ballot(k0 < e) != 0ull; k0 += LPR) {  // until the wave's longest list is done
+      uint32_t u = 0;
+      bool on = false;
+      if (k0 + w < e) {
+        u = row_idx[k0 + w];
+        on = (changed[u >> 6] >> (u & 63)) & 1ull;
       }
+      const uint64_t m = (__ballot(on) >> g0) & (LPR == 64 ? ~0ull : (1ull << LPR) - 1ull);  // the group's
+      any |= m != 0ull;
 #pragma unroll
-      for (int u = 0; u < U; ++u) acc = byte_max4(acc, val[u]);
+      for (int t = 0; t < LPR; t += U) {
+        uint4 r[U];
+#pragma unroll
+        for (int i = 0; i < U; ++i) {
+          const uint32_t x = (uint32_t)__shfl((int)u, g0 + t + i, 64);
+          r[i] = (m >> (t + i)) & 1ull ? cur[(uint64_t)x * LPR + w] : make_uint4(0, 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < U; ++i) acc.add(r[i]);
+      }
+      const uint64_t full = full_groups<LPR>(__ballot(!row_differs(acc.row(), bound)));
+      if ((full >> g0) & 1ull) e = b;  // at the bound: nothing left to gain
     }
-    if (mine) nxt[v * WPR + w] = acc;
+    bool diff = false, below = true;
+    if (mine && (any || stale)) {
+      const uint4 own = cur[v * LPR + w];
+      const uint4 now = row_max2(own, acc.row());
+      diff = row_differs(own, now);
+      below = row_differs(now, row_max2(now, bound));
+      if (diff || stale) nxt[v * LPR + w] = now;
+    }
+    const uint64_t dm = (__ballot(diff) >> g0) & (LPR == 64 ? ~0ull : (1ull << LPR) - 1ull);
+    // a lane whose own registers stay still writes them when others of the row change
+    if (dm && !diff && !stale) nxt[v * LPR + w] = cur[v * LPR + w];
+    const uint64_t bm = (__ballot(below) >> g0) & (LPR == 64 ? ~0ull : (1ull << LPR) - 1ull);
+    if (mine && w == 0) marks[v] = (uint8_t)((dm ? HANF_CHANGED : 0) | (bm ? 0 : HANF_DONE));
   }
 }
 
-// Pull with W 32-bit words (4 W registers) per lane and chunk, P >= 8: a counter row
-// of `row` words is handled in chunks of 64 W words (larger counters walk the in-edges
-// once per chunk), U in-edges in flight.
-template <int W, int U>
-__global__ __launch_bounds__(256) void k_hanf_pull_words(const uint64_t* __restrict__ col_ptr,
-                                                         const uint32_t* __restrict__ row_idx, uint32_t V,
-                                                         uint64_t row, const uint32_t* __restrict__ cur,
-                                                         uint32_t* __restrict__ nxt) {
+// The hubs' own rows, before their in-edges.
+__global__ __launch_bounds__(256) void k_hanf_hub_rows(const uint32_t* __restrict__ hubs,
+                                                       const unsigned long long* __restrict__ nhub, uint64_t wpr4,
+                                                       const uint4* __restrict__ bound_row,
+                                                       const uint4* __restrict__ cur, uint4* __restrict__ nxt,
+                                                       uint8_t* __restrict__ marks) {
   const int lane = threadIdx.x & 63;
-  const uint64_t wave_id = grid_wave_id(), nwaves = grid_waves();
-  for (uint64_t v = wave_id; v < V; v += nwaves) {
-    const uint64_t b = col_ptr[v], e = col_ptr[v + 1];
-    if (e - b > HANF_HUB_DEG) {  // a hub: its own row now, its in-edges in k_hanf_pull_hubs
-      for (uint64_t i = lane; i < row; i += 64) nxt[v * row + i] = cur[v * row + i];
-      continue;
+  const uint64_t n = *nhub, nwaves = grid_waves();
+  for (uint64_t h = grid_wave_id(); h < n; h += nwaves) {
+    const uint64_t v = hubs[h];
+    bool below = false;
+    for (uint64_t i = lane; i < wpr4; i += 64) {
+      const uint4 own = cur[v * wpr4 + i];
+      below |= row_differs(own, row_max2(own, bound_row[i]));
+      nxt[v * wpr4 + i] = own;
     }
-    for (uint64_t c0 = 0; c0 < row; c0 += 64 * W) {
-      uint32_t acc[W];
-#pragma unroll
-      for (int j = 0; j < W; ++j) acc[j] = cur[v * row + c0 + (uint64_t)j * 64 + lane];
-      for (uint64_t k0 = b; k0 < e; k0 += U) {
-        uint32_t val[U][W];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const bool ok = k0 + u < e;
-          const uint64_t urow = ok ? (uint64_t)row_idx[k0 + u] * row + c0 : 0;
-#pragma unroll
-          for (int j = 0; j < W; ++j) val[u][j] = ok ? cur[urow + (uint64_t)j * 64 + lane] : 0u;
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-          for (int j = 0; j < W; ++j) acc[j] = byte_max4(acc[j], val[u][j]);
-      }
-#pragma unroll
-      for (int j = 0; j < W; ++j) nxt[v * row + c0 + (uint64_t)j * 64 + lane] = acc[j];
-    }
+    const bool done = __ballot(below) == 0ull;
+    if (lane == 0) marks[v] = done ? HANF_DONE : 0;
   }
 }
 
 // Register-wise max of x into *p (a compare-and-swap loop: every retry sees a word that
-// only grew, so it ends).
-__device__ __forceinline__ void byte_max_merge(uint32_t* p, uint32_t x) {
+// only grew, so it ends); whether *p grew.
+__device__ __forceinline__ bool byte_max_merge(uint32_t* p, uint32_t x) {
   uint32_t old = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   for (;;) {
     const uint32_t nv = byte_max4(old, x);
-    if (nv == old) return;
+    if (nv == old) return false;
     const uint32_t prev = atomicCAS(p, old, nv);
-    if (prev == old) return;
+    if (prev == old) return true;
     old = prev;
   }
 }
 
-// Hub in-edges, one chunk per wave at a time: the chunk's register-wise max (rows of
-// wpr words; up to 64 words: 64 / wpr in-edges per step, larger rows 64 words per step
-// with the in-edges walked once per 64-word block) merged into the hub's next row.
+// Hub in-edges, one chunk per wave at a time, the chunk's max merged into the hub's next row.
+template <int LPR>
 __global__ __launch_bounds__(256) void k_hanf_pull_hubs(const uint64_t* __restrict__ col_ptr,
                                                         const uint32_t* __restrict__ row_idx,
                                                         const uint32_t* __restrict__ hubs,
                                                         const unsigned long long* __restrict__ nhub,
-                                                        const uint64_t* __restrict__ start, uint64_t wpr,
-                                                        const uint32_t* __restrict__ cur, uint32_t* __restrict__ nxt) {
+                                                        const uint64_t* __restrict__ start, uint64_t wpr4,
+                                                        const uint64_t* __restrict__ changed,
+                                                        const uint4* __restrict__ bound_row,
+                                                        const uint4* __restrict__ cur, uint4* __restrict__ nxt,
+                                                        uint8_t* __restrict__ marks) {
   const int lane = threadIdx.x & 63;
-  const uint64_t wave_id = grid_wave_id(), nwaves = grid_waves();
+  const uint64_t nwaves = grid_waves();
   const uint64_t n = *nhub;
   if (n == 0) return;
   const uint64_t total = start[n];
-  for (uint64_t c = wave_id; c < total; c += nwaves) {
+  for (uint64_t c = grid_wave_id(); c < total; c += nwaves) {
     uint64_t k0, k1;
     const uint32_t v = hub_chunk(col_ptr, hubs, start, n, HANF_HUB_CHUNK, c, &k0, &k1);
-    if (wpr <= 64) {
-      const uint64_t eps = 64 / wpr, slot = (uint64_t)lane / wpr, w = (uint64_t)lane % wpr;
-      uint32_t acc = 0;
-      for (uint64_t k = k0 + slot; k < k1; k += eps * HANF_HUB_U) {
-        uint32_t val[HANF_HUB_U];
-#pragma unroll
-        for (int u = 0; u < HANF_HUB_U; ++u) {
-          const uint64_t kk = k + (uint64_t)u * eps;
-          val[u] = kk < k1 ? cur[(uint64_t)row_idx[kk] * wpr + w] : 0u;
-        }
-#pragma unroll
-        for (int u = 0; u < HANF_HUB_U; ++u) acc = byte_max4(acc, val[u]);
-      }
-      for (uint64_t off = wpr; off < 64; off <<= 1) acc = byte_max4(acc, (uint32_t)__shfl_xor(acc, (int)off, 64));
-      if (slot == 0) byte_max_merge(&nxt[(uint64_t)v * wpr + w], acc);
-    } else {
-      for (uint64_t cw = lane; cw < wpr; cw += 64) {
-        uint32_t acc = 0;
-        for (uint64_t k = k0; k < k1; ++k) acc = byte_max4(acc, cur[(uint64_t)row_idx[k] * wpr + cw]);
-        byte_max_merge(&nxt[(uint64_t)v * wpr + cw], acc);
+    if (marks[v] & HANF_DONE) continue;  // uniform
+    for (uint64_t c0 = 0; c0 < wpr4; c0 += LPR) {
+      uint4 r;
+      if (!hanf_range<LPR>(k0, k1, row_idx, changed, cur, wpr4, c0, bound_row[c0 + lane % LPR], &r)) continue;
+      if (lane < LPR) {
+        uint32_t* p = reinterpret_cast<uint32_t*>(nxt + (uint64_t)v * wpr4 + c0 + lane);
+        const bool grew = byte_max_merge(p, r.x) | byte_max_merge(p + 1, r.y) | byte_max_merge(p + 2, r.z) |
+                          byte_max_merge(p + 3, r.w);
+        if (grew) marks[v] = HANF_CHANGED;
       }
     }
   }
@@ -278,9 +467,11 @@ __device__ __forceinline__ double hanf_alpha(int P) {
 
 // Estimates of counters of at most 1024 registers, summed per block in a fixed order:
 // m / 16 lanes per counter (16 registers each, one 16-byte load), 1024 / m counters per
-// wave step, so a wave keeps many counters' loads in flight instead of one.
+// wave step, so a wave keeps many counters' loads in flight instead of one.  Only changed
+// counters are read; the others' estimates are kept in est.
 __global__ __launch_bounds__(256) void k_hanf_estimate_rows(const uint8_t* __restrict__ regs, uint32_t V, int P,
-                                                            double* __restrict__ part) {
+                                                            const uint64_t* __restrict__ changed,
+                                                            double* __restrict__ est, double* __restrict__ part) {
   __shared__ double s_w[4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t m = 1u << P, L = m / 16, sub = (uint32_t)lane % L, slot = (uint32_t)lane / L, per = 64 / L;
@@ -291,7 +482,8 @@ __global__ __launch_bounds__(256) void k_hanf_estimate_rows(const uint8_t* __res
     const uint64_t v = v0 + slot;
     double s = 0.0;
     uint32_t zeros = 0;
-    if (v < V) {
+    const bool on = v < V && ((changed[v >> 6] >> (v & 63)) & 1ull);
+    if (on) {
       const uint4 q = *reinterpret_cast<const uint4*>(regs + v * m + (uint64_t)sub * 16);
       const uint32_t w4[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
@@ -307,7 +499,12 @@ __global__ __launch_bounds__(256) void k_hanf_estimate_rows(const uint8_t* __res
       s += __shfl_xor(s, (int)off, 64);
       zeros += (uint32_t)__shfl_xor((int)zeros, (int)off, 64);
     }
-    if (v < V && sub == 0) total += hanf_estimate(alpha, (double)m, s, zeros);
+    if (v < V && sub == 0) {
+      double x;
+      if (on) est[v] = x = hanf_estimate(alpha, (double)m, s, zeros);
+      else x = est[v];
+      total += x;
+    }
   }
   for (int off = 32; off > 0; off >>= 1) total += __shfl_down(total, off, 64);
   if (lane == 0) s_w[wave] = total;
@@ -319,7 +516,8 @@ __global__ __launch_bounds__(256) void k_hanf_estimate_rows(const uint8_t* __res
 // summed per block in a fixed order.
 // The register sum of 2^-reg is exact in FP64 (at most 2^16 terms of 2^-k, k <= 27).
 __global__ __launch_bounds__(256) void k_hanf_estimate(const uint8_t* __restrict__ regs, uint32_t V, int P,
-                                                       double* __restrict__ part) {
+                                                       const uint64_t* __restrict__ changed,
+                                                       double* __restrict__ est, double* __restrict__ part) {
   __shared__ double s_w[4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint64_t m = 1ull << P;
@@ -327,6 +525,10 @@ __global__ __launch_bounds__(256) void k_hanf_estimate(const uint8_t* __restrict
   const double alpha = hanf_alpha(P);
   double total = 0.0;  // lane 0's running sum over this wave's vertices, in order
   for (uint64_t v = wave_id; v < V; v += nwaves) {
+    if (!((changed[v >> 6] >> (v & 63)) & 1ull)) {  // uniform
+      total += est[v];
+      continue;
+    }
     double s = 0.0;
     uint32_t zeros = 0;
     for (uint64_t i = lane; i < m; i += 64) {
@@ -338,7 +540,9 @@ __global__ __launch_bounds__(256) void k_hanf_estimate(const uint8_t* __restrict
       s += __shfl_xor(s, off, 64);
       zeros += __shfl_xor(zeros, off, 64);
     }
-    total += hanf_estimate(alpha, (double)m, s, zeros);
+    const double x = hanf_estimate(alpha, (double)m, s, zeros);
+    if (lane == 0) est[v] = x;
+    total += x;
   }
   if (lane == 0) s_w[wave] = total;
   __syncthreads();
@@ -376,17 +580,6 @@ __global__ __launch_bounds__(256) void k_nstep_degree(const uint8_t* __restrict_
   }
 }
 
-// Any word of a differs from b: *flag = 1.
-__global__ void k_rows_differ(const uint32_t* __restrict__ a, const uint32_t* __restrict__ b, uint64_t n,
-                              unsigned int* __restrict__ flag) {
-  bool d = false;
-  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-    d |= a[i] != b[i];
-  if (__ballot(d) && (threadIdx.x & 63) == 0) *flag = 1u;
-}
-
-__global__ void k_flag_zero(unsigned int* f) { *f = 0u; }
-
 // counters in input-id order
 __global__ void k_hanf_rows_external(const uint8_t* __restrict__ in, const uint32_t* __restrict__ rank_of,
                                      uint32_t V, uint64_t m, uint8_t* __restrict__ out) {
@@ -401,33 +594,75 @@ __global__ void k_hanf_rows_external(const uint8_t* __restrict__ in, const uint3
 
 using namespace pe;
 
-// One HyperANF pull over the adjacency (ptr, idx): nxt[v] = register-wise max of cur[v]
-// and cur[u] over the adjacency of v.  hubs: the adjacency's hub table.
-static void hanf_pull(pe_ctx_s* ctx, const uint64_t* ptr, const uint32_t* idx, uint32_t V, int P, hub_table& hubs,
-                      const uint8_t* cur, uint8_t* nxt, unsigned grid) {
-  hipStream_t s = ctx->stream;
-  const uint64_t m = 1ull << P;
-  switch (P) {
-    case 6:
-      k_hanf_pull_lowdeg<16, 4><<<grid, 256, 0, s>>>(ptr, idx, V, HANF_LOW_DEG, (const uint32_t*)cur, (uint32_t*)nxt);
-      k_hanf_pull_small<4, 8><<<grid, 256, 0, s>>>(ptr, idx, V, HANF_LOW_DEG, (const uint32_t*)cur, (uint32_t*)nxt);
-      break;
-    case 7:
-      k_hanf_pull_lowdeg<32, 4><<<grid, 256, 0, s>>>(ptr, idx, V, HANF_LOW_DEG, (const uint32_t*)cur, (uint32_t*)nxt);
-      k_hanf_pull_small<2, 4><<<grid, 256, 0, s>>>(ptr, idx, V, HANF_LOW_DEG, (const uint32_t*)cur, (uint32_t*)nxt);
-      break;
-#define HANF_W(PP, W, U)                                                                                 \
-  case PP:                                                                                               \
-    k_hanf_pull_words<W, U><<<grid, 256, 0, s>>>(ptr, idx, V, m / 4, (const uint32_t*)cur, (uint32_t*)nxt); \
-    break;
-    HANF_W(8, 1, 8) HANF_W(9, 2, 4) HANF_W(10, 4, 4) HANF_W(11, 8, 2) HANF_W(12, 16, 2) HANF_W(13, 16, 2)
-    HANF_W(14, 16, 2) HANF_W(15, 16, 2) HANF_W(16, 16, 2)
-#undef HANF_W
+// The pull over one adjacency (ptr, idx): its passes' vertex lists and the changed rows.
+struct hanf_pull {
+  pe_ctx_s* ctx;
+  const uint64_t* ptr;
+  const uint32_t* idx;
+  uint32_t V;
+  int P;
+  uint64_t nwords;
+  hub_table hubs;
+  dbuf<uint32_t> mid;             // vertices of the wave pass
+  dbuf<unsigned long long> nmid;  // [0] their number, [1] whether the last pull changed a row
+  dbuf<uint64_t> changed;         // rows that the last pull changed (all before the first)
+  dbuf<uint64_t> marks;           // HANF_CHANGED and HANF_DONE bytes
+  dbuf<uint32_t> top;             // the bound row, a word per register
+  dbuf<uint8_t> bound;            // the bound row
+  unsigned grid;
+
+  // od (out-degrees over this adjacency's entries) or, without it, src_ptr tells which vertices
+  // some other vertex pulls from: those with od > 0, or with entries in src_ptr
+  hanf_pull(pe_ctx_s* c, const uint64_t* p, const uint32_t* i, uint32_t v, uint64_t nnz, int bits, const uint32_t* perm,
+            const uint32_t* od, const uint64_t* src_ptr)
+      : ctx(c), ptr(p), idx(i), V(v), P(bits), nwords(((uint64_t)v >> 6) + 1), mid(c, std::max<uint32_t>(1, v)),
+        nmid(c, 2), changed(c, nwords), marks(c, nwords * 8), top(c, 1ull << bits), bound(c, 1ull << bits) {
+    hipStream_t s = ctx->stream;
+    k_hanf_zero<<<64, 256, 0, s>>>(top.p, 1ull << P);
+    k_hanf_bound<<<persistent_grid(ctx, grid_for(V, 256), 4), 256, 0, s>>>(V, P, perm, od, src_ptr, top.p);
+    k_hanf_bound_row<<<64, 256, 0, s>>>(top.p, 1u << P, bound.p);
+    hub_table_build(ctx, ptr, V, nnz, HANF_HUB_DEG, HANF_HUB_CHUNK, hubs);
+    // rows of 64 lanes and more have no group pass: the wave pass takes every shorter list
+    k_hanf_zero<<<1, 64, 0, s>>>(reinterpret_cast<uint32_t*>(nmid.p), 4);
+    k_hanf_mid_bits<<<grid_for(nwords, 4, 8192), 256, 0, s>>>(ptr, V, nwords, P < 10 ? HANF_LOW_DEG : 0, changed.p);
+    frontier_compact(ctx, changed.p, nwords, V, mid.p, nmid.p);
+    k_hanf_fill_bits<<<grid_for(nwords, 256, 4096), 256, 0, s>>>(changed.p, nwords, V);
+    k_hanf_zero<<<grid_for(nwords * 16, 256, 8192), 256, 0, s>>>(reinterpret_cast<uint32_t*>(marks.p), nwords * 16);
+    PE_HIP(hipGetLastError());
+    grid = persistent_grid(ctx, grid_for(V, 4), 8);
   }
-  k_hanf_pull_hubs<<<grid, 256, 0, s>>>(ptr, idx, hubs.hubs.p, hubs.count.p, hubs.start.p, m / 4,
-                                        (const uint32_t*)cur, (uint32_t*)nxt);
-  PE_HIP(hipGetLastError());
-}
+
+  template <int LPR>
+  void launch(const uint4* cur, uint4* nxt) {
+    hipStream_t s = ctx->stream;
+    const uint64_t wpr4 = (1ull << P) / 16;
+    uint8_t* mk = reinterpret_cast<uint8_t*>(marks.p);
+    const uint4* br = reinterpret_cast<const uint4*>(bound.p);
+    if constexpr (LPR < 64) k_hanf_pull_low<LPR><<<grid, 256, 0, s>>>(ptr, idx, V, changed.p, br, cur, nxt, mk);
+    k_hanf_pull_wave<LPR><<<grid, 256, 0, s>>>(ptr, idx, mid.p, nmid.p, wpr4, changed.p, br, cur, nxt, mk);
+    k_hanf_hub_rows<<<grid_for(hubs.max_hubs, 4, 1024), 256, 0, s>>>(hubs.hubs.p, hubs.count.p, wpr4, br, cur, nxt, mk);
+    k_hanf_pull_hubs<LPR><<<grid, 256, 0, s>>>(ptr, idx, hubs.hubs.p, hubs.count.p, hubs.start.p, wpr4, changed.p, br,
+                                               cur, nxt, mk);
+  }
+
+  // nxt[v] = register-wise max of cur[v] and cur[u] over the adjacency of v; nxt holds the
+  // rows before the last pull (anything before the first)
+  void pull(const uint8_t* cur, uint8_t* nxt) {
+    const uint4* c = reinterpret_cast<const uint4*>(cur);
+    uint4* n = reinterpret_cast<uint4*>(nxt);
+    switch (P) {
+      case 6: launch<4>(c, n); break;
+      case 7: launch<8>(c, n); break;
+      case 8: launch<16>(c, n); break;
+      case 9: launch<32>(c, n); break;
+      default: launch<64>(c, n);
+    }
+    hipStream_t s = ctx->stream;
+    k_hanf_zero<<<1, 64, 0, s>>>(reinterpret_cast<uint32_t*>(nmid.p + 1), 2);
+    k_hanf_bits<<<grid_for(nwords * 8, 256, 1024), 256, 0, s>>>(marks.p, nwords, changed.p, nmid.p + 1);
+    PE_HIP(hipGetLastError());
+  }
+};
 
 extern "C" int pe_hyperanf(pe_graph_t* g, const pe_hyperanf_opts_t* opts, double* anfs, uint32_t cap,
                            uint32_t* nanfs, double* avg_distance, uint8_t* registers, double* seconds) {
@@ -443,14 +678,15 @@ extern "C" int pe_hyperanf(pe_graph_t* g, const pe_hyperanf_opts_t* opts, double
     const unsigned est_grid = persistent_grid(ctx, grid_for(V, 4), 4);
     dbuf<double> part(ctx, est_grid);
     std::vector<double> hpart(est_grid);
-    const unsigned pull_grid = persistent_grid(ctx, grid_for(V, 4), 8);
     const uint32_t* perm = g->relabeled ? g->perm.p : nullptr;
-    hub_table hubs;
+    dbuf<double> est(ctx, std::max<uint32_t>(1, V));
+    PE_HIP(hipEventRecord(ctx->t0, s));
+    hanf_pull pulls(ctx, g->col_ptr.p, g->row_idx.p, V, g->nnz, P, perm, g->od.p, nullptr);
     auto anf_of = [&](const uint8_t* regs) {
       if (P <= 10)
-        k_hanf_estimate_rows<<<est_grid, 256, 0, s>>>(regs, V, P, part.p);
+        k_hanf_estimate_rows<<<est_grid, 256, 0, s>>>(regs, V, P, pulls.changed.p, est.p, part.p);
       else
-        k_hanf_estimate<<<est_grid, 256, 0, s>>>(regs, V, P, part.p);
+        k_hanf_estimate<<<est_grid, 256, 0, s>>>(regs, V, P, pulls.changed.p, est.p, part.p);
       PE_HIP(hipGetLastError());
       PE_HIP(hipMemcpyAsync(hpart.data(), part.p, est_grid * sizeof(double), hipMemcpyDeviceToHost, s));
       PE_HIP(hipStreamSynchronize(s));
@@ -458,11 +694,6 @@ extern "C" int pe_hyperanf(pe_graph_t* g, const pe_hyperanf_opts_t* opts, double
       for (double x : hpart) t += x;
       return t;
     };
-    auto pull = [&](const uint8_t* cur, uint8_t* nxt) {
-      hanf_pull(ctx, g->col_ptr.p, g->row_idx.p, V, P, hubs, cur, nxt, pull_grid);
-    };
-    PE_HIP(hipEventRecord(ctx->t0, s));
-    hub_table_build(ctx, g->col_ptr.p, V, g->nnz, HANF_HUB_DEG, HANF_HUB_CHUNK, hubs);
     k_hanf_zero<<<grid_for(bytes / 4, 256, 65536), 256, 0, s>>>((uint32_t*)a.p, bytes / 4);
     k_hanf_init<<<grid_for(V, 256, 8192), 256, 0, s>>>(a.p, V, P, perm);
     PE_HIP(hipGetLastError());
@@ -472,7 +703,7 @@ extern "C" int pe_hyperanf(pe_graph_t* g, const pe_hyperanf_opts_t* opts, double
     uint8_t* cur = a.p;
     uint8_t* nxt = b.p;
     for (uint32_t it = 0; it < opts->iterations; ++it) {
-      pull(cur, nxt);
+      pulls.pull(cur, nxt);
       const double anf = anf_of(nxt);
       std::swap(cur, nxt);
       if (anf - last < DBL_EPSILON) break;  // hyperanf.hpp:189-191
@@ -526,27 +757,22 @@ extern "C" int pe_nstep_degrees(pe_graph_t* g, const uint64_t* target_words, uin
     }
     dbuf<uint8_t> a(ctx, bytes), b(ctx, bytes);
     dbuf<uint32_t> dev_deg(ctx, std::max<uint32_t>(1, V));
-    dbuf<unsigned int> flag(ctx, 1);
     const unsigned grid = persistent_grid(ctx, grid_for(V, 4), 8);
     PE_HIP(hipEventRecord(ctx->t0, s));
     // one pass per direction: the in pass gathers over in-edges (the reference's
     // propagate on the forward engine), the out pass over out-edges (on the reversed one)
-    auto pass = [&](const uint64_t* ptr, const uint32_t* idx, uint32_t* host_out) {
-      hub_table hubs;
-      hub_table_build(ctx, ptr, V, g->nnz, HANF_HUB_DEG, HANF_HUB_CHUNK, hubs);
+    auto pass = [&](const uint64_t* ptr, const uint32_t* idx, const uint32_t* od, const uint64_t* src_ptr,
+                    uint32_t* host_out) {
+      hanf_pull pulls(ctx, ptr, idx, V, g->nnz, P, perm, od, src_ptr);
       k_hanf_zero<<<grid_for(bytes / 4, 256, 65536), 256, 0, s>>>((uint32_t*)a.p, bytes / 4);
       k_hanf_init<<<grid_for(V, 256, 8192), 256, 0, s>>>(a.p, V, P, perm);
       PE_HIP(hipGetLastError());
       uint8_t* cur = a.p;
       uint8_t* nxt = b.p;
       for (uint32_t it = 0; it < step; ++it) {  // nstepdegrees.hpp:343-409
-        hanf_pull(ctx, ptr, idx, V, P, hubs, cur, nxt, grid);
-        k_flag_zero<<<1, 1, 0, s>>>(flag.p);
-        k_rows_differ<<<grid_for(bytes / 4, 256, 8192), 256, 0, s>>>((const uint32_t*)cur, (const uint32_t*)nxt,
-                                                                     bytes / 4, flag.p);
-        PE_HIP(hipGetLastError());
-        unsigned int changed = 0;
-        PE_HIP(hipMemcpyAsync(&changed, flag.p, 4, hipMemcpyDeviceToHost, s));
+        pulls.pull(cur, nxt);
+        unsigned long long changed = 0;
+        PE_HIP(hipMemcpyAsync(&changed, pulls.nmid.p + 1, 8, hipMemcpyDeviceToHost, s));
         PE_HIP(hipStreamSynchronize(s));
         std::swap(cur, nxt);
         if (!changed) break;  // no book grew: further steps change nothing
@@ -555,13 +781,13 @@ extern "C" int pe_nstep_degrees(pe_graph_t* g, const uint64_t* target_words, uin
       PE_HIP(hipGetLastError());
       download_external(g, dev_deg.p, host_out, 4);
     };
-    if (type & PE_NSTEP_IN) pass(g->col_ptr.p, g->row_idx.p, in_degrees);
+    if (type & PE_NSTEP_IN) pass(g->col_ptr.p, g->row_idx.p, g->od.p, nullptr, in_degrees);
     if (type & PE_NSTEP_OUT) {
       if (!g->directed && (type & PE_NSTEP_IN)) {
         std::memcpy(out_degrees, in_degrees, (size_t)V * 4);  // undirected: out = in (nstepdegrees.hpp:456-463)
       } else {
         PE_REQUIRE(g->has_csr || g->csr_is_csc, PE_ERR_STATE, "the out pass needs out-edges (PE_GRAPH_BUILD_CSR)");
-        pass(g->csr_ptr(), g->csr_idx(), out_degrees);
+        pass(g->csr_ptr(), g->csr_idx(), nullptr, g->col_ptr.p, out_degrees);
       }
     }
     PE_HIP(hipEventRecord(ctx->t1, s));

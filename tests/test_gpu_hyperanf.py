@@ -55,3 +55,32 @@ def test_rmat(ctx, scale, bits, directed, relabel):
     g = Graph.rmat(ctx, scale, 8, seed=21, directed=directed, relabel=relabel)
     _run(g, oracle.CSC(1 << scale, s, d, symmetrize=not directed), bits, 20)
     g.close()
+
+
+@pytest.mark.parametrize("bits", [6, 7, 8, 9, 10, 11])
+def test_changed_rows_and_length_classes(ctx, bits):
+    """Vertices of 31, 32, 4096 and 4097 in-edges (the last and the first of each pass) and a
+    long path, along which few rows change per iteration while the rest stay as they are;
+    an odd number of vertices, directed and symmetrized, relabeled and not."""
+    from plato_amd import Graph
+    rng = np.random.default_rng(bits)
+    rim, tail = 5000, 37
+    s, d = [], []
+    for h, n in enumerate((31, 32, 4096, 4097)):
+        s.append(rng.choice(rim, n, replace=False))
+        d.append(np.full(n, rim + h))
+    s.append(rng.integers(0, rim, rim))
+    d.append(rng.integers(0, rim, rim))
+    path = np.arange(tail + 1) + rim + 3
+    s.append(path[:-1])
+    d.append(path[1:])
+    s, d = np.concatenate(s).astype(np.uint32), np.concatenate(d).astype(np.uint32)
+    V = rim + 4 + tail
+    for directed in (True, False):
+        og = oracle.CSC(V, s, d, symmetrize=not directed)
+        if directed:
+            assert np.diff(og.col_ptr)[rim:rim + 4].tolist() == [31, 32, 4096, 4097]
+        print(f"case: hyperanf length classes bits={bits} directed={directed}", flush=True)
+        g = Graph.from_edges(ctx, s, d, V, directed=directed, relabel=directed)
+        assert _run(g, og, bits, 60).anfs.size > 30
+        g.close()
