@@ -21,11 +21,10 @@
 // in-neighbours is not touched, and its estimate is kept.  No row of a vertex that someone
 // pulls from can pass the register-wise max over the first counters of all such vertices (the
 // bound row): a pull stops at the first row that reaches it, and a vertex that has reached it
-// is done.  The pull's bound is the random
-// 2^P-byte rows of the first iterations, then the in-edge lists.  RMAT scale 23
-// symmetrized, P = 6, 8 pulls: 5.2 ms each with one 4-byte word per lane and every row read;
-// here 3.4, 3.4 and 2.5 ms, then 0.8 falling to 0.15 ms (without the bound row 3.4 four times,
-// then 0.8); the whole call 44.7 -> 16.0 ms.
+// is done.  The pull's bound is the random 2^P-byte rows of the second and third iteration,
+// then the in-edge lists.  RMAT scale 23 symmetrized, P = 6, 8 pulls: 5.2 ms each with one 4-byte word per lane and every row read;
+// here 1.8, 3.4 and 2.5 ms, then 0.8 falling to 0.15 ms (without the bound row 3.4 until the
+// fourth, then 0.8); the whole call 44.7 -> 14.0 ms.
 // Three passes by in-degree: fewer than HANF_LOW_DEG, a group of LPR lanes per vertex; up to
 // HANF_HUB_DEG, a wave per vertex; the hubs' in-edges in chunks over all waves, each merging
 // its chunk's maximum into the hub's row, so no wave walks a hub alone.
@@ -72,11 +71,36 @@ __device__ __forceinline__ void hanf_first(uint32_t id, int P, uint32_t* reg, ui
   *rank = r < q + 1u ? r : q + 1u;
 }
 
+// Counters of at most 2^HANF_CODE_P registers start as a 16-bit code, register << 6 | rank:
+// the first pull reads 2 bytes per in-edge instead of a row that holds one register.
+static constexpr int HANF_CODE_P = 10;
+__global__ void k_hanf_codes(uint16_t* __restrict__ code, uint32_t V, int P, const uint32_t* __restrict__ perm) {
+  for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x) {
+    uint32_t reg, rank;
+    hanf_first(perm ? perm[v] : (uint32_t)v, P, &reg, &rank);  // counters hash input ids
+    code[v] = (uint16_t)(reg << 6 | rank);
+  }
+}
+
+// the 16 registers from 16 w on of a row that starts as `code`
+__device__ __forceinline__ uint4 hanf_code_row(uint32_t code, uint32_t w) {
+  const uint32_t reg = code >> 6, at = (reg >> 4) == w ? (reg >> 2) & 3u : 4u;
+  const uint32_t x = (code & 63u) << ((reg & 3u) * 8u);
+  return make_uint4(at == 0 ? x : 0u, at == 1 ? x : 0u, at == 2 ? x : 0u, at == 3 ? x : 0u);
+}
+
+__global__ void k_hanf_init_rows(uint4* __restrict__ rows, uint32_t V, uint32_t log_wpr4,
+                                 const uint16_t* __restrict__ code) {
+  const uint64_t n = (uint64_t)V << log_wpr4, mask = (1ull << log_wpr4) - 1ull;
+  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
+    rows[i] = hanf_code_row(code[i >> log_wpr4], (uint32_t)(i & mask));
+}
+
 __global__ void k_hanf_init(uint8_t* __restrict__ regs, uint32_t V, int P, const uint32_t* __restrict__ perm) {
   const uint64_t m = 1ull << P;
   for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x) {
     uint32_t reg, rank;
-    hanf_first(perm ? perm[v] : (uint32_t)v, P, &reg, &rank);  // counters hash input ids
+    hanf_first(perm ? perm[v] : (uint32_t)v, P, &reg, &rank);
     regs[v * m + reg] = (uint8_t)rank;
   }
 }
@@ -260,17 +284,58 @@ __device__ __forceinline__ bool hanf_range(uint64_t b, uint64_t e, const uint32_
   return any;
 }
 
+// The same for the first pull, from the codes: one LDS maximum per in-edge into the wave's
+// registers (s, one word each).  Making each row from its code in registers instead took
+// 1.36 ms for the wave pass at RMAT scale 23, reading the rows 1.97 ms, this 0.91 ms (hubs 0.97,
+// 0.62 and 0.51 ms).
+template <int LPR>
+__device__ __forceinline__ bool hanf_first_range(uint64_t b, uint64_t e, const uint32_t* __restrict__ row_idx,
+                                                 const uint16_t* __restrict__ code, uint32_t* s, uint4* out) {
+  constexpr uint32_t M = 16 * LPR;
+  constexpr int U = 4;
+  const uint32_t lane = threadIdx.x & 63, w = lane % LPR;
+#pragma unroll
+  for (uint32_t i = 0; i < M; i += 64) s[i + lane] = 0u;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  for (uint64_t k0 = b; k0 < e; k0 += 64 * U) {
+    uint32_t c[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) {
+      const uint64_t k = k0 + (uint64_t)i * 64 + lane;
+      c[i] = k < e ? (uint32_t)code[row_idx[k]] : 0u;  // rank 0: no effect
+    }
+#pragma unroll
+    for (int i = 0; i < U; ++i)
+      if (c[i]) atomicMax(&s[c[i] >> 6], c[i] & 63u);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  uint32_t r[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t* q = s + w * 16 + i * 4;
+    r[i] = q[0] | q[1] << 8 | q[2] << 16 | q[3] << 24;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();  // read before the wave's next vertex clears them
+  *out = make_uint4(r[0], r[1], r[2], r[3]);
+  return b < e;
+}
+
 // A vertex's row is written to the next buffer when it changes now, or when it changed last
 // time (the next buffer then still holds the row before that).
-template <int LPR>
+template <int LPR, bool FIRST>
 __global__ __launch_bounds__(256) void k_hanf_pull_wave(const uint64_t* __restrict__ col_ptr,
                                                         const uint32_t* __restrict__ row_idx,
                                                         const uint32_t* __restrict__ queue,
                                                         const unsigned long long* __restrict__ nq, uint64_t wpr4,
                                                         const uint64_t* __restrict__ changed,
+                                                        const uint16_t* __restrict__ code,
                                                         const uint4* __restrict__ bound_row,
                                                         const uint4* __restrict__ cur, uint4* __restrict__ nxt,
                                                         uint8_t* __restrict__ marks) {
+  __shared__ uint32_t s_regs[FIRST ? 4 : 1][FIRST ? 16 * LPR : 1];
   const int lane = threadIdx.x & 63, w = lane % LPR;
   const uint64_t n = *nq, nwaves = grid_waves();
   for (uint64_t q = grid_wave_id(); q < n; q += nwaves) {
@@ -283,7 +348,9 @@ __global__ __launch_bounds__(256) void k_hanf_pull_wave(const uint64_t* __restri
     for (uint64_t c0 = 0; c0 < wpr4; c0 += LPR) {
       const uint4 bound = bound_row[c0 + w];
       uint4 r;
-      const bool any = hanf_range<LPR>(b, e, row_idx, changed, cur, wpr4, c0, bound, &r);
+      bool any;
+      if constexpr (FIRST) any = hanf_first_range<LPR>(b, e, row_idx, code, s_regs[threadIdx.x >> 6], &r);
+      else any = hanf_range<LPR>(b, e, row_idx, changed, cur, wpr4, c0, bound, &r);
       if (!any && !stale) {
         done = false;  // as it was: not done
         continue;
@@ -303,10 +370,11 @@ __global__ __launch_bounds__(256) void k_hanf_pull_wave(const uint64_t* __restri
 // A group of LPR lanes per vertex of fewer than HANF_LOW_DEG in-edges, 64 / LPR vertices per
 // wave step, LPR in-edges of each at a time (an id per lane), so that the vertices' short
 // chains of dependent loads overlap.
-template <int LPR>
+template <int LPR, bool FIRST>
 __global__ __launch_bounds__(256) void k_hanf_pull_low(const uint64_t* __restrict__ col_ptr,
                                                        const uint32_t* __restrict__ row_idx, uint32_t V,
                                                        const uint64_t* __restrict__ changed,
+                                                       const uint16_t* __restrict__ code,
                                                        const uint4* __restrict__ bound_row,
                                                        const uint4* __restrict__ cur, uint4* __restrict__ nxt,
                                                        uint8_t* __restrict__ marks) {
@@ -334,7 +402,8 @@ __global__ __launch_bounds__(256) void k_hanf_pull_low(const uint64_t* __restric
       bool on = false;
       if (k0 + w < e) {
         u = row_idx[k0 + w];
-        on = (changed[u >> 6] >> (u & 63)) & 1ull;
+        on = FIRST || ((changed[u >> 6] >> (u & 63)) & 1ull);
+        if (FIRST) u = code[u];
       }
       const uint64_t m = (__ballot(on) >> g0) & (LPR == 64 ? ~0ull : (1ull << LPR) - 1ull);  // the group's
       any |= m != 0ull;
@@ -344,7 +413,9 @@ __global__ __launch_bounds__(256) void k_hanf_pull_low(const uint64_t* __restric
 #pragma unroll
         for (int i = 0; i < U; ++i) {
           const uint32_t x = (uint32_t)__shfl((int)u, g0 + t + i, 64);
-          r[i] = (m >> (t + i)) & 1ull ? cur[(uint64_t)x * LPR + w] : make_uint4(0, 0, 0, 0);
+          r[i] = !((m >> (t + i)) & 1ull) ? make_uint4(0, 0, 0, 0)
+                 : FIRST                  ? hanf_code_row(x, (uint32_t)w)
+                                          : cur[(uint64_t)x * LPR + w];
         }
 #pragma unroll
         for (int i = 0; i < U; ++i) acc.add(r[i]);
@@ -403,16 +474,18 @@ __device__ __forceinline__ bool byte_max_merge(uint32_t* p, uint32_t x) {
 }
 
 // Hub in-edges, one chunk per wave at a time, the chunk's max merged into the hub's next row.
-template <int LPR>
+template <int LPR, bool FIRST>
 __global__ __launch_bounds__(256) void k_hanf_pull_hubs(const uint64_t* __restrict__ col_ptr,
                                                         const uint32_t* __restrict__ row_idx,
                                                         const uint32_t* __restrict__ hubs,
                                                         const unsigned long long* __restrict__ nhub,
                                                         const uint64_t* __restrict__ start, uint64_t wpr4,
                                                         const uint64_t* __restrict__ changed,
+                                                        const uint16_t* __restrict__ code,
                                                         const uint4* __restrict__ bound_row,
                                                         const uint4* __restrict__ cur, uint4* __restrict__ nxt,
                                                         uint8_t* __restrict__ marks) {
+  __shared__ uint32_t s_regs[FIRST ? 4 : 1][FIRST ? 16 * LPR : 1];
   const int lane = threadIdx.x & 63;
   const uint64_t nwaves = grid_waves();
   const uint64_t n = *nhub;
@@ -424,7 +497,8 @@ __global__ __launch_bounds__(256) void k_hanf_pull_hubs(const uint64_t* __restri
     if (marks[v] & HANF_DONE) continue;  // uniform
     for (uint64_t c0 = 0; c0 < wpr4; c0 += LPR) {
       uint4 r;
-      if (!hanf_range<LPR>(k0, k1, row_idx, changed, cur, wpr4, c0, bound_row[c0 + lane % LPR], &r)) continue;
+      if constexpr (FIRST) (void)hanf_first_range<LPR>(k0, k1, row_idx, code, s_regs[threadIdx.x >> 6], &r);
+      else if (!hanf_range<LPR>(k0, k1, row_idx, changed, cur, wpr4, c0, bound_row[c0 + lane % LPR], &r)) continue;
       if (lane < LPR) {
         uint32_t* p = reinterpret_cast<uint32_t*>(nxt + (uint64_t)v * wpr4 + c0 + lane);
         const bool grew = byte_max_merge(p, r.x) | byte_max_merge(p + 1, r.y) | byte_max_merge(p + 2, r.z) |
@@ -468,7 +542,8 @@ __device__ __forceinline__ double hanf_alpha(int P) {
 // Estimates of counters of at most 1024 registers, summed per block in a fixed order:
 // m / 16 lanes per counter (16 registers each, one 16-byte load), 1024 / m counters per
 // wave step, so a wave keeps many counters' loads in flight instead of one.  Only changed
-// counters are read; the others' estimates are kept in est.
+// counters are read; the others' estimates are kept in est.  Without `changed` every counter
+// is a first one: one register set, whose rank the small-range estimate does not use.
 __global__ __launch_bounds__(256) void k_hanf_estimate_rows(const uint8_t* __restrict__ regs, uint32_t V, int P,
                                                             const uint64_t* __restrict__ changed,
                                                             double* __restrict__ est, double* __restrict__ part) {
@@ -482,8 +557,11 @@ __global__ __launch_bounds__(256) void k_hanf_estimate_rows(const uint8_t* __res
     const uint64_t v = v0 + slot;
     double s = 0.0;
     uint32_t zeros = 0;
-    const bool on = v < V && ((changed[v >> 6] >> (v & 63)) & 1ull);
-    if (on) {
+    const bool on = v < V && (!changed || ((changed[v >> 6] >> (v & 63)) & 1ull));
+    if (!changed) {
+      s = sub == 0 ? (double)m : 0.0;
+      zeros = sub == 0 ? m - 1u : 0u;
+    } else if (on) {
       const uint4 q = *reinterpret_cast<const uint4*>(regs + v * m + (uint64_t)sub * 16);
       const uint32_t w4[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
@@ -525,7 +603,7 @@ __global__ __launch_bounds__(256) void k_hanf_estimate(const uint8_t* __restrict
   const double alpha = hanf_alpha(P);
   double total = 0.0;  // lane 0's running sum over this wave's vertices, in order
   for (uint64_t v = wave_id; v < V; v += nwaves) {
-    if (!((changed[v >> 6] >> (v & 63)) & 1ull)) {  // uniform
+    if (changed && !((changed[v >> 6] >> (v & 63)) & 1ull)) {  // uniform
       total += est[v];
       continue;
     }
@@ -609,6 +687,8 @@ struct hanf_pull {
   dbuf<uint64_t> marks;           // HANF_CHANGED and HANF_DONE bytes
   dbuf<uint32_t> top;             // the bound row, a word per register
   dbuf<uint8_t> bound;            // the bound row
+  dbuf<uint16_t> code;            // first counters, P <= HANF_CODE_P
+  bool first = true;              // no pull yet
   unsigned grid;
 
   // od (out-degrees over this adjacency's entries) or, without it, src_ptr tells which vertices
@@ -628,34 +708,54 @@ struct hanf_pull {
     frontier_compact(ctx, changed.p, nwords, V, mid.p, nmid.p);
     k_hanf_fill_bits<<<grid_for(nwords, 256, 4096), 256, 0, s>>>(changed.p, nwords, V);
     k_hanf_zero<<<grid_for(nwords * 16, 256, 8192), 256, 0, s>>>(reinterpret_cast<uint32_t*>(marks.p), nwords * 16);
+    if (P <= HANF_CODE_P) {
+      code.alloc(ctx, std::max<uint32_t>(1, V));
+      k_hanf_codes<<<grid_for(V, 256, 8192), 256, 0, s>>>(code.p, V, P, perm);
+    }
     PE_HIP(hipGetLastError());
     grid = persistent_grid(ctx, grid_for(V, 4), 8);
   }
 
-  template <int LPR>
+  // the first counters
+  void init(uint8_t* regs, uint64_t bytes, const uint32_t* perm) {
+    hipStream_t s = ctx->stream;
+    if (code.p) {
+      k_hanf_init_rows<<<grid_for((uint64_t)V << (P - 4), 256, 65536), 256, 0, s>>>(reinterpret_cast<uint4*>(regs), V,
+                                                                                   (uint32_t)P - 4u, code.p);
+    } else {
+      k_hanf_zero<<<grid_for(bytes / 4, 256, 65536), 256, 0, s>>>(reinterpret_cast<uint32_t*>(regs), bytes / 4);
+      k_hanf_init<<<grid_for(V, 256, 8192), 256, 0, s>>>(regs, V, P, perm);
+    }
+    PE_HIP(hipGetLastError());
+  }
+
+  template <int LPR, bool FIRST>
   void launch(const uint4* cur, uint4* nxt) {
     hipStream_t s = ctx->stream;
     const uint64_t wpr4 = (1ull << P) / 16;
     uint8_t* mk = reinterpret_cast<uint8_t*>(marks.p);
     const uint4* br = reinterpret_cast<const uint4*>(bound.p);
-    if constexpr (LPR < 64) k_hanf_pull_low<LPR><<<grid, 256, 0, s>>>(ptr, idx, V, changed.p, br, cur, nxt, mk);
-    k_hanf_pull_wave<LPR><<<grid, 256, 0, s>>>(ptr, idx, mid.p, nmid.p, wpr4, changed.p, br, cur, nxt, mk);
+    if constexpr (LPR < 64)
+      k_hanf_pull_low<LPR, FIRST><<<grid, 256, 0, s>>>(ptr, idx, V, changed.p, code.p, br, cur, nxt, mk);
+    k_hanf_pull_wave<LPR, FIRST><<<grid, 256, 0, s>>>(ptr, idx, mid.p, nmid.p, wpr4, changed.p, code.p, br, cur, nxt, mk);
     k_hanf_hub_rows<<<grid_for(hubs.max_hubs, 4, 1024), 256, 0, s>>>(hubs.hubs.p, hubs.count.p, wpr4, br, cur, nxt, mk);
-    k_hanf_pull_hubs<LPR><<<grid, 256, 0, s>>>(ptr, idx, hubs.hubs.p, hubs.count.p, hubs.start.p, wpr4, changed.p, br,
-                                               cur, nxt, mk);
+    k_hanf_pull_hubs<LPR, FIRST><<<grid, 256, 0, s>>>(ptr, idx, hubs.hubs.p, hubs.count.p, hubs.start.p, wpr4, changed.p,
+                                                      code.p, br, cur, nxt, mk);
   }
 
-  // nxt[v] = register-wise max of cur[v] and cur[u] over the adjacency of v; nxt holds the
+  // cur: the first counters before the first pull.  nxt[v] = register-wise max of cur[v] and cur[u] over the adjacency of v; nxt holds the
   // rows before the last pull (anything before the first)
   void pull(const uint8_t* cur, uint8_t* nxt) {
     const uint4* c = reinterpret_cast<const uint4*>(cur);
     uint4* n = reinterpret_cast<uint4*>(nxt);
+    const bool from_codes = first && code.p;
+    first = false;
     switch (P) {
-      case 6: launch<4>(c, n); break;
-      case 7: launch<8>(c, n); break;
-      case 8: launch<16>(c, n); break;
-      case 9: launch<32>(c, n); break;
-      default: launch<64>(c, n);
+      case 6: from_codes ? launch<4, true>(c, n) : launch<4, false>(c, n); break;
+      case 7: from_codes ? launch<8, true>(c, n) : launch<8, false>(c, n); break;
+      case 8: from_codes ? launch<16, true>(c, n) : launch<16, false>(c, n); break;
+      case 9: from_codes ? launch<32, true>(c, n) : launch<32, false>(c, n); break;
+      default: from_codes ? launch<64, true>(c, n) : launch<64, false>(c, n);
     }
     hipStream_t s = ctx->stream;
     k_hanf_zero<<<1, 64, 0, s>>>(reinterpret_cast<uint32_t*>(nmid.p + 1), 2);
@@ -683,10 +783,11 @@ extern "C" int pe_hyperanf(pe_graph_t* g, const pe_hyperanf_opts_t* opts, double
     PE_HIP(hipEventRecord(ctx->t0, s));
     hanf_pull pulls(ctx, g->col_ptr.p, g->row_idx.p, V, g->nnz, P, perm, g->od.p, nullptr);
     auto anf_of = [&](const uint8_t* regs) {
+      const uint64_t* changed = pulls.first ? nullptr : pulls.changed.p;
       if (P <= 10)
-        k_hanf_estimate_rows<<<est_grid, 256, 0, s>>>(regs, V, P, pulls.changed.p, est.p, part.p);
+        k_hanf_estimate_rows<<<est_grid, 256, 0, s>>>(regs, V, P, changed, est.p, part.p);
       else
-        k_hanf_estimate<<<est_grid, 256, 0, s>>>(regs, V, P, pulls.changed.p, est.p, part.p);
+        k_hanf_estimate<<<est_grid, 256, 0, s>>>(regs, V, P, changed, est.p, part.p);
       PE_HIP(hipGetLastError());
       PE_HIP(hipMemcpyAsync(hpart.data(), part.p, est_grid * sizeof(double), hipMemcpyDeviceToHost, s));
       PE_HIP(hipStreamSynchronize(s));
@@ -694,9 +795,7 @@ extern "C" int pe_hyperanf(pe_graph_t* g, const pe_hyperanf_opts_t* opts, double
       for (double x : hpart) t += x;
       return t;
     };
-    k_hanf_zero<<<grid_for(bytes / 4, 256, 65536), 256, 0, s>>>((uint32_t*)a.p, bytes / 4);
-    k_hanf_init<<<grid_for(V, 256, 8192), 256, 0, s>>>(a.p, V, P, perm);
-    PE_HIP(hipGetLastError());
+    pulls.init(a.p, bytes, perm);
     std::vector<double> out;
     double last = anf_of(a.p);
     out.push_back(last);
@@ -764,9 +863,7 @@ extern "C" int pe_nstep_degrees(pe_graph_t* g, const uint64_t* target_words, uin
     auto pass = [&](const uint64_t* ptr, const uint32_t* idx, const uint32_t* od, const uint64_t* src_ptr,
                     uint32_t* host_out) {
       hanf_pull pulls(ctx, ptr, idx, V, g->nnz, P, perm, od, src_ptr);
-      k_hanf_zero<<<grid_for(bytes / 4, 256, 65536), 256, 0, s>>>((uint32_t*)a.p, bytes / 4);
-      k_hanf_init<<<grid_for(V, 256, 8192), 256, 0, s>>>(a.p, V, P, perm);
-      PE_HIP(hipGetLastError());
+      pulls.init(a.p, bytes, perm);
       uint8_t* cur = a.p;
       uint8_t* nxt = b.p;
       for (uint32_t it = 0; it < step; ++it) {  // nstepdegrees.hpp:343-409
