@@ -60,3 +60,35 @@ def test_large_symmetrized(ctx):
     exp = oracle.cc_labels(oracle.CSC(1 << 20, s, d, symmetrize=True))
     assert np.array_equal(res.labels, exp)
     g.close()
+
+
+@pytest.mark.parametrize("directed", [False, True])
+@pytest.mark.parametrize("relabel", [False, True])
+def test_floor_and_length_classes(ctx, directed, relabel):
+    """The smallest ids have no out-edges (0 isolated, 1 only reached), a second component
+    never sees the smallest label, and vertices of 64, 65, 4096 and 4097 in-edges sit at the
+    ends of the pull's passes, the last one reached by the second component's ids only."""
+    from plato_amd import Graph
+    from plato_amd.algo import connected_components
+    rng = np.random.default_rng(3)
+    rim, V = 5000, 2 + 2 * 5000 + 8
+    s, d = [np.array([2])], [np.array([1])]
+    for h, n in enumerate((64, 65, 4096, 4097)):
+        for part in range(2):
+            s.append(2 + part * rim + rng.choice(rim, n, replace=False))
+            d.append(np.full(n, 2 + 2 * rim + 4 * part + h))
+    for part in range(2):  # chains, so that labels travel over several epochs
+        at = 2 + part * rim + rng.permutation(rim)[:600]
+        s.append(at[:-1])
+        d.append(at[1:])
+    s, d = np.concatenate(s).astype(np.uint32), np.concatenate(d).astype(np.uint32)
+    og = oracle.CSC(V, s, d, symmetrize=not directed)
+    if directed:
+        assert np.diff(og.col_ptr)[-4:].tolist() == [64, 65, 4096, 4097]
+    print(f"case: cc floor directed={directed} relabel={relabel}", flush=True)
+    g = Graph.from_edges(ctx, s, d, V, directed=directed, build_csr=True, relabel=relabel)
+    res = connected_components(g)
+    exp = oracle.cc_labels(og)
+    assert np.array_equal(res.labels, exp)
+    assert res.components == len(np.unique(exp))
+    g.close()
