@@ -209,3 +209,35 @@ def test_slot_errors(s13):
         b.admit(64, [1])         # out of range
     b.release(0)
     b.admit(0, [2])
+
+
+@pytest.mark.parametrize("slots,k", [([5], 1), (list(range(64)), 100), ([63, 0, 63, 7], 5000), ([1, 2], 200000)])
+def test_topk_selection(ctx, slots, k):
+    """Top-k against a sort of the slots' ranks: one slot and all, a slot asked for twice, lists
+    longer than the positive entries, and (a graph whose ranks are nearly all alike) a
+    threshold bin with far more entries than are wanted, which takes the second histogram."""
+    from plato_amd import Graph
+    from plato_amd.batch import PprBatch
+    V = 131073
+    for kind, relabel in (("ring", False), ("rmat", True)):
+        if kind == "ring":  # every vertex a seed of every query: ranks differ in their last bits only
+            v = np.arange(V, dtype=np.uint32)
+            s, d = np.concatenate([v, v[:50]]), np.concatenate([(v + 1) % V, (v[:50] * 7 + 3) % V]).astype(np.uint32)
+            seeds = v
+        else:
+            s, d = oracle.rmat_edges(17, 8, 5)
+            seeds = s[:3]
+        g = Graph.from_edges(ctx, s, d, V, relabel=relabel)
+        b = PprBatch(g, D, tol=1e-12, max_iters=3)
+        for q in sorted(set(slots)):
+            b.admit(q, seeds if kind == "ring" else [int(s[q])])
+        b.run_until_done(sorted(set(slots)), chunk=4)
+        print(f"case: topk {kind} k={k} slots={len(slots)}", flush=True)
+        ids, vals = b.topk(slots, k)
+        for i, q in enumerate(slots[:4]):
+            r = b.results([q])[0].astype(np.float32)
+            order = np.lexsort((np.arange(V), -r))[:k]
+            assert np.array_equal(vals[i][: len(order)], r[order])
+            assert np.array_equal(ids[i][: len(order)], order.astype(np.uint32))
+        b.close()
+        g.close()
