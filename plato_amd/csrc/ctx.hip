@@ -274,6 +274,7 @@ int pe_ctx_destroy(pe_ctx_t* ctx) {
   if (ctx->t1) (void)hipEventDestroy(ctx->t1);
   if (ctx->host_pinned) (void)hipHostFree(ctx->host_pinned);
   if (ctx->host_mail) (void)hipHostFree(ctx->host_mail);
+  staging_free(ctx->stage);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
   return PE_OK;
@@ -456,9 +457,7 @@ int pe_vec_upload(pe_vec_t* v, const void* host, uint64_t n) {
   if (!v || (!host && n)) return PE_ERR_INVALID;
   return guarded(v->ctx, [&] {
     PE_REQUIRE(n <= v->n, PE_ERR_RANGE, "upload longer than vector");
-    PE_HIP(hipMemcpyAsync(v->p, host, n * dtype_size(v->dtype), hipMemcpyHostToDevice,
-                          v->ctx->stream));
-    PE_HIP(hipStreamSynchronize(v->ctx->stream));
+    host_upload(v->ctx, v->p, host, n * dtype_size(v->dtype));
   });
 }
 
@@ -466,9 +465,7 @@ int pe_vec_download(pe_vec_t* v, void* host, uint64_t n) {
   if (!v || (!host && n)) return PE_ERR_INVALID;
   return guarded(v->ctx, [&] {
     PE_REQUIRE(n <= v->n, PE_ERR_RANGE, "download longer than vector");
-    PE_HIP(hipMemcpyAsync(host, v->p, n * dtype_size(v->dtype), hipMemcpyDeviceToHost,
-                          v->ctx->stream));
-    PE_HIP(hipStreamSynchronize(v->ctx->stream));
+    host_download(v->ctx, v->p, host, n * dtype_size(v->dtype));
   });
 }
 
@@ -477,19 +474,20 @@ int pe_vec_download_f64(pe_vec_t* v, double* host, uint64_t n) {
   return guarded(v->ctx, [&] {
     PE_REQUIRE(n <= v->n, PE_ERR_RANGE, "download longer than vector");
     if (v->dtype == PE_F64) {
-      PE_HIP(hipMemcpyAsync(host, v->p, n * 8, hipMemcpyDeviceToHost, v->ctx->stream));
-    } else {
-      dbuf<double> tmp(v->ctx, n ? n : 1);
-      unsigned g = grid_for(n, 256, 4096);
-      if (v->dtype == PE_F32)
-        k_to_f64<float><<<g, 256, 0, v->ctx->stream>>>((const float*)v->p, tmp.p, n);
-      else
-        k_to_f64<uint32_t><<<g, 256, 0, v->ctx->stream>>>((const uint32_t*)v->p, tmp.p, n);
-      PE_HIP(hipGetLastError());
-      PE_HIP(hipMemcpyAsync(host, tmp.p, n * 8, hipMemcpyDeviceToHost, v->ctx->stream));
-      PE_HIP(hipStreamSynchronize(v->ctx->stream));
+      host_download(v->ctx, v->p, host, n * 8);
+      return;
     }
-    PE_HIP(hipStreamSynchronize(v->ctx->stream));
+    staged_download(
+        v->ctx, n, 8,
+        [&](uint64_t u0, uint64_t m, void* slot) {
+          const unsigned g = grid_for(m, 256, 4096);
+          if (v->dtype == PE_F32)
+            k_to_f64<float><<<g, 256, 0, v->ctx->stream>>>((const float*)v->p + u0, (double*)slot, m);
+          else
+            k_to_f64<uint32_t><<<g, 256, 0, v->ctx->stream>>>((const uint32_t*)v->p + u0, (double*)slot, m);
+          PE_HIP(hipGetLastError());
+        },
+        [&](uint64_t u0, uint64_t m, void* slot) { std::memcpy(host + u0, slot, m * 8); });
   });
 }
 

@@ -502,22 +502,10 @@ void build_from_edges(pe_graph_s* g, dbuf<uint32_t>& ds, dbuf<uint32_t>& dd, dbu
 
 // ---- id mapping helpers (relabeled graphs) -----------------------------------------
 template <typename T>
-__global__ void k_gather_by_rank(const T* __restrict__ in, const uint32_t* __restrict__ rank_of, uint32_t V,
+__global__ void k_gather_by_rank(const T* __restrict__ in, const uint32_t* __restrict__ rank_of, uint64_t n,
                                  T* __restrict__ out) {
-  for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V;
-       v += (uint64_t)gridDim.x * blockDim.x)
+  for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < n; v += (uint64_t)gridDim.x * blockDim.x)
     out[v] = in[rank_of[v]];
-}
-
-void to_external_order(pe_graph_s* g, const void* in, void* out, size_t elem) {
-  hipStream_t s = g->ctx->stream;
-  if (elem == 8)
-    k_gather_by_rank<uint64_t><<<grid_for(g->V, 256, 8192), 256, 0, s>>>((const uint64_t*)in, g->rank_of.p, g->V,
-                                                                        (uint64_t*)out);
-  else
-    k_gather_by_rank<uint32_t><<<grid_for(g->V, 256, 8192), 256, 0, s>>>((const uint32_t*)in, g->rank_of.p, g->V,
-                                                                        (uint32_t*)out);
-  PE_HIP(hipGetLastError());
 }
 
 void to_internal_ids(pe_graph_s* g, const uint32_t* host_ids, uint32_t n, uint32_t* host_out) {
@@ -534,19 +522,37 @@ void to_internal_ids(pe_graph_s* g, const uint32_t* host_ids, uint32_t n, uint32
   PE_HIP(hipStreamSynchronize(s));
 }
 
-// Download a V-long device array in external (input) id order.
-void download_external(pe_graph_s* g, const void* dev, void* host, size_t elem) {
+// Download a V-long device array in external (input) id order: the reordering kernel writes
+// the pinned slots itself.
+void download_external(pe_graph_s* g, const void* dev, void* host, size_t elem, bool widen) {
   hipStream_t s = g->ctx->stream;
-  const uint64_t bytes = (uint64_t)g->V * elem;
-  if (g->relabeled) {
-    dbuf<uint8_t> tmp(g->ctx, std::max<uint64_t>(1, bytes));
-    to_external_order(g, dev, tmp.p, elem);
-    PE_HIP(hipMemcpyAsync(host, tmp.p, bytes, hipMemcpyDeviceToHost, s));
-    PE_HIP(hipStreamSynchronize(s));
-  } else {
-    PE_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, s));
-    PE_HIP(hipStreamSynchronize(s));
+  if (!g->relabeled && !widen) {
+    host_download(g->ctx, dev, host, (uint64_t)g->V * elem);
+    return;
   }
+  staged_download(
+      g->ctx, g->V, elem,
+      [&](uint64_t v0, uint64_t n, void* slot) {
+        if (!g->relabeled) {
+          PE_HIP(hipMemcpyAsync(slot, static_cast<const uint8_t*>(dev) + v0 * elem, n * elem, hipMemcpyDeviceToHost, s));
+          return;
+        }
+        const unsigned grid = grid_for(n, 256, 8192);
+        if (elem == 8)
+          k_gather_by_rank<uint64_t><<<grid, 256, 0, s>>>((const uint64_t*)dev, g->rank_of.p + v0, n, (uint64_t*)slot);
+        else
+          k_gather_by_rank<uint32_t><<<grid, 256, 0, s>>>((const uint32_t*)dev, g->rank_of.p + v0, n, (uint32_t*)slot);
+        PE_HIP(hipGetLastError());
+      },
+      [&](uint64_t v0, uint64_t n, void* slot) {
+        if (!widen) {
+          std::memcpy(static_cast<uint8_t*>(host) + v0 * elem, slot, n * elem);
+          return;
+        }
+        const float* f = static_cast<const float*>(slot);
+        double* out = static_cast<double*>(host) + v0;
+        for (uint64_t i = 0; i < n; ++i) out[i] = f[i];
+      });
 }
 
 }  // namespace pe
@@ -595,10 +601,9 @@ int pe_rmat_edges(pe_ctx_t* ctx, uint32_t scale, uint64_t seed, double a, double
     if (w) dw.alloc(ctx, n);
     k_rmat_edges<<<grid_for(n, 256, 1u << 16), 256, 0, s>>>(p, e0, n, ds.p, dd.p, w ? dw.p : nullptr);
     PE_HIP(hipGetLastError());
-    PE_HIP(hipMemcpyAsync(src, ds.p, n * 4, hipMemcpyDeviceToHost, s));
-    PE_HIP(hipMemcpyAsync(dst, dd.p, n * 4, hipMemcpyDeviceToHost, s));
-    if (w) PE_HIP(hipMemcpyAsync(w, dw.p, n * 4, hipMemcpyDeviceToHost, s));
-    PE_HIP(hipStreamSynchronize(s));
+    host_download(ctx, ds.p, src, n * 4);
+    host_download(ctx, dd.p, dst, n * 4);
+    if (w) host_download(ctx, dw.p, w, n * 4);
   });
 }
 
@@ -620,13 +625,11 @@ int pe_graph_create(pe_ctx_t* ctx, const uint32_t* src, const uint32_t* dst, con
     g->edges = E;
     dbuf<uint32_t> ds(ctx, std::max<uint64_t>(1, E)), dd(ctx, std::max<uint64_t>(1, E));
     dbuf<float> dw;
-    if (E) {
-      PE_HIP(hipMemcpyAsync(ds.p, src, E * 4, hipMemcpyHostToDevice, s));
-      PE_HIP(hipMemcpyAsync(dd.p, dst, E * 4, hipMemcpyHostToDevice, s));
-    }
+    host_upload(ctx, ds.p, src, E * 4);
+    host_upload(ctx, dd.p, dst, E * 4);
     if (weighted) {
       dw.alloc(ctx, std::max<uint64_t>(1, E));
-      if (E) PE_HIP(hipMemcpyAsync(dw.p, w, E * 4, hipMemcpyHostToDevice, s));
+      host_upload(ctx, dw.p, w, E * 4);
     }
     build_from_edges(g, ds, dd, dw, flags);
     *out = guard.release();
@@ -640,8 +643,7 @@ int pe_graph_permutation(pe_graph_t* g, uint32_t* rank_of) {
       for (uint32_t v = 0; v < g->V; ++v) rank_of[v] = v;
       return;
     }
-    PE_HIP(hipMemcpyAsync(rank_of, g->rank_of.p, (uint64_t)g->V * 4, hipMemcpyDeviceToHost, g->ctx->stream));
-    PE_HIP(hipStreamSynchronize(g->ctx->stream));
+    host_download(g->ctx, g->rank_of.p, rank_of, (uint64_t)g->V * 4);
   });
 }
 
@@ -678,14 +680,12 @@ int pe_graph_get_info(const pe_graph_t* g, pe_graph_info_t* info) {
 int pe_graph_download_csc(pe_graph_t* g, uint64_t* col_ptr, uint32_t* row_idx, float* wn) {
   if (!g) return PE_ERR_INVALID;
   return guarded(g->ctx, [&] {
-    hipStream_t s = g->ctx->stream;
-    if (col_ptr) PE_HIP(hipMemcpyAsync(col_ptr, g->col_ptr.p, ((uint64_t)g->V + 1) * 8, hipMemcpyDeviceToHost, s));
-    if (row_idx && g->nnz) PE_HIP(hipMemcpyAsync(row_idx, g->row_idx.p, g->nnz * 4, hipMemcpyDeviceToHost, s));
+    if (col_ptr) host_download(g->ctx, g->col_ptr.p, col_ptr, ((uint64_t)g->V + 1) * 8);
+    if (row_idx) host_download(g->ctx, g->row_idx.p, row_idx, g->nnz * 4);
     if (wn) {
       PE_REQUIRE(g->has_weights, PE_ERR_STATE, "graph has no weights");
-      if (g->nnz) PE_HIP(hipMemcpyAsync(wn, g->wn.p, g->nnz * 4, hipMemcpyDeviceToHost, s));
+      host_download(g->ctx, g->wn.p, wn, g->nnz * 4);
     }
-    PE_HIP(hipStreamSynchronize(s));
   });
 }
 
@@ -693,10 +693,8 @@ int pe_graph_download_csr(pe_graph_t* g, uint64_t* row_ptr, uint32_t* col_idx) {
   if (!g) return PE_ERR_INVALID;
   return guarded(g->ctx, [&] {
     PE_REQUIRE(g->has_csr, PE_ERR_STATE, "graph has no CSR (PE_GRAPH_BUILD_CSR)");
-    hipStream_t s = g->ctx->stream;
-    if (row_ptr) PE_HIP(hipMemcpyAsync(row_ptr, g->csr_ptr(), ((uint64_t)g->V + 1) * 8, hipMemcpyDeviceToHost, s));
-    if (col_idx && g->nnz) PE_HIP(hipMemcpyAsync(col_idx, g->csr_idx(), g->nnz * 4, hipMemcpyDeviceToHost, s));
-    PE_HIP(hipStreamSynchronize(s));
+    if (row_ptr) host_download(g->ctx, g->csr_ptr(), row_ptr, ((uint64_t)g->V + 1) * 8);
+    if (col_idx) host_download(g->ctx, g->csr_idx(), col_idx, g->nnz * 4);
   });
 }
 

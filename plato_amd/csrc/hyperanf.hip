@@ -824,11 +824,10 @@ extern "C" int pe_hyperanf(pe_graph_t* g, const pe_hyperanf_opts_t* opts, double
       if (g->relabeled) {
         k_hanf_rows_external<<<grid_for((uint64_t)V * m, 256, 65536), 256, 0, s>>>(cur, g->rank_of.p, V, m, nxt);
         PE_HIP(hipGetLastError());
-        PE_HIP(hipMemcpyAsync(registers, nxt, (uint64_t)V * m, hipMemcpyDeviceToHost, s));
+        host_download(ctx, nxt, registers, (uint64_t)V * m);
       } else {
-        PE_HIP(hipMemcpyAsync(registers, cur, (uint64_t)V * m, hipMemcpyDeviceToHost, s));
+        host_download(ctx, cur, registers, (uint64_t)V * m);
       }
-      PE_HIP(hipStreamSynchronize(s));
     }
     if (seconds) *seconds = ms * 1e-3;
   });

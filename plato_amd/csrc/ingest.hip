@@ -422,7 +422,7 @@ int pe_graph_create_csv(pe_ctx_t* ctx, const char* text, uint64_t nbytes, uint32
     const bool encode = (flags & PE_GRAPH_ENCODE_IDS) != 0;
     // text on the device
     dbuf<char> db(ctx, std::max<uint64_t>(1, nbytes));
-    if (nbytes) PE_HIP(hipMemcpyAsync(db.p, text, nbytes, hipMemcpyHostToDevice, s));
+    host_upload(ctx, db.p, text, nbytes);
     // newlines
     const uint64_t nseg = std::max<uint64_t>(1, (nbytes + CSV_SEG - 1) / CSV_SEG);
     PE_REQUIRE(nseg < 0x7FFFFFFFull, PE_ERR_RANGE, "text too large");
@@ -462,8 +462,7 @@ int pe_graph_create_csv(pe_ctx_t* ctx, const char* text, uint64_t nbytes, uint32
     nl.release();
     // errors: first offending line (host scan of the status bytes is enough: 1 B per line)
     std::vector<uint8_t> hst(nlines);
-    if (nlines) PE_HIP(hipMemcpyAsync(hst.data(), status.p, nlines, hipMemcpyDeviceToHost, s));
-    PE_HIP(hipStreamSynchronize(s));
+    host_download(ctx, status.p, hst.data(), nlines);
     for (uint64_t i = 0; i < nlines; ++i) {
       if (hst[i] == 2)
         fail(PE_ERR_RANGE, "line " + std::to_string(i + 1) + ": vertex id above 2^32 - 1 (use PE_GRAPH_ENCODE_IDS)");
@@ -554,8 +553,7 @@ int pe_graph_vertex_ids(pe_graph_t* g, uint64_t* original_ids) {
       for (uint32_t v = 0; v < g->V; ++v) original_ids[v] = v;
       return;
     }
-    PE_HIP(hipMemcpyAsync(original_ids, g->vid_decode.p, (uint64_t)g->V * 8, hipMemcpyDeviceToHost, g->ctx->stream));
-    PE_HIP(hipStreamSynchronize(g->ctx->stream));
+    host_download(g->ctx, g->vid_decode.p, original_ids, (uint64_t)g->V * 8);
   });
 }
 

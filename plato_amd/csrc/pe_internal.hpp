@@ -8,6 +8,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <memory>
 #include <stdexcept>
 #include <string>
@@ -46,6 +47,8 @@ struct kernel_timer {
   uint64_t launches = 0;
 };
 
+struct staging;
+
 }  // namespace pe
 
 struct pe_ctx_s {
@@ -66,6 +69,7 @@ struct pe_ctx_s {
   unsigned long long mail_seq = 0;
   // this device's static scratch array of pe_pull_sum_noalloc (its device address)
   void* noalloc_scratch = nullptr;
+  pe::staging* stage = nullptr;  // pinned ring of large transfers (transfer.hip), made by the first
 };
 
 namespace pe {
@@ -75,6 +79,17 @@ namespace pe {
 // the next call on this context.
 const unsigned long long* mail_post(pe_ctx_s* ctx, const unsigned long long* src, uint32_t n,
                                     unsigned long long* clear, uint32_t nclear);
+
+// Transfers to and from ordinary host memory (transfer.hip); all wait for the work queued on
+// the stream and for the data.  staged_download moves `units` of unit_bytes each in chunks:
+// launch(u0, n, slot) queues work that leaves units [u0, u0 + n) in the pinned slot (a copy, or
+// a kernel that writes there), consume(u0, n, slot) puts them where they belong, on a worker
+// thread (calls for different chunks overlap; it must not throw or call HIP).
+using stage_fn = std::function<void(uint64_t u0, uint64_t n, void* slot)>;
+void staged_download(pe_ctx_s* ctx, uint64_t units, size_t unit_bytes, const stage_fn& launch, const stage_fn& consume);
+void host_download(pe_ctx_s* ctx, const void* dev, void* host, size_t bytes);
+void host_upload(pe_ctx_s* ctx, void* dev, const void* host, size_t bytes);
+void staging_free(staging* st);
 
 // Allocation through the context keeps a ledger (admission control reads it).
 void* dmalloc(pe_ctx_s* ctx, size_t bytes);
@@ -365,9 +380,9 @@ void build_from_edges(pe_graph_s* g, dbuf<uint32_t>& ds, dbuf<uint32_t>& dd, dbu
 // pull_binned.hip: builds g->pb (no-op if built with the same options)
 void binned_build(pe_graph_s* g, const pe_binned_opts_t* opts);
 // relabeled graphs: input ids -> internal ids (host arrays), and V-long device
-// arrays downloaded in input id order (elem = 4 or 8 bytes)
+// arrays downloaded in input id order (elem = 4 or 8 bytes; widen: FP32 to an FP64 host array)
 void to_internal_ids(pe_graph_s* g, const uint32_t* host_ids, uint32_t n, uint32_t* host_out);
-void download_external(pe_graph_s* g, const void* dev, void* host, size_t elem);
+void download_external(pe_graph_s* g, const void* dev, void* host, size_t elem, bool widen = false);
 // sum of out-degrees over a bitmap's vertices (rank.hip)
 uint64_t active_edges_dev(pe_graph_s* g, const uint64_t* words, uint64_t nwords);
 // bitmap -> queue of its set ids below V, appended at *count (bfs.hip)

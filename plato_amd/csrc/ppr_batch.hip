@@ -500,14 +500,14 @@ __global__ void k_batch_set_slot(uint32_t* status, double* init_dist, uint32_t* 
   last_delta[slot] = 0.0;
 }
 
-// Columns of the current block -> dense [n][V] (internal order).
+// Entries [v0, v0 + n) (input ids; rank_of: input -> internal, nullptr when they are the same)
+// of one column of the current block.
 __global__ void k_batch_extract(const float* X0, const float* X1, const batch_ctl* __restrict__ ctl,
-                                uint32_t V, const uint32_t* __restrict__ slots, uint32_t n,
+                                const uint32_t* __restrict__ rank_of, uint64_t v0, uint64_t n, uint32_t slot,
                                 float* __restrict__ out) {
   const float* X = ctl->cur ? X1 : X0;
-  for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V;
-       v += (uint64_t)gridDim.x * blockDim.x)
-    for (uint32_t i = 0; i < n; ++i) out[(uint64_t)i * V + v] = X[v * BK + slots[i]];
+  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
+    out[i] = X[(rank_of ? (uint64_t)rank_of[v0 + i] : v0 + i) * BK + slot];
 }
 
 __global__ void k_batch_zero_words(unsigned int* __restrict__ p, uint64_t n) {
@@ -744,13 +744,6 @@ void check_slot(pe_ppr_batch_s* b, uint32_t slot) {
   PE_REQUIRE(slot < b->opts.k, PE_ERR_RANGE, "slot out of range");
 }
 
-// Slots given by the caller -> device list (all must be DONE)
-dbuf<uint32_t> device_slots(pe_ppr_batch_s* b, const uint32_t* slots, uint32_t n) {
-  dbuf<uint32_t> d(b->g->ctx, std::max<uint32_t>(1, n));
-  PE_HIP(hipMemcpyAsync(d.p, slots, (size_t)n * 4, hipMemcpyHostToDevice, b->g->ctx->stream));
-  return d;
-}
-
 void refresh_status(pe_ppr_batch_s* b) {
   hipStream_t s = b->g->ctx->stream;
   b->host_status.resize(BK);
@@ -907,14 +900,20 @@ int pe_ppr_batch_results(pe_ppr_batch_t* b, const uint32_t* slots, uint32_t n, d
     pe_graph_s* g = b->g;
     hipStream_t s = g->ctx->stream;
     const uint32_t V = g->V;
-    auto ds = device_slots(b, slots, n);
-    dbuf<float> dense(g->ctx, (uint64_t)n * std::max<uint32_t>(1, V));
-    k_batch_extract<<<grid_for(V, 256, 8192), 256, 0, s>>>(b->X0.p, b->X1.p, b->ctl.p, V, ds.p, n, dense.p);
-    PE_HIP(hipGetLastError());
-    std::vector<float> tmp(V);
     for (uint32_t i = 0; i < n; ++i) {
-      download_external(g, dense.p + (uint64_t)i * V, tmp.data(), 4);
-      for (uint32_t v = 0; v < V; ++v) ranks[(uint64_t)i * V + v] = tmp[v];
+      double* out = ranks + (uint64_t)i * V;
+      staged_download(
+          g->ctx, V, 4,
+          [&](uint64_t v0, uint64_t m, void* slot) {
+            k_batch_extract<<<grid_for(m, 256, 8192), 256, 0, s>>>(b->X0.p, b->X1.p, b->ctl.p,
+                                                                  g->relabeled ? g->rank_of.p : nullptr, v0, m,
+                                                                  slots[i], static_cast<float*>(slot));
+            PE_HIP(hipGetLastError());
+          },
+          [&](uint64_t v0, uint64_t m, void* slot) {
+            const float* f = static_cast<const float*>(slot);
+            for (uint64_t q = 0; q < m; ++q) out[v0 + q] = f[q];
+          });
     }
   });
 }

@@ -153,9 +153,7 @@ static void download_state(pe_graph_s* g, int prec, const void* dev, double* out
   if (prec == 64) {
     download_external(g, dev, out, 8);
   } else {
-    std::vector<float> tmp(g->V);
-    download_external(g, dev, tmp.data(), 4);
-    for (uint32_t v = 0; v < g->V; ++v) out[v] = tmp[v];
+    download_external(g, dev, out, 4, true);
   }
 }
 
