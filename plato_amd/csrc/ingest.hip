@@ -525,6 +525,7 @@ int pe_graph_create_csv(pe_ctx_t* ctx, const char* text, uint64_t nbytes, uint32
       k_encode<<<grid_for(E, 256, 1u << 20), 256, 0, s>>>(es.p, E, g->vid_decode.p, nu, ds.p);
       k_encode<<<grid_for(E, 256, 1u << 20), 256, 0, s>>>(ed.p, E, g->vid_decode.p, nu, dd.p);
       PE_HIP(hipGetLastError());
+      PE_HIP(hipStreamSynchronize(s));  // hoff has been read
       g->V = (uint32_t)nu;
       g->encoded = true;
     } else {

@@ -113,7 +113,7 @@ __global__ __launch_bounds__(BLOCK) void k_pull_tiles(
     const uint64_t* __restrict__ tile_edge, uint64_t T_tiles, T* buf0, T* buf1,
     const uint32_t* __restrict__ od, rank_args a, const iter_ctl* __restrict__ ctl,
     cpair<T>* __restrict__ tile_carry, cpair<T>* __restrict__ tile_head,
-    double* __restrict__ part_delta, double* __restrict__ part_rsum) {
+    double* __restrict__ part_delta, double* __restrict__ part_rsum, uint32_t* __restrict__ ticket) {
   constexpr int TILE = BLOCK * ITEMS;
   constexpr int WAVES = BLOCK / 64;
   __shared__ T s_val[TILE];
@@ -134,6 +134,7 @@ __global__ __launch_bounds__(BLOCK) void k_pull_tiles(
     final_iter = a.final_iter;
   }
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  if (blockIdx.x == 0 && tid == 0) *ticket = 0u;  // of the fix-up, the next launch
   double delta = 0.0, rsum = 0.0;
 
   uint64_t t = blockIdx.x;
@@ -292,14 +293,18 @@ __global__ __launch_bounds__(BLOCK) void k_pull_tiles(
 }
 
 // ---- fix-up of rows spanning tiles -------------------------------------------------------
-// Short spans (<= 8 tiles): one thread per row, carries summed in tile order.
+// Blocks [0, short_grid): short spans (<= 8 tiles), one thread per row, carries summed in tile
+// order.  The others: long spans (hub columns), one wave per row; lane j sums tiles t0+j,
+// t0+j+64, ... then a fixed butterfly combines the lanes.  The last block to end finishes the
+// iteration (RMAT scale 16, FP64: short, long and finish as three launches 11.2 us an
+// iteration, as one 6.7 us).
 template <typename T>
-__global__ __launch_bounds__(256) void k_pull_fixup_short(
+__global__ __launch_bounds__(256) void k_pull_fixup(
     const uint32_t* __restrict__ fix_row, const uint32_t* __restrict__ fix_t0,
-    const uint32_t* __restrict__ fix_t1, uint64_t n, const cpair<T>* __restrict__ tile_carry,
-    const cpair<T>* __restrict__ tile_head, T* buf0, T* buf1, const uint32_t* __restrict__ od,
-    rank_args a, const iter_ctl* __restrict__ ctl, double* __restrict__ part_delta,
-    double* __restrict__ part_rsum) {
+    const uint32_t* __restrict__ fix_t1, uint64_t nshort, uint64_t n, unsigned short_grid,
+    const cpair<T>* __restrict__ tile_carry, const cpair<T>* __restrict__ tile_head, T* buf0, T* buf1,
+    const uint32_t* __restrict__ od, rank_args a, iter_ctl* ctl, double* part_delta, double* part_rsum,
+    unsigned tile_grid, uint32_t* ticket, double* __restrict__ deltas, double* __restrict__ rsums) {
   __shared__ double s_red[8];
   bool final_iter = false;
   const T* x = buf0;
@@ -312,63 +317,38 @@ __global__ __launch_bounds__(256) void k_pull_fixup_short(
     final_iter = a.final_iter;
   }
   double delta = 0.0, rsum = 0.0;
-  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * blockDim.x) {
-    const uint32_t t0 = fix_t0[i], t1 = fix_t1[i];
-    cpair<T> s{(T)0, (T)0};
-    for (uint32_t t = t0; t < t1; ++t) s = cadd(s, tile_carry[t]);
-    s = cadd(s, tile_head[t1]);
-    delta += apply_row<T>(a, final_iter, fix_row[i], (double)s.hi + (double)s.lo, x, y, od, rsum);
-  }
-  block_reduce2<256>(delta, rsum, s_red);
-  if (threadIdx.x == 0) {
-    part_delta[blockIdx.x] = delta;
-    part_rsum[blockIdx.x] = rsum;
-  }
-}
-
-// Long spans (hub columns): one wave per row; lane j sums tiles t0+j, t0+j+64, ...
-// then a fixed butterfly combines the lanes.
-template <typename T>
-__global__ __launch_bounds__(256) void k_pull_fixup_long(
-    const uint32_t* __restrict__ fix_row, const uint32_t* __restrict__ fix_t0,
-    const uint32_t* __restrict__ fix_t1, uint64_t n, const cpair<T>* __restrict__ tile_carry,
-    const cpair<T>* __restrict__ tile_head, T* buf0, T* buf1, const uint32_t* __restrict__ od,
-    rank_args a, const iter_ctl* __restrict__ ctl, double* __restrict__ part_delta,
-    double* __restrict__ part_rsum) {
-  __shared__ double s_red[8];
-  bool final_iter = false;
-  const T* x = buf0;
-  T* y = buf1;
-  if (ctl) {
-    if (ctl->done) return;
-    final_iter = (ctl->t + 1 == ctl->iters);
-    if (ctl->cur) { x = buf1; y = buf0; }
-  } else {
-    final_iter = a.final_iter;
-  }
-  const int lane = threadIdx.x & 63;
-  const uint64_t wave_id = grid_wave_id();
-  const uint64_t nwaves = grid_waves();
-  double delta = 0.0, rsum = 0.0;
-  for (uint64_t i = wave_id; i < n; i += nwaves) {
-    const uint32_t t0 = fix_t0[i], t1 = fix_t1[i];
-    cpair<T> s{(T)0, (T)0};
-    for (uint32_t t = t0 + lane; t < t1; t += 64) s = cadd(s, tile_carry[t]);
-    for (int off = 32; off > 0; off >>= 1) {
-      cpair<T> o{__shfl_down(s.hi, off, 64), __shfl_down(s.lo, off, 64)};
-      if (lane < off) s = cadd(s, o);
-    }
-    if (lane == 0) {
+  if (blockIdx.x < short_grid) {
+    for (uint64_t i = blockIdx.x * (uint64_t)256 + threadIdx.x; i < nshort; i += (uint64_t)short_grid * 256) {
+      const uint32_t t0 = fix_t0[i], t1 = fix_t1[i];
+      cpair<T> s{(T)0, (T)0};
+      for (uint32_t t = t0; t < t1; ++t) s = cadd(s, tile_carry[t]);
       s = cadd(s, tile_head[t1]);
       delta += apply_row<T>(a, final_iter, fix_row[i], (double)s.hi + (double)s.lo, x, y, od, rsum);
     }
+  } else {
+    const int lane = threadIdx.x & 63;
+    const uint64_t nwaves = (uint64_t)(gridDim.x - short_grid) * 4;
+    for (uint64_t i = nshort + wave_uniform((blockIdx.x - short_grid) * (uint64_t)4 + (threadIdx.x >> 6)); i < n;
+         i += nwaves) {
+      const uint32_t t0 = fix_t0[i], t1 = fix_t1[i];
+      cpair<T> s{(T)0, (T)0};
+      for (uint32_t t = t0 + lane; t < t1; t += 64) s = cadd(s, tile_carry[t]);
+      for (int off = 32; off > 0; off >>= 1) {
+        cpair<T> o{__shfl_down(s.hi, off, 64), __shfl_down(s.lo, off, 64)};
+        if (lane < off) s = cadd(s, o);
+      }
+      if (lane == 0) {
+        s = cadd(s, tile_head[t1]);
+        delta += apply_row<T>(a, final_iter, fix_row[i], (double)s.hi + (double)s.lo, x, y, od, rsum);
+      }
+    }
   }
   block_reduce2<256>(delta, rsum, s_red);
   if (threadIdx.x == 0) {
-    part_delta[blockIdx.x] = delta;
-    part_rsum[blockIdx.x] = rsum;
+    part_delta[tile_grid + blockIdx.x] = delta;
+    part_rsum[tile_grid + blockIdx.x] = rsum;
   }
+  if (last_block(ticket)) iter_finish(part_delta, part_rsum, tile_grid + gridDim.x, ctl, deltas, rsums);
 }
 
 // ---- unfused apply (pe_rank_apply) -------------------------------------------------------
@@ -389,57 +369,12 @@ __global__ __launch_bounds__(256) void k_rank_apply(uint32_t V, const T* __restr
   }
 }
 
-// ---- end of an iteration: reduce the partials, advance the controller ----------------------
-// Plato's loop control (pagerank.hpp:100-146): after a non-final iteration,
-// delta < eps jumps to one more, final, iteration.  The optional normalised
-// tolerance does the same on delta / sum(rank).
+// end of an iteration of its own (unfused apply)
 __global__ __launch_bounds__(256) void k_iter_finish(const double* __restrict__ part_delta,
                                                      const double* __restrict__ part_rsum,
-                                                     unsigned n, iter_ctl* __restrict__ ctl,
-                                                     double* __restrict__ deltas,
+                                                     unsigned n, double* __restrict__ deltas,
                                                      double* __restrict__ rsums) {
-  __shared__ double sd[256], sr[256];
-  if (ctl && ctl->done) return;
-  double d = 0.0, r = 0.0;
-  for (unsigned i = threadIdx.x; i < n; i += blockDim.x) {
-    d += part_delta[i];
-    r += part_rsum[i];
-  }
-  sd[threadIdx.x] = d;
-  sr[threadIdx.x] = r;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) {
-      sd[threadIdx.x] += sd[threadIdx.x + w];
-      sr[threadIdx.x] += sr[threadIdx.x + w];
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x != 0) return;
-  const double delta = sd[0], rs = sr[0];
-  if (!ctl) {
-    deltas[0] = delta;
-    rsums[0] = rs;
-    return;
-  }
-  const bool final_iter = (ctl->t + 1 == ctl->iters);
-  const uint32_t k = ctl->executed;
-  if (k < ctl->cap) {
-    deltas[k] = final_iter ? 0.0 : delta;
-    rsums[k] = rs;
-  }
-  ctl->executed = k + 1;
-  ctl->last_delta = final_iter ? 0.0 : delta;
-  ctl->cur ^= 1u;
-  if (final_iter) {
-    ctl->done = 1;
-    return;
-  }
-  uint32_t t = ctl->t;
-  const bool hit_eps = ctl->eps > 0.0 && delta < ctl->eps;
-  const bool hit_tol = ctl->l1tol > 0.0 && rs > 0.0 && (delta / rs) < ctl->l1tol;
-  if ((hit_eps || hit_tol) && ctl->iters >= 2) t = ctl->iters - 2;
-  ctl->t = t + 1;
+  iter_finish(part_delta, part_rsum, n, nullptr, deltas, rsums);
 }
 
 // ---- host side ------------------------------------------------------------------------------
@@ -457,17 +392,17 @@ static void launch_tiles_t(pe_graph_s* g, T* b0, T* b1, const rank_args& a, cons
     case 1024:
       k_pull_tiles<T, W, 256, 4><<<G, 256, 0, s>>>(g->col_ptr.p, g->row_idx.p, wn, g->tile_row.p,
                                                    g->tile_edge.p, g->num_tiles, b0, b1, g->od.p, a,
-                                                   ctl, tc, th, wk.part_delta, wk.part_rsum);
+                                                   ctl, tc, th, wk.part_delta, wk.part_rsum, wk.ticket());
       break;
     case 4096:
       k_pull_tiles<T, W, 256, 16><<<G, 256, 0, s>>>(g->col_ptr.p, g->row_idx.p, wn, g->tile_row.p,
                                                     g->tile_edge.p, g->num_tiles, b0, b1, g->od.p, a,
-                                                    ctl, tc, th, wk.part_delta, wk.part_rsum);
+                                                    ctl, tc, th, wk.part_delta, wk.part_rsum, wk.ticket());
       break;
     default:
       k_pull_tiles<T, W, 256, 8><<<G, 256, 0, s>>>(g->col_ptr.p, g->row_idx.p, wn, g->tile_row.p,
                                                    g->tile_edge.p, g->num_tiles, b0, b1, g->od.p, a,
-                                                   ctl, tc, th, wk.part_delta, wk.part_rsum);
+                                                   ctl, tc, th, wk.part_delta, wk.part_rsum, wk.ticket());
   }
   PE_HIP(hipGetLastError());
 }
@@ -478,38 +413,36 @@ static void launch_iteration_t(pe_graph_s* g, T* b0, T* b1, bool weighted, const
   hipStream_t s = g->ctx->stream;
   if (weighted) launch_tiles_t<T, true>(g, b0, b1, a, ctl, wk);
   else launch_tiles_t<T, false>(g, b0, b1, a, ctl, wk);
-  const uint64_t nshort = g->num_fix - g->num_fix_long, nlong = g->num_fix_long;
+  const uint64_t nshort = g->num_fix - g->num_fix_long;
   auto* tc = reinterpret_cast<cpair<T>*>(wk.tile_carry);
   auto* th = reinterpret_cast<cpair<T>*>(wk.tile_head);
-  {
-    ktime_scope kt(wk.timed ? g->ctx : nullptr, PE_KT_PULL_FIXUP);
-    k_pull_fixup_short<T><<<wk.fix_grid, 256, 0, s>>>(
-        g->fix_row.p, g->fix_t0.p, g->fix_t1.p, nshort, tc, th, b0, b1, g->od.p, a, ctl,
-        wk.part_delta + wk.tile_grid, wk.part_rsum + wk.tile_grid);
-    k_pull_fixup_long<T><<<wk.fix_grid, 256, 0, s>>>(
-        g->fix_row.p + nshort, g->fix_t0.p + nshort, g->fix_t1.p + nshort, nlong, tc, th, b0, b1,
-        g->od.p, a, ctl, wk.part_delta + wk.tile_grid + wk.fix_grid,
-        wk.part_rsum + wk.tile_grid + wk.fix_grid);
-  }
+  ktime_scope kt(wk.timed ? g->ctx : nullptr, PE_KT_PULL_FIXUP);
+  k_pull_fixup<T><<<wk.fix_grid + wk.long_grid, 256, 0, s>>>(
+      g->fix_row.p, g->fix_t0.p, g->fix_t1.p, nshort, g->num_fix, wk.fix_grid, tc, th, b0, b1, g->od.p, a, ctl,
+      wk.part_delta, wk.part_rsum, wk.tile_grid, wk.ticket(), deltas, rsums);
   PE_HIP(hipGetLastError());
-  k_iter_finish<<<1, 256, 0, s>>>(wk.part_delta, wk.part_rsum, wk.tile_grid + 2 * wk.fix_grid, ctl,
-                                  deltas, rsums);
-  PE_HIP(hipGetLastError());
+}
+
+// blocks of the fix-up's short and long part (none for an empty part, one at least in all)
+static void fix_grids(pe_graph_s* g, unsigned* short_grid, unsigned* long_grid) {
+  const uint64_t nshort = g->num_fix - g->num_fix_long;
+  *long_grid = g->num_fix_long ? persistent_grid(g->ctx, (g->num_fix_long + 3) / 4, 2) : 0u;
+  *short_grid = nshort || !*long_grid ? persistent_grid(g->ctx, std::max<uint64_t>(1, (nshort + 255) / 256), 2) : 0u;
 }
 
 void rank_work::init(pe_graph_s* g, int precision) {
   pe_ctx_s* ctx = g->ctx;
   const size_t pair_bytes = precision == 64 ? 16 : 8;
   tile_grid = persistent_grid(ctx, g->num_tiles, 8);
-  fix_grid = persistent_grid(ctx, std::max<uint64_t>(1, (g->num_fix + 255) / 256), 2);
+  fix_grids(g, &fix_grid, &long_grid);
   own_tiles.alloc(ctx, 2 * g->num_tiles * pair_bytes);
   tile_carry = own_tiles.p;
   tile_head = own_tiles.p + g->num_tiles * pair_bytes;
   pb_parts = 0;
   if (precision != 64 && g->pull_layout == PE_PULL_BINNED && g->pb)
     pb_parts = binned_grid_gather(g) + binned_grid_split(g);
-  const size_t parts = std::max<size_t>(tile_grid + 2 * fix_grid, pb_parts);
-  own_parts.alloc(ctx, 2 * parts + 2);
+  const size_t parts = std::max<size_t>(tile_grid + fix_grid + long_grid, pb_parts);
+  own_parts.alloc(ctx, 2 * parts + 3);
   part_delta = own_parts.p;
   part_rsum = own_parts.p + parts;
   scalars = own_parts.p + 2 * parts;
@@ -521,9 +454,10 @@ static uint64_t align256(uint64_t b) { return (b + 255) & ~255ull; }
 uint64_t rank_work::arena_bytes(pe_graph_s* g, int precision) {
   const uint64_t pair_bytes = precision == 64 ? 16 : 8;
   const uint64_t tg = persistent_grid(g->ctx, g->num_tiles, 8);
-  const uint64_t fg = persistent_grid(g->ctx, std::max<uint64_t>(1, (g->num_fix + 255) / 256), 2);
-  const uint64_t parts = tg + 2 * fg;
-  return 2 * align256(g->num_tiles * pair_bytes) + 2 * align256(parts * 8) + align256(16);
+  unsigned fg = 0, lg = 0;
+  fix_grids(g, &fg, &lg);
+  const uint64_t parts = tg + fg + lg;
+  return 2 * align256(g->num_tiles * pair_bytes) + 2 * align256(parts * 8) + align256(24);
 }
 
 void rank_work::init_in(pe_graph_s* g, int precision, uint8_t* arena, uint64_t cap) {
@@ -536,8 +470,8 @@ void rank_work::init_in(pe_graph_s* g, int precision, uint8_t* arena, uint64_t c
   }
   const uint64_t pair_bytes = precision == 64 ? 16 : 8;
   tile_grid = persistent_grid(g->ctx, g->num_tiles, 8);
-  fix_grid = persistent_grid(g->ctx, std::max<uint64_t>(1, (g->num_fix + 255) / 256), 2);
-  const uint64_t parts = tile_grid + 2 * fix_grid;
+  fix_grids(g, &fix_grid, &long_grid);
+  const uint64_t parts = tile_grid + fix_grid + long_grid;
   uint8_t* p = arena;
   tile_carry = p;
   p += align256(g->num_tiles * pair_bytes);
@@ -577,10 +511,7 @@ void rank_iteration(pe_graph_s* g, int precision, void* b0, void* b1, bool weigh
                     double* rsums) {
   if (precision != 64 && a.mode == MODE_APPLY && a.mass > 0.0 && g->pull_layout == PE_PULL_BINNED && g->pb) {
     PE_REQUIRE(wk.pb_parts > 0, PE_ERR_STATE, "pull layout changed after the iteration was set up");
-    binned_iteration(g, (float*)b0, (float*)b1, weighted, a, ctl, wk.part_delta, wk.part_rsum);
-    k_iter_finish<<<1, 256, 0, g->ctx->stream>>>(wk.part_delta, wk.part_rsum, wk.pb_parts, ctl, deltas,
-                                                 rsums);
-    PE_HIP(hipGetLastError());
+    binned_iteration(g, (float*)b0, (float*)b1, weighted, a, ctl, wk, deltas, rsums);
     return;
   }
   if (precision == 64)
@@ -600,8 +531,7 @@ void rank_apply_only(pe_graph_s* g, int precision, const void* x, void* y, const
     k_rank_apply<float><<<G, 256, 0, s>>>(g->V, (const float*)x, (float*)y, g->od.p, a,
                                           wk.part_delta, wk.part_rsum);
   PE_HIP(hipGetLastError());
-  k_iter_finish<<<1, 256, 0, s>>>(wk.part_delta, wk.part_rsum, G, nullptr, wk.scalars,
-                                  wk.scalars + 1);
+  k_iter_finish<<<1, 256, 0, s>>>(wk.part_delta, wk.part_rsum, G, wk.scalars, wk.scalars + 1);
   PE_HIP(hipGetLastError());
 }
 

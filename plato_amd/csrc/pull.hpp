@@ -97,14 +97,83 @@ __device__ __forceinline__ void block_reduce2(double& a, double& b, double* sm) 
   }
 }
 
+// End of an iteration, by one whole block of 256 threads: reduces the n partials in a fixed
+// order and advances the controller.  Plato's loop control (pagerank.hpp:100-146): after a
+// non-final iteration, delta < eps jumps to one more, final, iteration.  The optional
+// normalised tolerance does the same on delta / sum(rank).
+__device__ __forceinline__ void iter_finish(const double* part_delta, const double* part_rsum, unsigned n,
+                                            iter_ctl* ctl, double* deltas, double* rsums) {
+  __shared__ double sd[256], sr[256];
+  double d = 0.0, r = 0.0;
+  for (unsigned i = threadIdx.x; i < n; i += 256) {
+    d += part_delta[i];
+    r += part_rsum[i];
+  }
+  sd[threadIdx.x] = d;
+  sr[threadIdx.x] = r;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) {
+      sd[threadIdx.x] += sd[threadIdx.x + w];
+      sr[threadIdx.x] += sr[threadIdx.x + w];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x != 0) return;
+  const double delta = sd[0], rs = sr[0];
+  if (!ctl) {
+    deltas[0] = delta;
+    rsums[0] = rs;
+    return;
+  }
+  const bool final_iter = (ctl->t + 1 == ctl->iters);
+  const uint32_t k = ctl->executed;
+  if (k < ctl->cap) {
+    deltas[k] = final_iter ? 0.0 : delta;
+    rsums[k] = rs;
+  }
+  ctl->executed = k + 1;
+  ctl->last_delta = final_iter ? 0.0 : delta;
+  ctl->cur ^= 1u;
+  if (final_iter) {
+    ctl->done = 1;
+    return;
+  }
+  uint32_t t = ctl->t;
+  const bool hit_eps = ctl->eps > 0.0 && delta < ctl->eps;
+  const bool hit_tol = ctl->l1tol > 0.0 && rs > 0.0 && (delta / rs) < ctl->l1tol;
+  if ((hit_eps || hit_tol) && ctl->iters >= 2) t = ctl->iters - 2;
+  ctl->t = t + 1;
+}
+
+// Whether the calling block is the last of its grid to get here; its partials and those of all
+// other blocks, and of the kernels before, are then visible to it.  Every thread calls it;
+// thread 0 has written the block's partials.  *ticket starts at 0 and ends at 0.  The last
+// block of an iteration's last kernel finishes the iteration itself: a launch less.
+__device__ __forceinline__ bool last_block(uint32_t* ticket) {
+  __shared__ uint32_t s_last;
+  if (threadIdx.x == 0) {
+    __threadfence();  // the partials before the ticket
+    const uint32_t k = atomicAdd(ticket, 1u);
+    s_last = k + 1 == gridDim.x ? 1u : 0u;
+    if (s_last) {
+      *ticket = 0u;
+      __threadfence();  // the ticket before the others' partials
+    }
+  }
+  __syncthreads();
+  return s_last != 0u;
+}
+
 struct rank_work {
-  unsigned tile_grid = 0, fix_grid = 0;
+  unsigned tile_grid = 0, fix_grid = 0, long_grid = 0;
   unsigned pb_parts = 0;                     // partials of a binned iteration (0: not binned)
   uint8_t* tile_carry = nullptr;             // compensated pair per tile
   uint8_t* tile_head = nullptr;
   double* part_delta = nullptr;              // per-block partials
   double* part_rsum = nullptr;
-  double* scalars = nullptr;                 // delta, rank sum (engine-level calls)
+  double* scalars = nullptr;                 // delta, rank sum (engine-level calls), last_block ticket
+  uint32_t* ticket() const { return reinterpret_cast<uint32_t*>(scalars + 2); }
   bool timed = true;                         // per-kernel event timing allowed
   dbuf<uint8_t> own_tiles;                   // storage when init() allocates it
   dbuf<double> own_parts;
@@ -132,7 +201,7 @@ void rank_iteration(pe_graph_s* g, int precision, void* b0, void* b1, bool weigh
 unsigned binned_grid_gather(pe_graph_s* g);
 unsigned binned_grid_split(pe_graph_s* g);
 void binned_iteration(pe_graph_s* g, float* b0, float* b1, bool weighted, const rank_args& a, iter_ctl* ctl,
-                      double* part_delta, double* part_rsum);
+                      rank_work& wk, double* deltas, double* rsums);
 // Bound on the total contribution of state x (rank_args::mass) for a binned iteration;
 // 0 when x has a negative or non-finite source value (such states take the merge-path
 // gather).  Synchronizes the stream.

@@ -366,12 +366,13 @@ __global__ __launch_bounds__(THREADS) void k_pb_gather(
   }
 }
 
-// Bins summed by several units: apply from the global accumulators, then clear them.
+// Bins summed by several units: apply from the global accumulators, then clear them.  The
+// last block to end finishes the iteration.
 __global__ __launch_bounds__(256) void k_pb_apply_split(
     const uint32_t* __restrict__ split_bin, uint32_t nsplit, int dst_bits, int frac, uint32_t V,
     unsigned long long* __restrict__ acc, float* buf0, float* buf1, const uint32_t* __restrict__ od,
-    rank_args a, const iter_ctl* __restrict__ ctl, double* __restrict__ part_delta,
-    double* __restrict__ part_rsum) {
+    rank_args a, iter_ctl* ctl, double* part_delta, double* part_rsum, unsigned gather_grid, uint32_t* ticket,
+    double* __restrict__ deltas, double* __restrict__ rsums) {
   __shared__ double s_red[8];
   bool final_iter = a.final_iter;
   const float* x = buf0;
@@ -397,9 +398,10 @@ __global__ __launch_bounds__(256) void k_pb_apply_split(
   }
   block_reduce2<256>(delta, rsum, s_red);
   if (threadIdx.x == 0) {
-    part_delta[blockIdx.x] = delta;
-    part_rsum[blockIdx.x] = rsum;
+    part_delta[gather_grid + blockIdx.x] = delta;
+    part_rsum[gather_grid + blockIdx.x] = rsum;
   }
+  if (last_block(ticket)) iter_finish(part_delta, part_rsum, gather_grid + gridDim.x, ctl, deltas, rsums);
 }
 
 // Total contribution of a state x along the edges: sum over sources of od(u) * x(u)
@@ -754,8 +756,8 @@ void binned_build(pe_graph_s* g, const pe_binned_opts_t* opts) {
   L->acc.alloc(ctx, nacc);
   k_pb_zero<<<grid_for(nacc, 256, 65536), 256, 0, s>>>(L->acc.p, nacc);
   PE_HIP(hipGetLastError());
-  L->work.alloc(ctx, 4);
-  k_pb_zero<<<1, 256, 0, s>>>(reinterpret_cast<unsigned long long*>(L->work.p), 2);
+  L->work.alloc(ctx, 6);
+  k_pb_zero<<<1, 256, 0, s>>>(reinterpret_cast<unsigned long long*>(L->work.p), 3);
   PE_HIP(hipGetLastError());
   PE_HIP(hipStreamSynchronize(s));
   g->pb = std::move(L);
@@ -782,7 +784,9 @@ unsigned binned_grid_split(pe_graph_s* g) {
 }
 
 void binned_iteration(pe_graph_s* g, float* b0, float* b1, bool weighted, const rank_args& a, iter_ctl* ctl,
-                      double* part_delta, double* part_rsum) {
+                      rank_work& wk, double* deltas, double* rsums) {
+  double* part_delta = wk.part_delta;
+  double* part_rsum = wk.part_rsum;
   PE_REQUIRE(g->pb, PE_ERR_STATE, "binned layout not built");
   const pb_layout& L = *g->pb;
   PE_REQUIRE(!weighted || L.weighted, PE_ERR_STATE, "weighted iteration on a layout built without weights");
@@ -818,7 +822,7 @@ void binned_iteration(pe_graph_s* g, float* b0, float* b1, bool weighted, const 
                                                    part_rsum, L.work.p + 2);
     PE_HIP(hipGetLastError());
     k_pb_apply_split<<<gs, 256, 0, s>>>(L.split_bin.p, L.nsplit, (int)L.dst_bits, frac, g->V, L.acc.p, b0, b1, g->od.p,
-                                        a, ctl, part_delta + g2, part_rsum + g2);
+                                        a, ctl, part_delta, part_rsum, g2, L.work.p + 4, deltas, rsums);
     PE_HIP(hipGetLastError());
   }
 }

@@ -51,10 +51,7 @@ uint64_t active_edges_dev(pe_graph_s* g, const uint64_t* words, uint64_t nwords)
   PE_HIP(hipMemsetAsync(c.p, 0, 8, s));
   k_active_edges<<<grid_for(nwords, 256, 4096), 256, 0, s>>>(words, nwords, g->V, g->od.p, c.p);
   PE_HIP(hipGetLastError());
-  unsigned long long h = 0;
-  PE_HIP(hipMemcpyAsync(&h, c.p, 8, hipMemcpyDeviceToHost, s));
-  PE_HIP(hipStreamSynchronize(s));
-  return h;
+  return mail_post(g->ctx, c.p, 1, nullptr, 0)[0];
 }
 
 // Push scatter of PPR (personalized_pagerank.hpp:225-239): every vertex of the
@@ -209,47 +206,28 @@ struct rank_run {
     k_init_ctl<<<1, 1, 0, s>>>(ctl.p, c);
     PE_HIP(hipGetLastError());
     PE_HIP(hipEventRecord(ctx->t0, s));
+    // Plain launches: an iteration is two or three kernels of at least 4 us each, which the host
+    // stays ahead of; capturing and instantiating a graph of 16 iterations, replayed past the
+    // last one, took longer than small iterations themselves (RMAT scale 16, FP64, 20 iterations
+    // of 20 us: 0.87 ms a call; launched one by one, with the fix-up fused: 0.47 ms).  With a stopping rule
+    // the controller is read after every 8 iterations; those queued past the end return at once.
     const bool early = eps > 0.0 || l1tol > 0.0;
-    if (iters > 0) {
-      if (ctx->timing) {
-        // per-kernel events: plain launches
-        uint32_t left = iters;
-        while (left > 0) {
-          const uint32_t chunk = std::min<uint32_t>(left, 8);
-          for (uint32_t i = 0; i < chunk; ++i)
-            rank_iteration(g, prec, b0.p, b1.p, weighted, args, ctl.p, wk, deltas.p, rsums.p);
-          left -= chunk;
-          if (early) {
-            PE_HIP(hipMemcpyAsync(&host_ctl, ctl.p, sizeof(iter_ctl), hipMemcpyDeviceToHost, s));
-            PE_HIP(hipStreamSynchronize(s));
-            if (host_ctl.done) break;
-          }
-        }
-      } else {
-        // capture a chunk of iterations once, replay it until the controller is done
-        const uint32_t chunk = early ? std::min<uint32_t>(iters, 8) : std::min<uint32_t>(iters, 16);
-        stream_graph sg;  // destroyed after the stream drains, also on an exception
-        sg.begin(s);
-        for (uint32_t i = 0; i < chunk; ++i)
-          rank_iteration(g, prec, b0.p, b1.p, weighted, args, ctl.p, wk, deltas.p, rsums.p);
-        sg.end();
-        uint32_t launched = 0;
-        while (launched < iters) {
-          sg.launch();
-          launched += chunk;
-          if (early) {
-            PE_HIP(hipMemcpyAsync(&host_ctl, ctl.p, sizeof(iter_ctl), hipMemcpyDeviceToHost, s));
-            PE_HIP(hipStreamSynchronize(s));
-            if (host_ctl.done) break;
-          }
-        }
-        PE_HIP(hipStreamSynchronize(s));
+    constexpr uint32_t CTL_WORDS = sizeof(iter_ctl) / 8;
+    static_assert(sizeof(iter_ctl) % 8 == 0, "the controller travels as 8-byte words");
+    auto read_ctl = [&] {
+      std::memcpy(&host_ctl, mail_post(ctx, reinterpret_cast<const unsigned long long*>(ctl.p), CTL_WORDS, nullptr, 0),
+                  sizeof(iter_ctl));
+    };
+    for (uint32_t i = 0; i < iters; ++i) {
+      rank_iteration(g, prec, b0.p, b1.p, weighted, args, ctl.p, wk, deltas.p, rsums.p);
+      if (early && (i & 7) == 7) {
+        read_ctl();
+        if (host_ctl.done) break;
       }
     }
     PE_HIP(hipEventRecord(ctx->t1, s));
-    PE_HIP(hipMemcpyAsync(&host_ctl, ctl.p, sizeof(iter_ctl), hipMemcpyDeviceToHost, s));
+    read_ctl();
     PE_HIP(hipEventSynchronize(ctx->t1));
-    PE_HIP(hipStreamSynchronize(s));
     float ms = 0.f;
     PE_HIP(hipEventElapsedTime(&ms, ctx->t0, ctx->t1));
     seconds = ms * 1e-3;
@@ -288,6 +266,13 @@ static rank_args make_args(double damping, double base, double seed_mass, const 
   a.final_iter = p ? p->final_iter : 0;
   a.mode = MODE_APPLY;
   return a;
+}
+
+// one device double, after the work queued on the stream
+static double mail_double(pe_ctx_s* ctx, const double* d) {
+  double h;
+  std::memcpy(&h, mail_post(ctx, reinterpret_cast<const unsigned long long*>(d), 1, nullptr, 0), 8);
+  return h;
 }
 
 static int vec_prec(const pe_vec_s* v) { return v->dtype == PE_F64 ? 64 : 32; }
@@ -366,9 +351,7 @@ int pe_rank_apply(pe_graph_t* g, pe_vec_t* x, pe_vec_t* y, const pe_apply_params
     const rank_args a = make_args(p->damping, p->base, p->seed_mass, p->seeds ? p->seeds->p : nullptr,
                                   p->divide_by_od, p);
     rank_apply_only(g, vec_prec(x), x->p, y->p, a, wk);
-    double h = 0.0;
-    PE_HIP(hipMemcpyAsync(&h, wk.scalars, 8, hipMemcpyDeviceToHost, g->ctx->stream));
-    PE_HIP(hipStreamSynchronize(g->ctx->stream));
+    const double h = mail_double(g->ctx, wk.scalars);
     if (delta) *delta = h;
   });
 }
@@ -389,9 +372,7 @@ int pe_rank_iterate(pe_graph_t* g, pe_vec_t* x, pe_vec_t* y, int weighted, const
       a.mass = binned_mass_bound(g, (const float*)x->p, weighted != 0);
     rank_iteration(g, vec_prec(x), x->p, y->p, weighted != 0, a, nullptr, wk, wk.scalars,
                    wk.scalars + 1);
-    double h = 0.0;
-    PE_HIP(hipMemcpyAsync(&h, wk.scalars, 8, hipMemcpyDeviceToHost, g->ctx->stream));
-    PE_HIP(hipStreamSynchronize(g->ctx->stream));
+    const double h = mail_double(g->ctx, wk.scalars);
     if (delta) *delta = h;
   });
 }
@@ -558,9 +539,7 @@ int pe_ppr_pushpull(pe_graph_t* g, uint32_t src, const pe_rank_opts_t* opts, dou
         PE_HIP(hipGetLastError());
         rank_apply_only(g, prec, x, y, a, wk);
       }
-      double delta = 0.0;
-      PE_HIP(hipMemcpyAsync(&delta, wk.scalars, 8, hipMemcpyDeviceToHost, s));
-      PE_HIP(hipStreamSynchronize(s));
+      const double delta = mail_double(ctx, wk.scalars);
       if (modes) modes[executed] = do_pull ? 0 : 1;
       if (deltas) deltas[executed] = final_iter ? 0.0 : delta;
       last = final_iter ? 0.0 : delta;

@@ -1,0 +1,67 @@
+"""GPU: the blocks a context keeps for reuse.  A reused block must behave like a fresh one, what
+is kept is bounded, and it is given back with the context and when memory is asked for that
+only the kept blocks can make room for."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [1, 127, 128, 129, 100003, 1 << 20])
+def test_reused_blocks_start_clean(ctx, n):
+    from plato_amd import Bitmap, DenseState
+    for m in (n, n, max(1, n - n // 8)):  # the same size, and one that a kept block also serves
+        v = DenseState(ctx, m, np.float32)
+        assert not v.numpy().any()
+        v.fill(7.0)
+        assert (v.numpy() == 7.0).all()
+        v.close()
+        b = Bitmap(ctx, m)
+        assert b.count() == 0
+        b.fill()
+        assert b.count() == m
+        b.close()
+
+
+def test_results_do_not_depend_on_kept_blocks():
+    """Algorithms on graphs of several sizes in one context, each after the others have left
+    their blocks behind, against a context of their own."""
+    from plato_amd import Context, Graph
+    from plato_amd.algo import (bfs_opts_t, breadth_first_search, connected_components, hyperanf, hyperanf_opts_t,
+                                kcore, pagerank, pagerank_opts_t)
+
+    def run(c, scale):
+        g = Graph.rmat(c, scale, 8, seed=scale, directed=False, relabel=scale % 2 == 0)
+        out = [pagerank(g, pagerank_opts_t(7, 0.85, 0.0), precision=64).rank]
+        g.set_pull_layout("binned")
+        out += [pagerank(g, pagerank_opts_t(7, 0.85, 0.0)).rank, breadth_first_search(g, bfs_opts_t(1)).levels,
+                connected_components(g).labels, kcore(g).coreness, hyperanf(g, hyperanf_opts_t(20, 7)).anfs]
+        g.close()
+        return out
+
+    with Context(0) as shared:
+        for scale in (14, 9, 13, 14, 10):
+            got = run(shared, scale)
+            with Context(0) as own:
+                want = run(own, scale)
+            print(f"case: pool scale={scale}", flush=True)
+            for a, b in zip(got, want):
+                assert np.array_equal(a, b)
+
+
+def test_kept_blocks_are_bounded_and_given_back():
+    from plato_amd import Context, DenseState
+    with Context(0) as meter:  # allocates nothing, so its view of free memory is the device's
+        free0 = meter.mem_info()["free"]
+        c = Context(0)
+        for i in range(6):  # 0.3 to 0.4 GiB each, no two alike
+            DenseState(c, (80 + 4 * i) << 20, np.float32).close()
+        assert c.mem_info()["ctx"] == 0
+        kept = free0 - meter.mem_info()["free"]
+        assert kept < (1 << 30) + (256 << 20), kept
+        # a block larger than what is free beside the kept ones
+        big = (meter.mem_info()["free"] + (256 << 20)) // 4
+        v = DenseState(c, big, np.float32)
+        v.close()
+        c.close()
+        assert free0 - meter.mem_info()["free"] < 256 << 20
