@@ -246,16 +246,39 @@ __global__ void k_mail_post(const unsigned long long* __restrict__ src, uint32_t
                             unsigned long long* __restrict__ mail, unsigned long long seq) {
   for (uint32_t i = 0; i < n; ++i) mail[1 + i] = src[i];
   for (uint32_t i = 0; i < nclear; ++i) clear[i] = 0ull;
+  mail_deliver(mail, seq);
+}
+
+// The words of a small download to the mailbox (one block), then the sequence number.
+__global__ __launch_bounds__(1024) void k_mail_words(const uint32_t* __restrict__ src, uint32_t n,
+                                                     uint32_t* __restrict__ words, unsigned long long* mail,
+                                                     unsigned long long seq) {
+  for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) words[i] = src[i];
   __threadfence_system();
-  __hip_atomic_store(&mail[0], seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  __syncthreads();
+  if (threadIdx.x == 0) mail_deliver(mail, seq);
+}
+
+const uint32_t* mail_words(pe_ctx_s* ctx, const uint32_t* src, uint32_t n) {
+  PE_REQUIRE(n <= MAIL_WORDS, PE_ERR_INTERNAL, "mail_words: too many words");
+  uint32_t* words = reinterpret_cast<uint32_t*>(ctx->host_mail) + 1024;
+  const unsigned long long seq = mail_next(ctx);
+  k_mail_words<<<1, 1024, 0, ctx->stream>>>(src, n, words, ctx->host_mail, seq);
+  PE_HIP(hipGetLastError());
+  (void)mail_wait(ctx, seq);
+  return words;
 }
 
 const unsigned long long* mail_post(pe_ctx_s* ctx, const unsigned long long* src, uint32_t n,
                                     unsigned long long* clear, uint32_t nclear) {
   PE_REQUIRE(n <= 64, PE_ERR_INTERNAL, "mail_post: more than 64 words");
-  const unsigned long long seq = ++ctx->mail_seq;
+  const unsigned long long seq = mail_next(ctx);
   k_mail_post<<<1, 1, 0, ctx->stream>>>(src, n, clear, nclear, ctx->host_mail, seq);
   PE_HIP(hipGetLastError());
+  return mail_wait(ctx, seq);
+}
+
+const unsigned long long* mail_wait(pe_ctx_s* ctx, unsigned long long seq) {
   // poll the sequence number; every 1024 polls ask the stream, so that a failed kernel
   // ends the wait with its error instead of spinning
   for (uint64_t k = 1;; ++k) {
@@ -301,7 +324,7 @@ int pe_ctx_create(int device, pe_ctx_t** out) {
     PE_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
     ctx->num_cus = cus;
     PE_HIP(hipHostMalloc(&ctx->host_pinned, 4096, hipHostMallocDefault));
-    PE_HIP(hipHostMalloc(reinterpret_cast<void**>(&ctx->host_mail), 4096, hipHostMallocCoherent));
+    PE_HIP(hipHostMalloc(reinterpret_cast<void**>(&ctx->host_mail), 4096 + MAIL_WORDS * 4, hipHostMallocCoherent));
     ctx->host_mail[0] = 0ull;
     ctx->noalloc_scratch = pull_scratch_setup(device);  // with the device current
   });

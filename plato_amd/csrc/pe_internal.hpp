@@ -85,7 +85,7 @@ struct pe_ctx_s {
   void* host_pinned = nullptr;  // 4 KiB
   // coherent pinned host words that a one-thread kernel writes at the end of a step and
   // the host polls: a step's counters reach the host without a copy or a stream wait
-  unsigned long long* host_mail = nullptr;  // 4 KiB; [0] = sequence number, [1..] = words
+  unsigned long long* host_mail = nullptr;  // 4 KiB: [0] = sequence number, [1..] = words; then mail_words'
   unsigned long long mail_seq = 0;
   // this device's static scratch array of pe_pull_sum_noalloc (its device address)
   void* noalloc_scratch = nullptr;
@@ -111,6 +111,19 @@ void staged_download(pe_ctx_s* ctx, uint64_t units, size_t unit_bytes, const sta
 void host_download(pe_ctx_s* ctx, const void* dev, void* host, size_t bytes);
 void host_upload(pe_ctx_s* ctx, void* dev, const void* host, size_t bytes);
 void staging_free(staging* st);
+
+// The same in two halves, for a kernel that delivers its words itself as its last act: it calls
+// mail_deliver from one thread with mail_address(ctx) and a number from mail_next(ctx), and
+// mail_wait returns the host copy.
+// mail_words brings up to MAIL_WORDS 4-byte words the same way.
+static constexpr uint32_t MAIL_WORDS = 16384;
+const uint32_t* mail_words(pe_ctx_s* ctx, const uint32_t* src, uint32_t n);
+inline unsigned long long mail_next(pe_ctx_s* ctx) { return ++ctx->mail_seq; }
+const unsigned long long* mail_wait(pe_ctx_s* ctx, unsigned long long seq);
+__device__ __forceinline__ void mail_deliver(unsigned long long* mail, unsigned long long seq) {
+  __threadfence_system();
+  __hip_atomic_store(&mail[0], seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // Allocation through the context keeps a ledger (admission control reads it).
 void* dmalloc(pe_ctx_s* ctx, size_t bytes);

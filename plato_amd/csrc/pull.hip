@@ -304,7 +304,7 @@ __global__ __launch_bounds__(256) void k_pull_fixup(
     const uint32_t* __restrict__ fix_t1, uint64_t nshort, uint64_t n, unsigned short_grid,
     const cpair<T>* __restrict__ tile_carry, const cpair<T>* __restrict__ tile_head, T* buf0, T* buf1,
     const uint32_t* __restrict__ od, rank_args a, iter_ctl* ctl, double* part_delta, double* part_rsum,
-    unsigned tile_grid, uint32_t* ticket, double* __restrict__ deltas, double* __restrict__ rsums) {
+    unsigned tile_grid, uint32_t* ticket, double* __restrict__ deltas, double* __restrict__ rsums, iter_mail mail) {
   __shared__ double s_red[8];
   bool final_iter = false;
   const T* x = buf0;
@@ -348,7 +348,7 @@ __global__ __launch_bounds__(256) void k_pull_fixup(
     part_delta[tile_grid + blockIdx.x] = delta;
     part_rsum[tile_grid + blockIdx.x] = rsum;
   }
-  if (last_block(ticket)) iter_finish(part_delta, part_rsum, tile_grid + gridDim.x, ctl, deltas, rsums);
+  if (last_block(ticket)) iter_finish(part_delta, part_rsum, tile_grid + gridDim.x, ctl, deltas, rsums, mail);
 }
 
 // ---- unfused apply (pe_rank_apply) -------------------------------------------------------
@@ -373,8 +373,8 @@ __global__ __launch_bounds__(256) void k_rank_apply(uint32_t V, const T* __restr
 __global__ __launch_bounds__(256) void k_iter_finish(const double* __restrict__ part_delta,
                                                      const double* __restrict__ part_rsum,
                                                      unsigned n, double* __restrict__ deltas,
-                                                     double* __restrict__ rsums) {
-  iter_finish(part_delta, part_rsum, n, nullptr, deltas, rsums);
+                                                     double* __restrict__ rsums, iter_mail mail) {
+  iter_finish(part_delta, part_rsum, n, nullptr, deltas, rsums, mail);
 }
 
 // ---- host side ------------------------------------------------------------------------------
@@ -419,7 +419,7 @@ static void launch_iteration_t(pe_graph_s* g, T* b0, T* b1, bool weighted, const
   ktime_scope kt(wk.timed ? g->ctx : nullptr, PE_KT_PULL_FIXUP);
   k_pull_fixup<T><<<wk.fix_grid + wk.long_grid, 256, 0, s>>>(
       g->fix_row.p, g->fix_t0.p, g->fix_t1.p, nshort, g->num_fix, wk.fix_grid, tc, th, b0, b1, g->od.p, a, ctl,
-      wk.part_delta, wk.part_rsum, wk.tile_grid, wk.ticket(), deltas, rsums);
+      wk.part_delta, wk.part_rsum, wk.tile_grid, wk.ticket(), deltas, rsums, wk.mail);
   PE_HIP(hipGetLastError());
 }
 
@@ -531,7 +531,7 @@ void rank_apply_only(pe_graph_s* g, int precision, const void* x, void* y, const
     k_rank_apply<float><<<G, 256, 0, s>>>(g->V, (const float*)x, (float*)y, g->od.p, a,
                                           wk.part_delta, wk.part_rsum);
   PE_HIP(hipGetLastError());
-  k_iter_finish<<<1, 256, 0, s>>>(wk.part_delta, wk.part_rsum, G, wk.scalars, wk.scalars + 1);
+  k_iter_finish<<<1, 256, 0, s>>>(wk.part_delta, wk.part_rsum, G, wk.scalars, wk.scalars + 1, wk.mail);
   PE_HIP(hipGetLastError());
 }
 

@@ -101,8 +101,14 @@ __device__ __forceinline__ void block_reduce2(double& a, double& b, double* sm) 
 // order and advances the controller.  Plato's loop control (pagerank.hpp:100-146): after a
 // non-final iteration, delta < eps jumps to one more, final, iteration.  The optional
 // normalised tolerance does the same on delta / sum(rank).
+// Without a controller the delta also goes to the host's mailbox when the call waits for it.
+struct iter_mail {
+  unsigned long long* mail = nullptr;
+  unsigned long long seq = 0;
+};
+
 __device__ __forceinline__ void iter_finish(const double* part_delta, const double* part_rsum, unsigned n,
-                                            iter_ctl* ctl, double* deltas, double* rsums) {
+                                            iter_ctl* ctl, double* deltas, double* rsums, iter_mail m) {
   __shared__ double sd[256], sr[256];
   double d = 0.0, r = 0.0;
   for (unsigned i = threadIdx.x; i < n; i += 256) {
@@ -124,6 +130,10 @@ __device__ __forceinline__ void iter_finish(const double* part_delta, const doub
   if (!ctl) {
     deltas[0] = delta;
     rsums[0] = rs;
+    if (m.mail) {
+      m.mail[1] = (unsigned long long)__double_as_longlong(delta);
+      mail_deliver(m.mail, m.seq);
+    }
     return;
   }
   const bool final_iter = (ctl->t + 1 == ctl->iters);
@@ -175,6 +185,7 @@ struct rank_work {
   double* scalars = nullptr;                 // delta, rank sum (engine-level calls), last_block ticket
   uint32_t* ticket() const { return reinterpret_cast<uint32_t*>(scalars + 2); }
   bool timed = true;                         // per-kernel event timing allowed
+  iter_mail mail;                            // of an engine call that waits for its delta
   dbuf<uint8_t> own_tiles;                   // storage when init() allocates it
   dbuf<double> own_parts;
   void init(pe_graph_s* g, int precision);

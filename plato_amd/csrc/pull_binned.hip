@@ -372,7 +372,7 @@ __global__ __launch_bounds__(256) void k_pb_apply_split(
     const uint32_t* __restrict__ split_bin, uint32_t nsplit, int dst_bits, int frac, uint32_t V,
     unsigned long long* __restrict__ acc, float* buf0, float* buf1, const uint32_t* __restrict__ od,
     rank_args a, iter_ctl* ctl, double* part_delta, double* part_rsum, unsigned gather_grid, uint32_t* ticket,
-    double* __restrict__ deltas, double* __restrict__ rsums) {
+    double* __restrict__ deltas, double* __restrict__ rsums, iter_mail mail) {
   __shared__ double s_red[8];
   bool final_iter = a.final_iter;
   const float* x = buf0;
@@ -401,7 +401,7 @@ __global__ __launch_bounds__(256) void k_pb_apply_split(
     part_delta[gather_grid + blockIdx.x] = delta;
     part_rsum[gather_grid + blockIdx.x] = rsum;
   }
-  if (last_block(ticket)) iter_finish(part_delta, part_rsum, gather_grid + gridDim.x, ctl, deltas, rsums);
+  if (last_block(ticket)) iter_finish(part_delta, part_rsum, gather_grid + gridDim.x, ctl, deltas, rsums, mail);
 }
 
 // Total contribution of a state x along the edges: sum over sources of od(u) * x(u)
@@ -822,7 +822,7 @@ void binned_iteration(pe_graph_s* g, float* b0, float* b1, bool weighted, const 
                                                    part_rsum, L.work.p + 2);
     PE_HIP(hipGetLastError());
     k_pb_apply_split<<<gs, 256, 0, s>>>(L.split_bin.p, L.nsplit, (int)L.dst_bits, frac, g->V, L.acc.p, b0, b1, g->od.p,
-                                        a, ctl, part_delta, part_rsum, g2, L.work.p + 4, deltas, rsums);
+                                        a, ctl, part_delta, part_rsum, g2, L.work.p + 4, deltas, rsums, wk.mail);
     PE_HIP(hipGetLastError());
   }
 }

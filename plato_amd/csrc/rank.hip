@@ -268,10 +268,11 @@ static rank_args make_args(double damping, double base, double seed_mass, const 
   return a;
 }
 
-// one device double, after the work queued on the stream
-static double mail_double(pe_ctx_s* ctx, const double* d) {
+// the delta that the kernels of an iteration with wk.mail deliver
+static void mail_expect(pe_ctx_s* ctx, rank_work& wk) { wk.mail = iter_mail{ctx->host_mail, mail_next(ctx)}; }
+static double mail_delta(pe_ctx_s* ctx, const rank_work& wk) {
   double h;
-  std::memcpy(&h, mail_post(ctx, reinterpret_cast<const unsigned long long*>(d), 1, nullptr, 0), 8);
+  std::memcpy(&h, mail_wait(ctx, wk.mail.seq), 8);
   return h;
 }
 
@@ -314,9 +315,10 @@ int pe_pull_sum(pe_graph_t* g, pe_vec_t* x, pe_vec_t* y, int weighted) {
     wk.init(g, vec_prec(x));
     rank_args a = make_args(1.0, 0.0, 0.0, nullptr, 0, nullptr);
     a.mode = MODE_RAW_SUM;
+    mail_expect(g->ctx, wk);
     rank_iteration(g, vec_prec(x), x->p, y->p, weighted != 0, a, nullptr, wk, wk.scalars,
                    wk.scalars + 1);
-    PE_HIP(hipStreamSynchronize(g->ctx->stream));
+    (void)mail_delta(g->ctx, wk);
   });
 }
 
@@ -350,8 +352,9 @@ int pe_rank_apply(pe_graph_t* g, pe_vec_t* x, pe_vec_t* y, const pe_apply_params
     wk.init(g, vec_prec(x));
     const rank_args a = make_args(p->damping, p->base, p->seed_mass, p->seeds ? p->seeds->p : nullptr,
                                   p->divide_by_od, p);
+    mail_expect(g->ctx, wk);
     rank_apply_only(g, vec_prec(x), x->p, y->p, a, wk);
-    const double h = mail_double(g->ctx, wk.scalars);
+    const double h = mail_delta(g->ctx, wk);
     if (delta) *delta = h;
   });
 }
@@ -370,9 +373,10 @@ int pe_rank_iterate(pe_graph_t* g, pe_vec_t* x, pe_vec_t* y, int weighted, const
                             p->divide_by_od, p);
     if (vec_prec(x) == 32 && g->pull_layout == PE_PULL_BINNED && g->pb)
       a.mass = binned_mass_bound(g, (const float*)x->p, weighted != 0);
+    mail_expect(g->ctx, wk);
     rank_iteration(g, vec_prec(x), x->p, y->p, weighted != 0, a, nullptr, wk, wk.scalars,
                    wk.scalars + 1);
-    const double h = mail_double(g->ctx, wk.scalars);
+    const double h = mail_delta(g->ctx, wk);
     if (delta) *delta = h;
   });
 }
@@ -513,6 +517,7 @@ int pe_ppr_pushpull(pe_graph_t* g, uint32_t src, const pe_rank_opts_t* opts, dou
       const bool final_iter = (opts->iterations - 1 == t);
       a.final_iter = final_iter ? 1 : 0;
       if (!do_pull) do_pull = active_edges_dev(g, active.p, nwords) > Ep / 20;  // (188-205)
+      mail_expect(ctx, wk);
       if (do_pull) {
         rank_iteration(g, prec, x, y, false, a, nullptr, wk, wk.scalars, wk.scalars + 1);
       } else {
@@ -539,7 +544,7 @@ int pe_ppr_pushpull(pe_graph_t* g, uint32_t src, const pe_rank_opts_t* opts, dou
         PE_HIP(hipGetLastError());
         rank_apply_only(g, prec, x, y, a, wk);
       }
-      const double delta = mail_double(ctx, wk.scalars);
+      const double delta = mail_delta(ctx, wk);
       if (modes) modes[executed] = do_pull ? 0 : 1;
       if (deltas) deltas[executed] = final_iter ? 0.0 : delta;
       last = final_iter ? 0.0 : delta;

@@ -24,7 +24,9 @@ static constexpr int ST_SLOTS = 8;
 static constexpr size_t ST_BYTES = 2u << 20;      // per slot
 static constexpr unsigned ST_THREADS = 6;         // workers at most
 static constexpr uint64_t ST_INLINE_CHUNKS = 3;   // up to this many the calling thread moves alone
-static constexpr size_t ST_SMALL = 256u << 10;    // the runtime's own copy is as fast up to here
+static constexpr size_t ST_SMALL = 256u << 10;    // the runtime's own copy is as fast up to here; up to
+                                                  // MAIL_WORDS words come by mail (nine engine calls and
+                                                  // two results of 16 KB: 312 -> 239 us with theirs)
 
 struct staging {
   uint8_t* ring = nullptr;
@@ -130,6 +132,10 @@ void staged_download(pe_ctx_s* ctx, uint64_t units, size_t unit_bytes, const sta
 }
 
 void host_download(pe_ctx_s* ctx, const void* dev, void* host, size_t bytes) {
+  if (bytes && bytes <= MAIL_WORDS * 4 && bytes % 4 == 0) {
+    std::memcpy(host, mail_words(ctx, static_cast<const uint32_t*>(dev), (uint32_t)(bytes / 4)), bytes);
+    return;
+  }
   if (bytes <= ST_SMALL) {
     if (bytes) PE_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, ctx->stream));
     PE_HIP(hipStreamSynchronize(ctx->stream));
