@@ -525,6 +525,166 @@ __global__ __launch_bounds__(256) void k_reached_edges(const uint32_t* __restric
   block_add2(acc, cntv, out, out + 1);
 }
 
+// ---- small graphs: a whole search in one block -------------------------------------------------
+// A search of a graph that a few thousand lanes cover is all launches and waits: three to
+// six kernels and a mail per level, about 30 us.  Here one block of SMALL_THREADS threads runs
+// it to the end: same levels, same push/pull rule, same counters.  Levels are read past the
+// L1 (relaxed atomic loads), since claims are made in L2.  The line, whole calls on RMAT graphs
+// in one block and level by level: 40 K entries 100 and 279 us, 66 K 140 and 268, 131 K
+// (16 K vertices, 6 levels) 289 and 333, 320 K 297 and 295, 640 K 585 and 313 us.
+static constexpr uint64_t SMALL_NNZ = 1ull << 17;
+static constexpr uint32_t SMALL_V = 1u << 15;  // a pull looks at every vertex
+static constexpr int SMALL_THREADS = 1024;
+static constexpr uint32_t SMALL_WAVE_DEG = 1024;  // longer lists take the whole block
+static constexpr uint32_t SMALL_LANE_DEG = 64;    // a pull lane scans that many in-edges, then a wave goes on
+static constexpr uint32_t SMALL_LISTS = SMALL_NNZ / SMALL_WAVE_DEG + 1;
+static constexpr uint32_t SMALL_MAIL_EPOCHS = 18;  // epochs whose log entries fit the mail
+
+struct bfs_small_out {
+  unsigned long long epochs, visited, reached_edges, alg_bytes;
+};
+struct bfs_small_log {
+  unsigned long long frontier, active, push;
+};
+
+__device__ __forceinline__ uint32_t level_of(const uint32_t* level, uint32_t v) {
+  return __hip_atomic_load(&level[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ __launch_bounds__(SMALL_THREADS) void k_bfs_small(
+    const uint64_t* __restrict__ col_ptr, const uint32_t* __restrict__ row_idx, const uint64_t* __restrict__ csr_ptr,
+    const uint32_t* __restrict__ csr_idx, const uint32_t* __restrict__ od, uint32_t V, uint32_t root, double Ep,
+    double threshold, uint32_t max_epochs, uint32_t* level, uint32_t* q0, uint32_t* q1, uint32_t* heavy,
+    bfs_small_log* log, unsigned long long* mail, unsigned long long seq) {
+  __shared__ uint32_t s_next, s_heavy, s_lists;
+  __shared__ uint32_t s_list[SMALL_LISTS];
+  __shared__ unsigned long long s_active, s_examined;
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr uint32_t WAVES = SMALL_THREADS / 64;
+  for (uint32_t v = tid; v < V; v += SMALL_THREADS) level[v] = v == root ? 0u : UNVIS;
+  if (tid == 0) q0[0] = root;
+  __threadfence();
+  uint32_t* qc = q0;
+  uint32_t* qn = q1;
+  uint32_t n = 1, epoch = 0;
+  unsigned long long A = od[root];
+  bfs_small_out out{0, 1, A, 0};
+  while (n != 0) {  // n, A and the choice are the same in every thread
+    const bool push = (double)A / Ep < threshold;  // dualmode.hpp:279
+    if (tid == 0) {
+      if (epoch < max_epochs) log[epoch] = bfs_small_log{n, A, push ? 1ull : 0ull};
+      s_next = 0;
+      s_heavy = 0;
+      s_lists = 0;
+      s_active = 0;
+      s_examined = 0;
+    }
+    __syncthreads();
+    const uint32_t L = epoch + 1;
+    unsigned long long active = 0, examined = 0;
+    // the claimed lanes' vertices to the next queue
+    auto append = [&](bool claimed, uint32_t w) {
+      const uint64_t m = __ballot(claimed);
+      if (!m) return;
+      uint32_t at = 0;
+      const int first = __ffsll((unsigned long long)m) - 1;
+      if ((int)lane == first) at = atomicAdd(&s_next, (uint32_t)__popcll(m));
+      at = (uint32_t)__shfl((int)at, first, 64);
+      if (claimed) {
+        qn[at + wave_prefix(m)] = w;
+        active += od[w];
+      }
+    };
+    if (push) {
+      auto edges = [&](uint32_t v, uint32_t i0, uint32_t step) {  // i0, step: multiples of 64 apart per wave
+        const uint64_t b = csr_ptr[v], e = csr_ptr[v + 1];
+        for (uint64_t k0 = b + (i0 & ~63u); k0 < e; k0 += step) {
+          const uint64_t k = k0 + lane;
+          bool claimed = false;
+          uint32_t w = 0;
+          if (k < e) {
+            w = csr_idx[k];
+            claimed = level_of(level, w) == UNVIS && atomicCAS(&level[w], UNVIS, L) == UNVIS;
+          }
+          append(claimed, w);
+        }
+      };
+      for (uint32_t q = wave; q < n; q += WAVES) {
+        const uint32_t v = qc[q];
+        if (csr_ptr[v + 1] - csr_ptr[v] > SMALL_WAVE_DEG) {
+          if (lane == 0) s_list[atomicAdd(&s_lists, 1u)] = v;
+        } else {
+          edges(v, 0u, 64u);
+        }
+      }
+      __syncthreads();
+      for (uint32_t i = 0; i < s_lists; ++i) edges(s_list[i], tid, SMALL_THREADS);
+    } else {
+      auto hit_at = [&](uint32_t u) { return level_of(level, u) == L - 1; };
+      for (uint32_t v0 = wave * 64; v0 < V; v0 += SMALL_THREADS) {
+        const uint32_t v = v0 + lane;
+        bool claimed = false, more = false;
+        if (v < V && level_of(level, v) == UNVIS) {
+          const uint64_t b = col_ptr[v], e = col_ptr[v + 1];
+          const uint64_t lim = std::min<uint64_t>(e, b + SMALL_LANE_DEG);
+          uint64_t k = b;
+          for (; k < lim && !claimed; ++k) claimed = hit_at(row_idx[k]);
+          examined += k - b;
+          more = !claimed && lim < e;
+          if (claimed) level[v] = L;
+        }
+        append(claimed, v);
+        if (more) heavy[atomicAdd(&s_heavy, 1u)] = v;
+      }
+      __syncthreads();
+      for (uint32_t h = wave; h < s_heavy; h += WAVES) {
+        const uint32_t v = heavy[h];
+        const uint64_t b = col_ptr[v] + SMALL_LANE_DEG, e = col_ptr[v + 1];
+        uint64_t scanned = e - b;
+        bool found = false;
+        for (uint64_t k0 = b; k0 < e && !found; k0 += 64) {
+          const bool hit = k0 + lane < e && hit_at(row_idx[k0 + lane]);
+          const uint64_t m = __ballot(hit);
+          found = m != 0ull;
+          if (found) scanned = k0 - b + (uint64_t)__builtin_ctzll(m) + 1;
+        }
+        if (lane == 0) examined += scanned;
+        if (found && lane == 0) level[v] = L;
+        append(found && lane == 0, v);
+      }
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+      active += __shfl_down(active, off, 64);
+      examined += __shfl_down(examined, off, 64);
+    }
+    if (lane == 0 && active) atomicAdd(&s_active, active);
+    if (lane == 0 && examined) atomicAdd(&s_examined, examined);
+    __threadfence();  // this level's stores are in L2
+    __syncthreads();
+    const uint32_t found = s_next;
+    out.alg_bytes += push ? 8ull * n + 4ull * A + 4ull * found
+                          : 8ull * (V - out.visited) + 4ull * s_examined + (unsigned long long)V / 8;
+    n = found;
+    A = s_active;
+    out.visited += n;
+    out.reached_edges += A;
+    ++epoch;
+    uint32_t* t = qc;
+    qc = qn;
+    qn = t;
+    __syncthreads();  // everyone has read the counters
+  }
+  if (tid < SMALL_MAIL_EPOCHS && tid < epoch && tid < max_epochs)
+    *reinterpret_cast<bfs_small_log*>(mail + 1 + sizeof(bfs_small_out) / 8 + tid * (sizeof(bfs_small_log) / 8)) = log[tid];
+  __threadfence_system();
+  __syncthreads();
+  if (tid == 0) {
+    out.epochs = epoch;
+    *reinterpret_cast<bfs_small_out*>(mail + 1) = out;
+    mail_deliver(mail, seq);
+  }
+}
+
 // Device state of one BFS engine, reused across roots.
 // top-down levels with at most this many active edges append to a queue (one wave per
 // vertex); larger ones run edge-balanced and leave the next frontier as a bitmap
@@ -684,13 +844,49 @@ struct bfs_state {
   }
 };
 
+static void bfs_small(pe_graph_s* g, uint32_t root, double threshold, int32_t* levels, uint8_t* modes,
+                      uint64_t* frontier, uint64_t* actv, uint32_t max_epochs, pe_bfs_stats_t* stats) {
+  pe_ctx_s* ctx = g->ctx;
+  hipStream_t s = ctx->stream;
+  const uint32_t V = g->V, cap = std::min<uint32_t>(max_epochs, V + 1);  // a search has at most V + 1 epochs
+  dbuf<uint32_t> buf(ctx, 4ull * V);  // levels, two queues, the vertices that a wave goes on with
+  dbuf<bfs_small_log> log(ctx, std::max<uint32_t>(1, cap));
+  static_assert(1 + sizeof(bfs_small_out) / 8 + SMALL_MAIL_EPOCHS * (sizeof(bfs_small_log) / 8) <= 64, "one mail");
+  const double Ep = (double)(g->directed ? g->edges : g->edges * 2);  // dualmode.hpp:261-262
+  const unsigned long long seq = mail_next(ctx);
+  PE_HIP(hipEventRecord(ctx->t0, s));
+  k_bfs_small<<<1, SMALL_THREADS, 0, s>>>(g->col_ptr.p, g->row_idx.p, g->csr_ptr(), g->csr_idx(), g->od.p, V, root, Ep,
+                                          threshold, cap, buf.p, buf.p + V, buf.p + 2ull * V, buf.p + 3ull * V, log.p,
+                                          ctx->host_mail, seq);
+  PE_HIP(hipGetLastError());
+  PE_HIP(hipEventRecord(ctx->t1, s));
+  const unsigned long long* h = mail_wait(ctx, seq);
+  const bfs_small_out out = *reinterpret_cast<const bfs_small_out*>(h);
+  std::vector<bfs_small_log> l(std::min<uint64_t>(out.epochs, cap));
+  std::memcpy(l.data(), h + sizeof(bfs_small_out) / 8,
+              std::min<size_t>(l.size(), SMALL_MAIL_EPOCHS) * sizeof(bfs_small_log));
+  if (l.size() > SMALL_MAIL_EPOCHS) host_download(ctx, log.p, l.data(), l.size() * sizeof(bfs_small_log));
+  for (size_t e = 0; e < l.size(); ++e) {
+    if (modes) modes[e] = (uint8_t)l[e].push;
+    if (frontier) frontier[e] = l[e].frontier;
+    if (actv) actv[e] = l[e].active;
+  }
+  if (levels) download_external(g, buf.p, levels, 4);
+  PE_HIP(hipEventSynchronize(ctx->t1));
+  float ms = 0.f;
+  PE_HIP(hipEventElapsedTime(&ms, ctx->t0, ctx->t1));
+  if (stats) {
+    stats->epochs = (uint32_t)out.epochs;
+    stats->visited = (uint32_t)out.visited;
+    stats->reached_edges = out.reached_edges;
+    stats->seconds = ms * 1e-3;
+    stats->alg_bytes = out.alg_bytes;
+  }
+}
+
 }  // namespace pe
 
 using namespace pe;
-
-extern "C" {
-
-}  // extern "C"
 
 struct pe_bfs_s {
   pe_graph_s* g;
@@ -806,6 +1002,10 @@ int pe_bfs(pe_graph_t* g, uint32_t root, double threshold, int32_t* levels, uint
     PE_REQUIRE(root < g->V, PE_ERR_RANGE, "root >= V");
     uint32_t iroot = root;
     to_internal_ids(g, &root, 1, &iroot);
+    if (g->nnz <= SMALL_NNZ && g->V <= SMALL_V && g->has_csr && !g->ctx->timing) {
+      bfs_small(g, iroot, threshold, levels, modes, frontier, active_edges, max_epochs, stats);
+      return;
+    }
     bfs_state st(g);
     double secs = 0.0;
     const int epochs = st.run(iroot, threshold, modes, frontier, active_edges, max_epochs, &secs);

@@ -192,3 +192,59 @@ def test_bfs_forced_direction_rmat(ctx, threshold):
         for root in [int(cand[0]), int(cand[len(cand) // 2]), int(np.argmax(og.od))]:
             res = _check_bfs(g, og, root, threshold)
             assert set(res.modes.tolist()) == ({1} if threshold > 1 else {0})
+
+
+@pytest.mark.parametrize("kind", ["path", "star", "hubs", "edge_of_range", "self_loops"])
+@pytest.mark.parametrize("directed", [False, True])
+def test_small_graphs_in_one_block(ctx, kind, directed):
+    """Searches that run whole in one block, at its edges: more levels than one mail holds,
+    lists around the 64 entries of a pull lane and the 1024 of a push wave, the largest graph
+    (2^17 entries, 2^15 vertices) and the first beyond it, vertices without edges."""
+    from plato_amd import Graph
+    from plato_amd.algo import bfs_opts_t, breadth_first_search
+    rng = np.random.default_rng(7)
+    sizes = [0]
+    if kind == "edge_of_range":
+        sizes = [0, 1]
+    for extra in sizes:
+        if kind == "path":
+            V = 700
+            s, d = np.arange(V - 1), np.arange(1, V)
+        elif kind == "star":
+            V = 3000
+            s, d = np.zeros(V - 1, int), np.arange(1, V)
+        elif kind == "hubs":
+            V = 6000
+            s = np.concatenate([np.full(n, 5000 + i) for i, n in enumerate((64, 65, 1024, 1025, 2600))] + [rng.integers(0, 5000, 2000)])
+            d = np.concatenate([rng.choice(5000, n, replace=False) for n in (64, 65, 1024, 1025, 2600)] + [rng.integers(0, 5010, 2000)])
+            if directed:  # long lists in both directions
+                s, d = np.concatenate([s, d]), np.concatenate([d, s])
+        elif kind == "edge_of_range":
+            V = (1 << 15) + (extra if directed else 0)
+            E = (1 << 17) // (1 if directed else 2) + extra
+            s, d = rng.integers(0, V, E), rng.integers(0, V, E)
+        else:
+            V = 9
+            s, d = np.array([0, 0, 1, 3, 3]), np.array([0, 1, 1, 3, 3])
+        s, d = s.astype(np.uint32), d.astype(np.uint32)
+        og = oracle.CSC(V, s, d, symmetrize=not directed)
+        g = Graph.from_edges(ctx, s, d, V, directed=directed, build_csr=True, relabel=kind == "hubs")
+        print(f"case: bfs small {kind} V={V} nnz={g.nnz} directed={directed}", flush=True)
+        for root in {0, V // 2, V - 1, int(np.argmax(og.od))}:
+            for threshold in (0.05, 0.0, 2.0):  # the rule, always pull, always push
+                res = breadth_first_search(g, bfs_opts_t(root), push_threshold=threshold)
+                ref = oracle.bfs(og, root, threshold)
+                assert np.array_equal(res.levels, ref["levels"])
+                assert res.epochs == ref["epochs"] and np.array_equal(res.modes, ref["modes"])
+                assert np.array_equal(res.frontier, ref["frontier"])
+                assert np.array_equal(res.active_edges, ref["active_edges"])
+                assert res.visited == ref["visited"]
+                assert res.reached_edges == int(og.od[ref["levels"] >= 0].sum())
+                ctx.set_kernel_timing(True)  # timed searches run level by level
+                by_level = breadth_first_search(g, bfs_opts_t(root), push_threshold=threshold)
+                ctx.set_kernel_timing(False)
+                assert np.array_equal(res.levels, by_level.levels) and res.alg_bytes == by_level.alg_bytes
+                if not g.info.relabeled:  # how far a list is read depends on the order of its ids
+                    assert res.alg_bytes == _alg_bytes(og, ref["levels"], ref["modes"], ref["frontier"],
+                                                       ref["active_edges"])
+        g.close()
