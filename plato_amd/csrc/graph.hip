@@ -129,11 +129,52 @@ static void split_keys(hipStream_t s, const uint64_t* keys, uint64_t nnz, int b,
   PE_HIP(hipGetLastError());
 }
 
-__global__ void k_out_degrees(const uint32_t* __restrict__ row_idx, uint64_t nnz,
-                              uint32_t* __restrict__ od) {
-  for (uint64_t e = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; e < nnz;
-       e += (uint64_t)gridDim.x * blockDim.x)
-    atomicAdd(&od[row_idx[e]], 1u);
+// Occurrences of every id in a list.  The ids of hubs come up so often that their atomics
+// serialize in the memory-side unit, so a block counts the first OD_SLOTS ids that hash to
+// different slots in LDS and sends only the others, and its counts at the end, to memory
+// (RMAT scale 24, 2 * 2^28 ids: 62 ms with an atomic each, 50 ms;
+// bound by the rest's atomics, 6 G/s).
+static constexpr uint32_t OD_SLOTS = 4096;
+static constexpr int OD_THREADS = 512;
+__global__ __launch_bounds__(OD_THREADS) void k_count_ids(const uint32_t* __restrict__ ids, uint64_t n,
+                                                          uint32_t* __restrict__ count) {
+  __shared__ uint32_t s_id[OD_SLOTS], s_n[OD_SLOTS];
+  for (uint32_t i = threadIdx.x; i < OD_SLOTS; i += OD_THREADS) {
+    s_id[i] = 0xFFFFFFFFu;  // no vertex: ids are below V <= 2^32 - 1
+    s_n[i] = 0u;
+  }
+  __syncthreads();
+  auto add = [&](uint32_t id) {
+    const uint32_t slot = (id * 2654435761u) >> 20;
+    uint32_t have = s_id[slot];
+    if (have == 0xFFFFFFFFu) have = atomicCAS(&s_id[slot], 0xFFFFFFFFu, id);
+    if (have == 0xFFFFFFFFu || have == id) atomicAdd(&s_n[slot], 1u);
+    else atomicAdd(&count[id], 1u);
+  };
+  // whole groups of four ids (the list starts on a 16-byte boundary), then the rest
+  const uint64_t n4 = n / 4, stride = (uint64_t)gridDim.x * OD_THREADS, tid = blockIdx.x * (uint64_t)OD_THREADS + threadIdx.x;
+  for (uint64_t i = tid; i < n4; i += stride) {
+    const uint4 q = reinterpret_cast<const uint4*>(ids)[i];
+    add(q.x);
+    add(q.y);
+    add(q.z);
+    add(q.w);
+  }
+  if (tid < (n & 3)) add(ids[n4 * 4 + tid]);
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < OD_SLOTS; i += OD_THREADS)
+    if (s_n[i]) atomicAdd(&count[s_id[i]], s_n[i]);
+}
+
+static void count_ids(pe_ctx_s* ctx, const uint32_t* ids, uint64_t n, uint32_t* count) {
+  if (!n) return;
+  k_count_ids<<<persistent_grid(ctx, grid_for(n, OD_THREADS * 16), 4), OD_THREADS, 0, ctx->stream>>>(ids, n, count);
+  PE_HIP(hipGetLastError());
+}
+
+__global__ void k_zero_u32(uint32_t* __restrict__ p, uint64_t n) {
+  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
+    p[i] = 0u;
 }
 
 __global__ void k_row_lengths(const uint64_t* __restrict__ ptr, uint32_t V, uint32_t* __restrict__ len) {
@@ -142,32 +183,44 @@ __global__ void k_row_lengths(const uint64_t* __restrict__ ptr, uint32_t V, uint
     len[v] = (uint32_t)(ptr[v + 1] - ptr[v]);
 }
 
-// ids with an edge: count, max id, max in-degree
-__global__ void k_vertex_stats(const uint64_t* __restrict__ col_ptr, const uint32_t* __restrict__ od,
-                               uint32_t V, const uint32_t* __restrict__ perm, unsigned int* __restrict__ out) {
+// ids with an edge: count, max id, max in-degree (one atomic each per block)
+__global__ __launch_bounds__(256) void k_vertex_stats(const uint64_t* __restrict__ col_ptr,
+                                                      const uint32_t* __restrict__ od, uint32_t V,
+                                                      const uint32_t* __restrict__ perm,
+                                                      unsigned long long* __restrict__ out) {
+  __shared__ unsigned int s_cnt[4], s_max[4], s_deg[4];
   unsigned int cnt = 0, mx = 0, mdeg = 0;
-  bool any = false;
-  for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V;
-       v += (uint64_t)gridDim.x * blockDim.x) {
+  for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t indeg = (uint32_t)(col_ptr[v + 1] - col_ptr[v]);
-    if (indeg > mdeg) mdeg = indeg;
+    mdeg = max(mdeg, indeg);
     if (indeg || od[v]) {
       ++cnt;
       mx = max(mx, perm ? perm[v] : (unsigned)v);
-      any = true;
     }
   }
   for (int off = 32; off > 0; off >>= 1) {
     cnt += __shfl_down(cnt, off, 64);
     mx = max(mx, (unsigned)__shfl_down(mx, off, 64));
     mdeg = max(mdeg, (unsigned)__shfl_down(mdeg, off, 64));
-    any = any || __shfl_down((int)any, off, 64);
   }
+  const int wave = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0) {
-    if (cnt) atomicAdd(&out[0], cnt);
-    if (any) atomicMax(&out[1], mx);
-    atomicMax(&out[2], mdeg);
+    s_cnt[wave] = cnt;
+    s_max[wave] = mx;
+    s_deg[wave] = mdeg;
   }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int w = 1; w < 4; ++w) {
+    cnt += s_cnt[w];
+    mx = max(mx, s_max[w]);
+    mdeg = max(mdeg, s_deg[w]);
+  }
+  if (cnt) {
+    atomicAdd(&out[0], (unsigned long long)cnt);
+    atomicMax(&out[1], (unsigned long long)mx);
+  }
+  atomicMax(&out[2], (unsigned long long)mdeg);
 }
 
 // Sum of out-weights per source, in CSR order (deterministic), FP64.
@@ -336,34 +389,40 @@ void graph_build_tiles(pe_graph_s* g, uint32_t tile_items) {
   PE_HIP(hipStreamSynchronize(s));
 }
 
-// Shared tail of both builders: keys already hold the CSC order.
-static void finish_build(pe_graph_s* g, dbuf<uint64_t>& keys, dbuf<float>* w, int b) {
+// keys: the CSC order
+static void build_csc_from_keys(pe_graph_s* g, dbuf<uint64_t>& keys, dbuf<float>* w, int b) {
   pe_ctx_s* ctx = g->ctx;
-  hipStream_t s = ctx->stream;
   const uint64_t nnz = g->nnz;
   sort_keys(ctx, keys, w, nnz, 2 * b);
   g->col_ptr.alloc(ctx, (uint64_t)g->V + 1);
   g->row_idx.alloc(ctx, std::max<uint64_t>(1, nnz));
-  split_keys(s, keys.p, nnz, b, g->V, g->col_ptr.p, g->row_idx.p);
+  split_keys(ctx->stream, keys.p, nnz, b, g->V, g->col_ptr.p, g->row_idx.p);
   if (w) g->wn = std::move(*w);
   keys.release();
-  g->od.alloc(ctx, std::max<uint32_t>(1, g->V));
-  PE_HIP(hipMemsetAsync(g->od.p, 0, (uint64_t)std::max<uint32_t>(1, g->V) * 4, s));
-  if (nnz) {
-    k_out_degrees<<<grid_for(nnz, 256, 1u << 20), 256, 0, s>>>(g->row_idx.p, nnz, g->od.p);
-    PE_HIP(hipGetLastError());
+}
+
+// Out-degrees: the lengths of the CSR's rows when there is one, else counted from the in-edges;
+// then the vertex statistics and the tiling.
+static void finish_build(pe_graph_s* g) {
+  pe_ctx_s* ctx = g->ctx;
+  hipStream_t s = ctx->stream;
+  const uint32_t Vs = std::max<uint32_t>(1, g->V);
+  g->od.alloc(ctx, Vs);
+  if (g->has_csr) {
+    k_row_lengths<<<grid_for(g->V, 256, 65536), 256, 0, s>>>(g->csr_ptr(), g->V, g->od.p);
+  } else {
+    k_zero_u32<<<grid_for(Vs, 256, 8192), 256, 0, s>>>(g->od.p, Vs);
+    count_ids(ctx, g->row_idx.p, g->nnz, g->od.p);
   }
-  dbuf<unsigned int> st(ctx, 3);
-  PE_HIP(hipMemsetAsync(st.p, 0, 12, s));
-  k_vertex_stats<<<grid_for(g->V, 256, 4096), 256, 0, s>>>(g->col_ptr.p, g->od.p, g->V,
+  dbuf<unsigned long long> st(ctx, 3);
+  k_zero_u32<<<1, 64, 0, s>>>(reinterpret_cast<uint32_t*>(st.p), 6);
+  k_vertex_stats<<<grid_for(g->V, 256, 1024), 256, 0, s>>>(g->col_ptr.p, g->od.p, g->V,
                                                           g->relabeled ? g->perm.p : nullptr, st.p);
   PE_HIP(hipGetLastError());
-  unsigned int hs[3];
-  PE_HIP(hipMemcpyAsync(hs, st.p, 12, hipMemcpyDeviceToHost, s));
-  PE_HIP(hipStreamSynchronize(s));
-  g->vertices = hs[0];
-  g->max_v_i = hs[1];
-  g->max_in_degree = hs[2];
+  const unsigned long long* hs = mail_post(ctx, st.p, 3, nullptr, 0);
+  g->vertices = (uint32_t)hs[0];
+  g->max_v_i = (uint32_t)hs[1];
+  g->max_in_degree = (uint32_t)hs[2];
   graph_build_tiles(g, 2048);
 }
 
@@ -400,15 +459,6 @@ static void normalise_weights(pe_graph_s* g, dbuf<uint64_t>& csr_keys, dbuf<floa
 // New id = rank of the vertex by (out-degree desc, id asc), out-degree counted over
 // the CSC entries (reversals included).  Sources with many out-edges get small,
 // adjacent ids, so the hot part of the gathered vector packs into few cache lines.
-__global__ void k_entry_out_degrees(const uint32_t* __restrict__ src, const uint32_t* __restrict__ dst,
-                                    uint64_t E, int sym, uint32_t* __restrict__ od) {
-  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < E;
-       i += (uint64_t)gridDim.x * blockDim.x) {
-    atomicAdd(&od[src[i]], 1u);
-    if (sym) atomicAdd(&od[dst[i]], 1u);
-  }
-}
-
 __global__ void k_degree_keys(const uint32_t* __restrict__ od, uint32_t V, uint64_t* __restrict__ keys) {
   for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V;
        v += (uint64_t)gridDim.x * blockDim.x)
@@ -436,9 +486,9 @@ static void build_relabel(pe_graph_s* g, dbuf<uint32_t>& ds, dbuf<uint32_t>& dd,
   hipStream_t s = ctx->stream;
   const uint32_t V = g->V;
   dbuf<uint32_t> od(ctx, V);
-  PE_HIP(hipMemsetAsync(od.p, 0, (uint64_t)V * 4, s));
-  if (g->edges)
-    k_entry_out_degrees<<<grid_for(g->edges, 256, 1u << 20), 256, 0, s>>>(ds.p, dd.p, g->edges, sym, od.p);
+  k_zero_u32<<<grid_for(V, 256, 8192), 256, 0, s>>>(od.p, V);
+  count_ids(ctx, ds.p, g->edges, od.p);
+  if (sym) count_ids(ctx, dd.p, g->edges, od.p);
   dbuf<uint64_t> keys(ctx, V);
   k_degree_keys<<<grid_for(V, 256, 8192), 256, 0, s>>>(od.p, V, keys.p);
   PE_HIP(hipGetLastError());
@@ -480,7 +530,7 @@ void build_from_edges(pe_graph_s* g, dbuf<uint32_t>& ds, dbuf<uint32_t>& dd, dbu
     dbuf<uint64_t> keys;
     dbuf<float> wk;
     make_keys(0, keys, weighted ? &wk : nullptr);
-    finish_build(g, keys, weighted ? &wk : nullptr, b);
+    build_csc_from_keys(g, keys, weighted ? &wk : nullptr, b);
   }
   if (weighted) {
     dbuf<uint64_t> keys;
@@ -497,6 +547,7 @@ void build_from_edges(pe_graph_s* g, dbuf<uint32_t>& ds, dbuf<uint32_t>& dd, dbu
     build_csr_from_keys(g, keys, b);
     g->has_csr = true;
   }
+  finish_build(g);
   PE_HIP(hipStreamSynchronize(s));
 }
 

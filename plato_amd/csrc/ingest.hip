@@ -21,42 +21,105 @@ namespace pe {
 static constexpr uint64_t CSV_SEG = 1ull << 16;  // bytes per newline-count segment
 
 // ---- lines ----------------------------------------------------------------------------------
-__global__ __launch_bounds__(1024) void k_csv_count(const char* __restrict__ b, uint64_t n,
-                                                    uint32_t* __restrict__ seg_count) {
-  __shared__ uint32_t s_cnt;
-  if (threadIdx.x == 0) s_cnt = 0;
-  __syncthreads();
+// 16 bytes per thread and step, newlines found a word at a time (460 MB of text: counted in
+// 0.43 ms and listed in 0.91 ms a byte per thread, 0.09 and 0.13 ms so, 4.9 and 3.6 TB/s).
+static constexpr int CSV_THREADS = 256;
+
+// bit 7 of every byte of x that is a newline
+__device__ __forceinline__ uint32_t csv_newlines4(uint32_t x) {
+  const uint32_t t = x ^ 0x0A0A0A0Au;
+  return ~(((t & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | t) & 0x80808080u;
+}
+
+// The newlines of the 16 bytes at p (a multiple of 16) below n, as four masks.
+__device__ __forceinline__ void csv_newlines16(const char* __restrict__ b, uint64_t n, uint64_t p, uint32_t (&m)[4]) {
+  const uint4 q = p < n ? *reinterpret_cast<const uint4*>(b + p) : make_uint4(0, 0, 0, 0);
+  const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    m[i] = csv_newlines4(w[i]);
+    const uint64_t at = p + 4 * i;
+    if (at + 4 > n) m[i] = at >= n ? 0u : m[i] & ((1u << (8 * (uint32_t)(n - at))) - 1u);  // past the text
+  }
+}
+
+__global__ __launch_bounds__(CSV_THREADS) void k_csv_count(const char* __restrict__ b, uint64_t n,
+                                                           uint32_t* __restrict__ seg_count) {
+  __shared__ uint32_t s_cnt[CSV_THREADS / 64];
   const uint64_t p0 = (uint64_t)blockIdx.x * CSV_SEG, p1 = std::min<uint64_t>(n, p0 + CSV_SEG);
   uint32_t c = 0;
-  for (uint64_t p = p0 + threadIdx.x; p < p1; p += blockDim.x) c += b[p] == '\n' ? 1u : 0u;
-  atomicAdd(&s_cnt, c);
+  for (uint64_t p = p0 + threadIdx.x * 16; p < p1; p += CSV_THREADS * 16) {
+    uint32_t m[4];
+    csv_newlines16(b, p1, p, m);
+    c += __popc(m[0]) + __popc(m[1]) + __popc(m[2]) + __popc(m[3]);
+  }
+  for (int off = 32; off > 0; off >>= 1) c += __shfl_down(c, off, 64);
+  if ((threadIdx.x & 63) == 0) s_cnt[threadIdx.x >> 6] = c;
   __syncthreads();
-  if (threadIdx.x == 0) seg_count[blockIdx.x] = s_cnt;
+  if (threadIdx.x == 0) seg_count[blockIdx.x] = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
 }
 
 // Positions of the newlines in order; seg_off is the exclusive scan of seg_count.
-__global__ __launch_bounds__(1024) void k_csv_newlines(const char* __restrict__ b, uint64_t n,
-                                                       const uint64_t* __restrict__ seg_off,
-                                                       uint64_t* __restrict__ nl) {
-  __shared__ uint32_t s_wave[16];
+__global__ __launch_bounds__(CSV_THREADS) void k_csv_newlines(const char* __restrict__ b, uint64_t n,
+                                                              const uint64_t* __restrict__ seg_off,
+                                                              uint64_t* __restrict__ nl) {
+  __shared__ uint32_t s_wave[CSV_THREADS / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint64_t p0 = (uint64_t)blockIdx.x * CSV_SEG, p1 = std::min<uint64_t>(n, p0 + CSV_SEG);
   uint64_t out = seg_off[blockIdx.x];
-  for (uint64_t base = p0; base < p1; base += 1024) {
-    const uint64_t p = base + threadIdx.x;
-    const bool hit = p < p1 && b[p] == '\n';
-    const uint64_t m = __ballot(hit);
-    if (lane == 0) s_wave[wave] = (uint32_t)__popcll(m);
+  for (uint64_t base = p0; base < p1; base += CSV_THREADS * 16) {
+    const uint64_t p = base + threadIdx.x * 16;
+    uint32_t m[4];
+    csv_newlines16(b, p1, p, m);
+    const uint32_t c = __popc(m[0]) + __popc(m[1]) + __popc(m[2]) + __popc(m[3]);
+    uint32_t incl = c;
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t t = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += t;
+    }
+    if (lane == 63) s_wave[wave] = incl;
     __syncthreads();
     uint32_t before = 0, total = 0;
-    for (int i = 0; i < 16; ++i) {
+#pragma unroll
+    for (int i = 0; i < CSV_THREADS / 64; ++i) {
       if (i < wave) before += s_wave[i];
       total += s_wave[i];
     }
-    if (hit) nl[out + before + (uint64_t)__popcll(m & ((1ull << lane) - 1ull))] = p;
+    uint64_t at = out + before + incl - c;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      for (uint32_t x = m[i]; x; x &= x - 1) nl[at++] = p + 4 * i + ((uint32_t)(__ffs((int)x) - 1) >> 3);
     out += total;
     __syncthreads();
   }
+}
+
+// One block: off[i] = sum of cnt[0..i), total[0] = sum of all.
+__global__ __launch_bounds__(1024) void k_csv_scan(const uint32_t* __restrict__ cnt, uint64_t n,
+                                                   uint64_t* __restrict__ off, unsigned long long* __restrict__ total) {
+  __shared__ uint64_t s_wave[16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint64_t carry = 0;
+  for (uint64_t i0 = 0; i0 < n; i0 += 1024) {
+    const uint64_t i = i0 + threadIdx.x;
+    const uint64_t c = i < n ? cnt[i] : 0ull;
+    uint64_t incl = c;
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint64_t t = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += t;
+    }
+    if (lane == 63) s_wave[wave] = incl;
+    __syncthreads();
+    uint64_t before = 0, sum = 0;
+    for (int k = 0; k < 16; ++k) {
+      before += k < wave ? s_wave[k] : 0ull;
+      sum += s_wave[k];
+    }
+    if (i < n) off[i] = carry + before + incl - c;
+    carry += sum;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) *total = carry;
 }
 
 // ---- fields ---------------------------------------------------------------------------------
@@ -78,7 +141,7 @@ __device__ __forceinline__ bool csv_field(const char* b, uint64_t& p, uint64_t e
 
 // strtoul(field, nullptr, 10): leading whitespace, optional sign, decimal digits up to
 // the first other byte; no digits -> 0; overflow -> 2^64 - 1; '-' negates modulo 2^64.
-__device__ uint64_t csv_strtoul(const char* b, uint64_t p, uint64_t e) {
+__device__ __forceinline__ uint64_t csv_strtoul(const char* b, uint64_t p, uint64_t e) {
   while (p < e && csv_space(b[p])) ++p;
   bool neg = false;
   if (p < e && (b[p] == '+' || b[p] == '-')) {
@@ -141,7 +204,7 @@ __device__ __forceinline__ u128i pow10_128(int k) {
 // midpoint.
 // inf, nan, hex, more than 15 significant digits, an exponent beyond that range, a
 // result next to a midpoint, or a float result that is subnormal or infinite set *bad.
-__device__ float csv_strtof(const char* b, uint64_t p, uint64_t e, bool& bad) {
+__device__ __forceinline__ float csv_strtof(const char* b, uint64_t p, uint64_t e, bool& bad) {
   while (p < e && csv_space(b[p])) ++p;
   bool neg = false;
   if (p < e && (b[p] == '+' || b[p] == '-')) {
@@ -260,58 +323,79 @@ __device__ float csv_strtof(const char* b, uint64_t p, uint64_t e, bool& bad) {
   return neg ? -f : f;
 }
 
-// One line per thread.  status: 0 skipped, 1 edge, 2 src or dst above the id limit,
+// One line b[p, e) to its edge.  Returns 0 skipped, 1 edge, 2 src or dst above the id limit,
 // 3 weight literal outside the exact range.
-__global__ void k_csv_parse(const char* __restrict__ b, uint64_t n, const uint64_t* __restrict__ nl, uint64_t nnl,
-                            uint64_t nlines, int weighted, uint64_t id_limit, uint8_t* __restrict__ status,
-                            uint64_t* __restrict__ src, uint64_t* __restrict__ dst, float* __restrict__ w) {
-  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < nlines;
-       i += (uint64_t)gridDim.x * blockDim.x) {
-    uint64_t p = i ? nl[i - 1] + 1 : 0;
-    uint64_t e = i < nnl ? nl[i] : n;
-    // a NUL byte ends the line's string
-    for (uint64_t q = p; q < e; ++q)
-      if (b[q] == '\0') {
-        e = q;
-        break;
-      }
-    uint8_t st = 0;
-    uint64_t s = 0, d = 0;
-    float wt = 0.0f;
-    uint64_t fs, fe;
-    if (p < e && csv_field(b, p, e, fs, fe)) {
-      s = csv_strtoul(b, fs, fe);
-      if (s > id_limit) {
-        st = 2;
-      } else if (csv_field(b, p, e, fs, fe)) {
-        d = csv_strtoul(b, fs, fe);
-        if (d > id_limit) {
-          st = 2;
-        } else if (!weighted) {
-          st = 1;
-        } else if (csv_field(b, p, e, fs, fe)) {
-          bool bad = false;
-          wt = csv_strtof(b, fs, fe, bad);
-          st = bad ? 3 : 1;
-        }
-      }
+__device__ __forceinline__ uint8_t csv_line(const char* b, uint64_t p, uint64_t e, int weighted, uint64_t id_limit,
+                                            uint64_t& s, uint64_t& d, float& wt) {
+  // a NUL byte ends the line's string
+  for (uint64_t q = p; q < e; ++q)
+    if (b[q] == '\0') {
+      e = q;
+      break;
     }
-    status[i] = st;
-    src[i] = s;
-    dst[i] = d;
-    if (weighted) w[i] = wt;
+  uint64_t fs, fe;
+  if (!(p < e && csv_field(b, p, e, fs, fe))) return 0;
+  s = csv_strtoul(b, fs, fe);
+  if (s > id_limit) return 2;
+  if (!csv_field(b, p, e, fs, fe)) return 0;
+  d = csv_strtoul(b, fs, fe);
+  if (d > id_limit) return 2;
+  if (!weighted) return 1;
+  if (!csv_field(b, p, e, fs, fe)) return 0;
+  bool bad = false;
+  wt = csv_strtof(b, fs, fe, bad);
+  return bad ? 3 : 1;
+}
+
+// One line per thread, CSV_THREADS consecutive lines per block, whose bytes are staged in LDS
+// (each is looked at several times) unless they are longer than CSV_STAGE (17 M lines of 27
+// bytes: 1.15 ms from global memory, 0.75 ms; bound by the digit loops' divergence).
+static constexpr uint32_t CSV_STAGE = 16384;
+__global__ __launch_bounds__(CSV_THREADS) void k_csv_parse(
+    const char* __restrict__ b, uint64_t n, const uint64_t* __restrict__ nl, uint64_t nnl, uint64_t nlines, int weighted,
+    uint64_t id_limit, uint8_t* __restrict__ status, uint64_t* __restrict__ src, uint64_t* __restrict__ dst,
+    float* __restrict__ w) {
+  __shared__ uint4 s_text[CSV_STAGE / 16];
+  for (uint64_t i0 = blockIdx.x * (uint64_t)CSV_THREADS; i0 < nlines; i0 += (uint64_t)gridDim.x * CSV_THREADS) {
+    const uint64_t i1 = std::min<uint64_t>(nlines, i0 + CSV_THREADS);  // lines [i0, i1)
+    const uint64_t t0 = (i0 ? nl[i0 - 1] + 1 : 0) & ~15ull, t1 = i1 - 1 < nnl ? nl[i1 - 1] : n;
+    const bool staged = t1 - t0 <= CSV_STAGE;  // uniform
+    if (staged)
+      for (uint64_t k = threadIdx.x; k * 16 < t1 - t0; k += CSV_THREADS)
+        s_text[k] = *reinterpret_cast<const uint4*>(b + t0 + k * 16);
+    __syncthreads();
+    const uint64_t i = i0 + threadIdx.x;
+    if (i < nlines) {
+      const uint64_t p = i ? nl[i - 1] + 1 : 0, e = i < nnl ? nl[i] : n;
+      uint64_t s = 0, d = 0;
+      float wt = 0.0f;
+      uint8_t st;
+      if (staged) st = csv_line(reinterpret_cast<const char*>(s_text), p - t0, e - t0, weighted, id_limit, s, d, wt);
+      else st = csv_line(b, p, e, weighted, id_limit, s, d, wt);
+      status[i] = st;
+      src[i] = s;
+      dst[i] = d;
+      if (weighted) w[i] = wt;
+    }
+    __syncthreads();
   }
 }
 
 // ---- compaction of the edges in file order ---------------------------------------------------
+// Entries of status 1 per segment, and the first entry above 1 (an error), if any, in *bad.
 __global__ __launch_bounds__(1024) void k_csv_count_ok(const uint8_t* __restrict__ status, uint64_t nlines,
-                                                       uint32_t* __restrict__ seg_count) {
+                                                       uint32_t* __restrict__ seg_count,
+                                                       unsigned long long* __restrict__ bad) {
   __shared__ uint32_t s_cnt;
   if (threadIdx.x == 0) s_cnt = 0;
   __syncthreads();
   const uint64_t p0 = (uint64_t)blockIdx.x * CSV_SEG, p1 = std::min<uint64_t>(nlines, p0 + CSV_SEG);
   uint32_t c = 0;
-  for (uint64_t p = p0 + threadIdx.x; p < p1; p += blockDim.x) c += status[p] == 1 ? 1u : 0u;
+  for (uint64_t p = p0 + threadIdx.x; p < p1; p += blockDim.x) {
+    const uint8_t st = status[p];
+    c += st == 1 ? 1u : 0u;
+    if (st > 1) atomicMin(bad, (unsigned long long)p);
+  }
   atomicAdd(&s_cnt, c);
   __syncthreads();
   if (threadIdx.x == 0) seg_count[blockIdx.x] = s_cnt;
@@ -364,48 +448,65 @@ __global__ void k_u64_heads(const uint64_t* __restrict__ k, uint64_t n, uint8_t*
     head[i] = (i == 0 || k[i] != k[i - 1]) ? 1 : 0;
 }
 
-// dense id of each original id: its index in the sorted distinct ids
-__global__ void k_encode(const uint64_t* __restrict__ ids, uint64_t n, const uint64_t* __restrict__ uniq,
-                         uint64_t nu, uint32_t* __restrict__ out) {
-  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
-    const uint64_t x = ids[i];
-    uint64_t lo = 0, hi = nu - 1;
+// First distinct id of each bucket of `1 << shift` values: start[k] = the first index whose id is
+// at or above k << shift (k <= nbuckets).
+__global__ void k_encode_buckets(const uint64_t* __restrict__ uniq, uint64_t nu, int shift, uint64_t nbuckets,
+                                 uint32_t* __restrict__ start) {
+  for (uint64_t k = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; k <= nbuckets;
+       k += (uint64_t)gridDim.x * blockDim.x) {
+    uint64_t lo = 0, hi = nu;
+    if (k == nbuckets) lo = nu;
     while (lo < hi) {
       const uint64_t mid = (lo + hi) >> 1;
-      if (uniq[mid] < x) lo = mid + 1;
+      if (uniq[mid] < (k << shift)) lo = mid + 1;
       else hi = mid;
     }
-    out[i] = (uint32_t)lo;
+    start[k] = (uint32_t)lo;
   }
 }
 
-__global__ void k_u64_to_u32(const uint64_t* __restrict__ a, uint64_t n, uint32_t* __restrict__ out,
-                             unsigned long long* __restrict__ maxv) {
-  uint64_t m = 0;
+// dense id of each original id: its index in the sorted distinct ids, searched in its bucket
+// only (hashed ids leave one or two there; 17 M lookups in 1 M ids: 1.02 ms over
+// all ids, 0.21 ms)
+__global__ void k_encode(const uint64_t* __restrict__ ids, uint64_t n, const uint64_t* __restrict__ uniq, int shift,
+                         const uint32_t* __restrict__ start, uint32_t* __restrict__ out) {
   for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
-    out[i] = (uint32_t)a[i];
-    m = a[i] > m ? a[i] : m;
+    const uint64_t x = ids[i], k = x >> shift;
+    uint32_t lo = start[k], hi = start[k + 1] - 1;  // x occurs, so its bucket is not empty
+    while (lo < hi) {
+      const uint32_t mid = lo + (hi - lo) / 2;
+      if (uniq[mid] < x) lo = mid + 1;
+      else hi = mid;
+    }
+    out[i] = lo;
   }
+}
+
+// largest value
+__global__ __launch_bounds__(256) void k_u64_max(const uint64_t* __restrict__ a, uint64_t n,
+                                                 unsigned long long* __restrict__ maxv) {
+  uint64_t m = 0;
+  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
+    m = a[i] > m ? a[i] : m;
   for (int off = 32; off > 0; off >>= 1) {
     const uint64_t o = __shfl_down(m, off, 64);
     m = o > m ? o : m;
   }
-  if ((threadIdx.x & 63) == 0) atomicMax(maxv, (unsigned long long)m);
+  if ((threadIdx.x & 63) == 0 && m > *(volatile unsigned long long*)maxv) atomicMax(maxv, (unsigned long long)m);
 }
 
-// Two-level ordered compaction helper on the host side of a segment count.
-static std::vector<uint64_t> exclusive_offsets(pe_ctx_s* ctx, const uint32_t* dcount, uint64_t nseg, uint64_t& total) {
-  std::vector<uint32_t> h(nseg);
-  PE_HIP(hipMemcpyAsync(h.data(), dcount, nseg * 4, hipMemcpyDeviceToHost, ctx->stream));
-  PE_HIP(hipStreamSynchronize(ctx->stream));
-  std::vector<uint64_t> off(nseg);
-  total = 0;
-  for (uint64_t i = 0; i < nseg; ++i) {
-    off[i] = total;
-    total += h[i];
-  }
-  return off;
+__global__ void k_u64_to_u32(const uint64_t* __restrict__ a, uint64_t n, uint32_t* __restrict__ out) {
+  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
+    out[i] = (uint32_t)a[i];
 }
+
+// The device words that the host reads along the way.
+struct csv_words {
+  unsigned long long total;  // of the last scan
+  unsigned long long bad;    // first line in error
+  unsigned long long max;    // largest id
+};
+__global__ void k_csv_words(csv_words* w) { *w = csv_words{0, ~0ull, 0}; }
 
 }  // namespace pe
 
@@ -420,33 +521,30 @@ int pe_graph_create_csv(pe_ctx_t* ctx, const char* text, uint64_t nbytes, uint32
     hipStream_t s = ctx->stream;
     const bool weighted = (flags & PE_GRAPH_WEIGHTED) != 0;
     const bool encode = (flags & PE_GRAPH_ENCODE_IDS) != 0;
-    // text on the device
-    dbuf<char> db(ctx, std::max<uint64_t>(1, nbytes));
+    // text on the device, in whole 16-byte words
+    dbuf<char> db(ctx, std::max<uint64_t>(16, (nbytes + 15) & ~15ull));
     host_upload(ctx, db.p, text, nbytes);
+    dbuf<csv_words> words(ctx, 1);
+    k_csv_words<<<1, 1, 0, s>>>(words.p);
+    PE_HIP(hipGetLastError());
+    auto read_words = [&] {
+      return *reinterpret_cast<const csv_words*>(
+          mail_post(ctx, reinterpret_cast<const unsigned long long*>(words.p), sizeof(csv_words) / 8, nullptr, 0));
+    };
     // newlines
     const uint64_t nseg = std::max<uint64_t>(1, (nbytes + CSV_SEG - 1) / CSV_SEG);
     PE_REQUIRE(nseg < 0x7FFFFFFFull, PE_ERR_RANGE, "text too large");
     dbuf<uint32_t> cnt(ctx, nseg);
-    uint64_t nnl = 0;
-    if (nbytes) {
-      k_csv_count<<<(unsigned)nseg, 1024, 0, s>>>(db.p, nbytes, cnt.p);
-      PE_HIP(hipGetLastError());
-    } else {
-      PE_HIP(hipMemsetAsync(cnt.p, 0, 4, s));
-    }
-    auto off = exclusive_offsets(ctx, cnt.p, nseg, nnl);
-    dbuf<uint64_t> doff(ctx, nseg), nl(ctx, std::max<uint64_t>(1, nnl));
-    PE_HIP(hipMemcpyAsync(doff.p, off.data(), nseg * 8, hipMemcpyHostToDevice, s));
-    if (nbytes) {
-      k_csv_newlines<<<(unsigned)nseg, 1024, 0, s>>>(db.p, nbytes, doff.p, nl.p);
-      PE_HIP(hipGetLastError());
-    }
+    dbuf<uint64_t> doff(ctx, nseg);
+    k_csv_count<<<(unsigned)nseg, CSV_THREADS, 0, s>>>(db.p, nbytes, cnt.p);
+    k_csv_scan<<<1, 1024, 0, s>>>(cnt.p, nseg, doff.p, &words.p->total);
+    PE_HIP(hipGetLastError());
+    const uint64_t nnl = read_words().total;
+    dbuf<uint64_t> nl(ctx, std::max<uint64_t>(1, nnl));
+    k_csv_newlines<<<(unsigned)nseg, CSV_THREADS, 0, s>>>(db.p, nbytes, doff.p, nl.p);
+    PE_HIP(hipGetLastError());
     // lines: one per newline, plus the text after the last newline when non-empty
-    uint64_t last_nl = 0;
-    if (nnl) PE_HIP(hipMemcpyAsync(&last_nl, nl.p + nnl - 1, 8, hipMemcpyDeviceToHost, s));
-    PE_HIP(hipStreamSynchronize(s));
-    const uint64_t tail_start = nnl ? last_nl + 1 : 0;
-    const uint64_t nlines = nnl + (tail_start < nbytes ? 1 : 0);
+    const uint64_t nlines = nnl + (nbytes && text[nbytes - 1] != '\n' ? 1 : 0);
     // parse
     const uint64_t id_limit = encode ? ~0ull : 0xFFFFFFFFull;
     dbuf<uint8_t> status(ctx, std::max<uint64_t>(1, nlines));
@@ -454,38 +552,39 @@ int pe_graph_create_csv(pe_ctx_t* ctx, const char* text, uint64_t nbytes, uint32
     dbuf<float> lw;
     if (weighted) lw.alloc(ctx, std::max<uint64_t>(1, nlines));
     if (nlines) {
-      k_csv_parse<<<grid_for(nlines, 256, 1u << 20), 256, 0, s>>>(db.p, nbytes, nl.p, nnl, nlines, weighted ? 1 : 0,
-                                                                  id_limit, status.p, ls.p, ld.p, lw.p);
+      k_csv_parse<<<grid_for(nlines, CSV_THREADS, 1u << 20), CSV_THREADS, 0, s>>>(
+          db.p, nbytes, nl.p, nnl, nlines, weighted ? 1 : 0, id_limit, status.p, ls.p, ld.p, lw.p);
       PE_HIP(hipGetLastError());
     }
     db.release();
     nl.release();
-    // errors: first offending line (host scan of the status bytes is enough: 1 B per line)
-    std::vector<uint8_t> hst(nlines);
-    host_download(ctx, status.p, hst.data(), nlines);
-    for (uint64_t i = 0; i < nlines; ++i) {
-      if (hst[i] == 2)
-        fail(PE_ERR_RANGE, "line " + std::to_string(i + 1) + ": vertex id above 2^32 - 1 (use PE_GRAPH_ENCODE_IDS)");
-      if (hst[i] == 3)
-        fail(PE_ERR_RANGE, "line " + std::to_string(i + 1) +
-                               ": weight literal outside the exactly-rounded decimal range");
-    }
-    // compact the edges in file order
+    // compact the edges in file order; the first offending line ends it
     const uint64_t lseg = std::max<uint64_t>(1, (nlines + CSV_SEG - 1) / CSV_SEG);
     dbuf<uint32_t> lcnt(ctx, lseg);
-    uint64_t E = 0;
-    if (nlines) {
-      k_csv_count_ok<<<(unsigned)lseg, 1024, 0, s>>>(status.p, nlines, lcnt.p);
-      PE_HIP(hipGetLastError());
-    } else {
-      PE_HIP(hipMemsetAsync(lcnt.p, 0, 4, s));
+    dbuf<uint64_t> dloff(ctx, lseg);
+    k_csv_count_ok<<<(unsigned)lseg, 1024, 0, s>>>(status.p, nlines, lcnt.p, &words.p->bad);
+    k_csv_scan<<<1, 1024, 0, s>>>(lcnt.p, lseg, dloff.p, &words.p->total);
+    PE_HIP(hipGetLastError());
+    const csv_words parsed = read_words();
+    if (parsed.bad != ~0ull) {
+      uint8_t st = 0;
+      PE_HIP(hipMemcpyAsync(&st, status.p + parsed.bad, 1, hipMemcpyDeviceToHost, s));
+      PE_HIP(hipStreamSynchronize(s));
+      const std::string line = "line " + std::to_string(parsed.bad + 1);
+      if (st == 2) fail(PE_ERR_RANGE, line + ": vertex id above 2^32 - 1 (use PE_GRAPH_ENCODE_IDS)");
+      fail(PE_ERR_RANGE, line + ": weight literal outside the exactly-rounded decimal range");
     }
-    auto loff = exclusive_offsets(ctx, lcnt.p, lseg, E);
-    dbuf<uint64_t> dloff(ctx, lseg), es(ctx, std::max<uint64_t>(1, E)), ed(ctx, std::max<uint64_t>(1, E));
+    const uint64_t E = parsed.total;
+    dbuf<uint64_t> es, ed;
     dbuf<float> ew;
-    if (weighted) ew.alloc(ctx, std::max<uint64_t>(1, E));
-    PE_HIP(hipMemcpyAsync(dloff.p, loff.data(), lseg * 8, hipMemcpyHostToDevice, s));
-    if (nlines) {
+    if (E == nlines) {  // every line is an edge: nothing to compact
+      es = std::move(ls);
+      ed = std::move(ld);
+      ew = std::move(lw);
+    } else if (E) {
+      es.alloc(ctx, E);
+      ed.alloc(ctx, E);
+      if (weighted) ew.alloc(ctx, E);
       k_csv_compact<<<(unsigned)lseg, 1024, 0, s>>>(status.p, nlines, dloff.p, ls.p, ld.p, weighted ? lw.p : nullptr,
                                                     es.p, ed.p, weighted ? ew.p : nullptr);
       PE_HIP(hipGetLastError());
@@ -501,44 +600,49 @@ int pe_graph_create_csv(pe_ctx_t* ctx, const char* text, uint64_t nbytes, uint32
     g->ctx = ctx;
     g->edges = E;
     dbuf<uint32_t> ds(ctx, E), dd(ctx, E);
+    k_u64_max<<<grid_for(E, 256, 1024), 256, 0, s>>>(es.p, E, &words.p->max);
+    k_u64_max<<<grid_for(E, 256, 1024), 256, 0, s>>>(ed.p, E, &words.p->max);
+    PE_HIP(hipGetLastError());
+    const uint64_t max_id = read_words().max;
     if (encode) {
+      int bits = 1;  // of the largest id: the sort and the buckets go no higher
+      while (bits < 64 && (max_id >> bits)) ++bits;
       dbuf<uint64_t> all(ctx, 2 * E);
       k_u64_concat<<<grid_for(E, 256, 1u << 20), 256, 0, s>>>(es.p, ed.p, E, all.p);
       PE_HIP(hipGetLastError());
-      sort_keys(ctx, all, nullptr, 2 * E, 64);
+      sort_keys(ctx, all, nullptr, 2 * E, bits);
       dbuf<uint8_t> head(ctx, 2 * E);
       k_u64_heads<<<grid_for(2 * E, 256, 1u << 20), 256, 0, s>>>(all.p, 2 * E, head.p);
       PE_HIP(hipGetLastError());
       const uint64_t hseg = (2 * E + CSV_SEG - 1) / CSV_SEG;
       dbuf<uint32_t> hcnt(ctx, hseg);
-      k_csv_count_ok<<<(unsigned)hseg, 1024, 0, s>>>(head.p, 2 * E, hcnt.p);
-      PE_HIP(hipGetLastError());
-      uint64_t nu = 0;
-      auto hoff = exclusive_offsets(ctx, hcnt.p, hseg, nu);
-      PE_REQUIRE(nu <= 0xFFFFFFFFull, PE_ERR_RANGE, "more than 2^32 - 1 distinct vertex ids");
       dbuf<uint64_t> dhoff(ctx, hseg);
-      PE_HIP(hipMemcpyAsync(dhoff.p, hoff.data(), hseg * 8, hipMemcpyHostToDevice, s));
+      k_csv_count_ok<<<(unsigned)hseg, 1024, 0, s>>>(head.p, 2 * E, hcnt.p, &words.p->bad);
+      k_csv_scan<<<1, 1024, 0, s>>>(hcnt.p, hseg, dhoff.p, &words.p->total);
+      PE_HIP(hipGetLastError());
+      const uint64_t nu = read_words().total;
+      PE_REQUIRE(nu <= 0xFFFFFFFFull, PE_ERR_RANGE, "more than 2^32 - 1 distinct vertex ids");
       g->vid_decode.alloc(ctx, nu);
       k_csv_compact<<<(unsigned)hseg, 1024, 0, s>>>(head.p, 2 * E, dhoff.p, all.p, nullptr, nullptr, g->vid_decode.p,
                                                     nullptr, nullptr);
       PE_HIP(hipGetLastError());
-      k_encode<<<grid_for(E, 256, 1u << 20), 256, 0, s>>>(es.p, E, g->vid_decode.p, nu, ds.p);
-      k_encode<<<grid_for(E, 256, 1u << 20), 256, 0, s>>>(ed.p, E, g->vid_decode.p, nu, dd.p);
+      // about one bucket per distinct id
+      int shift = std::min(bits, 63);
+      while (shift > 0 && (max_id >> (shift - 1)) < nu) --shift;
+      const uint64_t nbuckets = (max_id >> shift) + 1;
+      dbuf<uint32_t> start(ctx, nbuckets + 1);
+      k_encode_buckets<<<grid_for(nbuckets + 1, 256, 1u << 20), 256, 0, s>>>(g->vid_decode.p, nu, shift, nbuckets, start.p);
+      k_encode<<<grid_for(E, 256, 1u << 20), 256, 0, s>>>(es.p, E, g->vid_decode.p, shift, start.p, ds.p);
+      k_encode<<<grid_for(E, 256, 1u << 20), 256, 0, s>>>(ed.p, E, g->vid_decode.p, shift, start.p, dd.p);
       PE_HIP(hipGetLastError());
-      PE_HIP(hipStreamSynchronize(s));  // hoff has been read
       g->V = (uint32_t)nu;
       g->encoded = true;
     } else {
-      dbuf<unsigned long long> mx(ctx, 1);
-      PE_HIP(hipMemsetAsync(mx.p, 0, 8, s));
-      k_u64_to_u32<<<grid_for(E, 256, 65536), 256, 0, s>>>(es.p, E, ds.p, mx.p);
-      k_u64_to_u32<<<grid_for(E, 256, 65536), 256, 0, s>>>(ed.p, E, dd.p, mx.p);
+      PE_REQUIRE(max_id < 0xFFFFFFFFull, PE_ERR_RANGE, "vertex id 2^32 - 1 leaves no room for V");
+      k_u64_to_u32<<<grid_for(E, 256, 65536), 256, 0, s>>>(es.p, E, ds.p);
+      k_u64_to_u32<<<grid_for(E, 256, 65536), 256, 0, s>>>(ed.p, E, dd.p);
       PE_HIP(hipGetLastError());
-      unsigned long long m = 0;
-      PE_HIP(hipMemcpyAsync(&m, mx.p, 8, hipMemcpyDeviceToHost, s));
-      PE_HIP(hipStreamSynchronize(s));
-      PE_REQUIRE(m < 0xFFFFFFFFull, PE_ERR_RANGE, "vertex id 2^32 - 1 leaves no room for V");
-      g->V = (uint32_t)(m + 1);
+      g->V = (uint32_t)(max_id + 1);
     }
     es.release();
     ed.release();

@@ -107,3 +107,51 @@ def test_rmat_csv_matches_generated_graph(ctx):
     V = int(max(s.max(), d.max())) + 1
     assert g.V == V and g.info.edges == s.size
     assert _same_csc(g, s, d, V)
+
+
+@pytest.mark.parametrize("shape", ["dense", "hashed", "skewed", "top", "one_id"])
+def test_encoded_ids_of_any_spread(ctx, shape):
+    """Ids spread evenly, all low but a few near 2^64, around the top bit, and a single one:
+    compacted in ascending order, whatever their buckets hold."""
+    from plato_amd import Graph
+    rng = np.random.default_rng(3)
+    ids = {"dense": np.arange(5000, dtype=np.uint64), "hashed": rng.integers(0, 10 ** 12, 5000).astype(np.uint64),
+           "skewed": np.concatenate([np.arange(5000, dtype=np.uint64), np.array([2 ** 40, 2 ** 63, 2 ** 64 - 2], np.uint64)]),
+           "top": np.array([0, 2 ** 63 - 1, 2 ** 63, 2 ** 63 + 1, 2 ** 64 - 2, 2 ** 64 - 1], np.uint64),
+           "one_id": np.array([2 ** 64 - 1], np.uint64)}[shape]
+    src, dst = rng.choice(ids, 9000), rng.choice(ids, 9000)
+    text = "".join(f"{a},{b}\n" for a, b in zip(src.tolist(), dst.tolist())).encode()
+    print(f"case: csv encode {shape}", flush=True)
+    g = Graph.from_csv_bytes(ctx, text, build_csr=True, encode_ids=True)
+    uniq = np.unique(np.concatenate([src, dst]))
+    assert np.array_equal(g.vertex_ids(), uniq)
+    s, d = (np.searchsorted(uniq, x).astype(np.uint32) for x in (src, dst))
+    og = oracle.CSC(uniq.size, s, d)
+    assert _same_csc(g, s, d, uniq.size)
+    rp, ci = g.download_csr()
+    assert np.array_equal(rp, og.row_ptr) and np.array_equal(np.sort(ci), np.sort(og.col_idx))
+    assert np.array_equal(g.out_degrees(), np.bincount(s, minlength=uniq.size).astype(np.uint32))
+    g.close()
+
+
+@pytest.mark.parametrize("pad", [0, 1, 15, 16, 17, 40, 16300, 17000, 65535, 65536])
+def test_line_lengths_around_words_stages_and_segments(ctx, pad):
+    """Lines drawn out with leading commas past a 16-byte word, the staging buffer of a block of
+    lines and a 64 KiB segment, empty lines between, with and without a last newline; an error
+    behind them names its line."""
+    from plato_amd import Graph
+    from plato_amd._lib import PlatoHipError
+    lines = []
+    for i in range(600):
+        lines.append(b"," * (pad if i in (5, 6, 300) else i % 19) + b"%d,%d" % (i % 97, (i * 7) % 89))
+        if i % 11 == 0:
+            lines.append(b"")
+    for text in (b"\n".join(lines), b"\n".join(lines) + b"\n"):
+        s, d = oracle.parse_csv(text)
+        assert s.size == 600
+        print(f"case: csv lines pad={pad} bytes={len(text)}", flush=True)
+        g = Graph.from_csv_bytes(ctx, text)
+        assert g.info.edges == 600 and _same_csc(g, s, d, int(max(s.max(), d.max())) + 1)
+        g.close()
+        with pytest.raises(PlatoHipError, match=f"line {len(lines) + 2}:"):
+            Graph.from_csv_bytes(ctx, b"\n".join(lines) + b"\n1,2\n4294967296,1\n4294967297,1\n")
