@@ -17,12 +17,14 @@
 // estimate[v] along with the estimates: v is modified in an epoch exactly when cnt(v) <
 // estimate[v].  A vertex that drops from `old` to `now` takes one from cnt(u) of every
 // unmodified neighbour u with now < estimate[u] <= old and re-counts its own, so an epoch
-// reads the adjacencies of the modified vertices (twice) instead of those of all active
-// ones; the active set is still marked and counted, for the per-epoch log.  In epoch 0
-// everything is active; a vertex that keeps its adjacency length has cnt(v) equal to it.
+// reads the adjacencies of the modified vertices instead of those of all active ones, twice
+// where a vertex is newly modified and once where it was in the epoch before; the active set
+// is still marked and counted, for the per-epoch log.  In epoch 0 everything is active; a vertex
+// that keeps its adjacency length has cnt(v) equal to it.
 // RMAT scale 22 symmetrized, degree-relabeled, 39 epochs, whole call: 51 ms re-counting every
-// active vertex, 20 ms with the counts.  Bound by the random 4-byte reads of the estimates in
-// the first ten epochs, when most vertices are modified (0.5 ms per scan of the 2^27 entries).
+// active vertex, 20 ms with the counts, 16.1 ms with the drops found in the spread before.  Bound by
+// the random 4-byte reads of the values in the first ten epochs, when most vertices are modified
+// (0.5 ms per scan of the 2^27 entries).
 // Other adjacencies (in-edges or out-edges of a directed graph) have no counts: every
 // active vertex is re-counted.
 //
@@ -77,13 +79,16 @@ struct kc_giant {
 };
 
 __global__ void k_kc_init(const uint64_t* __restrict__ ptr, uint32_t V, uint32_t* __restrict__ core,
-                          uint32_t* __restrict__ est, uint32_t* __restrict__ cnt) {
+                          uint32_t* __restrict__ est, uint32_t* __restrict__ cnt, uint32_t* __restrict__ ahead) {
   for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x) {
     const uint64_t len = ptr[v + 1] - ptr[v];
     const uint32_t c = len ? (uint32_t)std::min<uint64_t>(len, 0xFFFFFFFEull) : KC_UNSET;
     core[v] = c;
     est[v] = c;
-    if (cnt) cnt[v] = c;
+    if (cnt) {
+      cnt[v] = c;
+      ahead[v] = KC_UNSET;
+    }
   }
 }
 
@@ -190,13 +195,54 @@ __global__ __launch_bounds__(1024) void k_kc_classify(uint64_t* __restrict__ can
 }
 
 // ---- h-index: lanes and waves -------------------------------------------------------------
+// Largest i in [1, top] with (count of bins >= i) >= i from a wave's histogram (top <= KC_HIST;
+// 0: none): lane l owns bins [PER l, PER l + PER), and the bins of the lanes above it are
+// suffix-summed.  Every lane gets the answer.
+__device__ __forceinline__ uint32_t kc_wave_pick(const uint32_t* hist, uint32_t top) {
+  const int lane = threadIdx.x & 63;
+  const uint32_t j0 = (uint32_t)lane * KC_PER;
+  uint32_t own = 0;
+  for (uint32_t j = j0; j < j0 + KC_PER && j <= top; ++j) own += hist[j];
+  uint32_t incl = own;
+  for (int off = 1; off < 64; off <<= 1) {
+    const uint32_t t = __shfl_down(incl, off, 64);
+    if (lane + off < 64) incl += t;
+  }
+  uint32_t best = 0, sum = incl - own;
+  for (int j = (int)std::min(j0 + KC_PER - 1, top); j >= (int)j0 && j >= 1; --j) {
+    sum += hist[j];
+    if (sum >= (uint32_t)j) {
+      best = (uint32_t)j;
+      break;
+    }
+  }
+  for (int off = 32; off > 0; off >>= 1) best = std::max(best, (uint32_t)__shfl_xor(best, off, 64));
+  return best;
+}
+
+// the same from one lane's byte histogram
+__device__ __forceinline__ uint32_t kc_lane_pick(const uint8_t* h, uint32_t top) {
+  uint32_t sum = 0;
+  for (uint32_t j = top; j > 0; --j) {
+    sum += h[j];
+    if (sum >= j) return j;
+  }
+  return 0;
+}
+
+__device__ __forceinline__ void kc_wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 // The wave pass's vertices first (the longer ones), then one lane per vertex of the small
 // queue.  A wave's LDS share serves both: KC_PER words per lane as one histogram of the
-// wave, or KC_SMALL + 1 bytes per lane.
+// wave, or KC_SMALL + 1 bytes per lane.  ahead: the answers that the last spread found already
+// (see there), nullptr without counts.
 __global__ __launch_bounds__(KC_THREADS) void k_kc_hindex(
     const uint32_t* __restrict__ qsmall, const uint32_t* __restrict__ qbig, const kc_counters* __restrict__ cnt_in,
     const uint64_t* __restrict__ ptr, const uint32_t* __restrict__ idx, const uint32_t* __restrict__ est,
-    uint32_t* __restrict__ core) {
+    uint32_t* __restrict__ ahead, uint32_t* __restrict__ core) {
   __shared__ uint32_t hist_all[KC_THREADS / 64][64 * KC_PER];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   uint32_t* hist = hist_all[wave];
@@ -204,11 +250,18 @@ __global__ __launch_bounds__(KC_THREADS) void k_kc_hindex(
   const uint64_t wave_id = grid_wave_id(), nwaves = grid_waves();
   for (uint64_t q = wave_id; q < nbig; q += nwaves) {
     const uint32_t v = qbig[q];
+    const uint32_t known = ahead ? ahead[v] : KC_UNSET;
+    if (known != KC_UNSET) {  // uniform
+      if (lane == 0) {
+        core[v] = known;
+        ahead[v] = KC_UNSET;
+      }
+      continue;
+    }
     const uint64_t b = ptr[v], e = ptr[v + 1];
     const uint32_t top = (uint32_t)std::min<uint64_t>(e - b, (uint64_t)est[v]);  // at most KC_HIST
     for (uint32_t j = lane; j <= top; j += 64) hist[j] = 0;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+    kc_wave_fence();
     for (uint64_t k0 = b; k0 < e; k0 += 64 * KC_U) {
       uint32_t eu[KC_U];
 #pragma unroll
@@ -220,35 +273,21 @@ __global__ __launch_bounds__(KC_THREADS) void k_kc_hindex(
       for (int i = 0; i < KC_U; ++i)
         if (k0 + (uint64_t)i * 64 + lane < e) atomicAdd(&hist[eu[i] < top ? eu[i] : top], 1u);
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    // largest i in [1, top] with (count of bins >= i) >= i: lane l owns bins
-    // [PER l, PER l + PER), and the bins of the lanes above it are suffix-summed
-    const uint32_t j0 = (uint32_t)lane * KC_PER;
-    uint32_t own = 0;
-    for (uint32_t j = j0; j < j0 + KC_PER && j <= top; ++j) own += hist[j];
-    uint32_t incl = own;
-    for (int off = 1; off < 64; off <<= 1) {
-      const uint32_t t = __shfl_down(incl, off, 64);
-      if (lane + off < 64) incl += t;
-    }
-    uint32_t best = 0, sum = incl - own;
-    for (int j = (int)std::min(j0 + KC_PER - 1, top); j >= (int)j0 && j >= 1; --j) {
-      sum += hist[j];
-      if (sum >= (uint32_t)j) {
-        best = (uint32_t)j;
-        break;
-      }
-    }
-    for (int off = 32; off > 0; off >>= 1) best = std::max(best, (uint32_t)__shfl_xor(best, off, 64));
+    kc_wave_fence();
+    const uint32_t best = kc_wave_pick(hist, top);
     if (lane == 0 && best && best < core[v]) core[v] = best;
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+    kc_wave_fence();
   }
   uint8_t* h = reinterpret_cast<uint8_t*>(hist) + lane * (KC_SMALL + 1);
   for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < nsmall;
        i += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t v = qsmall[i];
+    const uint32_t known = ahead ? ahead[v] : KC_UNSET;
+    if (known != KC_UNSET) {
+      core[v] = known;
+      ahead[v] = KC_UNSET;
+      continue;
+    }
     const uint64_t b = ptr[v], e = ptr[v + 1];
     if (b == e) {
       core[v] = 0;  // kcore.hpp:214-218
@@ -260,14 +299,7 @@ __global__ __launch_bounds__(KC_THREADS) void k_kc_hindex(
       const uint32_t eu = est[idx[k]];
       ++h[eu < cap ? eu : cap];
     }
-    uint32_t sum = 0, best = 0;
-    for (uint32_t j = cap; j > 0; --j) {
-      sum += h[j];
-      if (sum >= j) {
-        best = j;
-        break;
-      }
-    }
+    const uint32_t best = kc_lane_pick(h, cap);
     if (best && best < core[v]) core[v] = best;
   }
 }
@@ -332,12 +364,22 @@ __device__ void kc_block_pick(const uint32_t* hist, uint32_t nb, uint32_t base, 
 // One block per queued vertex of up to KC_GIANT neighbours.
 __global__ __launch_bounds__(KC_HTHREADS) void k_kc_huge(
     const uint32_t* __restrict__ qhuge_end, const kc_counters* __restrict__ cnt_in, const uint64_t* __restrict__ ptr,
-    const uint32_t* __restrict__ idx, const uint32_t* __restrict__ est, uint32_t* __restrict__ core) {
+    const uint32_t* __restrict__ idx, const uint32_t* __restrict__ est, uint32_t* ahead,
+    uint32_t* __restrict__ core) {
   __shared__ uint32_t hist[KC_HTHREADS * KC_HPER];
   const int tid = threadIdx.x;
   const uint64_t nhuge = cnt_in->nhuge;
   for (uint64_t q = blockIdx.x; q < nhuge; q += gridDim.x) {
     const uint32_t v = *(qhuge_end - q);
+    const uint32_t known = ahead ? ahead[v] : KC_UNSET;
+    if (known != KC_UNSET) {  // uniform
+      __syncthreads();  // every thread has read it
+      if (tid == 0) {
+        core[v] = known;
+        ahead[v] = KC_UNSET;
+      }
+      continue;
+    }
     const uint64_t b = ptr[v], e = ptr[v + 1];
     const uint32_t cap = (uint32_t)std::min<uint64_t>(e - b, (uint64_t)est[v]);
     int shift = kc_first_shift(cap);
@@ -512,51 +554,135 @@ struct kc_spread {
     }
     return c;
   }
+  // with counts: the same, and the capped new values into hist[0..now]
+  __device__ __forceinline__ void range_hist(uint64_t b, uint64_t e, uint32_t i0, uint32_t step, uint32_t old,
+                                             uint32_t now, uint32_t* hist) const {
+    for (uint64_t k0 = b; k0 < e; k0 += (uint64_t)step * KC_U) {
+      uint32_t u[KC_U], cu[KC_U];
+#pragma unroll
+      for (int i = 0; i < KC_U; ++i) {
+        const uint64_t k = k0 + (uint64_t)i * step + i0;
+        u[i] = k < e ? idx[k] : 0u;
+        cu[i] = k < e ? core[u[i]] : 0u;
+      }
+#pragma unroll
+      for (int i = 0; i < KC_U; ++i)
+        if (k0 + (uint64_t)i * step + i0 < e) {
+          (void)one(u[i], cu[i], old, now);
+          atomicAdd(&hist[cu[i] < now ? cu[i] : now], 1u);
+        }
+    }
+  }
+  // one lane's list
+  __device__ __forceinline__ void range_lane(uint64_t b, uint64_t e, uint32_t old, uint32_t now, uint8_t* h) const {
+    for (uint64_t k0 = b; k0 < e; k0 += KC_U) {
+      uint32_t u[KC_U], cu[KC_U];
+#pragma unroll
+      for (int i = 0; i < KC_U; ++i) {
+        u[i] = k0 + i < e ? idx[k0 + i] : 0u;
+        cu[i] = k0 + i < e ? core[u[i]] : 0u;
+      }
+#pragma unroll
+      for (int i = 0; i < KC_U; ++i)
+        if (k0 + i < e) {
+          (void)one(u[i], cu[i], old, now);
+          ++h[cu[i] < now ? cu[i] : now];
+        }
+    }
+  }
 };
 
+// With counts a spread's walk also takes the histogram of the neighbours' new values, capped at
+// the vertex's own: it holds both its count and, when that falls short, its h-index of the next
+// epoch, whose estimates are these values.  The vertex is then a candidate of the next epoch
+// for sure, and `ahead` carries the answer there instead of a second walk (RMAT scale 22, all
+// epochs: h-index passes 7.0 -> 3.0 ms, spreads 10.2 -> 10.5 ms).  A block's vertex with a value above
+// KC_HHIST and a giant have too many values for that and are walked again.
 __global__ __launch_bounds__(KC_THREADS) void k_kc_spread(
     const uint32_t* __restrict__ qsmall, const uint32_t* __restrict__ qbig, const kc_counters* __restrict__ cnt_in,
-    const uint64_t* __restrict__ ptr, kc_spread sp) {
-  const int lane = threadIdx.x & 63;
+    const uint64_t* __restrict__ ptr, kc_spread sp, uint32_t* __restrict__ ahead) {
+  __shared__ uint32_t hist_all[KC_THREADS / 64][64 * KC_PER];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t* hist = hist_all[wave];
   const uint64_t nbig = cnt_in->nbig, nsmall = cnt_in->nsmall;
   const uint64_t wave_id = grid_wave_id(), nwaves = grid_waves();
   for (uint64_t q = wave_id; q < nbig; q += nwaves) {
     const uint32_t v = qbig[q];
     const uint32_t old = sp.est[v], now = sp.core[v];
     if (old == now) continue;  // uniform
-    uint32_t c = sp.range(ptr[v], ptr[v + 1], (uint32_t)lane, 64u, old, now);
-    if (sp.cnt_v) {
-      for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
-      if (lane == 0) sp.cnt_v[v] = c;
+    if (!sp.cnt_v) {
+      (void)sp.range(ptr[v], ptr[v + 1], (uint32_t)lane, 64u, old, now);
+      continue;
     }
+    for (uint32_t j = lane; j <= now; j += 64) hist[j] = 0;
+    kc_wave_fence();
+    sp.range_hist(ptr[v], ptr[v + 1], (uint32_t)lane, 64u, old, now, hist);
+    kc_wave_fence();
+    const uint32_t c = hist[now];
+    const uint32_t best = c < now ? kc_wave_pick(hist, now) : 0u;
+    if (lane == 0) {
+      sp.cnt_v[v] = c;
+      if (best) ahead[v] = best;
+    }
+    kc_wave_fence();
   }
+  uint8_t* h = reinterpret_cast<uint8_t*>(hist) + lane * (KC_SMALL + 1);
   for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < nsmall;
        i += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t v = qsmall[i];
     const uint32_t old = sp.est[v], now = sp.core[v];
     if (old == now) continue;
-    const uint32_t c = sp.range(ptr[v], ptr[v + 1], 0u, 1u, old, now);
-    if (sp.cnt_v) sp.cnt_v[v] = c;
+    if (!sp.cnt_v || old == KC_UNSET) {
+      (void)sp.range(ptr[v], ptr[v + 1], 0u, 1u, old, now);
+      continue;
+    }
+    for (uint32_t j = 0; j <= now; ++j) h[j] = 0;
+    sp.range_lane(ptr[v], ptr[v + 1], old, now, h);
+    const uint32_t c = h[now];
+    sp.cnt_v[v] = c;
+    if (c < now) {
+      const uint32_t best = kc_lane_pick(h, now);
+      if (best) ahead[v] = best;
+    }
   }
 }
 
 __global__ __launch_bounds__(KC_HTHREADS) void k_kc_spread_huge(const uint32_t* __restrict__ qhuge_end,
                                                                 const kc_counters* __restrict__ cnt_in,
-                                                                const uint64_t* __restrict__ ptr, kc_spread sp) {
+                                                                const uint64_t* __restrict__ ptr, kc_spread sp,
+                                                                uint32_t* __restrict__ ahead) {
+  __shared__ uint32_t hist[KC_HTHREADS * KC_HPER];
   __shared__ uint32_t s_c;
+  const uint32_t tid = threadIdx.x;
   const uint64_t nhuge = cnt_in->nhuge;
   for (uint64_t q = blockIdx.x; q < nhuge; q += gridDim.x) {
     const uint32_t v = *(qhuge_end - q);
     const uint32_t old = sp.est[v], now = sp.core[v];
     if (old == now) continue;  // uniform
-    if (threadIdx.x == 0) s_c = 0u;
-    __syncthreads();
-    uint32_t c = sp.range(ptr[v], ptr[v + 1], threadIdx.x, KC_HTHREADS, old, now);
-    if (sp.cnt_v) {
-      for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
-      if ((threadIdx.x & 63) == 0) atomicAdd(&s_c, c);
+    if (!sp.cnt_v) {
+      (void)sp.range(ptr[v], ptr[v + 1], tid, KC_HTHREADS, old, now);
+      continue;
+    }
+    if (now <= KC_HHIST) {  // uniform
+      for (uint32_t j = tid; j <= now; j += KC_HTHREADS) hist[j] = 0;
       __syncthreads();
-      if (threadIdx.x == 0) sp.cnt_v[v] = s_c;
+      sp.range_hist(ptr[v], ptr[v + 1], tid, KC_HTHREADS, old, now, hist);
+      __syncthreads();
+      const uint32_t c = hist[now];
+      uint32_t best = 0, over;
+      if (c < now) kc_block_pick(hist, now, 0u, 0, 0u, &best, &over);
+      if (tid == 0) {
+        sp.cnt_v[v] = c;
+        if (best) ahead[v] = best;
+      }
+    } else {
+      if (tid == 0) s_c = 0u;
+      __syncthreads();
+      uint32_t c = sp.range(ptr[v], ptr[v + 1], tid, KC_HTHREADS, old, now);
+      for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
+      if ((tid & 63) == 0) atomicAdd(&s_c, c);
+      __syncthreads();
+      if (tid == 0) sp.cnt_v[v] = s_c;
     }
     __syncthreads();
   }
@@ -660,13 +786,16 @@ extern "C" int pe_kcore(pe_graph_t* g, int out_edges, uint32_t* coreness, uint64
     const bool counts = g->csr_is_csc;  // the adjacency is its own reverse
     const uint64_t nwords = ((uint64_t)V >> 6) + 1;
     const uint32_t Vs = std::max<uint32_t>(1, V);
-    dbuf<uint32_t> core(ctx, Vs), est(ctx, Vs), qsmall(ctx, Vs), qbig(ctx, Vs), cnt_v;
+    dbuf<uint32_t> core(ctx, Vs), est(ctx, Vs), qsmall(ctx, Vs), qbig(ctx, Vs), cnt_v, ahead;
     dbuf<uint64_t> cand(ctx, nwords), act, nxt(ctx, nwords * 8);  // nxt: one byte per vertex
-    if (counts) cnt_v.alloc(ctx, Vs);
+    if (counts) {
+      cnt_v.alloc(ctx, Vs);
+      ahead.alloc(ctx, Vs);
+    }
     uint32_t* qhuge_end = qbig.p + (Vs - 1);
     dbuf<kc_counters> cnt(ctx, 2);  // two sets: consecutive epochs alternate
     PE_HIP(hipEventRecord(ctx->t0, s));
-    k_kc_init<<<grid_for(V, 256, 8192), 256, 0, s>>>(ptr, V, core.p, est.p, cnt_v.p);
+    k_kc_init<<<grid_for(V, 256, 8192), 256, 0, s>>>(ptr, V, core.p, est.p, cnt_v.p, ahead.p);
     k_kc_fill<<<grid_for(nwords, 256, 4096), 256, 0, s>>>(cand.p, nwords, V);  // active_current.fill()
     k_kc_zero<<<grid_for(nwords * 8, 256, 4096), 256, 0, s>>>(nxt.p, nwords * 8);
     PE_HIP(hipGetLastError());
@@ -698,8 +827,8 @@ extern "C" int pe_kcore(pe_graph_t* g, int out_edges, uint32_t* coreness, uint64
         const unsigned hgrid = (unsigned)std::min<uint64_t>(huge_max, ncand);
         k_kc_classify<<<grid_for(nwords, 16 * KC_CW_WORDS, (unsigned)std::max(1, ctx->num_cus) * 2), 1024, 0, s>>>(
             cand.p, act.p, nwords, V, ptr, est.p, qsmall.p, qbig.p, qhuge_end, c);
-        k_kc_huge<<<hgrid, KC_HTHREADS, 0, s>>>(qhuge_end, c, ptr, idx, est.p, core.p);
-        k_kc_hindex<<<grid, KC_THREADS, 0, s>>>(qsmall.p, qbig.p, c, ptr, idx, est.p, core.p);
+        k_kc_huge<<<hgrid, KC_HTHREADS, 0, s>>>(qhuge_end, c, ptr, idx, est.p, ahead.p, core.p);
+        k_kc_hindex<<<grid, KC_THREADS, 0, s>>>(qsmall.p, qbig.p, c, ptr, idx, est.p, ahead.p, core.p);
         if (ngiant) {
           // rounds: 14 bits of the answer each after the first
           int rounds = 1;
@@ -713,8 +842,8 @@ extern "C" int pe_kcore(pe_graph_t* g, int out_edges, uint32_t* coreness, uint64
           }
           k_kc_spread_giant<<<huge_max, KC_HTHREADS, 0, s>>>(ptr, gl, giants.count.p, giants.start.p, act.p, sp);
         }
-        k_kc_spread_huge<<<hgrid, KC_HTHREADS, 0, s>>>(qhuge_end, c, ptr, sp);
-        k_kc_spread<<<grid, KC_THREADS, 0, s>>>(qsmall.p, qbig.p, c, ptr, sp);
+        k_kc_spread_huge<<<hgrid, KC_HTHREADS, 0, s>>>(qhuge_end, c, ptr, sp, ahead.p);
+        k_kc_spread<<<grid, KC_THREADS, 0, s>>>(qsmall.p, qbig.p, c, ptr, sp, ahead.p);
         k_kc_commit<<<grid_for(ncand, KC_THREADS, full_grid), KC_THREADS, 0, s>>>(
             qsmall.p, qbig.p, qhuge_end, gl, giants.count.p, act.p, core.p, est.p, cnt_v.p, cand.p, c);
         k_kc_next<<<grid_for(nwords * 8, 256, (unsigned)std::max(1, ctx->num_cus) * 2), 256, 0, s>>>(nxt.p, cand.p, nwords, counts ? 0 : 1, c);

@@ -152,3 +152,22 @@ def test_adjacency_length_classes(ctx, length, directed):
     g = Graph.from_edges(ctx, s, d, V, directed=directed, relabel=length % 2 == 1)
     _check(g, og)
     g.close()
+
+
+@pytest.mark.parametrize("length", [60, 64, 1500, 4096, 5000, 40000])
+def test_values_that_fall_epoch_after_epoch(ctx, length):
+    """Hubs of `length` neighbours over a skewed rim: they drop in several epochs running, so the
+    value of a drop comes from the previous epoch's walk in the pass of each adjacency length."""
+    from plato_amd import Graph
+    rng = np.random.default_rng(length)
+    rim, hubs = max(2 * length, 300), 6
+    m = 12 * rim
+    s = np.concatenate([np.full(length, rim + h) for h in range(hubs)] + [(rim * rng.random(m) ** 3).astype(np.int64)])
+    d = np.concatenate([rng.choice(rim, length, replace=False) for _ in range(hubs)]
+                       + [(rim * rng.random(m) ** 2).astype(np.int64)])
+    s, d = s.astype(np.uint32), d.astype(np.uint32)
+    V = rim + hubs
+    print(f"case: kcore falling values length={length}", flush=True)
+    g = Graph.from_edges(ctx, s, d, V, directed=False)
+    _check(g, oracle.CSC(V, s, d, symmetrize=True))
+    g.close()
