@@ -128,7 +128,7 @@ __device__ __forceinline__ float ld_row(const float* X, uint32_t u, uint32_t str
 
 // A column's sum (or a long column's chunk sum) runs as BS interleaved Kahan sums: edge k
 // of the column (counted from its first edge, or the chunk's) goes to sub-sum k % BS, and
-// the sub-sums are combined in order 0..BS-1 with TwoSum.  Every pass kernel below, however
+// the sub-sums are combined in order 0..BS-1 with TwoSum.  Every form of the pass below, however
 // many edges it puts in one row load, keeps exactly this arithmetic, so a column's bits do
 // not depend on how many other columns are in the pass.
 static constexpr int BS = 4;
@@ -232,7 +232,7 @@ __device__ __forceinline__ uint64_t lane_u64(uint64_t v, int i) {
   return ((uint64_t)hi << 32) | lo;
 }
 
-// Which columns a pass must write, and which pass kernel runs.  A column is covered while
+// Which columns a pass must write, and which form of the pass runs.  A column is covered while
 // LOADING, ACTIVE or FINAL, and for the first pass after it turns DONE (that pass copies its
 // final value into the other buffer; after it both buffers hold it).  EMPTY and settled DONE
 // columns are left alone: nothing reads an EMPTY column, and a settled one is the same in
@@ -241,47 +241,41 @@ __device__ __forceinline__ uint64_t lane_u64(uint64_t v, int i) {
 // block); at most 16 or 32 put 4 or 2 edges in a row load of the wide block; more run one
 // edge per load, every column written.  The limits come from the batch options (these
 // widths by default; a kernel can be turned off).
-__global__ void k_batch_plan(batch_ctl* __restrict__ ctl, const uint32_t* __restrict__ status) {
-  const int j = threadIdx.x;  // one wave, lane j = column j
-  const uint32_t st = status[j];
+//
+// One wave, lane j = column j.  The plan follows from the column states and the last pass
+// alone, so it is made again wherever a state changes (the end of a pass, an admission, a
+// release) and is ready when the next pass starts.
+__device__ __forceinline__ void batch_plan(batch_ctl* __restrict__ ctl, uint32_t j, uint32_t st) {
   const bool covered = st == COL_LOADING || st == COL_ACTIVE || st == COL_FINAL || (st == COL_DONE && ctl->pend[j]);
   const uint64_t mask = __ballot(covered);
   const uint32_t n = (uint32_t)__popcll(mask);
   const uint32_t r = (uint32_t)__popcll(mask & ((1ull << j) - 1ull));
   const bool packed = n >= 1 && n <= ctl->max_packed;
   // the packed block is valid if the last pass was packed over exactly these columns
-  const uint32_t last_n = ctl->pk_n;
   const bool same = !covered || (r < (uint32_t)BATCH_PACKED_W && ctl->pk_cols[r] == (uint8_t)j);
-  const bool valid = packed && last_n == n && __ballot(!same) == 0ull;
-  __syncthreads();  // every lane has read the last plan before it is overwritten
+  const bool valid = packed && ctl->pk_n == n && __ballot(!same) == 0ull;
   ctl->qof[j] = covered ? (uint8_t)r : (uint8_t)0xFF;
-  if (covered) {
-    ctl->cols[r] = (uint8_t)j;
-    if (packed) ctl->pk_cols[r] = (uint8_t)j;
-  }
+  if (covered) ctl->cols[r] = (uint8_t)j;
   if (j == 0) {
     ctl->ncols = n;
     ctl->mode = packed ? BATCH_MODE_PACKED : n <= ctl->max_edges4 ? 4u : n <= ctl->max_edges2 ? 2u : 1u;
     ctl->pk_valid = valid ? 1u : 0u;
-    ctl->pk_n = packed ? n : 0xFFFFFFFFu;
   }
 }
 
-// One pass over the tasks with P edges per row load; runs only if the plan chose it.
+// One pass over the tasks with P edges per row load.
 // PK: the packed pass (P = 4, at most BATCH_PACKED_W columns): rows come from the packed
 // block when the plan allows it, else from the wide one, and every new value goes to both.
 template <int P, bool PK>
-__global__ __launch_bounds__(256) void k_batch_tasks(
-    const uint64_t* __restrict__ col_ptr, const uint32_t* __restrict__ row_idx,
+__device__ __forceinline__ void batch_pass(
+    double (&s_red)[4][BK], const uint64_t* __restrict__ col_ptr, const uint32_t* __restrict__ row_idx,
     const uint32_t* __restrict__ od, const uint64_t* __restrict__ seedmask,
     const bt_task* __restrict__ tasks, uint64_t ntasks, float* X0, float* X1, float* P0, float* P1,
     const batch_ctl* __restrict__ ctl, const uint32_t* __restrict__ status,
     const double* __restrict__ init_dist, double damping, float2* __restrict__ partial,
     double* __restrict__ part_delta) {
   static_assert(!PK || P == 4, "the packed pass puts 4 edges in a load");
-  if (ctl->mode != (PK ? BATCH_MODE_PACKED : (uint32_t)P)) return;
   constexpr int W = BK / P;
-  __shared__ double s_red[4][BK];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int p = lane / W, q = lane % W;
   const uint32_t cur = ctl->cur;
@@ -365,6 +359,33 @@ __global__ __launch_bounds__(256) void k_batch_tasks(
   }
 }
 
+// The pass that the plan chose.  All forms in one kernel: each has at most 64 registers, so
+// none costs another its waves, where a kernel per form launched three that return at once
+// (5 us each per pass).
+__global__ __launch_bounds__(256) void k_batch_tasks(
+    const uint64_t* __restrict__ col_ptr, const uint32_t* __restrict__ row_idx,
+    const uint32_t* __restrict__ od, const uint64_t* __restrict__ seedmask,
+    const bt_task* __restrict__ tasks, uint64_t ntasks, float* X0, float* X1, float* P0, float* P1,
+    const batch_ctl* __restrict__ ctl, const uint32_t* __restrict__ status,
+    const double* __restrict__ init_dist, double damping, float2* __restrict__ partial,
+    double* __restrict__ part_delta) {
+  __shared__ double s_red[4][BK];
+  switch (ctl->mode) {
+    case 1u:
+      return batch_pass<1, false>(s_red, col_ptr, row_idx, od, seedmask, tasks, ntasks, X0, X1, P0, P1, ctl, status,
+                                  init_dist, damping, partial, part_delta);
+    case 2u:
+      return batch_pass<2, false>(s_red, col_ptr, row_idx, od, seedmask, tasks, ntasks, X0, X1, P0, P1, ctl, status,
+                                  init_dist, damping, partial, part_delta);
+    case 4u:
+      return batch_pass<4, false>(s_red, col_ptr, row_idx, od, seedmask, tasks, ntasks, X0, X1, P0, P1, ctl, status,
+                                  init_dist, damping, partial, part_delta);
+    default:
+      return batch_pass<4, true>(s_red, col_ptr, row_idx, od, seedmask, tasks, ntasks, X0, X1, P0, P1, ctl, status,
+                                 init_dist, damping, partial, part_delta);
+  }
+}
+
 // Long columns: chunk partials combined in chunk order, then applied.
 __global__ __launch_bounds__(256) void k_batch_fixup(
     const uint32_t* __restrict__ od, const uint64_t* __restrict__ seedmask,
@@ -418,8 +439,11 @@ __global__ __launch_bounds__(256) void k_batch_fixup(
   }
 }
 
-// Per-column delta, state transitions, buffer flip.  One block of 64 threads.
+// Per-column delta, state transitions, buffer flip, the next pass's plan.  One block: a
+// group's sum is a chain of adds in a fixed order, but FIN_U of its loads are in flight at a
+// time (2048 blocks' partials: 47 -> 26 us).
 static constexpr int FIN_GROUPS = 16;
+static constexpr int FIN_U = 16;
 
 __global__ __launch_bounds__(FIN_GROUPS * BK) void k_batch_finish(const double* __restrict__ part_delta, uint32_t nparts,
                                batch_ctl* __restrict__ ctl, uint32_t* __restrict__ status,
@@ -431,16 +455,24 @@ __global__ __launch_bounds__(FIN_GROUPS * BK) void k_batch_finish(const double* 
   const int j = threadIdx.x & (BK - 1), grp = threadIdx.x / BK;
   {
     double d = 0.0;
-    for (uint32_t b = grp; b < nparts; b += FIN_GROUPS) d += part_delta[(uint64_t)b * BK + j];
+    uint32_t b = grp;
+    for (; b + (FIN_U - 1) * FIN_GROUPS < nparts; b += FIN_U * FIN_GROUPS) {
+      double x[FIN_U];
+#pragma unroll
+      for (int i = 0; i < FIN_U; ++i) x[i] = part_delta[(uint64_t)(b + i * FIN_GROUPS) * BK + j];
+#pragma unroll
+      for (int i = 0; i < FIN_U; ++i) d += x[i];
+    }
+    for (; b < nparts; b += FIN_GROUPS) d += part_delta[(uint64_t)b * BK + j];
     s_sum[grp][j] = d;
   }
   __syncthreads();
   if (threadIdx.x < BK) {
     double d = 0.0;
     for (int q = 0; q < FIN_GROUPS; ++q) d += s_sum[q][j];
-    const uint32_t st = status[j];
+    uint32_t st = status[j];
     if (st == COL_LOADING) {
-      status[j] = COL_ACTIVE;
+      st = COL_ACTIVE;
       iters[j] = 0;
     } else if (st == COL_ACTIVE) {
       const uint32_t it = iters[j] + 1;
@@ -448,28 +480,63 @@ __global__ __launch_bounds__(FIN_GROUPS * BK) void k_batch_finish(const double* 
       last_delta[j] = d;
       // delta < tol jumps to one more, final, iteration; the cap makes the
       // max_iters-th iteration the final one
-      if (d < tol || it + 1 >= max_iters) status[j] = COL_FINAL;
+      if (d < tol || it + 1 >= max_iters) st = COL_FINAL;
     } else if (st == COL_FINAL) {
       iters[j] = iters[j] + 1;
-      status[j] = COL_DONE;
+      st = COL_DONE;
       ctl->pend[j] = 1u;  // the next pass copies the final value into the other buffer
     } else if (st == COL_DONE) {
       ctl->pend[j] = 0u;
     }
+    status[j] = st;
+    const bool packed = ctl->mode == BATCH_MODE_PACKED;
+    if (packed && (uint32_t)j < ctl->ncols) ctl->pk_cols[j] = ctl->cols[j];
+    if (j == 0) {
+      ctl->pk_n = packed ? ctl->ncols : 0xFFFFFFFFu;
+      ctl->cur ^= 1u;
+      ctl->iteration += 1;
+    }
   }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    ctl->cur ^= 1u;
-    ctl->iteration += 1;
-  }
+  __syncthreads();  // the packed columns, before the plan reads them
+  if (threadIdx.x < BK) batch_plan(ctl, (uint32_t)j, status[j]);
 }
 
-__global__ void k_batch_seed_bits(uint64_t* __restrict__ seedmask, const uint32_t* __restrict__ ids,
-                                  uint32_t n, uint32_t slot, int set) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    if (set) atomicOr((unsigned long long*)&seedmask[ids[i]], 1ull << slot);
-    else atomicAnd((unsigned long long*)&seedmask[ids[i]], ~(1ull << slot));
+// Seed ids (input ids, each once) of an admission or a release: up to SEEDS_INLINE come with
+// the launch itself, so such a call is one kernel with no copy and no wait (64 admissions and
+// releases with two copies, three kernels and waits each: 5.5 ms of host time; now below 0.5 ms).
+static constexpr uint32_t SEEDS_INLINE = 64;
+struct seed_list {
+  uint32_t n;
+  const uint32_t* ids;  // device, nullptr: `few`
+  uint32_t few[SEEDS_INLINE];
+  __device__ __forceinline__ uint32_t internal(uint32_t i, const uint32_t* __restrict__ rank_of) const {
+    const uint32_t v = ids ? ids[i] : few[i];
+    return rank_of ? rank_of[v] : v;
   }
+};
+
+// the first wave of block 0: the slot's state, and the plan that follows from it
+__device__ __forceinline__ void set_slot(batch_ctl* __restrict__ ctl, uint32_t* __restrict__ status,
+                                         double* __restrict__ init_dist, uint32_t* __restrict__ iters,
+                                         double* __restrict__ last_delta, uint32_t slot, uint32_t st, double dist) {
+  if (blockIdx.x != 0 || threadIdx.x >= BK) return;
+  const uint32_t j = threadIdx.x;
+  if (j == slot) {
+    status[slot] = st;
+    init_dist[slot] = dist;
+    iters[slot] = 0;
+    last_delta[slot] = 0.0;
+  }
+  batch_plan(ctl, j, j == slot ? st : status[j]);
+}
+
+__global__ void k_batch_admit(seed_list seeds, const uint32_t* __restrict__ rank_of, uint64_t* __restrict__ seedmask,
+                              batch_ctl* __restrict__ ctl, uint32_t* __restrict__ status,
+                              double* __restrict__ init_dist, uint32_t* __restrict__ iters,
+                              double* __restrict__ last_delta, uint32_t slot, double dist) {
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < seeds.n; i += gridDim.x * blockDim.x)
+    atomicOr((unsigned long long*)&seedmask[seeds.internal(i, rank_of)], 1ull << slot);
+  set_slot(ctl, status, init_dist, iters, last_delta, slot, COL_LOADING, dist);
 }
 
 // A released slot's seeds stop being seeds: their entries in that column go to 0 in both
@@ -477,27 +544,24 @@ __global__ void k_batch_seed_bits(uint64_t* __restrict__ seedmask, const uint32_
 // In the packed block a row holds whatever columns the last packed pass covered, so a seed
 // that is left without in-edges and without seeds (a vertex the passes skip) gets its whole
 // packed row cleared; the rows of other vertices are rewritten by every pass.
-__global__ void k_batch_zero_slot(float* X0, float* X1, float* P0, float* P1, const uint64_t* __restrict__ col_ptr,
-                                  const uint64_t* __restrict__ seedmask, const uint32_t* __restrict__ ids, uint32_t n,
-                                  uint32_t slot) {
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-    const uint32_t v = ids[i];
+__global__ void k_batch_release(seed_list seeds, const uint32_t* __restrict__ rank_of,
+                                const uint64_t* __restrict__ col_ptr, float* X0, float* X1, float* P0, float* P1,
+                                uint64_t* __restrict__ seedmask, batch_ctl* __restrict__ ctl,
+                                uint32_t* __restrict__ status, double* __restrict__ init_dist,
+                                uint32_t* __restrict__ iters, double* __restrict__ last_delta, uint32_t slot) {
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < seeds.n; i += gridDim.x * blockDim.x) {
+    const uint32_t v = seeds.internal(i, rank_of);
+    const uint64_t bit = 1ull << slot;
+    const uint64_t left = atomicAnd((unsigned long long*)&seedmask[v], ~bit) & ~bit;
     X0[(uint64_t)v * BK + slot] = 0.0f;
     X1[(uint64_t)v * BK + slot] = 0.0f;
-    if (seedmask[v] == 0ull && col_ptr[v] == col_ptr[v + 1])
+    if (left == 0ull && col_ptr[v] == col_ptr[v + 1])
       for (int k = 0; k < BATCH_PACKED_W; ++k) {
         P0[(uint64_t)v * BATCH_PACKED_W + k] = 0.0f;
         P1[(uint64_t)v * BATCH_PACKED_W + k] = 0.0f;
       }
   }
-}
-
-__global__ void k_batch_set_slot(uint32_t* status, double* init_dist, uint32_t* iters, double* last_delta,
-                                 uint32_t slot, uint32_t st, double dist) {
-  status[slot] = st;
-  init_dist[slot] = dist;
-  iters[slot] = 0;
-  last_delta[slot] = 0.0;
+  set_slot(ctl, status, init_dist, iters, last_delta, slot, COL_EMPTY, 0.0);
 }
 
 // Entries [v0, v0 + n) (input ids; rank_of: input -> internal, nullptr when they are the same)
@@ -627,7 +691,7 @@ struct pe_ppr_batch_s {
   dbuf<double> init_dist, last_delta;
   uint64_t ntasks = 0, nlong = 0, nchunks = 0;
   unsigned task_grid = 0, fix_grid = 0;
-  std::vector<std::vector<uint32_t>> slot_seeds;  // internal ids per slot
+  std::vector<std::vector<uint32_t>> slot_seeds;  // input ids per slot, each once
   std::vector<uint32_t> host_status;
   stream_graph sg;  // the captured iterations, replayed by step()
   uint32_t graph_iters = 0;
@@ -697,20 +761,9 @@ struct pe_ppr_batch_s {
     hipStream_t s = g->ctx->stream;
     {
       ktime_scope kt(g->ctx, PE_KT_PPR_BLOCK);
-      // the plan picks one of the four pass kernels; the others return at once
-      k_batch_plan<<<1, BK, 0, s>>>(ctl.p, status.p);
-      k_batch_tasks<4, true><<<task_grid, 256, 0, s>>>(g->col_ptr.p, g->row_idx.p, g->od.p, seedmask.p, tasks.p,
-                                                       ntasks, X0.p, X1.p, P0.p, P1.p, ctl.p, status.p, init_dist.p,
-                                                       opts.damping, partial.p, part_delta.p);
-      k_batch_tasks<4, false><<<task_grid, 256, 0, s>>>(g->col_ptr.p, g->row_idx.p, g->od.p, seedmask.p, tasks.p,
-                                                        ntasks, X0.p, X1.p, P0.p, P1.p, ctl.p, status.p, init_dist.p,
-                                                        opts.damping, partial.p, part_delta.p);
-      k_batch_tasks<2, false><<<task_grid, 256, 0, s>>>(g->col_ptr.p, g->row_idx.p, g->od.p, seedmask.p, tasks.p,
-                                                        ntasks, X0.p, X1.p, P0.p, P1.p, ctl.p, status.p, init_dist.p,
-                                                        opts.damping, partial.p, part_delta.p);
-      k_batch_tasks<1, false><<<task_grid, 256, 0, s>>>(g->col_ptr.p, g->row_idx.p, g->od.p, seedmask.p, tasks.p,
-                                                        ntasks, X0.p, X1.p, P0.p, P1.p, ctl.p, status.p, init_dist.p,
-                                                        opts.damping, partial.p, part_delta.p);
+      k_batch_tasks<<<task_grid, 256, 0, s>>>(g->col_ptr.p, g->row_idx.p, g->od.p, seedmask.p, tasks.p, ntasks, X0.p,
+                                              X1.p, P0.p, P1.p, ctl.p, status.p, init_dist.p, opts.damping, partial.p,
+                                              part_delta.p);
     }
     k_batch_fixup<<<fix_grid, 256, 0, s>>>(g->od.p, seedmask.p, longs.p, nlong, X0.p, X1.p, P0.p, P1.p, ctl.p, status.p,
                                            init_dist.p, opts.damping, partial.p,
@@ -749,6 +802,26 @@ void refresh_status(pe_ppr_batch_s* b) {
   b->host_status.resize(BK);
   PE_HIP(hipMemcpyAsync(b->host_status.data(), b->status.p, BK * 4, hipMemcpyDeviceToHost, s));
   PE_HIP(hipStreamSynchronize(s));
+}
+
+// Calls f(seeds, grid, block) with the list where the kernel can read it; waits only for a
+// list that had to be copied.
+template <class F>
+void with_seeds(pe_ctx_s* ctx, const std::vector<uint32_t>& ids, F f) {
+  seed_list l{};
+  l.n = (uint32_t)ids.size();
+  if (ids.size() <= SEEDS_INLINE) {
+    std::copy(ids.begin(), ids.end(), l.few);
+    f(l, 1u, (unsigned)BK);
+    PE_HIP(hipGetLastError());
+    return;
+  }
+  dbuf<uint32_t> d(ctx, ids.size());
+  PE_HIP(hipMemcpyAsync(d.p, ids.data(), ids.size() * 4, hipMemcpyHostToDevice, ctx->stream));
+  l.ids = d.p;
+  f(l, grid_for(ids.size(), 256, 64), 256u);
+  PE_HIP(hipGetLastError());
+  PE_HIP(hipStreamSynchronize(ctx->stream));
 }
 
 }  // namespace
@@ -792,6 +865,8 @@ int pe_ppr_batch_create(pe_graph_t* g, const pe_ppr_batch_opts_t* opts, pe_ppr_b
     b->last_delta.alloc(ctx, BK);
     batch_ctl c0{};
     c0.pk_n = 0xFFFFFFFFu;  // no packed pass yet
+    c0.mode = 4u;           // the plan of no covered column
+    std::fill(std::begin(c0.qof), std::end(c0.qof), (uint8_t)0xFF);
     auto limit = [](uint32_t v, uint32_t widest) {
       return v == 0 ? widest : v == PE_BATCH_PLAN_OFF ? 0u : std::min(v, widest);
     };
@@ -828,22 +903,18 @@ int pe_ppr_batch_admit(pe_ppr_batch_t* b, uint32_t slot, const uint32_t* seeds, 
   if (!b || !seeds || nseeds == 0) return PE_ERR_INVALID;
   return guarded(b->g->ctx, [&] {
     check_slot(b, slot);
-    refresh_status(b);
+    // only admissions and releases make a slot EMPTY or not, so the host's copy knows
     PE_REQUIRE(b->host_status[slot] == COL_EMPTY, PE_ERR_STATE, "slot is not free (release it first)");
     pe_graph_s* g = b->g;
     for (uint32_t i = 0; i < nseeds; ++i) PE_REQUIRE(seeds[i] < g->V, PE_ERR_RANGE, "seed vertex >= V");
-    std::vector<uint32_t> ids(nseeds);
-    to_internal_ids(g, seeds, nseeds, ids.data());
+    std::vector<uint32_t> ids(seeds, seeds + nseeds);
     std::sort(ids.begin(), ids.end());
     ids.erase(std::unique(ids.begin(), ids.end()), ids.end());
-    hipStream_t s = g->ctx->stream;
-    dbuf<uint32_t> d(g->ctx, ids.size());
-    PE_HIP(hipMemcpyAsync(d.p, ids.data(), ids.size() * 4, hipMemcpyHostToDevice, s));
-    k_batch_seed_bits<<<grid_for(ids.size(), 256, 64), 256, 0, s>>>(b->seedmask.p, d.p, (uint32_t)ids.size(), slot, 1);
-    k_batch_set_slot<<<1, 1, 0, s>>>(b->status.p, b->init_dist.p, b->iters.p, b->last_delta.p, slot, COL_LOADING,
-                                     1.0 / (double)ids.size());
-    PE_HIP(hipGetLastError());
-    PE_HIP(hipStreamSynchronize(s));
+    with_seeds(g->ctx, ids, [&](const seed_list& l, unsigned grid, unsigned block) {
+      k_batch_admit<<<grid, block, 0, g->ctx->stream>>>(l, g->relabeled ? g->rank_of.p : nullptr, b->seedmask.p,
+                                                        b->ctl.p, b->status.p, b->init_dist.p, b->iters.p,
+                                                        b->last_delta.p, slot, 1.0 / (double)l.n);
+    });
     b->slot_seeds[slot] = std::move(ids);
     b->host_status[slot] = COL_LOADING;
   });
@@ -853,20 +924,15 @@ int pe_ppr_batch_release(pe_ppr_batch_t* b, uint32_t slot) {
   if (!b) return PE_ERR_INVALID;
   return guarded(b->g->ctx, [&] {
     check_slot(b, slot);
-    hipStream_t s = b->g->ctx->stream;
+    pe_graph_s* g = b->g;
     auto& ids = b->slot_seeds[slot];
-    if (!ids.empty()) {
-      dbuf<uint32_t> d(b->g->ctx, ids.size());
-      PE_HIP(hipMemcpyAsync(d.p, ids.data(), ids.size() * 4, hipMemcpyHostToDevice, s));
-      k_batch_seed_bits<<<grid_for(ids.size(), 256, 64), 256, 0, s>>>(b->seedmask.p, d.p, (uint32_t)ids.size(), slot, 0);
-      k_batch_zero_slot<<<grid_for(ids.size(), 256, 64), 256, 0, s>>>(b->X0.p, b->X1.p, b->P0.p, b->P1.p,
-                                                                     b->g->col_ptr.p, b->seedmask.p, d.p,
-                                                                     (uint32_t)ids.size(), slot);
-      ids.clear();
-    }
-    k_batch_set_slot<<<1, 1, 0, s>>>(b->status.p, b->init_dist.p, b->iters.p, b->last_delta.p, slot, COL_EMPTY, 0.0);
-    PE_HIP(hipGetLastError());
-    PE_HIP(hipStreamSynchronize(s));
+    with_seeds(g->ctx, ids, [&](const seed_list& l, unsigned grid, unsigned block) {
+      k_batch_release<<<grid, block, 0, g->ctx->stream>>>(l, g->relabeled ? g->rank_of.p : nullptr, g->col_ptr.p,
+                                                          b->X0.p, b->X1.p, b->P0.p, b->P1.p, b->seedmask.p, b->ctl.p,
+                                                          b->status.p, b->init_dist.p, b->iters.p, b->last_delta.p,
+                                                          slot);
+    });
+    ids.clear();
     b->host_status[slot] = COL_EMPTY;
   });
 }

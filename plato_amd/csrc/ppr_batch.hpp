@@ -27,7 +27,7 @@ struct bt_long {
 struct batch_ctl {
   uint32_t cur;        // 0: state in X0, 1: in X1
   uint32_t iteration;  // passes run since creation
-  // the pass plan (k_batch_plan): the pass kernel to run (1, 2, 4: edges per row load
+  // the pass plan (batch_plan): the form of the pass to run (1, 2, 4: edges per row load
   // over the wide block; BATCH_MODE_PACKED: the packed block), and the columns it writes
   uint32_t mode;
   uint32_t ncols;

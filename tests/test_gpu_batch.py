@@ -241,3 +241,42 @@ def test_topk_selection(ctx, slots, k):
             assert np.array_equal(ids[i][: len(order)], order.astype(np.uint32))
         b.close()
         g.close()
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 700])
+def test_seed_list_lengths(s13, n):
+    """Lists that come with the launch (up to 64 distinct seeds) and longer ones that are copied,
+    given unsorted and with repeats; the slot is released and admitted again between passes."""
+    from plato_amd.batch import PprBatch
+    g, og = s13
+    rng = np.random.default_rng(n)
+    seeds = rng.choice(g.V, n, replace=False).astype(np.uint32)
+    b = PprBatch(g, D, tol=1e-7, max_iters=300)
+    runs = []
+    for _ in range(2):
+        b.admit(7, np.concatenate([seeds, seeds[::3]]))
+        b.run_until_done([7])
+        runs.append(b.results([7])[0])
+        b.release(7)
+        assert (b.poll()[0] == 0).all()
+    assert np.array_equal(runs[0], runs[1])
+    ref, _ = oracle.ppr(og, [int(v) for v in seeds], 2000, D, 0.0)
+    assert float(np.abs(runs[0] - ref).sum()) <= 1e-6
+
+
+@pytest.mark.parametrize("task_edges", [64, 128, 4096])
+def test_deltas_over_many_partials(s13, task_edges):
+    """A pass's deltas are the sums over its blocks' partials, few or several hundred of them.
+    The ranks are FP32, so the deltas of two task splits differ by their rounding (1e-7 each,
+    against 2e-3 for one lost block of 500)."""
+    from plato_amd.batch import PprBatch
+    g, og = s13
+    got = []
+    for te in (4096, task_edges):
+        b = PprBatch(g, D, tol=0.0, max_iters=6, task_edges=te)
+        for slot in (0, 31, 63):
+            b.admit(slot, [int(np.argmax(og.od)) + slot])
+        b.step(4)
+        got.append(b.poll()[2][[0, 31, 63]])
+    assert (got[0] > 0).all()
+    np.testing.assert_allclose(got[1], got[0], rtol=1e-5)
