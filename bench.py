@@ -101,7 +101,8 @@ def profiled_traffic(kernel, scale):
 
 def measure_pull(ctx, g, layout, steps, warmup, weighted=False):
     """Time `steps` FP32 PageRank iterations on one pull layout: per-kernel HIP events on the
-    library stream (timed run), then the same iterations replayed from a captured graph."""
+    library stream (timed run), then the same iterations without them (graph_ms, a name from when
+    those iterations were replayed from a captured graph; they are plain launches)."""
     from plato_amd import _lib as L
     from plato_amd.algo import pagerank as plain, pagerank_opts_t, weighted_pagerank
     pagerank = weighted_pagerank if weighted else plain
@@ -133,7 +134,7 @@ def measure_pull(ctx, g, layout, steps, warmup, weighted=False):
                           "layout_build_s": round(layout_s, 2), "run_records": int(info.binned_runs),
                           "layout_bytes": int(info.binned_bytes)})
     log(f"[bench] {'weighted ' if weighted else ''}{layout}: {out['ms_per_step']:.3f} ms/iteration (timed), {out['graph_ms']:.3f} ms "
-        f"(graph replay), kernel {out['kernel_ms']:.3f} ms")
+        f"(without events), kernel {out['kernel_ms']:.3f} ms")
     return out
 
 

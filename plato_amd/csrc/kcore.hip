@@ -21,7 +21,7 @@
 // where a vertex is newly modified and once where it was in the epoch before; the active set
 // is still marked and counted, for the per-epoch log.  In epoch 0 everything is active; a vertex
 // that keeps its adjacency length has cnt(v) equal to it.
-// RMAT scale 22 symmetrized, degree-relabeled, 39 epochs, whole call: 51 ms re-counting every
+// RMAT scale 22 symmetrized, degree-relabeled, 38 epochs, whole call: 51 ms re-counting every
 // active vertex, 20 ms with the counts, 16.1 ms with the drops found in the spread before.  Bound by
 // the random 4-byte reads of the values in the first ten epochs, when most vertices are modified
 // (0.5 ms per scan of the 2^27 entries).

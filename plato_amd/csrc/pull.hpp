@@ -21,9 +21,8 @@ struct rank_args {
                           // fixed-point scale
 };
 
-// Device-resident loop controller: lets iterations be enqueued (or replayed
-// from a captured graph) without host round-trips.  Kernels return at once
-// when done is set; the finish kernel advances t and flips cur.
+// Device-resident loop controller: lets iterations be enqueued without host round-trips.
+// Kernels return at once when done is set; the finish advances t and flips cur.
 struct iter_ctl {
   uint32_t iters;       // pagerank_opts_t::iteration_
   uint32_t t;           // the reference's epoch_i
