@@ -22,8 +22,8 @@
 // is still marked and counted, for the per-epoch log.  In epoch 0 everything is active; a vertex
 // that keeps its adjacency length has cnt(v) equal to it.
 // RMAT scale 22 symmetrized, degree-relabeled, 38 epochs, whole call: 51 ms re-counting every
-// active vertex, 20 ms with the counts, 16.1 ms with the drops found in the spread before.  Bound by
-// the random 4-byte reads of the values in the first ten epochs, when most vertices are modified
+// active vertex, 20 ms with the counts, 16.1 ms with the drops found in the spread before, 15.6 ms with
+// the marks in the values.  Bound by the random 4-byte reads of the values in the first ten epochs, when most vertices are modified
 // (0.5 ms per scan of the 2^27 entries).
 // Other adjacencies (in-edges or out-edges of a directed graph) have no counts: every
 // active vertex is re-counted.
@@ -519,20 +519,30 @@ __global__ __launch_bounds__(KC_HTHREADS) void k_kc_giant_pick(
 // The modified vertices (core below est) activate their neighbours; with counts (cnt_v) each
 // also takes itself out of the counts of the unmodified neighbours it fell below, marking those
 // that the last one leaves short as candidates, and returns how many neighbours it keeps at or
-// above its own new value.  act_bytes: the next active set, one byte per
-// vertex: a mark is a plain store of 1 that any number of waves may repeat, where an atomic OR
-// on a shared bitmap word is serialized in the memory-side atomic unit (RMAT scale 22, all epochs: 35 ms of
-// spreading with bits, 10 ms with bytes).
+// above its own new value.  The next active set is marked with plain stores that any number of
+// waves may repeat, where an atomic OR on a shared bitmap word is serialized in the memory-side
+// atomic unit (RMAT scale 22, all epochs: 35 ms of spreading with bits, 10 ms with bytes).  The
+// mark is the top bit of the neighbour's coreness, which stands still meanwhile, so a
+// neighbour costs one random read, where values of 31 bits suffice (act_bytes is nullptr then:
+// with counts, and below 2^31 entries, so no length needs the bit; the lane and wave spreads 5.4 -> 4.2 ms, the
+// blocks' 4.5 -> 4.8); else one byte per vertex.
+static constexpr uint32_t KC_MARK = 0x80000000u;
 struct kc_spread {
   const uint32_t* idx;
   const uint32_t* est;
-  const uint32_t* core;
+  uint32_t* core;
   uint32_t* cnt_v;
   uint8_t* act_bytes;
   uint64_t* cand;
-  __device__ __forceinline__ uint32_t one(uint32_t u, uint32_t cu, uint32_t old, uint32_t now) const {
-    if (!act_bytes[u]) act_bytes[u] = 1;
+  __device__ __forceinline__ uint32_t value(uint32_t raw) const { return act_bytes ? raw : raw & ~KC_MARK; }
+  __device__ __forceinline__ uint32_t one(uint32_t u, uint32_t raw, uint32_t old, uint32_t now) const {
+    if (act_bytes) {
+      if (!act_bytes[u]) act_bytes[u] = 1;
+    } else if (!(raw & KC_MARK)) {
+      core[u] = raw | KC_MARK;
+    }
     if (!cnt_v) return 0u;
+    const uint32_t cu = value(raw);
     if (cu > now && cu <= old && est[u] == cu && atomicSub(&cnt_v[u], 1u) == cu) kc_set_bit(cand, u);
     return cu >= now ? 1u : 0u;
   }
@@ -569,7 +579,8 @@ struct kc_spread {
       for (int i = 0; i < KC_U; ++i)
         if (k0 + (uint64_t)i * step + i0 < e) {
           (void)one(u[i], cu[i], old, now);
-          atomicAdd(&hist[cu[i] < now ? cu[i] : now], 1u);
+          const uint32_t x = value(cu[i]);
+          atomicAdd(&hist[x < now ? x : now], 1u);
         }
     }
   }
@@ -586,7 +597,8 @@ struct kc_spread {
       for (int i = 0; i < KC_U; ++i)
         if (k0 + i < e) {
           (void)one(u[i], cu[i], old, now);
-          ++h[cu[i] < now ? cu[i] : now];
+          const uint32_t x = value(cu[i]);
+          ++h[x < now ? x : now];
         }
     }
   }
@@ -608,7 +620,7 @@ __global__ __launch_bounds__(KC_THREADS) void k_kc_spread(
   const uint64_t wave_id = grid_wave_id(), nwaves = grid_waves();
   for (uint64_t q = wave_id; q < nbig; q += nwaves) {
     const uint32_t v = qbig[q];
-    const uint32_t old = sp.est[v], now = sp.core[v];
+    const uint32_t old = sp.est[v], now = sp.value(sp.core[v]);
     if (old == now) continue;  // uniform
     if (!sp.cnt_v) {
       (void)sp.range(ptr[v], ptr[v + 1], (uint32_t)lane, 64u, old, now);
@@ -630,7 +642,7 @@ __global__ __launch_bounds__(KC_THREADS) void k_kc_spread(
   for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < nsmall;
        i += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t v = qsmall[i];
-    const uint32_t old = sp.est[v], now = sp.core[v];
+    const uint32_t old = sp.est[v], now = sp.value(sp.core[v]);
     if (old == now) continue;
     if (!sp.cnt_v || old == KC_UNSET) {
       (void)sp.range(ptr[v], ptr[v + 1], 0u, 1u, old, now);
@@ -657,7 +669,7 @@ __global__ __launch_bounds__(KC_HTHREADS) void k_kc_spread_huge(const uint32_t* 
   const uint64_t nhuge = cnt_in->nhuge;
   for (uint64_t q = blockIdx.x; q < nhuge; q += gridDim.x) {
     const uint32_t v = *(qhuge_end - q);
-    const uint32_t old = sp.est[v], now = sp.core[v];
+    const uint32_t old = sp.est[v], now = sp.value(sp.core[v]);
     if (old == now) continue;  // uniform
     if (!sp.cnt_v) {
       (void)sp.range(ptr[v], ptr[v + 1], tid, KC_HTHREADS, old, now);
@@ -700,7 +712,7 @@ __global__ __launch_bounds__(KC_HTHREADS) void k_kc_spread_giant(const uint64_t*
     uint64_t k0, k1;
     const uint32_t v = hub_chunk(ptr, giants, start, n, KC_GCHUNK, c, &k0, &k1);
     if (!((act[v >> 6] >> (v & 63)) & 1ull)) continue;  // uniform
-    const uint32_t old = sp.est[v], now = sp.core[v];
+    const uint32_t old = sp.est[v], now = sp.value(sp.core[v]);
     if (old == now) continue;
     uint32_t k = sp.range(k0, k1, threadIdx.x, KC_HTHREADS, old, now);
     if (sp.cnt_v) {
@@ -716,7 +728,7 @@ __global__ __launch_bounds__(KC_HTHREADS) void k_kc_spread_giant(const uint64_t*
 __global__ __launch_bounds__(KC_THREADS) void k_kc_commit(
     const uint32_t* __restrict__ qsmall, const uint32_t* __restrict__ qbig, const uint32_t* __restrict__ qhuge_end,
     const uint32_t* __restrict__ giants, const unsigned long long* __restrict__ ngiant,
-    const uint64_t* __restrict__ act, const uint32_t* __restrict__ core, uint32_t* __restrict__ est,
+    const uint64_t* __restrict__ act, const uint32_t* __restrict__ core, uint32_t mark, uint32_t* __restrict__ est,
     const uint32_t* __restrict__ cnt_v, uint64_t* __restrict__ cand, kc_counters* __restrict__ cnt) {
   const uint64_t ns = cnt->nsmall, nb = cnt->nbig, nh = cnt->nhuge, ng = giants ? *ngiant : 0ull;
   unsigned long long nmod = 0;
@@ -733,7 +745,7 @@ __global__ __launch_bounds__(KC_THREADS) void k_kc_commit(
       v = giants[i - ns - nb - nh];
       if (!((act[v >> 6] >> (v & 63)) & 1ull)) continue;
     }
-    const uint32_t c = core[v], old = est[v];
+    const uint32_t c = core[v] & ~mark, old = est[v];
     if (c == old) continue;
     est[v] = c;
     nmod += old != KC_UNSET ? 1u : 0u;
@@ -769,6 +781,29 @@ __global__ __launch_bounds__(256) void k_kc_next(uint64_t* __restrict__ act_byte
   block_add2(a, c, &cnt->next_active, &cnt->next_cand);
 }
 
+// the same where the marks are top bits of the values
+__global__ __launch_bounds__(1024) void k_kc_next_marked(uint32_t* __restrict__ core, uint64_t V,
+                                                         const uint64_t* __restrict__ cand, uint64_t nwords,
+                                                         kc_counters* __restrict__ cnt) {
+  const uint64_t i0 = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x, step = (uint64_t)gridDim.x * blockDim.x;
+  unsigned long long a = 0, c = 0;
+  uint4* quads = reinterpret_cast<uint4*>(core);
+  for (uint64_t i = i0; i < V / 4; i += step) {
+    const uint4 x = quads[i];
+    const uint32_t n = (x.x >> 31) + (x.y >> 31) + (x.z >> 31) + (x.w >> 31);
+    if (n) quads[i] = make_uint4(x.x & ~KC_MARK, x.y & ~KC_MARK, x.z & ~KC_MARK, x.w & ~KC_MARK);
+    a += n;
+  }
+  if (i0 < V % 4) {
+    const uint64_t v = V - V % 4 + i0;
+    const uint32_t x = core[v];
+    a += x >> 31;
+    core[v] = x & ~KC_MARK;
+  }
+  for (uint64_t i = i0; i < nwords; i += step) c += (unsigned long long)__popcll(cand[i]);
+  block_add2(a, c, &cnt->next_active, &cnt->next_cand);
+}
+
 }  // namespace pe
 
 using namespace pe;
@@ -787,7 +822,9 @@ extern "C" int pe_kcore(pe_graph_t* g, int out_edges, uint32_t* coreness, uint64
     const uint64_t nwords = ((uint64_t)V >> 6) + 1;
     const uint32_t Vs = std::max<uint32_t>(1, V);
     dbuf<uint32_t> core(ctx, Vs), est(ctx, Vs), qsmall(ctx, Vs), qbig(ctx, Vs), cnt_v, ahead;
-    dbuf<uint64_t> cand(ctx, nwords), act, nxt(ctx, nwords * 8);  // nxt: one byte per vertex
+    const bool marked = counts && g->nnz < (1ull << 31);  // active marks in the values' top bits
+    dbuf<uint64_t> cand(ctx, nwords), act, nxt;             // nxt: else, one byte per vertex
+    if (!marked) nxt.alloc(ctx, nwords * 8);
     if (counts) {
       cnt_v.alloc(ctx, Vs);
       ahead.alloc(ctx, Vs);
@@ -797,7 +834,7 @@ extern "C" int pe_kcore(pe_graph_t* g, int out_edges, uint32_t* coreness, uint64
     PE_HIP(hipEventRecord(ctx->t0, s));
     k_kc_init<<<grid_for(V, 256, 8192), 256, 0, s>>>(ptr, V, core.p, est.p, cnt_v.p, ahead.p);
     k_kc_fill<<<grid_for(nwords, 256, 4096), 256, 0, s>>>(cand.p, nwords, V);  // active_current.fill()
-    k_kc_zero<<<grid_for(nwords * 8, 256, 4096), 256, 0, s>>>(nxt.p, nwords * 8);
+    if (!marked) k_kc_zero<<<grid_for(nwords * 8, 256, 4096), 256, 0, s>>>(nxt.p, nwords * 8);
     PE_HIP(hipGetLastError());
     // giants and their histograms (one per giant, KC_HHIST + 1 bins)
     hub_table giants;
@@ -845,8 +882,10 @@ extern "C" int pe_kcore(pe_graph_t* g, int out_edges, uint32_t* coreness, uint64
         k_kc_spread_huge<<<hgrid, KC_HTHREADS, 0, s>>>(qhuge_end, c, ptr, sp, ahead.p);
         k_kc_spread<<<grid, KC_THREADS, 0, s>>>(qsmall.p, qbig.p, c, ptr, sp, ahead.p);
         k_kc_commit<<<grid_for(ncand, KC_THREADS, full_grid), KC_THREADS, 0, s>>>(
-            qsmall.p, qbig.p, qhuge_end, gl, giants.count.p, act.p, core.p, est.p, cnt_v.p, cand.p, c);
-        k_kc_next<<<grid_for(nwords * 8, 256, (unsigned)std::max(1, ctx->num_cus) * 2), 256, 0, s>>>(nxt.p, cand.p, nwords, counts ? 0 : 1, c);
+            qsmall.p, qbig.p, qhuge_end, gl, giants.count.p, act.p, core.p, marked ? KC_MARK : 0u, est.p, cnt_v.p, cand.p, c);
+        const unsigned next_max = (unsigned)std::max(1, ctx->num_cus) * 2;
+        if (marked) k_kc_next_marked<<<grid_for(V, 4096, next_max), 1024, 0, s>>>(core.p, V, cand.p, nwords, c);
+        else k_kc_next<<<grid_for(nwords * 8, 256, next_max), 256, 0, s>>>(nxt.p, cand.p, nwords, counts ? 0 : 1, c);
         PE_HIP(hipGetLastError());
         const kc_counters* h = reinterpret_cast<const kc_counters*>(
             mail_post(ctx, reinterpret_cast<const unsigned long long*>(c), KC_CW,
