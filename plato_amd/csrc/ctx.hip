@@ -4,77 +4,45 @@
 
 namespace pe {
 
+// hipFree waits for the work that may still use a block
 void pool_trim(pe_ctx_s* ctx) {
-  block_pool& b = ctx->pool;
-  for (auto& k : b.kept) {
-    b.size_of.erase(k.second.p);
-    (void)hipFree(k.second.p);  // waits for the work that may still use it
-  }
-  b.kept.clear();
-  b.kept_bytes = 0;
+  while (void* p = ctx->pool.oldest_over(0)) (void)hipFree(p);
 }
 
 void* dmalloc(pe_ctx_s* ctx, size_t bytes) {
   block_pool& b = ctx->pool;
-  const size_t want = (std::max<size_t>(bytes, 1) + 511) & ~(size_t)511;
-  void* p = nullptr;
-  auto it = b.kept.lower_bound(want);
-  if (it != b.kept.end() && it->first <= want + want / 4) {
-    p = it->second.p;
-    b.kept_bytes -= it->first;
-    b.kept.erase(it);
-    ctx->allocated += bytes;
-    if (ctx->allocated > ctx->peak_allocated) ctx->peak_allocated = ctx->allocated;
-    return p;
+  const size_t want = block_pool::block_size(bytes);
+  void* p = b.take(want);
+  if (!p) {
+    hipError_t e = hipMalloc(&p, want);
+    if (e != hipSuccess && b.kept_bytes()) {
+      (void)hipGetLastError();
+      pool_trim(ctx);
+      e = hipMalloc(&p, want);
+    }
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      char buf[160];
+      std::snprintf(buf, sizeof(buf), "hipMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(e));
+      fail(PE_ERR_OOM, buf);
+    }
+    try {
+      b.add(p, want);
+    } catch (...) {
+      (void)hipFree(p);
+      throw;
+    }
   }
-  hipError_t e = hipMalloc(&p, want);
-  if (e != hipSuccess && !b.kept.empty()) {
-    (void)hipGetLastError();
-    pool_trim(ctx);
-    e = hipMalloc(&p, want);
-  }
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    char buf[160];
-    std::snprintf(buf, sizeof(buf), "hipMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(e));
-    fail(PE_ERR_OOM, buf);
-  }
-  try {
-    b.size_of.emplace(p, want);
-  } catch (...) {
-    (void)hipFree(p);
-    throw;
-  }
-  ctx->allocated += bytes;
-  if (ctx->allocated > ctx->peak_allocated) ctx->peak_allocated = ctx->allocated;
+  b.charge(bytes);
   return p;
 }
 
 void dfree(pe_ctx_s* ctx, void* p, size_t bytes) {
   if (!p) return;
-  ctx->allocated -= bytes;
   block_pool& b = ctx->pool;
-  auto it = b.size_of.find(p);
-  if (it == b.size_of.end()) return;
-  const size_t size = it->second;
-  if (size <= block_pool::BLOCK_BYTES) {
-    try {
-      b.kept.emplace(size, block_pool::entry{p, ++b.clock});
-      b.kept_bytes += size;
-      while (b.kept_bytes > block_pool::POOL_BYTES) {
-        auto old = std::min_element(b.kept.begin(), b.kept.end(),
-                                    [](const auto& x, const auto& y) { return x.second.age < y.second.age; });
-        b.size_of.erase(old->second.p);
-        b.kept_bytes -= old->first;
-        (void)hipFree(old->second.p);
-        b.kept.erase(old);
-      }
-      return;
-    } catch (...) {  // no host memory for the entry: give the block back
-    }
-  }
-  b.size_of.erase(it);
-  (void)hipFree(p);
+  b.credit(bytes);
+  if (b.give(p)) (void)hipFree(p);
+  while (void* old = b.oldest_over(block_pool::POOL_BYTES)) (void)hipFree(old);
 }
 
 ktime_scope::ktime_scope(pe_ctx_s* c, int w) : ctx(c), which(w) {
@@ -373,9 +341,9 @@ int pe_ctx_mem_info(pe_ctx_t* ctx, uint64_t* free_bytes, uint64_t* total_bytes,
     size_t f = 0, t = 0;
     PE_HIP(hipSetDevice(ctx->device));
     PE_HIP(hipMemGetInfo(&f, &t));
-    if (free_bytes) *free_bytes = f + ctx->pool.kept_bytes;  // kept blocks go back when memory runs short
+    if (free_bytes) *free_bytes = f + ctx->pool.kept_bytes();  // kept blocks go back when memory runs short
     if (total_bytes) *total_bytes = t;
-    if (ctx_bytes) *ctx_bytes = ctx->allocated;
+    if (ctx_bytes) *ctx_bytes = ctx->pool.used_bytes();
   });
 }
 

@@ -9,13 +9,12 @@
 #include <cstdio>
 #include <cstring>
 #include <functional>
-#include <map>
 #include <memory>
 #include <stdexcept>
 #include <string>
-#include <unordered_map>
 #include <vector>
 
+#include "block_pool.hpp"
 #include "plato_hip.h"
 
 namespace pe {
@@ -51,32 +50,12 @@ struct kernel_timer {
 
 struct staging;
 
-// Device blocks that a context keeps after they are freed, for its next allocations of about
-// the same size: an algorithm's scratch is allocated and freed by every call, and a hipFree
-// waits for the device (BFS scale 24, 14 blocks of 0.5 GB in all: 5.2 ms a call without, 2.7 ms
-// with; nine engine calls at scale 12: 0.56 and 0.32 ms).  Bounded by POOL_BYTES, the blocks
-// kept longest leaving first; given back when an allocation fails and when the context goes.
-// All work of a context is on one stream, so a block's next user runs after its last one.
-struct block_pool {
-  static constexpr size_t POOL_BYTES = 1ull << 30, BLOCK_BYTES = 512ull << 20;
-  struct entry {
-    void* p;
-    uint64_t age;
-  };
-  std::multimap<size_t, entry> kept;          // free blocks by size
-  uint64_t clock = 0;
-  std::unordered_map<void*, size_t> size_of;  // every block of the context
-  size_t kept_bytes = 0;
-};
-
 }  // namespace pe
 
 struct pe_ctx_s {
   int device = 0;
   hipStream_t stream = nullptr;
   std::string last_error;
-  uint64_t allocated = 0;       // bytes currently held by this context
-  uint64_t peak_allocated = 0;
   hipEvent_t t0 = nullptr, t1 = nullptr;
   int timing = 0;               // per-kernel event timing on/off
   pe::kernel_timer timers[PE_KT_COUNT];
@@ -89,7 +68,7 @@ struct pe_ctx_s {
   unsigned long long mail_seq = 0;
   // this device's static scratch array of pe_pull_sum_noalloc (its device address)
   void* noalloc_scratch = nullptr;
-  pe::block_pool pool;
+  pe::block_pool pool;          // its device blocks, in use and kept
   pe::staging* stage = nullptr;  // pinned ring of large transfers (transfer.hip), made by the first
 };
 
