@@ -24,14 +24,16 @@ class block_pool {
  public:
   static constexpr size_t POOL_BYTES = 1ull << 30, BLOCK_BYTES = 512ull << 20;
 
-  // the size of the block that serves a request of `bytes`
-  static size_t block_size(size_t bytes) { return (std::max<size_t>(bytes, 1) + 511) & ~(size_t)511; }
+  // the size of the block that serves a request of `bytes`: whole units of 512, as far as size_t goes
+  static size_t block_size(size_t bytes) {
+    return bytes > SIZE_MAX - 511 ? bytes : (std::max<size_t>(bytes, 1) + 511) & ~(size_t)511;
+  }
 
   // a kept block of `want` to a quarter more bytes, or nullptr
   void* take(size_t want) {
     std::lock_guard<std::mutex> lock(mu);
     auto it = kept.lower_bound(want);
-    if (it == kept.end() || it->first > want + want / 4) return nullptr;
+    if (it == kept.end() || it->first - want > want / 4) return nullptr;
     void* p = it->second.p;
     kept_total -= it->first;
     kept.erase(it);

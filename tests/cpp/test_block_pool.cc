@@ -18,7 +18,29 @@ static void release(void* p) {
   --live;
 }
 
+// a request near the largest size_t keeps its size (a multiple of 512 would wrap to nothing) and
+// is served by no smaller block that is kept
+static int wrong_sizes() {
+  int bad = 0;
+  for (size_t bytes : {(size_t)0, (size_t)1, (size_t)511, (size_t)512, (size_t)513, (size_t)1 << 40})
+    bad += pe::block_pool::block_size(bytes) % 512 != 0 || pe::block_pool::block_size(bytes) < std::max<size_t>(bytes, 1);
+  pe::block_pool p;
+  void* small = &bad;
+  p.add(small, 512);
+  bad += p.give(small);
+  for (size_t off : {0, 7, 510, 511, 512, 1000}) {
+    const size_t bytes = SIZE_MAX - off;
+    bad += pe::block_pool::block_size(bytes) < bytes;
+    bad += p.take(pe::block_pool::block_size(bytes)) != nullptr;
+  }
+  return bad;
+}
+
 int main() {
+  if (int n = wrong_sizes()) {
+    std::printf("wrong sizes: %d\n", n);
+    return 1;
+  }
   constexpr int THREADS = 4, ROUNDS = 20000;
   std::atomic<int> bad{0};
   auto work = [&](unsigned id) {
