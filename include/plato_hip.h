@@ -66,9 +66,15 @@ int pe_ctx_create(int device, pe_ctx_t** out);
 int pe_ctx_destroy(pe_ctx_t* ctx);
 const char* pe_ctx_last_error(const pe_ctx_t* ctx);
 int pe_ctx_sync(pe_ctx_t* ctx);
-/* free/total device memory and the bytes this context holds */
+/* free/total device memory and the bytes this context's objects hold.  Device blocks that
+ * are freed stay with the context, up to 1 GiB, for its next allocations; they count as
+ * free here (another context's do not).  They are given back when an allocation of any
+ * context of the process on that device fails (which then tries again), by pe_ctx_trim,
+ * and with the context; other allocators on the device do not see them as free. */
 int pe_ctx_mem_info(pe_ctx_t* ctx, uint64_t* free_bytes, uint64_t* total_bytes,
                     uint64_t* ctx_bytes);
+/* Gives the freed blocks that the context keeps back to the device (waits for its work). */
+int pe_ctx_trim(pe_ctx_t* ctx);
 /* event timer on the context stream (stop synchronizes) */
 int pe_ctx_timer_start(pe_ctx_t* ctx);
 int pe_ctx_timer_stop(pe_ctx_t* ctx, double* ms);

@@ -126,6 +126,7 @@ SIGNATURES = {
     "pe_ctx_last_error": [_vp],
     "pe_ctx_sync": [_vp],
     "pe_ctx_mem_info": [_vp, _P(_u64), _P(_u64), _P(_u64)],
+    "pe_ctx_trim": [_vp],
     "pe_ctx_timer_start": [_vp],
     "pe_ctx_timer_stop": [_vp, _P(_dbl)],
     "pe_ctx_set_kernel_timing": [_vp, _i32],

@@ -16,7 +16,8 @@ namespace pe {
 // the same size: an algorithm's scratch is allocated and freed by every call, and a hipFree
 // waits for the device (BFS scale 24, 14 blocks of 0.5 GB in all: 5.2 ms a call without, 2.7 ms
 // with; nine engine calls at scale 12: 0.56 and 0.32 ms).  Bounded by POOL_BYTES, the blocks
-// kept longest leaving first; given back when an allocation fails and when the context goes.
+// kept longest leaving first; given back when an allocation of any context on the device fails,
+// when the caller asks for it, and when the context goes.
 // All work of a context is on one stream, so a block's next user runs after its last one.
 // Every member may be called from several threads: a context's calls come from one at a time,
 // but its objects may be destroyed by another meanwhile (a garbage collector's).

@@ -9,16 +9,49 @@ void pool_trim(pe_ctx_s* ctx) {
   while (void* p = ctx->pool.oldest_over(0)) (void)hipFree(p);
 }
 
+// The contexts of the process, for trim_device.
+struct ctx_list {
+  std::mutex mu;
+  std::vector<pe_ctx_s*> all;
+};
+static ctx_list& contexts() {
+  static ctx_list* l = new ctx_list;  // never destroyed: contexts may outlive static objects
+  return *l;
+}
+
+static void list_ctx(pe_ctx_s* ctx) {
+  std::lock_guard<std::mutex> lock(contexts().mu);
+  contexts().all.push_back(ctx);
+}
+
+static void unlist_ctx(pe_ctx_s* ctx) {
+  ctx_list& l = contexts();
+  std::lock_guard<std::mutex> lock(l.mu);
+  l.all.erase(std::remove(l.all.begin(), l.all.end(), ctx), l.all.end());
+}
+
+// Gives the kept blocks of every context on the device back; whether there were any.
+static bool trim_device(int device) {
+  ctx_list& l = contexts();
+  std::lock_guard<std::mutex> lock(l.mu);
+  bool any = false;
+  for (pe_ctx_s* c : l.all)
+    if (c->device == device && c->pool.kept_bytes()) {
+      pool_trim(c);
+      any = true;
+    }
+  return any;
+}
+
 void* dmalloc(pe_ctx_s* ctx, size_t bytes) {
   block_pool& b = ctx->pool;
   const size_t want = block_pool::block_size(bytes);
   void* p = b.take(want);
   if (!p) {
     hipError_t e = hipMalloc(&p, want);
-    if (e != hipSuccess && b.kept_bytes()) {
+    if (e != hipSuccess) {
       (void)hipGetLastError();
-      pool_trim(ctx);
-      e = hipMalloc(&p, want);
+      if (trim_device(ctx->device)) e = hipMalloc(&p, want);
     }
     if (e != hipSuccess) {
       (void)hipGetLastError();
@@ -295,6 +328,7 @@ int pe_ctx_create(int device, pe_ctx_t** out) {
     PE_HIP(hipHostMalloc(reinterpret_cast<void**>(&ctx->host_mail), 4096 + MAIL_WORDS * 4, hipHostMallocCoherent));
     ctx->host_mail[0] = 0ull;
     ctx->noalloc_scratch = pull_scratch_setup(device);  // with the device current
+    list_ctx(ctx);
   });
   if (rc != PE_OK) {
     std::fprintf(stderr, "pe_ctx_create: %s\n", ctx->last_error.c_str());
@@ -308,6 +342,7 @@ int pe_ctx_create(int device, pe_ctx_t** out) {
 
 int pe_ctx_destroy(pe_ctx_t* ctx) {
   if (!ctx) return PE_ERR_INVALID;
+  unlist_ctx(ctx);
   (void)hipSetDevice(ctx->device);
   (void)hipStreamSynchronize(ctx->stream);
   for (auto& t : ctx->timers) {
@@ -345,6 +380,11 @@ int pe_ctx_mem_info(pe_ctx_t* ctx, uint64_t* free_bytes, uint64_t* total_bytes,
     if (total_bytes) *total_bytes = t;
     if (ctx_bytes) *ctx_bytes = ctx->pool.used_bytes();
   });
+}
+
+int pe_ctx_trim(pe_ctx_t* ctx) {
+  if (!ctx) return PE_ERR_INVALID;
+  return guarded(ctx, [&] { pool_trim(ctx); });
 }
 
 int pe_ctx_timer_start(pe_ctx_t* ctx) {

@@ -64,6 +64,10 @@ class Context:
         check(self.lib.pe_ctx_mem_info(self.h, C.byref(f), C.byref(t), C.byref(c)), self.h)
         return dict(free=f.value, total=t.value, ctx=c.value)
 
+    def trim(self):
+        """Give the device blocks that the context keeps for reuse (at most 1 GiB) back."""
+        check(self.lib.pe_ctx_trim(self.h), self.h)
+
     def num_cus(self):
         n = C.c_int()
         check(self.lib.pe_ctx_num_cus(self.h, C.byref(n)), self.h)

@@ -65,3 +65,27 @@ def test_kept_blocks_are_bounded_and_given_back():
         v.close()
         c.close()
         assert free0 - meter.mem_info()["free"] < 256 << 20
+
+
+@pytest.mark.parametrize("how", ["allocation", "trim"])
+def test_kept_blocks_of_another_context(how):
+    """Blocks that one context keeps are given back when an allocation of another fails, and by
+    a trim."""
+    from plato_amd import Context, DenseState
+    from plato_amd._lib import PlatoHipError
+    with Context(0) as a, Context(0) as b:
+        free0 = b.mem_info()["free"]  # b has no blocks: the device's free memory
+        for i in range(2):
+            DenseState(a, (96 + 4 * i) << 20, np.float32).close()
+        free = b.mem_info()["free"]
+        assert free0 - free > 600 << 20, free0 - free  # a keeps both, 0.77 GiB
+        if how == "allocation":
+            held = [DenseState(b, (free - (2 << 30)) // 4, np.float32)]
+            with pytest.raises(PlatoHipError, match="out of memory"):
+                for _ in range(16):  # 0.6 GiB each, more than a pool keeps
+                    held.append(DenseState(b, 150 << 20, np.float32))
+            for v in held:
+                v.close()
+        else:
+            a.trim()
+        assert free0 - b.mem_info()["free"] < 256 << 20
