@@ -386,6 +386,12 @@ typedef struct {
  * the size of the next active set (the reference's modified / need_modified log). */
 int pe_kcore(pe_graph_t* g, int out_edges, uint32_t* coreness, uint64_t* epoch_modified,
              uint64_t* epoch_next, uint32_t cap, pe_kcore_stats_t* stats);
+/* pe_kcore with a lower bound on the adjacency entries from which on a symmetrized graph's
+ * active marks take a byte per vertex (2^31 in pe_kcore, and at most; below, they sit in the
+ * top bits of the values).  The results are the same: it lets the form that only the
+ * largest graphs take run on any graph. */
+int pe_kcore_byte_marks(pe_graph_t* g, int out_edges, uint64_t byte_marks_from, uint32_t* coreness,
+                        uint64_t* epoch_modified, uint64_t* epoch_next, uint32_t cap, pe_kcore_stats_t* stats);
 
 /* ---- connected components -------------------------------------------------- */
 

@@ -140,6 +140,7 @@ SIGNATURES = {
     "pe_trustrank_select": [_vp, _vp, _vp, _vp, _vp, _vp],
     "pe_trustrank": [_vp, _vp, _vp, _vp, _vp, _vp, _vp],
     "pe_kcore": [_vp, C.c_int, _vp, _vp, _vp, _u32, _vp],
+    "pe_kcore_byte_marks": [_vp, C.c_int, _u64, _vp, _vp, _vp, _u32, _vp],
     "pe_connected_components": [_vp, _vp, _vp, _vp, _u32, _vp],
     "pe_nstep_degrees": [_vp, _vp, _u32, _u32, _i32, _vp, _vp, _P(_dbl)],
     "pe_hyperanf": [_vp, _vp, _vp, _u32, _vp, _vp, _vp, _vp],

@@ -809,8 +809,12 @@ __global__ __launch_bounds__(1024) void k_kc_next_marked(uint32_t* __restrict__ 
 
 using namespace pe;
 
-extern "C" int pe_kcore(pe_graph_t* g, int out_edges, uint32_t* coreness, uint64_t* epoch_modified,
-                        uint64_t* epoch_next, uint32_t cap, pe_kcore_stats_t* stats) {
+// byte_marks_from: adjacency entries from which on the active marks are bytes (see kc_spread);
+// the values have 31 bits below 2^31 entries
+static constexpr uint64_t KC_MARKED_BELOW = 1ull << 31;
+
+static int kcore_run(pe_graph_t* g, int out_edges, uint64_t byte_marks_from, uint32_t* coreness,
+                     uint64_t* epoch_modified, uint64_t* epoch_next, uint32_t cap, pe_kcore_stats_t* stats) {
   if (!g || !coreness) return PE_ERR_INVALID;
   return guarded(g->ctx, [&] {
     PE_REQUIRE(!out_edges || g->has_csr, PE_ERR_STATE, "out-edge k-core needs PE_GRAPH_BUILD_CSR");
@@ -823,7 +827,8 @@ extern "C" int pe_kcore(pe_graph_t* g, int out_edges, uint32_t* coreness, uint64
     const uint64_t nwords = ((uint64_t)V >> 6) + 1;
     const uint32_t Vs = std::max<uint32_t>(1, V);
     dbuf<uint32_t> core(ctx, Vs), est(ctx, Vs), qsmall(ctx, Vs), qbig(ctx, Vs), cnt_v, ahead;
-    const bool marked = counts && g->nnz < (1ull << 31);  // active marks in the values' top bits
+    // active marks in the values' top bits
+    const bool marked = counts && g->nnz < std::min(byte_marks_from, KC_MARKED_BELOW);
     dbuf<uint64_t> cand(ctx, nwords), act, nxt;             // nxt: else, one byte per vertex
     if (!marked) nxt.alloc(ctx, nwords * 8);
     if (counts) {
@@ -915,4 +920,15 @@ extern "C" int pe_kcore(pe_graph_t* g, int out_edges, uint32_t* coreness, uint64
       stats->seconds = ms * 1e-3;
     }
   });
+}
+
+extern "C" int pe_kcore(pe_graph_t* g, int out_edges, uint32_t* coreness, uint64_t* epoch_modified,
+                        uint64_t* epoch_next, uint32_t cap, pe_kcore_stats_t* stats) {
+  return kcore_run(g, out_edges, KC_MARKED_BELOW, coreness, epoch_modified, epoch_next, cap, stats);
+}
+
+extern "C" int pe_kcore_byte_marks(pe_graph_t* g, int out_edges, uint64_t byte_marks_from, uint32_t* coreness,
+                                   uint64_t* epoch_modified, uint64_t* epoch_next, uint32_t cap,
+                                   pe_kcore_stats_t* stats) {
+  return kcore_run(g, out_edges, byte_marks_from, coreness, epoch_modified, epoch_next, cap, stats);
 }

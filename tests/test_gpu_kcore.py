@@ -171,3 +171,58 @@ def test_values_that_fall_epoch_after_epoch(ctx, length):
     g = Graph.from_edges(ctx, s, d, V, directed=False)
     _check(g, oracle.CSC(V, s, d, symmetrize=True))
     g.close()
+
+
+def _lengths(length):
+    rng = np.random.default_rng(length)
+    rim, hubs = max(4 * length // 3, 200), 8
+    s = np.concatenate([np.full(length, rim + h) for h in range(hubs)] + [rng.integers(0, rim, 6 * rim)])
+    d = np.concatenate([rng.choice(rim, length, replace=False) for _ in range(hubs)] + [rng.integers(0, rim, 6 * rim)])
+    return rim + hubs, s, d
+
+
+def _falling(length):
+    rng = np.random.default_rng(length)
+    rim, hubs = max(2 * length, 300), 6
+    m = 12 * rim
+    s = np.concatenate([np.full(length, rim + h) for h in range(hubs)] + [(rim * rng.random(m) ** 3).astype(np.int64)])
+    d = np.concatenate([rng.choice(rim, length, replace=False) for _ in range(hubs)]
+                       + [(rim * rng.random(m) ** 2).astype(np.int64)])
+    return rim + hubs, s, d
+
+
+def _multi(n):
+    a, b = np.triu_indices(n, 1)
+    m = np.random.default_rng(n).integers(870, 1060, a.size)
+    return n + 1, np.repeat(a, m), np.repeat(b, m)
+
+
+def _giant(rim):
+    rng = np.random.default_rng(8)
+    r = np.arange(1, rim + 1)
+    chords = rng.integers(1, rim + 1, (2, 3 * rim))
+    return rim + 1, np.concatenate([np.zeros(rim, int), r, chords[0]]), np.concatenate([r, r % rim + 1, chords[1]])
+
+
+@pytest.mark.parametrize("make,size", [(_lengths, n) for n in (64, 65, 1025, 4096, 4097, 65536, 65537)]
+                         + [(_falling, n) for n in (60, 1500, 5000, 40000)] + [(_multi, 18), (_multi, 80), (_giant, 70000)])
+def test_byte_marks_with_counts(ctx, make, size):
+    """The form that symmetrized graphs of 2^31 entries and more take (counts, and the active
+    marks as bytes), on graphs of every adjacency class with values that fall over several
+    epochs: coreness and log against the oracle, and the marks in the values beside it."""
+    import ctypes as C
+    from plato_amd import Graph
+    from plato_amd._lib import KcoreStats, check
+    V, s, d = make(size)
+    s, d = s.astype(np.uint32), d.astype(np.uint32)
+    core, mod, nxt = oracle.kcore(oracle.CSC(V, s, d, symmetrize=True))
+    for relabel in (False, True):
+        print(f"case: kcore byte marks {make.__name__} {size} relabel={relabel}", flush=True)
+        g = Graph.from_edges(ctx, s, d, V, directed=False, relabel=relabel)
+        for limit in (0, g.nnz, g.nnz + 1, 1 << 63):  # bytes, bytes, values, values (2^31 at most)
+            got, m, n, st = np.zeros(V, np.uint32), np.zeros(4096, np.uint64), np.zeros(4096, np.uint64), KcoreStats()
+            check(g.lib.pe_kcore_byte_marks(g.h, 0, limit, got.ctypes.data, m.ctypes.data, n.ctypes.data, 4096,
+                                            C.byref(st)), ctx.h)
+            assert np.array_equal(got, core)
+            assert np.array_equal(m[:st.epochs], mod) and np.array_equal(n[:st.epochs], nxt)
+        g.close()
