@@ -383,7 +383,10 @@ typedef struct {
  * set (a BCSR passed as "incomings", as example/kcore_simple.cc does; needs
  * PE_GRAPH_BUILD_CSR).  Writes coreness[V] in input ids (0xFFFFFFFF never remains: vertices
  * without neighbours get 0), and per epoch e < cap the number of modified vertices and
- * the size of the next active set (the reference's modified / need_modified log). */
+ * the size of the next active set (the reference's modified / need_modified log).
+ * Device workspace: at most 20 bytes a vertex (16 without counts, that is on directed
+ * graphs; plus 1 where active marks are bytes), two bits a vertex, and 64 KiB per vertex
+ * of more than 65536 neighbours. */
 int pe_kcore(pe_graph_t* g, int out_edges, uint32_t* coreness, uint64_t* epoch_modified,
              uint64_t* epoch_next, uint32_t cap, pe_kcore_stats_t* stats);
 /* pe_kcore with a lower bound on the adjacency entries from which on a symmetrized graph's

@@ -48,6 +48,10 @@
 namespace pe {
 
 static constexpr uint32_t KC_UNSET = 0xFFFFFFFFu;
+// A count with this bit is none: the vertex falls short, and the other bits are its value of the
+// next epoch (of a vertex of at most KC_GIANT neighbours).  Counts of more than 2^31 neighbours
+// have the bit too, which at most makes such a vertex a candidate that keeps its value.
+static constexpr uint32_t KC_AHEAD = 0x80000000u;
 static constexpr uint32_t KC_SMALL = 64;    // neighbours handled by one lane
 static constexpr uint32_t KC_HIST = 1024;   // histogram bins 0..KC_HIST of the wave-per-vertex pass
 static constexpr uint32_t KC_PER = 17;      // bins per lane in its scan (64 * 17 > KC_HIST)
@@ -80,16 +84,13 @@ struct kc_giant {
 };
 
 __global__ void k_kc_init(const uint64_t* __restrict__ ptr, uint32_t V, uint32_t* __restrict__ core,
-                          uint32_t* __restrict__ est, uint32_t* __restrict__ cnt, uint32_t* __restrict__ ahead) {
+                          uint32_t* __restrict__ est, uint32_t* __restrict__ cnt) {
   for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < V; v += (uint64_t)gridDim.x * blockDim.x) {
     const uint64_t len = ptr[v + 1] - ptr[v];
     const uint32_t c = len ? (uint32_t)std::min<uint64_t>(len, 0xFFFFFFFEull) : KC_UNSET;
     core[v] = c;
     est[v] = c;
-    if (cnt) {
-      cnt[v] = c;
-      ahead[v] = KC_UNSET;
-    }
+    if (cnt) cnt[v] = len ? c : 0u;
   }
 }
 
@@ -238,12 +239,12 @@ __device__ __forceinline__ void kc_wave_fence() {
 
 // The wave pass's vertices first (the longer ones), then one lane per vertex of the small
 // queue.  A wave's LDS share serves both: KC_PER words per lane as one histogram of the
-// wave, or KC_SMALL + 1 bytes per lane.  ahead: the answers that the last spread found already
-// (see there), nullptr without counts.
+// wave, or KC_SMALL + 1 bytes per lane.  cnt_v: the counts, with the answers that the last spread
+// found already (KC_AHEAD), nullptr without counts.
 __global__ __launch_bounds__(KC_THREADS) void k_kc_hindex(
     const uint32_t* __restrict__ qsmall, const uint32_t* __restrict__ qbig, const kc_counters* __restrict__ cnt_in,
     const uint64_t* __restrict__ ptr, const uint32_t* __restrict__ idx, const uint32_t* __restrict__ est,
-    uint32_t* __restrict__ ahead, uint32_t* __restrict__ core) {
+    const uint32_t* __restrict__ cnt_v, uint32_t* __restrict__ core) {
   __shared__ uint32_t hist_all[KC_THREADS / 64][64 * KC_PER];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   uint32_t* hist = hist_all[wave];
@@ -251,12 +252,9 @@ __global__ __launch_bounds__(KC_THREADS) void k_kc_hindex(
   const uint64_t wave_id = grid_wave_id(), nwaves = grid_waves();
   for (uint64_t q = wave_id; q < nbig; q += nwaves) {
     const uint32_t v = qbig[q];
-    const uint32_t known = ahead ? ahead[v] : KC_UNSET;
-    if (known != KC_UNSET) {  // uniform
-      if (lane == 0) {
-        core[v] = known;
-        ahead[v] = KC_UNSET;
-      }
+    const uint32_t known = cnt_v ? cnt_v[v] : 0u;
+    if (known & KC_AHEAD) {  // uniform
+      if (lane == 0) core[v] = known & ~KC_AHEAD;
       continue;
     }
     const uint64_t b = ptr[v], e = ptr[v + 1];
@@ -283,10 +281,9 @@ __global__ __launch_bounds__(KC_THREADS) void k_kc_hindex(
   for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < nsmall;
        i += (uint64_t)gridDim.x * blockDim.x) {
     const uint32_t v = qsmall[i];
-    const uint32_t known = ahead ? ahead[v] : KC_UNSET;
-    if (known != KC_UNSET) {
-      core[v] = known;
-      ahead[v] = KC_UNSET;
+    const uint32_t known = cnt_v ? cnt_v[v] : 0u;
+    if (known & KC_AHEAD) {
+      core[v] = known & ~KC_AHEAD;
       continue;
     }
     const uint64_t b = ptr[v], e = ptr[v + 1];
@@ -365,20 +362,16 @@ __device__ void kc_block_pick(const uint32_t* hist, uint32_t nb, uint32_t base, 
 // One block per queued vertex of up to KC_GIANT neighbours.
 __global__ __launch_bounds__(KC_HTHREADS) void k_kc_huge(
     const uint32_t* __restrict__ qhuge_end, const kc_counters* __restrict__ cnt_in, const uint64_t* __restrict__ ptr,
-    const uint32_t* __restrict__ idx, const uint32_t* __restrict__ est, uint32_t* ahead,
-    uint32_t* __restrict__ core) {
+    const uint32_t* __restrict__ idx, const uint32_t* __restrict__ est,
+    const uint32_t* __restrict__ cnt_v, uint32_t* __restrict__ core) {
   __shared__ uint32_t hist[KC_HTHREADS * KC_HPER];
   const int tid = threadIdx.x;
   const uint64_t nhuge = cnt_in->nhuge;
   for (uint64_t q = blockIdx.x; q < nhuge; q += gridDim.x) {
     const uint32_t v = *(qhuge_end - q);
-    const uint32_t known = ahead ? ahead[v] : KC_UNSET;
-    if (known != KC_UNSET) {  // uniform
-      __syncthreads();  // every thread has read it
-      if (tid == 0) {
-        core[v] = known;
-        ahead[v] = KC_UNSET;
-      }
+    const uint32_t known = cnt_v ? cnt_v[v] : 0u;
+    if (known & KC_AHEAD) {  // uniform
+      if (tid == 0) core[v] = known & ~KC_AHEAD;
       continue;
     }
     const uint64_t b = ptr[v], e = ptr[v + 1];
@@ -608,12 +601,13 @@ struct kc_spread {
 // With counts a spread's walk also takes the histogram of the neighbours' new values, capped at
 // the vertex's own: it holds both its count and, when that falls short, its h-index of the next
 // epoch, whose estimates are these values.  The vertex is then a candidate of the next epoch
-// for sure, and `ahead` carries the answer there instead of a second walk (RMAT scale 22, all
+// for sure, drops there, and counts anew, so its count's place carries the answer there
+// (KC_AHEAD) and saves a second walk (RMAT scale 22, all
 // epochs: h-index passes 7.0 -> 3.0 ms, spreads 10.2 -> 10.5 ms).  A block's vertex with a value above
 // KC_HHIST and a giant have too many values for that and are walked again.
 __global__ __launch_bounds__(KC_THREADS) void k_kc_spread(
     const uint32_t* __restrict__ qsmall, const uint32_t* __restrict__ qbig, const kc_counters* __restrict__ cnt_in,
-    const uint64_t* __restrict__ ptr, kc_spread sp, uint32_t* __restrict__ ahead) {
+    const uint64_t* __restrict__ ptr, kc_spread sp) {
   __shared__ uint32_t hist_all[KC_THREADS / 64][64 * KC_PER];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   uint32_t* hist = hist_all[wave];
@@ -633,10 +627,7 @@ __global__ __launch_bounds__(KC_THREADS) void k_kc_spread(
     kc_wave_fence();
     const uint32_t c = hist[now];
     const uint32_t best = c < now ? kc_wave_pick(hist, now) : 0u;
-    if (lane == 0) {
-      sp.cnt_v[v] = c;
-      if (best) ahead[v] = best;
-    }
+    if (lane == 0) sp.cnt_v[v] = best ? best | KC_AHEAD : c;
     kc_wave_fence();
   }
   uint8_t* h = reinterpret_cast<uint8_t*>(hist) + lane * (KC_SMALL + 1);
@@ -652,18 +643,14 @@ __global__ __launch_bounds__(KC_THREADS) void k_kc_spread(
     for (uint32_t j = 0; j <= now; ++j) h[j] = 0;
     sp.range_lane(ptr[v], ptr[v + 1], old, now, h);
     const uint32_t c = h[now];
-    sp.cnt_v[v] = c;
-    if (c < now) {
-      const uint32_t best = kc_lane_pick(h, now);
-      if (best) ahead[v] = best;
-    }
+    const uint32_t best = c < now ? kc_lane_pick(h, now) : 0u;
+    sp.cnt_v[v] = best ? best | KC_AHEAD : c;
   }
 }
 
 __global__ __launch_bounds__(KC_HTHREADS) void k_kc_spread_huge(const uint32_t* __restrict__ qhuge_end,
                                                                 const kc_counters* __restrict__ cnt_in,
-                                                                const uint64_t* __restrict__ ptr, kc_spread sp,
-                                                                uint32_t* __restrict__ ahead) {
+                                                                const uint64_t* __restrict__ ptr, kc_spread sp) {
   __shared__ uint32_t hist[KC_HTHREADS * KC_HPER];
   __shared__ uint32_t s_c;
   const uint32_t tid = threadIdx.x;
@@ -684,10 +671,7 @@ __global__ __launch_bounds__(KC_HTHREADS) void k_kc_spread_huge(const uint32_t* 
       const uint32_t c = hist[now];
       uint32_t best = 0, over;
       if (c < now) kc_block_pick(hist, now, 0u, 0, 0u, &best, &over);
-      if (tid == 0) {
-        sp.cnt_v[v] = c;
-        if (best) ahead[v] = best;
-      }
+      if (tid == 0) sp.cnt_v[v] = best ? best | KC_AHEAD : c;
     } else {
       if (tid == 0) s_c = 0u;
       __syncthreads();
@@ -750,7 +734,10 @@ __global__ __launch_bounds__(KC_THREADS) void k_kc_commit(
     if (c == old) continue;
     est[v] = c;
     nmod += old != KC_UNSET ? 1u : 0u;
-    if (cnt_v && cnt_v[v] < c) kc_set_bit(cand, v);
+    if (cnt_v) {
+      const uint32_t n = cnt_v[v];
+      if (n < c || (n & KC_AHEAD)) kc_set_bit(cand, v);
+    }
   }
   block_add2(nmod, 0, &cnt->modified, &cnt->modified);
 }
@@ -826,19 +813,19 @@ static int kcore_run(pe_graph_t* g, int out_edges, uint64_t byte_marks_from, uin
     const bool counts = g->csr_is_csc;  // the adjacency is its own reverse
     const uint64_t nwords = ((uint64_t)V >> 6) + 1;
     const uint32_t Vs = std::max<uint32_t>(1, V);
-    dbuf<uint32_t> core(ctx, Vs), est(ctx, Vs), qsmall(ctx, Vs), qbig(ctx, Vs), cnt_v, ahead;
+    dbuf<uint32_t> core(ctx, Vs), est(ctx, Vs), qsmall(ctx, Vs), cnt_v;
+    // the other queues: every vertex in them holds more than KC_SMALL of the entries
+    const uint64_t nlong = std::min<uint64_t>(Vs, g->nnz / (KC_SMALL + 1) + 1);
+    dbuf<uint32_t> qbig(ctx, nlong);
     // active marks in the values' top bits
     const bool marked = counts && g->nnz < std::min(byte_marks_from, KC_MARKED_BELOW);
     dbuf<uint64_t> cand(ctx, nwords), act, nxt;             // nxt: else, one byte per vertex
     if (!marked) nxt.alloc(ctx, nwords * 8);
-    if (counts) {
-      cnt_v.alloc(ctx, Vs);
-      ahead.alloc(ctx, Vs);
-    }
-    uint32_t* qhuge_end = qbig.p + (Vs - 1);
+    if (counts) cnt_v.alloc(ctx, Vs);
+    uint32_t* qhuge_end = qbig.p + (nlong - 1);
     dbuf<kc_counters> cnt(ctx, 2);  // two sets: consecutive epochs alternate
     PE_HIP(hipEventRecord(ctx->t0, s));
-    k_kc_init<<<grid_for(V, 256, 8192), 256, 0, s>>>(ptr, V, core.p, est.p, cnt_v.p, ahead.p);
+    k_kc_init<<<grid_for(V, 256, 8192), 256, 0, s>>>(ptr, V, core.p, est.p, cnt_v.p);
     k_kc_fill<<<grid_for(nwords, 256, 4096), 256, 0, s>>>(cand.p, nwords, V);  // active_current.fill()
     if (!marked) k_kc_zero<<<grid_for(nwords * 8, 256, 4096), 256, 0, s>>>(nxt.p, nwords * 8);
     PE_HIP(hipGetLastError());
@@ -870,8 +857,8 @@ static int kcore_run(pe_graph_t* g, int out_edges, uint64_t byte_marks_from, uin
         const unsigned hgrid = (unsigned)std::min<uint64_t>(huge_max, ncand);
         k_kc_classify<<<grid_for(nwords, 16 * KC_CW_WORDS, (unsigned)std::max(1, ctx->num_cus) * 2), 1024, 0, s>>>(
             cand.p, act.p, nwords, V, ptr, est.p, qsmall.p, qbig.p, qhuge_end, c);
-        k_kc_huge<<<hgrid, KC_HTHREADS, 0, s>>>(qhuge_end, c, ptr, idx, est.p, ahead.p, core.p);
-        k_kc_hindex<<<grid, KC_THREADS, 0, s>>>(qsmall.p, qbig.p, c, ptr, idx, est.p, ahead.p, core.p);
+        k_kc_huge<<<hgrid, KC_HTHREADS, 0, s>>>(qhuge_end, c, ptr, idx, est.p, cnt_v.p, core.p);
+        k_kc_hindex<<<grid, KC_THREADS, 0, s>>>(qsmall.p, qbig.p, c, ptr, idx, est.p, cnt_v.p, core.p);
         if (ngiant) {
           // rounds: 14 bits of the answer each after the first
           int rounds = 1;
@@ -885,8 +872,8 @@ static int kcore_run(pe_graph_t* g, int out_edges, uint64_t byte_marks_from, uin
           }
           k_kc_spread_giant<<<huge_max, KC_HTHREADS, 0, s>>>(ptr, gl, giants.count.p, giants.start.p, act.p, sp);
         }
-        k_kc_spread_huge<<<hgrid, KC_HTHREADS, 0, s>>>(qhuge_end, c, ptr, sp, ahead.p);
-        k_kc_spread<<<grid, KC_THREADS, 0, s>>>(qsmall.p, qbig.p, c, ptr, sp, ahead.p);
+        k_kc_spread_huge<<<hgrid, KC_HTHREADS, 0, s>>>(qhuge_end, c, ptr, sp);
+        k_kc_spread<<<grid, KC_THREADS, 0, s>>>(qsmall.p, qbig.p, c, ptr, sp);
         k_kc_commit<<<grid_for(ncand, KC_THREADS, full_grid), KC_THREADS, 0, s>>>(
             qsmall.p, qbig.p, qhuge_end, gl, giants.count.p, act.p, core.p, marked ? KC_MARK : 0u, est.p, cnt_v.p, cand.p, c);
         const unsigned next_max = (unsigned)std::max(1, ctx->num_cus) * 2;

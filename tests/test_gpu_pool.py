@@ -89,3 +89,33 @@ def test_kept_blocks_of_another_context(how):
         else:
             a.trim()
         assert free0 - b.mem_info()["free"] < 256 << 20
+
+
+def _workspace(run, build):
+    """Bytes of device memory that a call takes beside the graph: what its context keeps after it
+    (every block, none of them used twice), seen from a context without blocks."""
+    from plato_amd import Context
+    with Context(0) as c, Context(0) as meter:
+        g = build(c)
+        c.trim()
+        before = meter.mem_info()["free"]
+        run(g)
+        c.sync()
+        got = before - meter.mem_info()["free"]
+        g.close()
+    return got
+
+
+@pytest.mark.parametrize("ef", [1, 16])
+def test_kcore_workspace(ef):
+    """k-core of a symmetrized graph: 20 bytes a vertex and its bitmaps (beside the transfer's
+    pinned slots, which are host memory)."""
+    from plato_amd import Graph
+    from plato_amd.algo import kcore
+    V = 1 << 24
+    # a first call in another context, so that what the runtime sets up once is not counted
+    _workspace(kcore, lambda c: Graph.rmat(c, 10, 4, directed=False))
+    got = _workspace(kcore, lambda c: Graph.rmat(c, 24, ef, seed=2, directed=False, relabel=True))
+    print(f"case: kcore workspace ef={ef} {got / V:.2f} bytes a vertex", flush=True)
+    assert got > 14 * V  # the measure sees the blocks
+    assert got < 20.5 * V + (24 << 20)  # blocks come in units of 2 MiB; 24 bytes a vertex would not pass
