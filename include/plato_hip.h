@@ -410,7 +410,8 @@ typedef struct {
  * the smallest input id from which each vertex is reachable (on a symmetrized graph,
  * the smallest id of its component), and per epoch e < cap the mode (1 push, 0 pull)
  * and the sum of the slots' returns (the reference's logged actives; they depend on
- * the order in which labels spread, the labels do not). */
+ * the order in which labels spread, the labels do not).
+ * Device workspace: at most 13.25 bytes a vertex. */
 int pe_connected_components(pe_graph_t* g, uint32_t* labels, uint8_t* modes, uint64_t* actives, uint32_t cap,
                             pe_cc_stats_t* stats);
 

@@ -258,7 +258,7 @@ extern "C" int pe_connected_components(pe_graph_t* g, uint32_t* labels, uint8_t*
     const uint32_t V = g->V;
     const uint64_t nwords = ((uint64_t)V >> 6) + 1;
     const uint32_t Vs = std::max<uint32_t>(1, V);
-    dbuf<uint32_t> label(ctx, Vs), queue(ctx, Vs), heavy(ctx, g->nnz / (CC_PULL_CAP + 1) + 1);
+    dbuf<uint32_t> label(ctx, Vs), queue(ctx, Vs), heavy(ctx, std::min<uint64_t>(Vs, g->nnz / (CC_PULL_CAP + 1) + 1));
     dbuf<uint64_t> cur(ctx, nwords), nxt(ctx, nwords), marks(ctx, nwords * 8);
     dbuf<cc_counters> cnt(ctx, 3);  // set 0 holds for the whole call, the others are an epoch's
     cc_counters* c0 = cnt.p;

@@ -119,3 +119,15 @@ def test_kcore_workspace(ef):
     print(f"case: kcore workspace ef={ef} {got / V:.2f} bytes a vertex", flush=True)
     assert got > 14 * V  # the measure sees the blocks
     assert got < 20.5 * V + (24 << 20)  # blocks come in units of 2 MiB; 24 bytes a vertex would not pass
+
+
+def test_components_workspace_of_a_dense_graph():
+    """Components of a graph with many more entries than vertices: at most 13.3 bytes a vertex."""
+    from plato_amd import Graph
+    from plato_amd.algo import connected_components
+    V = 1 << 20
+    _workspace(connected_components, lambda c: Graph.rmat(c, 10, 4))
+    got = _workspace(connected_components, lambda c: Graph.rmat(c, 20, 1024, seed=2))
+    print(f"case: components workspace {got / V:.2f} bytes a vertex", flush=True)
+    assert got > 12 * V
+    assert got < 13.5 * V + (24 << 20)
