@@ -426,7 +426,10 @@ typedef struct {
  * in-edges: anfs[0..cap) gets the neighbourhood-function estimates (the initial one
  * first), *nanfs their number, *avg_distance GetAvgDistance of them (the reference's
  * return value), registers (optional, [V << bits] bytes in input-id order) the final
- * counters, *seconds the device time. */
+ * counters, *seconds the device time.
+ * Device workspace: two sets of counters, at most 5.3 bytes a vertex, and 8 (10 up to 10
+ * bits) bytes a vertex more that make the call faster and are left out when memory is
+ * short. */
 int pe_hyperanf(pe_graph_t* g, const pe_hyperanf_opts_t* opts, double* anfs, uint32_t cap, uint32_t* nanfs,
                 double* avg_distance, uint8_t* registers, double* seconds);
 

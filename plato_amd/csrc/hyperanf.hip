@@ -542,8 +542,9 @@ __device__ __forceinline__ double hanf_alpha(int P) {
 // Estimates of counters of at most 1024 registers, summed per block in a fixed order:
 // m / 16 lanes per counter (16 registers each, one 16-byte load), 1024 / m counters per
 // wave step, so a wave keeps many counters' loads in flight instead of one.  Only changed
-// counters are read; the others' estimates are kept in est.  Without `changed` every counter
-// is a first one: one register set, whose rank the small-range estimate does not use.
+// counters are read; the others' estimates are kept in est (nullptr: every counter is read).
+// Without `changed` every counter is a first one: one register set, whose rank the small-range
+// estimate does not use.
 __global__ __launch_bounds__(256) void k_hanf_estimate_rows(const uint8_t* __restrict__ regs, uint32_t V, int P,
                                                             const uint64_t* __restrict__ changed,
                                                             double* __restrict__ est, double* __restrict__ part) {
@@ -557,7 +558,7 @@ __global__ __launch_bounds__(256) void k_hanf_estimate_rows(const uint8_t* __res
     const uint64_t v = v0 + slot;
     double s = 0.0;
     uint32_t zeros = 0;
-    const bool on = v < V && (!changed || ((changed[v >> 6] >> (v & 63)) & 1ull));
+    const bool on = v < V && (!changed || !est || ((changed[v >> 6] >> (v & 63)) & 1ull));
     if (!changed) {
       s = sub == 0 ? (double)m : 0.0;
       zeros = sub == 0 ? m - 1u : 0u;
@@ -578,9 +579,8 @@ __global__ __launch_bounds__(256) void k_hanf_estimate_rows(const uint8_t* __res
       zeros += (uint32_t)__shfl_xor((int)zeros, (int)off, 64);
     }
     if (v < V && sub == 0) {
-      double x;
-      if (on) est[v] = x = hanf_estimate(alpha, (double)m, s, zeros);
-      else x = est[v];
+      const double x = on ? hanf_estimate(alpha, (double)m, s, zeros) : est[v];
+      if (on && est) est[v] = x;
       total += x;
     }
   }
@@ -603,7 +603,7 @@ __global__ __launch_bounds__(256) void k_hanf_estimate(const uint8_t* __restrict
   const double alpha = hanf_alpha(P);
   double total = 0.0;  // lane 0's running sum over this wave's vertices, in order
   for (uint64_t v = wave_id; v < V; v += nwaves) {
-    if (changed && !((changed[v >> 6] >> (v & 63)) & 1ull)) {  // uniform
+    if (changed && est && !((changed[v >> 6] >> (v & 63)) & 1ull)) {  // uniform
       total += est[v];
       continue;
     }
@@ -619,7 +619,7 @@ __global__ __launch_bounds__(256) void k_hanf_estimate(const uint8_t* __restrict
       zeros += __shfl_xor(zeros, off, 64);
     }
     const double x = hanf_estimate(alpha, (double)m, s, zeros);
-    if (lane == 0) est[v] = x;
+    if (lane == 0 && est) est[v] = x;
     total += x;
   }
   if (lane == 0) s_w[wave] = total;
@@ -672,6 +672,17 @@ __global__ void k_hanf_rows_external(const uint8_t* __restrict__ in, const uint3
 
 using namespace pe;
 
+// An array that makes a call faster but that it can do without: empty when memory is short.
+template <typename T>
+static void hanf_alloc_optional(dbuf<T>& b, pe_ctx_s* ctx, size_t n) {
+  try {
+    b.alloc(ctx, n);
+  } catch (const error& e) {
+    if (e.code != PE_ERR_OOM) throw;
+    b = dbuf<T>();
+  }
+}
+
 // The pull over one adjacency (ptr, idx): its passes' vertex lists and the changed rows.
 struct hanf_pull {
   pe_ctx_s* ctx;
@@ -687,15 +698,21 @@ struct hanf_pull {
   dbuf<uint64_t> marks;           // HANF_CHANGED and HANF_DONE bytes
   dbuf<uint32_t> top;             // the bound row, a word per register
   dbuf<uint8_t> bound;            // the bound row
-  dbuf<uint16_t> code;            // first counters, P <= HANF_CODE_P
+  dbuf<uint16_t> code;            // first counters, P <= HANF_CODE_P (empty when memory is short)
   bool first = true;              // no pull yet
   unsigned grid;
+
+  // vertices of the wave pass at most: below 10 bits each has HANF_LOW_DEG of the entries
+  static uint64_t max_mid(uint32_t V, uint64_t nnz, int bits) {
+    const uint64_t Vs = std::max<uint32_t>(1, V);
+    return bits < 10 ? std::min(Vs, nnz / HANF_LOW_DEG + 1) : Vs;
+  }
 
   // od (out-degrees over this adjacency's entries) or, without it, src_ptr tells which vertices
   // some other vertex pulls from: those with od > 0, or with entries in src_ptr
   hanf_pull(pe_ctx_s* c, const uint64_t* p, const uint32_t* i, uint32_t v, uint64_t nnz, int bits, const uint32_t* perm,
             const uint32_t* od, const uint64_t* src_ptr)
-      : ctx(c), ptr(p), idx(i), V(v), P(bits), nwords(((uint64_t)v >> 6) + 1), mid(c, std::max<uint32_t>(1, v)),
+      : ctx(c), ptr(p), idx(i), V(v), P(bits), nwords(((uint64_t)v >> 6) + 1), mid(c, max_mid(v, nnz, bits)),
         nmid(c, 2), changed(c, nwords), marks(c, nwords * 8), top(c, 1ull << bits), bound(c, 1ull << bits) {
     hipStream_t s = ctx->stream;
     k_hanf_zero<<<64, 256, 0, s>>>(top.p, 1ull << P);
@@ -709,7 +726,9 @@ struct hanf_pull {
     k_hanf_fill_bits<<<grid_for(nwords, 256, 4096), 256, 0, s>>>(changed.p, nwords, V);
     k_hanf_zero<<<grid_for(nwords * 16, 256, 8192), 256, 0, s>>>(reinterpret_cast<uint32_t*>(marks.p), nwords * 16);
     if (P <= HANF_CODE_P) {
-      code.alloc(ctx, std::max<uint32_t>(1, V));
+      hanf_alloc_optional(code, ctx, std::max<uint32_t>(1, V));
+    }
+    if (code.p) {
       k_hanf_codes<<<grid_for(V, 256, 8192), 256, 0, s>>>(code.p, V, P, perm);
     }
     PE_HIP(hipGetLastError());
@@ -779,9 +798,10 @@ extern "C" int pe_hyperanf(pe_graph_t* g, const pe_hyperanf_opts_t* opts, double
     dbuf<double> part(ctx, est_grid);
     std::vector<double> hpart(est_grid);
     const uint32_t* perm = g->relabeled ? g->perm.p : nullptr;
-    dbuf<double> est(ctx, std::max<uint32_t>(1, V));
     PE_HIP(hipEventRecord(ctx->t0, s));
     hanf_pull pulls(ctx, g->col_ptr.p, g->row_idx.p, V, g->nnz, P, perm, g->od.p, nullptr);
+    dbuf<double> est;
+    hanf_alloc_optional(est, ctx, std::max<uint32_t>(1, V));
     auto anf_of = [&](const uint8_t* regs) {
       const uint64_t* changed = pulls.first ? nullptr : pulls.changed.p;
       if (P <= 10)

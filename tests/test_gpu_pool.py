@@ -131,3 +131,30 @@ def test_components_workspace_of_a_dense_graph():
     print(f"case: components workspace {got / V:.2f} bytes a vertex", flush=True)
     assert got > 12 * V
     assert got < 13.5 * V + (24 << 20)
+
+
+def test_hyperanf_when_memory_is_short():
+    """HyperANF with the device filled up but for its counters and 0.2 GiB: the kept estimates
+    (0.5 GiB) and the codes of the first counters are left out, the results are the same."""
+    from plato_amd import Context, DenseState, Graph
+    from plato_amd._lib import PlatoHipError
+    from plato_amd.algo import hyperanf, hyperanf_opts_t
+    MB = 1 << 20
+    with Context(0) as a, Context(0) as b:
+        g = Graph.rmat(a, 26, 1, seed=4)
+        opts = hyperanf_opts_t(3, 6)
+        want = hyperanf(g, opts)
+        a.trim()
+        held = [DenseState(b, (b.mem_info()["free"] - (12 << 30)) // 4, np.float32)]
+        for size, most in ((64 * MB, 400), (16 * MB, 8)):
+            with pytest.raises(PlatoHipError, match="out of memory"):
+                for _ in range(most):
+                    held.append(DenseState(b, size // 4, np.float32))
+        for v in held[1:1 + (2 * 64 * (1 << 26) // MB + 192) // 64]:  # 8 GiB of counters, and 192 MiB
+            v.close()
+        print("case: hyperanf in 8.2 GiB", flush=True)
+        got = hyperanf(g, opts)
+        assert np.array_equal(got.anfs, want.anfs) and got.avg_distance == want.avg_distance
+        for v in held:
+            v.close()
+        g.close()
