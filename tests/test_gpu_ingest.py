@@ -155,3 +155,15 @@ def test_line_lengths_around_words_stages_and_segments(ctx, pad):
         g.close()
         with pytest.raises(PlatoHipError, match=f"line {len(lines) + 2}:"):
             Graph.from_csv_bytes(ctx, b"\n".join(lines) + b"\n1,2\n4294967296,1\n4294967297,1\n")
+
+
+@pytest.mark.parametrize("first", [0, 1000, 65535, 65536, 65537, 199999])
+def test_first_of_many_errors(ctx, first):
+    """200 000 lines that are all wrong from one on, around the ends of a counting segment of
+    65536 lines: the first of them is named."""
+    from plato_amd import Graph
+    from plato_amd._lib import PlatoHipError
+    text = b"1,2\n" * first + b"4294967296,1\n1,4294967297\n" * ((200000 - first + 1) // 2)
+    print(f"case: csv first error {first}", flush=True)
+    with pytest.raises(PlatoHipError, match=f"line {first + 1}:"):
+        Graph.from_csv_bytes(ctx, text)
