@@ -637,6 +637,8 @@ int pe_graph_create_csv(pe_ctx_t* ctx, const char* text, uint64_t nbytes, uint32
       k_csv_compact<<<(unsigned)hseg, 1024, 0, s>>>(head.p, 2 * E, dhoff.p, all.p, nullptr, nullptr, g->vid_decode.p,
                                                     nullptr, nullptr);
       PE_HIP(hipGetLastError());
+      all.release();  // 18 bytes an edge, before the buckets take up to 16
+      head.release();
       // about one bucket per distinct id
       int shift = std::min(bits, 63);
       while (shift > 0 && (max_id >> (shift - 1)) < nu) --shift;
