@@ -71,3 +71,33 @@ def test_two_contexts_in_two_threads(ctx):
     for t in threads:
         t.join()
     assert not errors, errors
+
+
+@pytest.mark.parametrize("direction", ["download", "upload"])
+def test_waiting_for_queued_work_costs_one_core(ctx, direction):
+    """A transfer behind device work that is still running: only the calling thread (and the
+    runtime's own) may be busy until the work is done."""
+    import time
+    from plato_amd import DenseState
+    a, b, v = (DenseState(ctx, n, np.float32) for n in (1 << 29, 1 << 29, 1 << 23))
+    host = np.arange(v.n, dtype=np.float32)
+    v.upload(host)
+
+    def timed(copies):
+        for _ in range(copies):
+            a.copy_from(b)  # 2 GiB, left running
+        t, c = time.perf_counter(), time.process_time()
+        if direction == "download":
+            assert np.array_equal(v.numpy(), host)
+        else:
+            v.upload(host)
+        return time.perf_counter() - t, time.process_time() - c
+
+    alone, _ = timed(0)
+    wall, cpu = timed(300)
+    print(f"case: transfer behind work {direction}: {wall * 1e3:.0f} ms ({alone * 1e3:.1f} alone), {cpu * 1e3:.0f} ms of CPU", flush=True)
+    assert wall > 0.1 and wall > 5 * alone  # it did wait
+    assert cpu < 2.5 * wall
+    assert np.array_equal(v.numpy(), host)
+    for x in (a, b, v):
+        x.close()
