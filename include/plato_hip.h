@@ -9,9 +9,15 @@
  *  - Host pointers are borrowed for the duration of the call only.  Device
  *    objects (graphs, vectors, bitmaps, batches, servers) are owned by their
  *    handle and freed by the matching *_destroy.
- *  - Work is issued on the context's stream; functions that return results to
- *    host memory synchronize that stream before returning.
- *  - A context is driven by one host thread at a time.
+ *  - Work is issued on the context's stream.  Functions that return results to
+ *    host memory wait for them, and for every write of the work that made them
+ *    (not always for the whole stream: the kernel that delivered them may still be
+ *    on its way out).  Functions without results may return before their work has
+ *    run; a device error in it is reported by a later call on the context.
+ *    pe_ctx_sync waits for everything.
+ *  - A context is driven by one host thread at a time.  Its objects may be
+ *    destroyed on another thread meanwhile (a garbage collector's), except during
+ *    pe_ppr_batch_step, which may be recording the stream.
  *
  * Each declaration names the reference interface it replaces (paths relative
  * to the reference repository root).  The reference is a header-only C++
@@ -506,7 +512,8 @@ int pe_ppr_batch_create(pe_graph_t* g, const pe_ppr_batch_opts_t* opts, pe_ppr_b
 int pe_ppr_batch_destroy(pe_ppr_batch_t* b);
 /* device bytes held by the batch (rank blocks, seed masks, task lists) */
 int pe_ppr_batch_bytes(const pe_ppr_batch_t* b, uint64_t* bytes);
-/* put a query (seed set, input ids) into an EMPTY slot; it starts LOADING */
+/* put a query (seed set, input ids) into an EMPTY slot; it starts LOADING (at most 64
+ * distinct seeds: enqueued, without waiting; so is the release of such a slot) */
 int pe_ppr_batch_admit(pe_ppr_batch_t* b, uint32_t slot, const uint32_t* seeds, uint32_t nseeds);
 /* free a slot (any state) */
 int pe_ppr_batch_release(pe_ppr_batch_t* b, uint32_t slot);
