@@ -258,3 +258,21 @@ def test_autotune_choices_are_valid_and_keep_results(ctx, tmp_path):
     out, found = L.TuneResult(), C.c_int()
     assert g.lib.pe_autotune_load(g.h, path, C.byref(out), C.byref(found)) == 0
     assert found.value == 1 and out.tile_items == r["tile_items"]
+
+
+@pytest.mark.parametrize("V", [1, 2, 63, 64, 65, 130, 4099, 300001])
+@pytest.mark.parametrize("relabel", [False, True])
+def test_vertex_statistics_of_sparse_graphs(ctx, V, relabel):
+    """Vertices with an edge, the largest of them and the largest in-degree, where most vertices
+    of a wave have none and the last vertex with an edge sits anywhere in it."""
+    from plato_amd import Graph
+    rng = np.random.default_rng(V)
+    for E in sorted({1, 3, max(1, V // 40), max(1, V // 3)}):
+        for top in {V, max(1, V // 2)}:
+            s, d = rng.integers(0, top, (2, E)).astype(np.uint32)
+            print(f"case: vertex statistics V={V} E={E} ids below {top} relabel={relabel}", flush=True)
+            g = Graph.from_edges(ctx, s, d, V, relabel=relabel)
+            assert g.info.vertices == np.unique(np.concatenate([s, d])).size
+            assert g.info.max_v_i == max(s.max(), d.max())
+            assert g.info.max_in_degree == np.bincount(d).max()
+            g.close()

@@ -101,3 +101,19 @@ def test_waiting_for_queued_work_costs_one_core(ctx, direction):
     assert np.array_equal(v.numpy(), host)
     for x in (a, b, v):
         x.close()
+
+
+# results of up to 16384 words come by mail: its ends in 4- and 8-byte elements, and a count that
+# gives each of the kernel's 1024 threads more than one
+MAIL_SIZES = [2, 1023, 1024, 1025, 8191, 8192, 8193, 16383, 16384, 16385, 32768, 32769]
+
+
+@pytest.mark.parametrize("n", MAIL_SIZES)
+def test_small_results(ctx, n):
+    print(f"case: small transfer n={n}", flush=True)
+    _round_trip(ctx, n, n)
+
+
+@pytest.mark.parametrize("V", MAIL_SIZES)
+def test_small_reordered(ctx, V):
+    test_reordered_and_widened(ctx, V)
