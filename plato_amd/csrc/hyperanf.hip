@@ -22,9 +22,9 @@
 // pulls from can pass the register-wise max over the first counters of all such vertices (the
 // bound row): a pull stops at the first row that reaches it, and a vertex that has reached it
 // is done.  The pull's bound is the random 2^P-byte rows of the second and third iteration,
-// then the in-edge lists.  RMAT scale 23 symmetrized, P = 6, 8 pulls: 5.2 ms each with one 4-byte word per lane and every row read;
-// here 1.8, 3.4 and 2.5 ms, then 0.8 falling to 0.15 ms (without the bound row 3.4 until the
-// fourth, then 0.8); the whole call 44.7 -> 13.4 ms.
+// then the in-edge lists.  RMAT scale 23 symmetrized, P = 6, 8 pulls: 5.2 ms each with one
+// 4-byte word per lane and every row read; here 1.8, 3.4 and 2.5 ms, then 0.8 falling to 0.15 ms
+// (without the bound row 3.4 until the fourth, then 0.8); the whole call 44.7 -> 13.4 ms.
 // Three passes by in-degree: fewer than HANF_LOW_DEG, a group of LPR lanes per vertex; up to
 // HANF_HUB_DEG, a wave per vertex; the hubs' in-edges in chunks over all waves, each merging
 // its chunk's maximum into the hub's row, so no wave walks a hub alone.

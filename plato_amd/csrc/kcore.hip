@@ -25,7 +25,7 @@
 // active vertex, 20 ms with the counts, 16.1 ms with the drops found in the spread before,
 // 15.6 ms with the marks in the values.  Bound by the rate of the random 4-byte reads of the
 // values in the first ten epochs, when most vertices are modified (1.2 ms per walk of the 2^27
-// entries, 120 G/s; twice as many in flight per lane: 16.3 ms).
+// entries, 112 G/s; twice as many in flight per lane: 16.3 ms).
 // Other adjacencies (in-edges or out-edges of a directed graph) have no counts: every
 // active vertex is re-counted.
 //
